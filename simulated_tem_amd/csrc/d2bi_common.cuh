@@ -219,6 +219,21 @@ static void fill_i32(int* p, int64_t n, int v, hipStream_t s)
 
 // ------------------------------------------------------------------ generic scan
 
+// Inclusive prefix sum over the 64 lanes of a wave in six DPP steps: within
+// each row of 16 lanes (row_shr 1, 2, 4, 8 with zero fill), then row 0's
+// total into row 1 and row 2's into row 3 (row_bcast:15), then rows 0-1's
+// into rows 2-3 (row_bcast:31).  All lanes must be active.
+__device__ __forceinline__ int wave_incl_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
 static constexpr int SCAN_BLOCK = 256;
 static constexpr int SCAN_ITEMS = 4;
 static constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;

@@ -84,6 +84,246 @@ __global__ __launch_bounds__(256) void k_voxel_fp64(VoxParams P, const int* __re
     if (out_r2m) out_r2m[o] = r2min;
 }
 
+// Region form (default).  A workgroup of four waves per 8 x 8 x 8 region, a
+// wave per column of two 4 x 4 x 4 subtiles (staging: d2bi_region.cuh).  Per axis, the
+// squared offset of a candidate from a voxel depends on the voxel's index
+// along that axis only, so neighbourList1b's range
+//     dd = (d1^2 + d2^2) + d3^2,   d = a (frac + (k - zi))
+// (Lib_LinkCell3D.f90:1565-1596) is an add of squares that are evaluated once
+// per candidate and axis position, with the reference's expression: every
+// range is the reference's to the bit, and so are the members and the nearest
+// range.  A voxel whose cell is not next to the candidate's along an axis
+// gets an infinite square there (the 27-cell rule).  The weight factorises the
+// same way,
+//     exp(-(d0 - i h)^2 / 2s^2) = exp(-d0^2 / 2s^2) exp(d0 h / s^2)^i b_i,
+// two exponentials per candidate and axis; b_i = exp(-(i h)^2 / 2s^2) depends
+// on the voxel alone and multiplies its sums at the end.  Lane (xy, part) walks every fourth candidate of the subtile's list
+// for the four voxels along z at its x and y: an add, a compare, a select, a
+// multiply and two FMAs per pair, in FP64.
+//
+// Bound: FP64 VALU issue (an add, multiply or compare ~4.7 cycles per wave,
+// measured) in the pair loop; the per-voxel 27-cell walk above evaluates 180
+// pairs per voxel with an exponential per member and gathers every point from
+// memory.  MFMA does not help: v_mfma_f64_4x4x4 takes 16 cycles for the two
+// FMAs' 10 and does not overlap the vector pipe.
+
+static constexpr int F64R_NW = 4;                    // waves per workgroup
+// Candidates whose records are held at once.  A workgroup's phases (cells,
+// points, records, pairs) are parted by barriers and start with loads, so it
+// is the number of workgroups per CU that hides their latencies: 64 records
+// (30 KB of LDS) ran 1.58 ms on a 400 x 360 x 200 field, 88 1.75, 128 (three
+// workgroups instead of four) 2.31, regions of 8 x 8 x 16 with eight waves
+// 2.18, of 8 x 8 x 4 1.89, and the per-voxel walk 10.4 ms.
+static constexpr int F64R_REC = 64;
+
+template <int NA>
+struct F64Record {
+    double2 x[REG], y[REG];                          // (square, weight) per voxel position
+    double z[REG];                                   // squares
+    double wz[REG / TILE];                           // weight of each subtile's first voxel
+    double ratio;                                    // weight ratio along z
+    double2 cs[NA];                                  // cos and sin of g.r
+};
+
+template <int NA, bool MIN, bool DIAG>
+__global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_region(
+    RegionParams R, const int* __restrict__ cell_start, const double4* __restrict__ frac,
+    const float4* __restrict__ p32, const double2* __restrict__ cs64, int64_t cs_stride, double* __restrict__ out_re,
+    double* __restrict__ out_im, int64_t out_stride, double* __restrict__ out_rho, int* __restrict__ out_cnt,
+    double* __restrict__ out_r2m)
+{
+    constexpr int NW = F64R_NW, NT = 64 * NW, NS = REG / TILE;
+    typedef F64Record<NA> Rec;
+    __shared__ RegionStage<NW> S;
+    // the link cells are done with once a pass is staged, the records after it
+    __shared__ union {
+        RegionCells<NW> cells;
+        Rec rec[F64R_REC + 1];                       // the last one pads lists
+    } U;
+    __shared__ unsigned short lists[NW][F64R_REC + 4];           // byte offsets of records
+    static_assert(sizeof U.rec < 65536, "16-bit record offsets");
+    const int region = region_of(R, blockIdx.x);
+    if (region >= R.nreg) return;
+    const VoxParams& P = R.v;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    RegionBox B;
+    region_box(R, region, S, B);
+
+    // the wave's subtiles (two along z) and the lane's voxels: x, y, and four
+    // along z in each
+    const int s0 = (wave & 1) * TILE, s1 = (wave >> 1) * TILE;
+    const int part = lane >> 4, lx = s0 + (lane & 3), ly = s1 + ((lane >> 2) & 3);
+    const bool active = B.o[0] + s0 <= B.l[0] && B.o[1] + s1 <= B.l[1];
+    double sre[NS][NA][TILE], sim[NS][NA][TILE], dmin[NS][TILE];
+    int cnt[NS][TILE];
+#pragma unroll
+    for (int z = 0; z < NS; z++)
+#pragma unroll
+        for (int i = 0; i < TILE; i++) {
+#pragma unroll
+            for (int a = 0; a < NA; a++) { sre[z][a][i] = 0.0; sim[z][a][i] = 0.0; }
+            dmin[z][i] = 3.4028234663852886e38;
+            cnt[z][i] = 0;
+        }
+
+    // records of a chunk: four threads per candidate, three for the axes, each
+    // also with a share of the phases.  A thread's inputs are loaded before
+    // the previous chunk's pairs.
+    constexpr int NI = (4 * F64R_REC + NT - 1) / NT, NC = NA > 2 ? NA / 2 : 1;
+    double in_f[NI], in_c[NI][NC];
+    auto load = [&](int c0, int nc) {
+#pragma unroll
+        for (int j = 0; j < NI; j++) {
+            const int t = threadIdx.x + j * NT, role = t & 3;
+            if (t >= 4 * nc) continue;
+            const int slot = __float_as_int(S.pos[c0 + (t >> 2)].w);
+            in_f[j] = reinterpret_cast<const double*>(frac + slot)[min(role, 2)];
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+                const int e = (role * NC + q) & (2 * NA - 1);
+                in_c[j][q] = reinterpret_cast<const double*>(cs64 + (e >> 1) * cs_stride + slot)[e & 1];
+            }
+        }
+    };
+    auto record = [&](int c0, int nc) {
+#pragma unroll
+        for (int j = 0; j < NI; j++) {
+            const int t = threadIdx.x + j * NT, i = t >> 2, role = t & 3;
+            if (t >= 4 * nc) continue;
+            const int ax = role;
+            if (ax == 3) continue;
+            Rec& q = U.rec[i];
+            const int u = ((S.upk[c0 + i] >> (8 * ax)) & 255) - 1;
+            const double side = ax == 0 ? P.a[0] : ax == 1 ? P.a[1] : P.a[2];
+            const double h = ax == 0 ? R.h[0] : ax == 1 ? R.h[1] : R.h[2];
+            const double d0 = side * (in_f[j] + (u - S.zi[ax][0]));
+            const double ratio = exp((2.0 * d0) * (h * P.i2s2));
+            double w = exp(-(d0 * d0) * P.i2s2);
+            if (ax == 2) q.ratio = ratio;
+#pragma unroll
+            for (int v = 0; v < REG; v++) {
+                const int k = u - S.lc[ax][v];
+                const double d = side * (in_f[j] + (k - S.zi[ax][v]));
+                const double d2 = (unsigned)(k + 1) <= 2u ? d * d : HUGE_VAL;
+                if (ax == 2) {
+                    q.z[v] = d2;
+                    if (v % TILE == 0) q.wz[v / TILE] = w;
+                } else {
+                    (ax == 0 ? q.x : q.y)[v] = make_double2(d2, w);
+                }
+                w = w * ratio;
+            }
+        }
+        // phases
+#pragma unroll
+        for (int j = 0; j < NI; j++) {
+            const int t = threadIdx.x + j * NT;
+            if (t >= 4 * nc) continue;
+#pragma unroll
+            for (int q = 0; q < NC; q++) {
+                const int e = ((t & 3) * NC + q) & (2 * NA - 1);
+                reinterpret_cast<double*>(U.rec[t >> 2].cs)[e] = in_c[j][q];
+            }
+        }
+        // the padding record: no voxel is in range of it
+        Rec& q = U.rec[F64R_REC];
+        if (threadIdx.x < REG) {
+            q.x[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
+            q.y[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
+        } else if (threadIdx.x < sizeof(Rec) / 8 - 3 * REG) {
+            reinterpret_cast<double*>(&q)[threadIdx.x + 3 * REG] = 0.0;      // past x and y
+        }
+    };
+
+    for (int t_next = 0, T = 1; t_next < T;) {
+        int K;
+        region_cells(R, B, S, U.cells, cell_start, K, T);
+        const int n = region_stage(R, B, S, U.cells, p32, K, T, t_next);
+        // equal chunks of at most F64R_REC candidates
+        const int nch = (n + F64R_REC - 1) / F64R_REC, per = nch > 0 ? (n + nch - 1) / nch : 0;
+        __syncthreads();                             // staged points written, cells read
+        load(0, min(per, n));
+        for (int c0 = 0; c0 < n; c0 += per) {
+            const int nc = min(per, n - c0);
+            if (c0 > 0) __syncthreads();             // earlier records read
+            record(c0, nc);
+            __syncthreads();
+            if (c0 + per < n) load(c0 + per, min(per, n - c0 - per));
+            if (!active) continue;
+#pragma unroll
+            for (int z = 0; z < NS; z++) {
+                const int s[3] = {s0, s1, z * TILE};
+                if (B.o[2] + s[2] > B.l[2]) continue;
+                float tc[3], th[3];
+                subtile_box(S, s, tc, th);
+                const int nl = subtile_list(S, R.rc_cull2, c0, nc, tc, th, (int)sizeof(Rec), F64R_REC, lists[wave]);
+                const char* rec = reinterpret_cast<const char*>(U.rec);
+#pragma unroll 1
+                for (int k = 0; k < nl; k += 4) {
+                    const Rec& q = *reinterpret_cast<const Rec*>(rec + lists[wave][k + part]);
+                    const double2 qx = q.x[lx], qy = q.y[ly];
+                    const double s12 = qx.x + qy.x, ratio = q.ratio;
+                    double p = (qx.y * qy.y) * q.wz[z];
+                    double2 cs[NA];
+#pragma unroll
+                    for (int a = 0; a < NA; a++) cs[a] = q.cs[a];
+#pragma unroll
+                    for (int v = 0; v < TILE; v++) {
+                        const double dd = s12 + q.z[z * TILE + v];
+                        const bool in = dd <= P.rc2;
+                        // a pair out of range keeps the low word of its
+                        // weight: < 1e-313, dropped from the sums at the end
+                        const double w = __hiloint2double(in ? __double2hiint(p) : 0, __double2loint(p));
+#pragma unroll
+                        for (int a = 0; a < NA; a++) {
+                            sre[z][a][v] = fma(w, cs[a].x, sre[z][a][v]);
+                            sim[z][a][v] = fma(w, cs[a].y, sim[z][a][v]);
+                        }
+                        if (MIN) dmin[z][v] = fmin(dmin[z][v], dd);
+                        if (DIAG) cnt[z][v] += in ? 1 : 0;
+                        p = p * ratio;
+                    }
+                }
+            }
+        }
+        __syncthreads();                             // staged points and records read
+    }
+    if (!active) return;
+
+    // lane (xy, part) finishes the voxel `part` along z of each subtile
+    auto drop = [](double v) { return fabs(v) < 1.0e-280 ? 0.0 : v; };
+#pragma unroll
+    for (int z = 0; z < NS; z++) {
+        const int vx = B.o[0] + lx, vy = B.o[1] + ly, vz = B.o[2] + z * TILE + part;
+        const double scale = (R.b[0][lx] * R.b[1][ly]) * R.b[2][z * TILE + part];
+        const bool out = vx < P.Mx && vy < P.My && vz < P.Mz;
+        const int64_t o = (int64_t)vx + (int64_t)P.Mx * (vy + (int64_t)P.My * vz);
+#pragma unroll
+        for (int a = 0; a < NA; a++) {
+            const double re = drop(part_sum(sre[z][a][0], sre[z][a][1], sre[z][a][2], sre[z][a][3])) * scale;
+            const double im = drop(part_sum(sim[z][a][0], sim[z][a][1], sim[z][a][2], sim[z][a][3])) * scale;
+            double ww = hypot(re, im);
+            ww = 1 / (1.0e-16 > ww ? 1.0e-16 : ww);
+            if (out) {
+                out_re[a * out_stride + o] = re * ww;
+                out_im[a * out_stride + o] = im * ww;
+            }
+        }
+        double r2 = 3.4028234663852886e38;
+        if (MIN) {
+            // over every candidate: the nearest is a member if there is one
+            const double v = part_min(dmin[z][0], dmin[z][1], dmin[z][2], dmin[z][3]);
+            if (v <= P.rc2) r2 = v;
+        }
+        if (out) out_rho[o] = P.use_density ? rho_of(r2, P.sigma) : 1.0;
+        if (DIAG) {
+            const float c = part_sum((float)cnt[z][0], (float)cnt[z][1], (float)cnt[z][2], (float)cnt[z][3]);
+            if (out && out_cnt) out_cnt[o] = (int)c;
+            if (out && out_r2m) out_r2m[o] = r2;
+        }
+    }
+}
+
 // ------------------------------------------------------------------ (c) integrate, FP64
 
 struct IntParams {

@@ -36,6 +36,7 @@
 #include "d2bi_common.cuh"
 #include "d2bi_bin.cuh"
 #include "d2bi_axis.cuh"
+#include "d2bi_region.cuh"
 #include "d2bi_fp64.cuh"
 #include "d2bi_voxel_tile.cuh"
 #include "d2bi_integrate_fast.cuh"

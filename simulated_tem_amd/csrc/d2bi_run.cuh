@@ -111,6 +111,75 @@ static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParam
     return D2BI_OK;
 }
 
+// Launch parameters of the region kernels for a plan; false where they do not
+// apply: a region spanning more link cells than its table holds (voxels
+// coarser than about a third of the lattice parameter).
+static bool region_params(const d2bi_plan* p, const AxisTables& tab, const VoxParams& V, RegionParams* R)
+{
+    R->v = V;
+    const int M[3] = {p->Mx, p->My, p->Mz}, E[3] = {p->Ex, p->Ey, p->Ez};
+    int n[3];
+    int64_t worst = 1;
+    for (int a = 0; a < 3; a++) {
+        int mx = 0;
+        for (int t0 = 0; t0 < M[a]; t0 += REG)
+            mx = std::max(mx, tab.cell[a][std::min(M[a], t0 + REG) - 1] - tab.cell[a][t0] + 3);
+        worst *= mx;
+        n[a] = (M[a] + REG - 1) / REG;
+        R->cellf[a] = (float)p->a_col[4 * a];
+        // voxel sides: the link cells divide the voxel box, in x and y with a
+        // margin of deltaM voxels on both sides (plan_image)
+        R->h[a] = p->a_col[4 * a] * E[a] / (M[a] + (a < 2 ? 2 * p->deltaM : 0));
+        for (int i = 0; i < REG; i++) R->b[a][i] = std::exp(-((i * R->h[a]) * (i * R->h[a])) * p->i2s2);
+    }
+    if (worst > REG_MAXC) return false;
+    R->nrx = n[0];
+    R->nry = n[1];
+    R->nrz = n[2];
+    R->nreg = n[0] * n[1] * n[2];
+    R->per_xcd = ((n[1] * n[2] + 7) / 8) * n[0];
+    R->rc_cull2 = (float)(p->rc2 * (1.0 + 1.0e-4));
+    return true;
+}
+
+// FP64 voxelisation of na aperture points (1, 2 or 4; phases cs at a stride
+// of cs_stride slots, fields at a stride of out_stride voxels) from workspace
+// w's binned points; cnt and r2m: optional diagnostics.  The per-voxel walk
+// takes over where a region spans too many link cells.
+static int launch_voxel_fp64(const d2bi_plan* p, const AxisTables& tab, const VoxParams& V, int na, Workspace& w,
+                             const double2* cs, int64_t cs_stride, int64_t out_stride, int* cnt, double* r2m,
+                             hipStream_t s)
+{
+    RegionParams R;
+    if (region_params(p, tab, V, &R)) {
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(8 * R.per_xcd), dim3(64 * F64R_NW), 0, s, R, w.cell_start.as<int>(),
+                               w.slot_frac.as<double4>(), w.slot_p32.as<float4>(), cs, cs_stride, w.f64_re.as<double>(),
+                               w.f64_im.as<double>(), out_stride, w.f64_rho.as<double>(), cnt, r2m);
+        };
+        const bool dens = V.use_density != 0;
+        if (cnt || r2m) go(k_voxel_fp64_region<1, true, true>);
+        else if (dens && na == 4) go(k_voxel_fp64_region<4, true, false>);
+        else if (dens && na == 2) go(k_voxel_fp64_region<2, true, false>);
+        else if (dens) go(k_voxel_fp64_region<1, true, false>);
+        else if (na == 4) go(k_voxel_fp64_region<4, false, false>);
+        else if (na == 2) go(k_voxel_fp64_region<2, false, false>);
+        else go(k_voxel_fp64_region<1, false, false>);
+    } else {
+        const dim3 grid((p->Mx + 7) / 8, (p->My + 7) / 8, (p->Mz + 3) / 4);
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, V, w.cell_start.as<int>(), w.slot_frac.as<double4>(), cs,
+                               cs_stride, w.f64_re.as<double>(), w.f64_im.as<double>(), out_stride,
+                               w.f64_rho.as<double>(), cnt, r2m);
+        };
+        if (na == 4) go(k_voxel_fp64<4>);
+        else if (na == 2) go(k_voxel_fp64<2>);
+        else go(k_voxel_fp64<1>);
+    }
+    HIPCHK(hipGetLastError());
+    return D2BI_OK;
+}
+
 // Launch parameters of a variant.  A 4 x 4 x 8 tile that spans more link
 // cells than the per-tile table holds falls back to the 4 x 4 x 4 row kernel
 // (*variant becomes 1), and so does an 8 x 4 x 4 tile (variant 3) that
@@ -265,12 +334,8 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
         CHK(w.f64_re.ensure(sizeof(double) * nvox));
         CHK(w.f64_im.ensure(sizeof(double) * nvox));
         CHK(w.f64_rho.ensure(sizeof(double) * nvox));
-        dim3 grid((p->Mx + 7) / 8, (p->My + 7) / 8, (p->Mz + 3) / 4);
         if (T) CHK(T->record(2));
-        hipLaunchKernelGGL(k_voxel_fp64<1>, grid, dim3(256), 0, s, V, w.cell_start.as<int>(),
-                           w.slot_frac.as<double4>(), w.slot_cs64.as<double2>(), (int64_t)0, w.f64_re.as<double>(),
-                           w.f64_im.as<double>(), (int64_t)0, w.f64_rho.as<double>(), dcnt, (double*)dr2);
-        HIPCHK(hipGetLastError());
+        CHK(launch_voxel_fp64(p, tab, V, 1, w, w.slot_cs64.as<double2>(), 0, 0, dcnt, (double*)dr2, s));
         if (T) CHK(T->record(3));
         return D2BI_OK;
     }
@@ -553,16 +618,7 @@ static int run_voxel_apps(const d2bi_record* r, const d2bi_plan* p, const AxisTa
         CHK(w.f64_re.ensure(sizeof(double) * nvox * na));
         CHK(w.f64_im.ensure(sizeof(double) * nvox * na));
         CHK(w.f64_rho.ensure(sizeof(double) * nvox));
-        dim3 grid((p->Mx + 7) / 8, (p->My + 7) / 8, (p->Mz + 3) / 4);
-        auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, V, w.cell_start.as<int>(), w.slot_frac.as<double4>(),
-                               w.app_cs.as<double2>(), nr, w.f64_re.as<double>(), w.f64_im.as<double>(), nvox,
-                               w.f64_rho.as<double>(), (int*)nullptr, (double*)nullptr);
-        };
-        if (na == 4) go(k_voxel_fp64<4>);
-        else go(k_voxel_fp64<2>);
-        HIPCHK(hipGetLastError());
-        return D2BI_OK;
+        return launch_voxel_fp64(p, tab, V, na, w, w.app_cs.as<double2>(), nr, nvox, nullptr, nullptr, s);
     }
     const bool dens = r->use_density != 0;
     CHK(w.f32_field.ensure((dens ? sizeof(float4) : sizeof(float2)) * nvox * na));

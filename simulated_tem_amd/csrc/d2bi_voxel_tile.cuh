@@ -16,21 +16,6 @@ static constexpr int GUARD_STRIDE = 16;              // ... 16 x 8 B = 128 B apa
 static constexpr int TILE_MAXC = 128;                // cells in a tile's unwrapped range (<= 5^3)
 static constexpr int ROW_BLOCK = 32;                 // row kernel: steps per guard test and Kahan merge
 
-// Inclusive prefix sum over the 64 lanes of a wave in six DPP steps: within
-// each row of 16 lanes (row_shr 1, 2, 4, 8 with zero fill), then row 0's
-// total into row 1 and row 2's into row 3 (row_bcast:15), then rows 0-1's
-// into rows 2-3 (row_bcast:31).  All lanes must be active.
-__device__ __forceinline__ int wave_incl_scan(int v)
-{
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-    return v;
-}
-
 struct FastParams {
     VoxParams v;
     int ntx, nty, ntz;          // tiles per axis
