@@ -19,7 +19,7 @@ struct Cond {
     int nblk = 0, ncell = 0, variant = 0;
     bool dens = false;
     int64_t nr = 0, nbc = 0, nvox = 0, plane = 0;
-    int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axs = 0, o_axq = 0, o_img = 0, o_aa = 0;
+    int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axs = 0, o_axq = 0, o_img = 0;
     AxisDev ax;
 };
 
@@ -30,7 +30,7 @@ struct Cond {
 static constexpr int MAX_BRANCH = 4;
 
 struct Batch {
-    Buf mask, blkcnt, blkoff, axc, axz, axs, axq, img, aa, guard, mpc;
+    Buf mask, blkcnt, blkoff, axc, axz, axs, axq, img, guard, mpc;
     std::vector<unsigned char> key;
     uint64_t gen = 0;
     hipGraphExec_t exec = nullptr;
@@ -50,7 +50,7 @@ struct Batch {
     void release()
     {
         reset();
-        Buf* all[] = {&mask, &blkcnt, &blkoff, &axc, &axz, &axs, &axq, &img, &aa, &guard, &mpc};
+        Buf* all[] = {&mask, &blkcnt, &blkoff, &axc, &axz, &axs, &axq, &img, &guard, &mpc};
         for (Buf* b : all) b->release();
         for (int k = 0; k < MAX_BRANCH - 1; k++) {
             ws[k].release_all();
@@ -130,7 +130,7 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w
     double* d_img = B.img.as<double>() + c.o_img;
     if (mode == D2BI_MODE_FP64) {
         CHK(launch_voxel_fp64(p, c.tab, V, 1, w, w.slot_cs64.as<double2>(), 0, 0, nullptr, nullptr, s));
-        return launch_integrate_fp64(p, B.aa.as<double>() + c.o_aa, d_img, s, 0, 0.0, &w);
+        return launch_integrate_fp64(p, c.dens, d_img, s, w);
     }
     FastParams F;
     int variant = c.variant;
@@ -233,7 +233,7 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
     if (!replay) {
         B.reset();
         std::vector<Cond> C(nRec);
-        int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axs = 0, o_axq = 0, o_img = 0, o_aa = 0;
+        int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axs = 0, o_axq = 0, o_img = 0;
         int64_t max_scan = 1;
         for (int i = 0; i < nRec; i++) {
             Cond& c = C[i];
@@ -256,7 +256,6 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
             c.o_axq = o_axq; o_axq += 2 * (int64_t)c.plan.Mx + c.plan.My + 2 * (int64_t)c.plan.Mz;
             c.o_axs = o_axs; o_axs += c.plan.Ex + c.plan.Ey + c.plan.Ez + 3;
             c.o_img = o_img; o_img += c.plane;
-            c.o_aa = o_aa; o_aa += c.plan.nPrec;
             max_scan = std::max(max_scan, std::max(scan_tmp_ints(c.nbc), scan_tmp_ints(c.ncell)));
         }
         CHK(B.mask.ensure(sizeof(uint32_t) * o_mask));
@@ -267,14 +266,13 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
         CHK(B.axs.ensure(sizeof(int) * o_axs));
         CHK(B.axq.ensure(sizeof(QL) * o_axq));
         CHK(B.img.ensure(sizeof(double) * o_img));
-        CHK(B.aa.ensure(sizeof(double) * std::max<int64_t>(o_aa, 1)));
         CHK(B.guard.ensure(sizeof(unsigned long long) * nRec));
         CHK(B.mpc.ensure(sizeof(int) * nRec));
         CHK(g.ws.scan_tmp.ensure(sizeof(int) * max_scan));       // the eager counting pass
-        // tables and precession coefficients stay resident in the batch buffers
+        // tables stay resident in the batch buffers
         {
             std::vector<int> hc(o_ax), hs(o_axs);
-            std::vector<double> hz(o_ax), haa(std::max<int64_t>(o_aa, 1));
+            std::vector<double> hz(o_ax);
             std::vector<QL> hq(o_axq);
             for (int i = 0; i < nRec; i++) {
                 Cond& c = C[i];
@@ -294,13 +292,11 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
                     oc += (int64_t)c.tab.cell[a].size();
                     os += (int64_t)c.tab.start[a].size();
                 }
-                std::copy(c.plan.aa, c.plan.aa + c.plan.nPrec, haa.begin() + c.o_aa);
             }
             HIPCHK(hipMemcpy(B.axc.p, hc.data(), sizeof(int) * o_ax, hipMemcpyHostToDevice));
             HIPCHK(hipMemcpy(B.axz.p, hz.data(), sizeof(double) * o_ax, hipMemcpyHostToDevice));
             HIPCHK(hipMemcpy(B.axs.p, hs.data(), sizeof(int) * o_axs, hipMemcpyHostToDevice));
             HIPCHK(hipMemcpy(B.axq.p, hq.data(), sizeof(QL) * o_axq, hipMemcpyHostToDevice));
-            HIPCHK(hipMemcpy(B.aa.p, haa.data(), sizeof(double) * haa.size(), hipMemcpyHostToDevice));
         }
         // counting pass: sizes of every condition
         int* scan_tmp = g.ws.scan_tmp.as<int>();

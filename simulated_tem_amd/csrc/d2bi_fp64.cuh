@@ -1,5 +1,5 @@
-// d2bi_fp64.cuh -- the FP64 path: voxelisation over the 27 neighbour cells and
-// the RK4 column march in the reference's arithmetic.
+// d2bi_fp64.cuh -- FP64 voxelisation: by regions, and the per-voxel walk over
+// the 27 neighbour cells.
 //
 // One part of the single translation unit d2bi_gpu.hip, which includes the
 // parts in order so that kernels and the device helpers they call compile
@@ -315,93 +315,14 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
             const double v = part_min(dmin[z][0], dmin[z][1], dmin[z][2], dmin[z][3]);
             if (v <= P.rc2) r2 = v;
         }
-        if (out) out_rho[o] = P.use_density ? rho_of(r2, P.sigma) : 1.0;
+        // without the density field rho = 1, which the integrators do not read
+        if (MIN && out) out_rho[o] = P.use_density ? rho_of(r2, P.sigma) : 1.0;
         if (DIAG) {
             const float c = part_sum((float)cnt[z][0], (float)cnt[z][1], (float)cnt[z][2], (float)cnt[z][3]);
             if (out && out_cnt) out_cnt[o] = (int)c;
             if (out && out_r2m) out_r2m[o] = r2;
         }
     }
-}
-
-// ------------------------------------------------------------------ (c) integrate, FP64
-
-struct IntParams {
-    int Mx, My, Mz, nPrec;
-    double b0, bg, dz;
-    const double* aa;           // device array of 2 pi s_g per precession point
-    int accumulate;             // add the column sum to img instead of writing
-    double div;                 // written value: sum / div
-};
-
-// dynamicalTwoBeamIntegrationColumn_phaserho (Lib_DynamicalTwoBeamImaging.f90:2316-2480):
-// one thread per pixel column, per-double-step renormalisation, precession
-// average (:1897-1900, 1951).
-__global__ __launch_bounds__(256) void k_integrate_fp64(IntParams P, const double* __restrict__ fre,
-                                                        const double* __restrict__ fim,
-                                                        const double* __restrict__ frho,
-                                                        double* __restrict__ img)
-{
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t plane = (int64_t)P.Mx * P.My;
-    if (col >= plane) return;
-    const int nz = P.Mz;
-    const double b0 = P.b0, bg = P.bg, dz = P.dz;
-    double acc = 0.0;
-    for (int prec = 0; prec < P.nPrec; prec++) {
-        const double a = P.aa[prec];
-        double phi0r = 1.0, phi0i = 0.0, phigr = 0.0, phigi = 0.0;
-        double dphi0r, dphi0i, dphigr, dphigi;
-        double phi0r1, phi0i1, phigr1, phigi1, phi0r2, phi0i2, phigr2, phigi2;
-        // coefficients at sample k (sample Mz is sample 0, :1894-1895)
-        auto coef = [&](int k, double& c0, double& ca, double& cgr, double& cgi) {
-            const int64_t o = col + plane * (k == nz ? 0 : k);
-            const double rh = frho[o];
-            c0 = b0 * rh;
-            ca = b0 * rh + a;
-            cgr = (bg * rh) * fre[o];
-            cgi = (bg * rh) * fim[o];
-        };
-        double c0a, caa, cgra, cgia;
-        if (nz >= 2) coef(0, c0a, caa, cgra, cgia);
-        for (int ii = 0; ii <= nz - 2; ii += 2) {
-            double c0b, cab, cgrb, cgib, c0c, cac, cgrc, cgic;
-            coef(ii + 1, c0b, cab, cgrb, cgib);
-            coef(ii + 2, c0c, cac, cgrc, cgic);
-#define DERIV(c0, ca, cgr, cgi)                                      \
-    dphi0r = ((-(c0 * phi0i)) - cgi * phigr) - cgr * phigi;          \
-    dphi0i = ((c0 * phi0r) + cgr * phigr) - cgi * phigi;             \
-    dphigr = ((cgi * phi0r) - cgr * phi0i) - ca * phigi;             \
-    dphigi = ((cgr * phi0r) + cgi * phi0i) + ca * phigr;
-            DERIV(c0a, caa, cgra, cgia)
-            phi0r2 = phi0r; phi0i2 = phi0i; phigr2 = phigr; phigi2 = phigi;
-            phi0r1 = phi0r + (dphi0r * dz) / 3; phi0i1 = phi0i + (dphi0i * dz) / 3;
-            phigr1 = phigr + (dphigr * dz) / 3; phigi1 = phigi + (dphigi * dz) / 3;
-            phi0r = phi0r + dphi0r * dz; phi0i = phi0i + dphi0i * dz;
-            phigr = phigr + dphigr * dz; phigi = phigi + dphigi * dz;
-            DERIV(c0b, cab, cgrb, cgib)
-            phi0r = phi0r2 + dphi0r * dz; phi0i = phi0i2 + dphi0i * dz;
-            phigr = phigr2 + dphigr * dz; phigi = phigi2 + dphigi * dz;
-            phi0r1 = phi0r1 + ((dphi0r * 2) * dz) / 3; phi0i1 = phi0i1 + ((dphi0i * 2) * dz) / 3;
-            phigr1 = phigr1 + ((dphigr * 2) * dz) / 3; phigi1 = phigi1 + ((dphigi * 2) * dz) / 3;
-            DERIV(c0b, cab, cgrb, cgib)
-            phi0r = phi0r2 + (dphi0r * 2) * dz; phi0i = phi0i2 + (dphi0i * 2) * dz;
-            phigr = phigr2 + (dphigr * 2) * dz; phigi = phigi2 + (dphigi * 2) * dz;
-            phi0r1 = phi0r1 + ((dphi0r * 2) * dz) / 3; phi0i1 = phi0i1 + ((dphi0i * 2) * dz) / 3;
-            phigr1 = phigr1 + ((dphigr * 2) * dz) / 3; phigi1 = phigi1 + ((dphigi * 2) * dz) / 3;
-            DERIV(c0c, cac, cgrc, cgic)
-#undef DERIV
-            phi0r = phi0r1 + (dphi0r * dz) / 3; phi0i = phi0i1 + (dphi0i * dz) / 3;
-            phigr = phigr1 + (dphigr * dz) / 3; phigi = phigi1 + (dphigi * dz) / 3;
-            double phimag = ((phi0r * phi0r + phi0i * phi0i) + phigr * phigr) + phigi * phigi;
-            phimag = 1 / sqrt(phimag);
-            phi0r = phi0r * phimag; phi0i = phi0i * phimag;
-            phigr = phigr * phimag; phigi = phigi * phimag;
-            c0a = c0c; caa = cac; cgra = cgrc; cgia = cgic;
-        }
-        acc = acc + (phigr * phigr + phigi * phigi);
-    }
-    img[col] = P.accumulate ? img[col] + acc : acc / P.div;
 }
 
 }  // namespace d2bi

@@ -502,21 +502,52 @@ static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, d
     return D2BI_OK;
 }
 
-// accumulate: add each column's sum over precession points to d_img;
-// otherwise write sum / nPrec (div = 0) or sum / div.
-// The FP64 field is read from workspace w (the library's by default).
-static int launch_integrate_fp64(const d2bi_plan* p, const double* d_aa, double* d_img, hipStream_t s,
-                                 int accumulate = 0, double div = 0.0, Workspace* wp = nullptr,
-                                 int64_t field_off = 0)
+// FP64 integration of all precession points, in passes of up to 16.
+// accumulate: add each column's sum over precession points to d_img; otherwise
+// write sum / nPrec (div = 0) or sum / div.  The field is read from workspace
+// w, field_off voxels on.
+static int launch_integrate_fp64(const d2bi_plan* p, bool dens, double* d_img, hipStream_t s, Workspace& w,
+                                 int accumulate = 0, double div = 0.0, int64_t field_off = 0)
 {
-    Workspace& w = wp ? *wp : g.ws;
     const int64_t plane = (int64_t)p->Mx * p->My;
-    IntParams P{p->Mx, p->My, p->Mz, p->nPrec, p->b0, p->bg, p->dz, d_aa, accumulate,
-                div == 0.0 ? (double)p->nPrec : div};
-    hipLaunchKernelGGL(k_integrate_fp64, dim3((unsigned)((plane + 255) / 256)), dim3(256), 0, s, P,
-                       w.f64_re.as<double>() + field_off, w.f64_im.as<double>() + field_off,
-                       w.f64_rho.as<double>(), d_img);
-    HIPCHK(hipGetLastError());
+    // a lane per column: small workgroups spread a small image over the CUs
+    const int block = plane < 256 * 1024 ? 64 : 256;
+    for (int p0 = 0; p0 < p->nPrec;) {
+        const int left = p->nPrec - p0;
+        const int inst = left <= 4 ? left : left <= 6 ? 6 : left <= 8 ? 8 : left <= 12 ? 12 : 16;
+        const int np = std::min(left, inst);
+        IntParams P;
+        P.Mx = p->Mx; P.My = p->My; P.Mz = p->Mz; P.np = np;
+        P.b0 = p->b0; P.bg = p->bg; P.dz = p->dz;
+        for (int i = 0; i < 16; i++) {
+            P.aa[i] = i < np ? p->aa[p0 + i] : 0.0;
+            P.al[i] = 2.0 * p->dz * P.aa[i];
+        }
+        P.accumulate = accumulate || p0 > 0;
+        P.div = accumulate || p0 + np < p->nPrec ? 0.0 : div == 0.0 ? (double)p->nPrec : div;
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)((plane + block - 1) / block)), dim3(block), 0, s, P,
+                               w.f64_re.as<double>() + field_off, w.f64_im.as<double>() + field_off,
+                               w.f64_rho.as<double>(), d_img);
+        };
+        auto pick = [&](auto np_c) {
+            constexpr int N = decltype(np_c)::value;
+            if (dens) go(k_integrate_fp64<N, true>);
+            else go(k_integrate_fp64<N, false>);
+        };
+        switch (inst) {
+            case 1: pick(std::integral_constant<int, 1>{}); break;
+            case 2: pick(std::integral_constant<int, 2>{}); break;
+            case 3: pick(std::integral_constant<int, 3>{}); break;
+            case 4: pick(std::integral_constant<int, 4>{}); break;
+            case 6: pick(std::integral_constant<int, 6>{}); break;
+            case 8: pick(std::integral_constant<int, 8>{}); break;
+            case 12: pick(std::integral_constant<int, 12>{}); break;
+            default: pick(std::integral_constant<int, 16>{}); break;
+        }
+        HIPCHK(hipGetLastError());
+        p0 += np;
+    }
     return D2BI_OK;
 }
 
@@ -525,14 +556,9 @@ static int run_integrate(const d2bi_plan* p, bool dens, int mode, hipStream_t s,
                          Timer* T = nullptr)
 {
     if (mode == D2BI_MODE_FP64) {
-        CHK(w.aa.ensure(sizeof(double) * D2BI_MAX_PREC));
-        double* d_aa = w.aa.as<double>();
-        HIPCHK(hipMemcpyAsync(d_aa, p->aa, sizeof(double) * p->nPrec, hipMemcpyHostToDevice, s));
         if (T) CHK(T->record(4));
-        CHK(launch_integrate_fp64(p, d_aa, d_img, s, 0, 0.0, &w));
+        CHK(launch_integrate_fp64(p, dens, d_img, s, w));
         if (T) CHK(T->record(5));
-        // the aa copy reads p->aa (caller memory): finish before returning
-        HIPCHK(hipStreamSynchronize(s));
         return D2BI_OK;
     }
     if (T) CHK(T->record(4));
@@ -691,7 +717,6 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
     const int64_t plane = (int64_t)plan.Mx * plan.My;
     const int64_t nvox = plane * plan.Mz;
     CHK(w.img.ensure(sizeof(double) * plane));
-    CHK(w.aa.ensure(sizeof(double) * D2BI_MAX_PREC));
     double* d_img = w.img.as<double>();
     const bool dens = r->use_density != 0;
     const double total = (double)nApp * nPrec;
@@ -708,12 +733,8 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
     auto integrate_point = [&](int app, int64_t f64_off, const void* f32) -> int {
         const d2bi_plan pk = point_plan(app);
         if (f64) {
-            double* d_aa = w.aa.as<double>();
-            HIPCHK(hipMemcpyAsync(d_aa, pk.aa, sizeof(double) * nPrec, hipMemcpyHostToDevice, s));
             // point 0 writes its sum (div 1), the others add theirs
-            CHK(launch_integrate_fp64(&pk, d_aa, d_img, s, app > 0 ? 1 : 0, 1.0, &w, f64_off));
-            // pk.aa (host) is read by the copy above: finish before it goes
-            HIPCHK(hipStreamSynchronize(s));
+            CHK(launch_integrate_fp64(&pk, dens, d_img, s, w, app > 0 ? 1 : 0, 1.0, f64_off));
         } else {
             CHK(launch_integrate_fast(&pk, dens, f32, d_img, s, app > 0, 1.0 / total, &w));
         }
