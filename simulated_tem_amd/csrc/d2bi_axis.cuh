@@ -36,8 +36,6 @@ struct AxisTables {
     std::vector<int> cell[3];
     std::vector<double> zi[3];
     std::vector<QL> ql[NQL];       // x, y, z for 4-voxel tiles; z, x for 8-voxel tiles
-    std::vector<int> start[3];     // first voxel of each link cell (size E+1)
-    int lo[3], hi[3];              // active link-cell range
 };
 
 static bool diagonal(const double* m)
@@ -54,7 +52,6 @@ static int axis_tables(const d2bi_record* r, const d2bi_plan* p, AxisTables* t)
     for (int a = 0; a < 3; a++) {
         t->cell[a].resize(M[a]);
         t->zi[a].resize(M[a]);
-        t->start[a].assign(E[a] + 1, M[a]);
         const double av = r->gk_a[4 * a], ia = p->ia_col[4 * a];
         for (int i = 0; i < M[a]; i++) {
             double xx = av * i - p->lc_delta[a];
@@ -76,21 +73,13 @@ static int axis_tables(const d2bi_record* r, const d2bi_plan* p, AxisTables* t)
                 t->ql[k][i] = QL{(float)(side * (t->zi[a][i] + lc)), lc};
             }
         }
-        for (int i = M[a] - 1; i >= 0; i--) t->start[a][t->cell[a][i]] = i;
-        // cells with no voxels take the start of the next occupied cell
-        for (int c = E[a] - 1; c >= 0; c--)
-            if (t->start[a][c] > t->start[a][c + 1]) t->start[a][c] = t->start[a][c + 1];
-        t->lo[a] = t->cell[a][0];
-        t->hi[a] = t->cell[a][M[a] - 1];
     }
     return D2BI_OK;
 }
 
-// Upload tables: ints [cellx|celly|cellz], doubles [zix|ziy|ziz], ints [startx|starty|startz]
 struct AxisDev {
     const int* cell[3];
     const double* zi[3];
-    const int* start[3];
     const QL* ql[NQL];
 };
 
@@ -99,17 +88,15 @@ struct AxisDev {
 static int upload_axis(const AxisTables& t, AxisDev* d, hipStream_t s, Workspace& w)
 {
     size_t nc = t.cell[0].size() + t.cell[1].size() + t.cell[2].size();
-    size_t ns = t.start[0].size() + t.start[1].size() + t.start[2].size();
     size_t nq = 0;
     for (int k = 0; k < NQL; k++) nq += t.ql[k].size();
     CHK(w.ax_cell.ensure(sizeof(int) * nc));
     CHK(w.ax_zi.ensure(sizeof(double) * nc));
-    CHK(w.ax_start.ensure(sizeof(int) * ns));
     CHK(w.ax_ql.ensure(sizeof(QL) * nq));
     if (w.ax_cell.arena) {
         // a workspace that must not allocate: copy from the tables
         // themselves, not through the (growable) pinned staging buffer
-        size_t oc = 0, os = 0, oq = 0;
+        size_t oc = 0, oq = 0;
         for (int k = 0; k < NQL; k++) {
             d->ql[k] = w.ax_ql.as<QL>() + oq;
             HIPCHK(hipMemcpyAsync((void*)d->ql[k], t.ql[k].data(), sizeof(QL) * t.ql[k].size(),
@@ -119,27 +106,22 @@ static int upload_axis(const AxisTables& t, AxisDev* d, hipStream_t s, Workspace
         for (int a = 0; a < 3; a++) {
             d->cell[a] = w.ax_cell.as<int>() + oc;
             d->zi[a] = w.ax_zi.as<double>() + oc;
-            d->start[a] = w.ax_start.as<int>() + os;
             HIPCHK(hipMemcpyAsync((void*)d->cell[a], t.cell[a].data(), sizeof(int) * t.cell[a].size(),
                                   hipMemcpyHostToDevice, s));
             HIPCHK(hipMemcpyAsync((void*)d->zi[a], t.zi[a].data(), sizeof(double) * t.zi[a].size(),
                                   hipMemcpyHostToDevice, s));
-            HIPCHK(hipMemcpyAsync((void*)d->start[a], t.start[a].data(), sizeof(int) * t.start[a].size(),
-                                  hipMemcpyHostToDevice, s));
             oc += t.cell[a].size();
-            os += t.start[a].size();
         }
         return D2BI_OK;
     }
-    size_t bytes = sizeof(int) * nc + sizeof(double) * nc + sizeof(int) * ns + sizeof(QL) * nq;
+    size_t bytes = sizeof(int) * nc + sizeof(double) * nc + sizeof(QL) * nq;
     void* hp;
     CHK(pinned(bytes, &hp));
     char* h = (char*)hp;
-    int* hc = (int*)h;
-    double* hz = (double*)(h + sizeof(int) * nc);
-    int* hs = (int*)(h + sizeof(int) * nc + sizeof(double) * nc);
-    QL* hq = (QL*)(h + sizeof(int) * nc + sizeof(double) * nc + sizeof(int) * ns);
-    size_t oc = 0, os = 0, oq = 0;
+    double* hz = (double*)h;
+    QL* hq = (QL*)(h + sizeof(double) * nc);
+    int* hc = (int*)(h + sizeof(double) * nc + sizeof(QL) * nq);
+    size_t oc = 0, oq = 0;
     for (int k = 0; k < NQL; k++) {
         std::memcpy(hq + oq, t.ql[k].data(), sizeof(QL) * t.ql[k].size());
         d->ql[k] = w.ax_ql.as<QL>() + oq;
@@ -148,16 +130,12 @@ static int upload_axis(const AxisTables& t, AxisDev* d, hipStream_t s, Workspace
     for (int a = 0; a < 3; a++) {
         std::memcpy(hc + oc, t.cell[a].data(), sizeof(int) * t.cell[a].size());
         std::memcpy(hz + oc, t.zi[a].data(), sizeof(double) * t.zi[a].size());
-        std::memcpy(hs + os, t.start[a].data(), sizeof(int) * t.start[a].size());
         d->cell[a] = w.ax_cell.as<int>() + oc;
         d->zi[a] = w.ax_zi.as<double>() + oc;
-        d->start[a] = w.ax_start.as<int>() + os;
         oc += t.cell[a].size();
-        os += t.start[a].size();
     }
     HIPCHK(hipMemcpyAsync(w.ax_cell.p, hc, sizeof(int) * nc, hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(w.ax_zi.p, hz, sizeof(double) * nc, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(w.ax_start.p, hs, sizeof(int) * ns, hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(w.ax_ql.p, hq, sizeof(QL) * nq, hipMemcpyHostToDevice, s));
     // the pinned buffer is reused by later calls: they wait for this event
     HIPCHK(hipEventRecord(g.ev[9], s));

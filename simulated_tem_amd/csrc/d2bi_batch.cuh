@@ -19,7 +19,7 @@ struct Cond {
     int nblk = 0, ncell = 0, variant = 0;
     bool dens = false;
     int64_t nr = 0, nbc = 0, nvox = 0, plane = 0;
-    int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axs = 0, o_axq = 0, o_img = 0;
+    int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axq = 0, o_img = 0;
     AxisDev ax;
 };
 
@@ -30,7 +30,7 @@ struct Cond {
 static constexpr int MAX_BRANCH = 4;
 
 struct Batch {
-    Buf mask, blkcnt, blkoff, axc, axz, axs, axq, img, guard, mpc;
+    Buf mask, blkcnt, blkoff, axc, axz, axq, img, guard, mpc;
     std::vector<unsigned char> key;
     uint64_t gen = 0;
     hipGraphExec_t exec = nullptr;
@@ -50,7 +50,7 @@ struct Batch {
     void release()
     {
         reset();
-        Buf* all[] = {&mask, &blkcnt, &blkoff, &axc, &axz, &axs, &axq, &img, &guard, &mpc};
+        Buf* all[] = {&mask, &blkcnt, &blkoff, &axc, &axz, &axq, &img, &guard, &mpc};
         for (Buf* b : all) b->release();
         for (int k = 0; k < MAX_BRANCH - 1; k++) {
             ws[k].release_all();
@@ -93,7 +93,7 @@ static int enqueue_count(const Cond& c, Batch& B, int* scan_tmp, hipStream_t s)
     if (c.n > 0)
         hipLaunchKernelGGL(k_bin_classify, dim3(c.nblk), dim3(BIN_BLOCK), 0, s, c.d_x, c.BP, mask, cnt, c.nblk);
     else
-        fill_i32(cnt, c.nbc, 0, s);
+        zero_i32(s, cnt, c.nbc);
     HIPCHK(hipGetLastError());
     return scan_exclusive_tmp(cnt, off, c.nbc, scan_tmp, s);
 }
@@ -106,23 +106,11 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w
     const d2bi_plan* p = &c.plan;
     int* mpc = B.mpc.as<int>() + idx;
     unsigned long long* gc = B.guard.as<unsigned long long>() + idx;
-    fill_i32(w.cell_cnt.as<int>(), c.ncell + 1, 0, s);
-    fill_i32(mpc, 1, 0, s);
     unsigned long long* gp = w.guard_part.as<unsigned long long>();
-    fill_i32((int*)gc, 2, 0, s);
-    if (mode == D2BI_MODE_FAST) fill_i32((int*)gp, 2 * GUARD_SLOTS * GUARD_STRIDE, 0, s);
-    if (c.n > 0 && c.nr > 0)
-        hipLaunchKernelGGL(k_bin_scatter, dim3(c.nblk), dim3(BIN_BLOCK), 0, s, c.d_x, c.BP,
-                           B.mask.as<uint32_t>() + c.o_mask, B.blkoff.as<int>() + c.o_blk, c.nblk,
-                           w.pt_cell.as<int>(), w.pt_slot.as<int>(), w.pt_frac.as<double>(),
-                           w.pt_gdotr.as<double>(), w.pt_j.as<int>(),
-                           w.cell_cnt.as<int>());
-    CHK(scan_exclusive_tmp(w.cell_cnt.as<int>(), w.cell_start.as<int>(), c.ncell, scan_tmp, s));
-    if (c.nr > 0)
-        hipLaunchKernelGGL(k_bin_place, dim3((unsigned)((c.nr + 255) / 256)), dim3(256), 0, s, c.nr,
-                           w.pt_cell.as<int>(), w.pt_slot.as<int>(), w.cell_start.as<int>(), w.cell_ids.as<int>());
-    launch_bin_finish(c.ncell, c.nr, c.BP, mpc, s, w, c.d_x, B.blkoff.as<int>() + c.o_blk, c.nblk);
-    HIPCHK(hipGetLastError());
+    zero_i32(s, w.cell_cnt.as<int>(), c.ncell + 1, mpc, 1, (int*)gc, 2, (int*)gp,
+             mode == D2BI_MODE_FAST ? 2 * GUARD_SLOTS * GUARD_STRIDE : 0);
+    CHK(launch_bin_points(c.d_x, c.BP, B.mask.as<uint32_t>() + c.o_mask, B.blkoff.as<int>() + c.o_blk, c.nblk, c.ncell,
+                          c.nr, scan_tmp, mpc, s, w));
     VoxParams V;
     d2bi_record dummy;
     dummy.use_density = c.dens ? 1 : 0;
@@ -138,7 +126,7 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w
     // the tile order timed eagerly before capture (nothing is timed here)
     set_tile_order(&F, tune_choose(tile_order_key(p, c.tab, c.dens, c.variant), "D2BI_TILE_ORDER", TILE_ORDERS, 3,
                                    2, false, s, [](int) {}));
-    launch_tile<false>(F, variant, c.dens, w.cell_start.as<int>(), w.slot_frac.as<double4>(),
+    launch_tile<false>(F, variant, c.dens, w.cell_start.as<int>(), w.slot_frac.as<Frac3>(),
                        w.slot_p32.as<float4>(), w.slot_sn32.as<float>(), w.f32_field.as<float4>(), nullptr, nullptr,
                        gp, s);
     HIPCHK(hipGetLastError());
@@ -158,21 +146,14 @@ static void branch_buffers(Workspace& w, const BranchSizes& z, F f)
 {
     f(w.pt_cell, sizeof(int) * z.max_nr);
     f(w.pt_slot, sizeof(int) * z.max_nr);
-    if (z.mode == D2BI_MODE_FP64) {
-        f(w.pt_frac, sizeof(double) * 3 * z.max_nr);
-        f(w.pt_gdotr, sizeof(double) * z.max_nr);
-        f(w.slot_id, sizeof(int) * z.max_nr);
-        f(w.slot_cs64, sizeof(double2) * z.max_nr);
-    } else {
-        f(w.pt_j, sizeof(int) * z.max_nr);
-    }
+    f(w.pt_j, sizeof(int) * z.max_nr);
     f(w.cell_ids, sizeof(int) * z.max_nr);
-    f(w.slot_frac, sizeof(double4) * z.max_nr);
+    f(w.slot_frac, sizeof(Frac3) * z.max_nr);
     f(w.slot_p32, sizeof(float4) * z.max_nr);
-    f(w.slot_sn32, sizeof(float) * z.max_nr);
+    if (z.mode == D2BI_MODE_FP64) f(w.slot_cs64, sizeof(double2) * z.max_nr);
+    else f(w.slot_sn32, sizeof(float) * z.max_nr);
     f(w.cell_cnt, sizeof(int) * z.max_cell);
     f(w.cell_start, sizeof(int) * z.max_cell);
-    f(w.blk_max, sizeof(int) * (z.max_cell / 256 + 2));
     if (z.mode == D2BI_MODE_FP64) {
         f(w.f64_re, sizeof(double) * z.max_vox);
         f(w.f64_im, sizeof(double) * z.max_vox);
@@ -233,7 +214,7 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
     if (!replay) {
         B.reset();
         std::vector<Cond> C(nRec);
-        int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axs = 0, o_axq = 0, o_img = 0;
+        int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axq = 0, o_img = 0;
         int64_t max_scan = 1;
         for (int i = 0; i < nRec; i++) {
             Cond& c = C[i];
@@ -244,7 +225,7 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
             c.d_x = atoms[i]->x;
             c.n = atoms[i]->n;
             c.BP.n = c.n;
-            c.nblk = (int)std::max<int64_t>(1, (c.n + BIN_TILE - 1) / BIN_TILE);
+            c.nblk = bin_blocks(c.n);
             c.nbc = (int64_t)c.BP.nuvw * c.nblk;
             c.ncell = c.plan.Ex * c.plan.Ey * c.plan.Ez;
             c.dens = recs[i].use_density != 0;
@@ -254,7 +235,6 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
             c.o_blk = o_blk; o_blk += c.nbc + 1;
             c.o_ax = o_ax; o_ax += c.plan.Mx + c.plan.My + c.plan.Mz;
             c.o_axq = o_axq; o_axq += 2 * (int64_t)c.plan.Mx + c.plan.My + 2 * (int64_t)c.plan.Mz;
-            c.o_axs = o_axs; o_axs += c.plan.Ex + c.plan.Ey + c.plan.Ez + 3;
             c.o_img = o_img; o_img += c.plane;
             max_scan = std::max(max_scan, std::max(scan_tmp_ints(c.nbc), scan_tmp_ints(c.ncell)));
         }
@@ -263,7 +243,6 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
         CHK(B.blkoff.ensure(sizeof(int) * o_blk));
         CHK(B.axc.ensure(sizeof(int) * o_ax));
         CHK(B.axz.ensure(sizeof(double) * o_ax));
-        CHK(B.axs.ensure(sizeof(int) * o_axs));
         CHK(B.axq.ensure(sizeof(QL) * o_axq));
         CHK(B.img.ensure(sizeof(double) * o_img));
         CHK(B.guard.ensure(sizeof(unsigned long long) * nRec));
@@ -271,12 +250,12 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
         CHK(g.ws.scan_tmp.ensure(sizeof(int) * max_scan));       // the eager counting pass
         // tables stay resident in the batch buffers
         {
-            std::vector<int> hc(o_ax), hs(o_axs);
+            std::vector<int> hc(o_ax);
             std::vector<double> hz(o_ax);
             std::vector<QL> hq(o_axq);
             for (int i = 0; i < nRec; i++) {
                 Cond& c = C[i];
-                int64_t oc = c.o_ax, os = c.o_axs, oq = c.o_axq;
+                int64_t oc = c.o_ax, oq = c.o_axq;
                 for (int k = 0; k < NQL; k++) {
                     std::copy(c.tab.ql[k].begin(), c.tab.ql[k].end(), hq.begin() + oq);
                     c.ax.ql[k] = B.axq.as<QL>() + oq;
@@ -285,17 +264,13 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
                 for (int a = 0; a < 3; a++) {
                     std::copy(c.tab.cell[a].begin(), c.tab.cell[a].end(), hc.begin() + oc);
                     std::copy(c.tab.zi[a].begin(), c.tab.zi[a].end(), hz.begin() + oc);
-                    std::copy(c.tab.start[a].begin(), c.tab.start[a].end(), hs.begin() + os);
                     c.ax.cell[a] = B.axc.as<int>() + oc;
                     c.ax.zi[a] = B.axz.as<double>() + oc;
-                    c.ax.start[a] = B.axs.as<int>() + os;
                     oc += (int64_t)c.tab.cell[a].size();
-                    os += (int64_t)c.tab.start[a].size();
                 }
             }
             HIPCHK(hipMemcpy(B.axc.p, hc.data(), sizeof(int) * o_ax, hipMemcpyHostToDevice));
             HIPCHK(hipMemcpy(B.axz.p, hz.data(), sizeof(double) * o_ax, hipMemcpyHostToDevice));
-            HIPCHK(hipMemcpy(B.axs.p, hs.data(), sizeof(int) * o_axs, hipMemcpyHostToDevice));
             HIPCHK(hipMemcpy(B.axq.p, hq.data(), sizeof(QL) * o_axq, hipMemcpyHostToDevice));
         }
         // counting pass: sizes of every condition

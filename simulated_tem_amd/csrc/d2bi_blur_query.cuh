@@ -104,7 +104,7 @@ struct QueryParams {
 // and a general (not necessarily cuboidal) cell.
 __global__ void k_lc_query(QueryParams Q, int64_t nq, const double* __restrict__ q,
                            const int* __restrict__ cell_start, const int* __restrict__ slot_id,
-                           const double4* __restrict__ frac, int* __restrict__ nout,
+                           const Frac3* __restrict__ frac, int* __restrict__ nout,
                            int* __restrict__ idout, double* __restrict__ r2out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -128,7 +128,7 @@ __global__ void k_lc_query(QueryParams Q, int64_t nq, const double* __restrict__
                 const double dzi1 = kx - zi[0];
                 const int c = jx + Q.Nx * (jy + Q.Ny * jz);
                 for (int s = cell_start[c]; s < cell_start[c + 1]; s++) {
-                    const double4 f = frac[s];
+                    const Frac3 f = frac[s];
                     const double dzj1 = f.x + dzi1, dzj2 = f.y + dzi2, dzj3 = f.z + dzi3;
                     double d[3];
                     for (int k = 0; k < 3; k++) d[k] = (Q.a[k] * dzj1 + Q.a[3 + k] * dzj2) + Q.a[6 + k] * dzj3;

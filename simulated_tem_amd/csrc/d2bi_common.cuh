@@ -101,17 +101,17 @@ struct Workspace {
     // binning
     Buf x;                      // atoms (temporary upload)
     Buf mask, blk_cnt, blk_off;
-    Buf pt_cell, pt_slot, pt_frac, pt_gdotr;
-    Buf pt_j;                   // atom number of each point (FAST imaging, FP64 aperture sums)
-    Buf cell_cnt, cell_start, cell_ids;
+    Buf pt_cell, pt_slot, pt_j;             // link cell, arrival in it and atom number of each point
+    Buf pt_gdotr;                           // g.r of each point (link-cell API)
+    Buf cell_cnt, cell_start, cell_ids;     // cell_ids: points by cell, unordered inside each
     Buf slot_id, slot_frac, slot_cs64, slot_p32, slot_sn32;
+    Buf slot_src;                           // atom and replica of each slot (aperture sums)
     Buf app_cs;                 // per-slot phases of the aperture points of one shared pass
     Buf scan_tmp;
-    Buf blk_max;                // per-block largest cell count (link-cell sort)
     Buf guard_part;             // FAST guard re-test counters, one per 128-byte line
     Buf counters;               // misc device counters (guard count, max per cell)
     // voxel axis tables
-    Buf ax_cell, ax_zi, ax_start, ax_ql;
+    Buf ax_cell, ax_zi, ax_ql;
     // fields and image
     Buf f64_re, f64_im, f64_rho, f32_field;
     Buf cnt, r2m;
@@ -123,9 +123,9 @@ struct Workspace {
     size_t pinned_cap = 0;
     template <class F> void each(F f)
     {
-        Buf* all[] = {&x, &mask, &blk_cnt, &blk_off, &pt_cell, &pt_slot, &pt_frac, &pt_gdotr, &pt_j,
+        Buf* all[] = {&x, &mask, &blk_cnt, &blk_off, &pt_cell, &pt_slot, &pt_j, &pt_gdotr,
                       &cell_cnt, &cell_start, &cell_ids, &slot_id, &slot_frac, &slot_cs64,
-                      &slot_p32, &slot_sn32, &app_cs, &scan_tmp, &blk_max, &guard_part, &counters, &ax_cell, &ax_zi, &ax_start, &ax_ql, &f64_re,
+                      &slot_p32, &slot_sn32, &slot_src, &app_cs, &scan_tmp, &guard_part, &counters, &ax_cell, &ax_zi, &ax_ql, &f64_re,
                       &f64_im, &f64_rho, &f32_field, &cnt, &r2m, &img, &tune_img, &blur_in, &blur_tmp,
                       &blur_out, &blur_w, &blur_wy, &blur_k};
         for (Buf* b : all) f(*b);
@@ -204,17 +204,29 @@ namespace d2bi {
 
 // ------------------------------------------------------------------ fills
 
-// Fill kernels clear counters and flags (rather than hipMemsetAsync, which
-// must not be recorded into a captured graph).
-__global__ void k_fill_i32(int* __restrict__ p, int64_t n, int v)
+// Kernels clear counters and flags (rather than hipMemsetAsync, which must not
+// be recorded into a captured graph): up to four arrays in one launch.
+struct ZeroRanges {
+    int* p[4];
+    int64_t n[4];
+};
+
+__global__ void k_zero(ZeroRanges Z)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        if (i >= 0 && i < Z.n[r]) Z.p[r][i] = 0;
+        i -= Z.n[r];
+    }
 }
 
-static void fill_i32(int* p, int64_t n, int v, hipStream_t s)
+static void zero_i32(hipStream_t s, int* p0, int64_t n0, int* p1 = nullptr, int64_t n1 = 0, int* p2 = nullptr,
+                     int64_t n2 = 0, int* p3 = nullptr, int64_t n3 = 0)
 {
-    if (n > 0) hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
+    const ZeroRanges Z{{p0, p1, p2, p3}, {n0, n1, n2, n3}};
+    const int64_t n = n0 + n1 + n2 + n3;
+    if (n > 0) hipLaunchKernelGGL(k_zero, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, Z);
 }
 
 // ------------------------------------------------------------------ generic scan
@@ -238,16 +250,12 @@ static constexpr int SCAN_BLOCK = 256;
 static constexpr int SCAN_ITEMS = 4;
 static constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
-// Block-wide exclusive scan of one int per thread (wave64 shuffles + LDS).
-__device__ inline int block_exclusive_scan(int v, int* total, int* lds /*[SCAN_BLOCK/64 + 1]*/)
+// Block-wide exclusive scan of one int per thread (wave64 prefix sums + LDS);
+// lds holds a word per wave and one more.
+__device__ inline int block_exclusive_scan(int v, int* total, int* lds)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int t = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += t;
-    }
+    const int incl = wave_incl_scan(v);
     if (lane == 63) lds[wave] = incl;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -262,23 +270,80 @@ __device__ inline int block_exclusive_scan(int v, int* total, int* lds /*[SCAN_B
     return r;
 }
 
+// Largest value of the block, in every thread.
+__device__ inline int block_max(int v, int* lds)
+{
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    for (int w = 0; w < (int)(blockDim.x >> 6); w++) v = max(v, lds[w]);
+    __syncthreads();
+    return v;
+}
+
+// Short arrays (a small condition's block counts or link cells) in one
+// workgroup and one launch: on an 80^3 condition the launch gaps of a
+// three-phase scan cost more than its work (3 x ~5 us against 5).
+static constexpr int SCAN_ONE_BLOCK = 1024;
+static constexpr int SCAN_ONE_ITEMS = 16;
+static constexpr int SCAN_ONE = SCAN_ONE_BLOCK * SCAN_ONE_ITEMS;
+
+__global__ __launch_bounds__(SCAN_ONE_BLOCK) void k_scan_one(const int* __restrict__ in, int n, int* __restrict__ out,
+                                                             int* __restrict__ max_out)
+{
+    __shared__ int lds[SCAN_ONE_BLOCK / 64 + 1];
+    const int per = (n + SCAN_ONE_BLOCK - 1) / SCAN_ONE_BLOCK, base = (int)threadIdx.x * per;
+    int v[SCAN_ONE_ITEMS], s = 0, m = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_ITEMS; i++) v[i] = i < per && base + i < n ? in[base + i] : 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_ITEMS; i++) {
+        s += v[i];
+        m = max(m, v[i]);
+    }
+    int tot;
+    int e = block_exclusive_scan(s, &tot, lds);
+#pragma unroll
+    for (int i = 0; i < SCAN_ONE_ITEMS; i++) {
+        if (i < per && base + i < n) out[base + i] = e;
+        e += v[i];
+    }
+    if (threadIdx.x == 0) out[n] = tot;
+    if (max_out) {
+        m = block_max(m, lds);
+        if (threadIdx.x == 0) *max_out = m;
+    }
+}
+
+// Longer ones: sums (and largest values) per tile of 1024, then each tile's
+// scan behind the sum of the tiles before it, which its workgroup adds up
+// itself up to SCAN_SELF tiles; beyond, one workgroup scans the sums between.
+static constexpr int SCAN_SELF = 4096;
+
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(const int* __restrict__ in, int64_t n,
-                                                            int* __restrict__ sums)
+                                                            int* __restrict__ sums, int* __restrict__ maxs)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
     int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-    int s = 0;
+    int s = 0, m = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++)
-        if (base + i < n) s += in[base + i];
+        if (base + i < n) {
+            s += in[base + i];
+            m = max(m, in[base + i]);
+        }
     int tot;
     block_exclusive_scan(s, &tot, lds);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
+    m = block_max(m, lds);
+    if (threadIdx.x == 0) {
+        sums[blockIdx.x] = tot;
+        maxs[blockIdx.x] = m;
+    }
 }
 
 // Single-block exclusive scan of the block sums (any length), in place.
-__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(int* __restrict__ sums, int64_t nb,
-                                                          int* __restrict__ total_out)
+__global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(int* __restrict__ sums, int64_t nb)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
     int carry = 0;
@@ -290,14 +355,22 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(int* __restrict__ sums
         if (i < nb) sums[i] = e + carry;
         carry += tot;
     }
-    if (threadIdx.x == 0) *total_out = carry;
 }
 
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const int* __restrict__ in, int64_t n,
-                                                           const int* __restrict__ sums,
-                                                           int* __restrict__ out)
+                                                           const int* __restrict__ sums, int scanned,
+                                                           const int* __restrict__ maxs, int* __restrict__ out,
+                                                           int* __restrict__ max_out)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
+    int before = 0;
+    if (scanned) {
+        before = sums[blockIdx.x];
+    } else {
+        int p = 0;
+        for (int b = threadIdx.x; b < (int)blockIdx.x; b += SCAN_BLOCK) p += sums[b];
+        block_exclusive_scan(p, &before, lds);
+    }
     int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     int v[SCAN_ITEMS];
     int s = 0;
@@ -307,37 +380,49 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const int* __restrict
         s += v[i];
     }
     int tot;
-    int e = block_exclusive_scan(s, &tot, lds) + sums[blockIdx.x];
+    int e = block_exclusive_scan(s, &tot, lds) + before;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++) {
         if (base + i < n) out[base + i] = e;
         e += v[i];
     }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + tot;
+    if (max_out && blockIdx.x == 0) {
+        int m = 0;
+        for (int b = threadIdx.x; b < (int)gridDim.x; b += SCAN_BLOCK) m = max(m, maxs[b]);
+        m = block_max(m, lds);
+        if (threadIdx.x == 0) *max_out = m;
+    }
 }
 
 static int64_t scan_tmp_ints(int64_t n)
 {
-    return std::max<int64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE) + 1;
+    return 2 * std::max<int64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE);
 }
 
-// out[0..n-1] = exclusive scan of in, out[n] = total.  in may equal out.
-// sums: scan_tmp_ints(n) ints of scratch (no allocation here, so the call can
-// be captured into a graph).
-static int scan_exclusive_tmp(const int* in, int* out, int64_t n, int* sums, hipStream_t s)
+// out[0..n-1] = exclusive scan of in, out[n] = total, *max_out (optional) the
+// largest value, 0 if n = 0.  tmp: scan_tmp_ints(n) ints of scratch (no
+// allocation here, so the call can be captured into a graph).
+static int scan_exclusive_tmp(const int* in, int* out, int64_t n, int* tmp, hipStream_t s, int* max_out = nullptr)
 {
-    int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-    if (nb < 1) nb = 1;
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, s, sums, nb, out + n);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, out);
+    if (n <= SCAN_ONE) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_BLOCK), 0, s, in, (int)n, out, max_out);
+    } else {
+        const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
+        int *sums = tmp, *maxs = tmp + nb;
+        hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, maxs);
+        if (nb > SCAN_SELF) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, s, sums, nb);
+        hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums,
+                           nb > SCAN_SELF ? 1 : 0, maxs, out, max_out);
+    }
     HIPCHK(hipGetLastError());
     return D2BI_OK;
 }
 
-static int scan_exclusive(const int* in, int* out, int64_t n, hipStream_t s, Workspace& w)
+static int scan_exclusive(const int* in, int* out, int64_t n, hipStream_t s, Workspace& w, int* max_out = nullptr)
 {
     CHK(w.scan_tmp.ensure(sizeof(int) * scan_tmp_ints(n)));
-    return scan_exclusive_tmp(in, out, n, w.scan_tmp.as<int>(), s);
+    return scan_exclusive_tmp(in, out, n, w.scan_tmp.as<int>(), s, max_out);
 }
 
 }  // namespace d2bi

@@ -20,7 +20,7 @@ namespace d2bi {
 // that point's phases.
 template <int NA>
 __global__ __launch_bounds__(256) void k_voxel_fp64(VoxParams P, const int* __restrict__ cell_start,
-                                                    const double4* __restrict__ frac,
+                                                    const Frac3* __restrict__ frac,
                                                     const double2* __restrict__ cs64, int64_t cs_stride,
                                                     double* __restrict__ out_re,
                                                     double* __restrict__ out_im, int64_t out_stride,
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void k_voxel_fp64(VoxParams P, const int* __re
                 const int c = jx + P.Ex * (jy + P.Ey * jz);
                 const int s1 = cell_start[c + 1];
                 for (int s = cell_start[c]; s < s1; s++) {
-                    const double4 f = frac[s];
+                    const Frac3 f = frac[s];
                     const double d1 = P.a[0] * (f.x + dzi1);
                     const double d2 = P.a[1] * (f.y + dzi2);
                     const double d3 = P.a[2] * (f.z + dzi3);
@@ -127,7 +127,7 @@ struct F64Record {
 
 template <int NA, bool MIN, bool DIAG>
 __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_region(
-    RegionParams R, const int* __restrict__ cell_start, const double4* __restrict__ frac,
+    RegionParams R, const int* __restrict__ cell_start, const Frac3* __restrict__ frac,
     const float4* __restrict__ p32, const double2* __restrict__ cs64, int64_t cs_stride, double* __restrict__ out_re,
     double* __restrict__ out_im, int64_t out_stride, double* __restrict__ out_rho, int* __restrict__ out_cnt,
     double* __restrict__ out_r2m)

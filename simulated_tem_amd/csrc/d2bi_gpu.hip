@@ -356,6 +356,7 @@ int d2bi_gpu_linkcells(const d2bi_record* rec, const double* x, int64_t ld, int6
     CHK(plan_image(rec, nAtoms, 0.0, 1, &plan));
     BinParams BP;
     CHK(bin_params(rec, &plan, &BP));
+    BP.keep_ids = 1;
     Binned b;
     CHK(run_binning(d_x, nAtoms, BP, &b, g.stream, g.ws));
     HIPCHK(hipStreamSynchronize(g.stream));
@@ -365,11 +366,7 @@ int d2bi_gpu_linkcells(const d2bi_record* rec, const double* x, int64_t ld, int6
     Workspace& w = g.ws;
     if (cell_start) HIPCHK(hipMemcpy(cell_start, w.cell_start.p, sizeof(int) * (b.ncell + 1), hipMemcpyDeviceToHost));
     if (ids && b.nr) HIPCHK(hipMemcpy(ids, w.slot_id.p, sizeof(int) * b.nr, hipMemcpyDeviceToHost));
-    if (frac && b.nr) {
-        std::vector<double> f(4 * b.nr);
-        HIPCHK(hipMemcpy(f.data(), w.slot_frac.p, sizeof(double) * 4 * b.nr, hipMemcpyDeviceToHost));
-        for (int64_t i = 0; i < b.nr; i++) { frac[3 * i] = f[4 * i]; frac[3 * i + 1] = f[4 * i + 1]; frac[3 * i + 2] = f[4 * i + 2]; }
-    }
+    if (frac && b.nr) HIPCHK(hipMemcpy(frac, w.slot_frac.p, sizeof(Frac3) * b.nr, hipMemcpyDeviceToHost));
     if (gdotr && b.nr) HIPCHK(hipMemcpy(gdotr, w.pt_gdotr.p, sizeof(double) * b.nr, hipMemcpyDeviceToHost));
     return D2BI_OK;
 }
@@ -392,6 +389,7 @@ int d2bi_gpu_lc_query(const double a[9], int32_t Nx, int32_t Ny, int32_t Nz, con
     BP.nuvw = 1;
     BP.Ex = Nx; BP.Ey = Ny; BP.Ez = Nz;
     BP.generic = 1;
+    BP.keep_ids = 1;
     BP.cell_a[0] = a[0]; BP.cell_a[1] = a[4]; BP.cell_a[2] = a[8];
     Binned b;
     CHK(run_binning(d_x, nP, BP, &b, s, g.ws));
@@ -415,7 +413,7 @@ int d2bi_gpu_lc_query(const double a[9], int32_t Nx, int32_t Ny, int32_t Nz, con
         if (e == hipSuccess) {
             hipLaunchKernelGGL(k_lc_query, dim3((unsigned)((nQ + 255) / 256)), dim3(256), 0, s, Q, nQ,
                                dq.as<double>(), w.cell_start.as<int>(), w.slot_id.as<int>(),
-                               w.slot_frac.as<double4>(), dn.as<int>(), did.as<int>(), dr2.as<double>());
+                               w.slot_frac.as<Frac3>(), dn.as<int>(), did.as<int>(), dr2.as<double>());
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipStreamSynchronize(s);

@@ -154,7 +154,7 @@ static int launch_voxel_fp64(const d2bi_plan* p, const AxisTables& tab, const Vo
     if (region_params(p, tab, V, &R)) {
         auto go = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(8 * R.per_xcd), dim3(64 * F64R_NW), 0, s, R, w.cell_start.as<int>(),
-                               w.slot_frac.as<double4>(), w.slot_p32.as<float4>(), cs, cs_stride, w.f64_re.as<double>(),
+                               w.slot_frac.as<Frac3>(), w.slot_p32.as<float4>(), cs, cs_stride, w.f64_re.as<double>(),
                                w.f64_im.as<double>(), out_stride, w.f64_rho.as<double>(), cnt, r2m);
         };
         const bool dens = V.use_density != 0;
@@ -168,7 +168,7 @@ static int launch_voxel_fp64(const d2bi_plan* p, const AxisTables& tab, const Vo
     } else {
         const dim3 grid((p->Mx + 7) / 8, (p->My + 7) / 8, (p->Mz + 3) / 4);
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, V, w.cell_start.as<int>(), w.slot_frac.as<double4>(), cs,
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, V, w.cell_start.as<int>(), w.slot_frac.as<Frac3>(), cs,
                                cs_stride, w.f64_re.as<double>(), w.f64_im.as<double>(), out_stride,
                                w.f64_rho.as<double>(), cnt, r2m);
         };
@@ -228,7 +228,7 @@ static void pick_tile(bool diag, bool dens, int variant, bool thin_z, Go go)
 
 template <bool DIAG>
 static void launch_tile(const FastParams& F, int variant, bool dens, const int* cell_start,
-                        const double4* slot_frac, const float4* p32, const float* sn32, float4* field, int* cnt,
+                        const Frac3* slot_frac, const float4* p32, const float* sn32, float4* field, int* cnt,
                         float* r2m, unsigned long long* gc, hipStream_t s)
 {
     pick_tile(DIAG, dens, variant, F.thin_z != 0, [&](auto kern) {
@@ -356,7 +356,7 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
         set_tile_order(&Fv, order);
         pick_tile(want_diag, dens, v, Fv.thin_z != 0, [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(8 * Fv.per_xcd), dim3(64), 0, s, Fv, w.cell_start.as<int>(),
-                               w.slot_frac.as<double4>(), w.slot_p32.as<float4>(),
+                               w.slot_frac.as<Frac3>(), w.slot_p32.as<float4>(),
                                w.slot_sn32.as<float>(), w.f32_field.as<float4>(), dcnt, (float*)dr2, gp);
         });
         return D2BI_OK;
@@ -380,7 +380,7 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
         order = tune_choose(tile_order_key(p, tab, dens, variant), "D2BI_TILE_ORDER", TILE_ORDERS, 3, 2, true, s,
                             [&](int o) { (void)run_variant(variant, o); });
     }
-    fill_i32((int*)gp, (int64_t)(gp_bytes / sizeof(int)), 0, s);   // tuning launches counted too
+    zero_i32(s, (int*)gp, (int64_t)(gp_bytes / sizeof(int)));   // tuning launches counted too
     if (T) CHK(T->record(2));
     CHK(run_variant(variant, order));
     HIPCHK(hipGetLastError());
@@ -661,10 +661,10 @@ static int run_voxel_apps(const d2bi_record* r, const d2bi_plan* p, const AxisTa
     const size_t gp_bytes = sizeof(unsigned long long) * GUARD_SLOTS * GUARD_STRIDE;
     CHK(w.guard_part.ensure(gp_bytes));
     unsigned long long* gp = w.guard_part.as<unsigned long long>();
-    fill_i32((int*)gp, (int64_t)(gp_bytes / sizeof(int)), 0, s);
+    zero_i32(s, (int*)gp, (int64_t)(gp_bytes / sizeof(int)));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(8 * F.per_xcd), dim3(64), 0, s, F, w.cell_start.as<int>(),
-                           w.slot_frac.as<double4>(), w.slot_p32.as<float4>(), w.slot_sn32.as<float>(),
+                           w.slot_frac.as<Frac3>(), w.slot_p32.as<float4>(), w.slot_sn32.as<float>(),
                            w.f32_field.as<float4>(), (int*)nullptr, (float*)nullptr, gp);
     };
     auto pick = [&](auto dens_c, auto row_c, auto na_c) {
@@ -753,7 +753,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
         return D2BI_OK;
     };
 
-    if (!aperture_shared() || (f64 && n > (int64_t)INT32_MAX)) {
+    if (!aperture_shared()) {
         // every point binned and voxelised on its own
         for (int app = 0; app < nApp; app++) {
             d2bi_plan pk = point_plan(app);
@@ -772,7 +772,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
         BinParams BP;
         CHK(bin_params(r, &p0, &BP));
         BP.fast = f64 ? 0 : 1;
-        BP.keep_j = f64 ? 1 : 0;
+        BP.keep_src = 1;
         Binned b;
         CHK(run_binning(d_x, n, BP, &b, s, w));
         const int64_t nr = b.nr;
@@ -783,7 +783,6 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
         variant = effective_variant(&plan, tab, variant);
         const int na_max = (f64 || variant == 1 || variant == 2) ? 4 : 1;
         if (na_max > 1) CHK(w.app_cs.ensure((f64 ? sizeof(double2) : sizeof(float2)) * std::max<int64_t>(nr, 1) * na_max));
-        const int nblk = (int)std::max<int64_t>(1, (n + BIN_TILE - 1) / BIN_TILE);
         for (int app = 0; app < nApp;) {
             const int left = nApp - app;
             const int na = na_max >= 4 && left >= 4 ? 4 : (na_max >= 2 && left >= 2 ? 2 : 1);
@@ -794,8 +793,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
                     for (int i = 0; i < 3; i++) G.g[a][i] = gshift[3 * (app + a) + i];
                 const dim3 grid((unsigned)((nr + 255) / 256));
                 auto go = [&](auto kern) {
-                    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, nr, w.cell_ids.as<int>(), w.pt_j.as<int>(), d_x,
-                                       BP, w.blk_off.as<int>(), nblk, G, nr,
+                    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, nr, w.slot_src.as<int2>(), d_x, BP, G, nr,
                                        na > 1 ? w.app_cs.as<double2>() : w.slot_cs64.as<double2>(),
                                        w.app_cs.as<float2>(), w.slot_p32.as<float4>(), w.slot_sn32.as<float>());
                 };

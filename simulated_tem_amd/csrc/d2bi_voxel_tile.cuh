@@ -106,7 +106,7 @@ struct FastParams {
 // that pass's to the bit.
 template <bool DENSITY, bool DIAG, int ROW, int TZ, int TX = 4, int NA = 1>
 __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __restrict__ cell_start,
-                                                   const double4* __restrict__ slot_frac,
+                                                   const Frac3* __restrict__ slot_frac,
                                                    const float4* __restrict__ p32,
                                                    const float* __restrict__ sn32,
                                                    float4* __restrict__ field,
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
     auto exact_at = [&](int lx, int vx, int u, int slot) -> bool {
         const int kx = (u & 255) - 1 - lx, ky = ((u >> 8) & 255) - 1 - lcy, kz = (u >> 16) - 1 - lcz;
         if (kx < -1 || kx > 1 || ky < -1 || ky > 1 || kz < -1 || kz > 1) return false;
-        const double4 f = slot_frac[slot];                              // FP64 offset in cell
+        const Frac3 f = slot_frac[slot];                              // FP64 offset in cell
         const double zix = P.ax.zi[0][vx], ziy = P.ax.zi[1][jy], ziz = P.ax.zi[2][jz];
         const double d1 = P.a[0] * (f.x + (kx - zix));
         const double d2 = P.a[1] * (f.y + (ky - ziy));

@@ -57,3 +57,25 @@ def test_fp64_field(grid, density):
     assert np.array_equal(r2m, or2m)
     assert np.max(np.abs(ph - oph)) < 1e-12
     assert np.max(np.abs(rho - orho)) < 1e-14
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 256, 257, 5000])
+def test_linkcells_counts(n):
+    """Binning at the edges of its workgroups (256 atoms), and of the scans:
+    the link cells of 5000 atoms in a box of 40 x 40 x 36 cells are more than
+    one workgroup scans alone (16,384), those of the small box fewer.  Cells,
+    order inside each, offsets and g.r bit for bit, and a crowded cell (every
+    atom of the last 60 within one) ranked by point number."""
+    for voxels in ((24, 20, 18), (240, 240, 216)):
+        cfg = synth.scaled("c0", cells=(7, 7, 7))
+        cfg.update(sg=[0.01], d=tuple(v * A0 / 4 for v in voxels))
+        box = np.array([v * A0 / 4 for v in voxels])
+        x = np.random.default_rng(n).random((n, 3)) * box
+        x[-60:] = 0.4 * box + 0.02 * (x[-60:] - x[-60:].mean(axis=0) if n else x[-60:])
+        x, conds = synth.conditions(cfg, x, box)
+        im = conds[0][0]
+        cs, ids, frac, gd = im.linkcells(x)
+        oc = orc.Condition(im.rec, x)
+        ocs, oids, ofrac = oc.cells()
+        assert np.array_equal(cs, ocs) and np.array_equal(ids, oids) and np.array_equal(frac, ofrac)
+        assert np.array_equal(gd, oc.gdotr())
