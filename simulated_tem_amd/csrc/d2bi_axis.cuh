@@ -36,6 +36,7 @@ struct AxisTables {
     std::vector<int> cell[3];
     std::vector<double> zi[3];
     std::vector<QL> ql[NQL];       // x, y, z for 4-voxel tiles; z, x for 8-voxel tiles
+    std::vector<char> packed;      // the tables as uploaded without pinned memory
 };
 
 static bool diagonal(const double* m)
@@ -83,63 +84,53 @@ struct AxisDev {
     const QL* ql[NQL];
 };
 
-// Copy the axis tables into workspace w.  t must stay alive until the
-// stream has executed the copies.
-static int upload_axis(const AxisTables& t, AxisDev* d, hipStream_t s, Workspace& w)
+// The axis tables of one condition as one block: doubles zi, then QL, then
+// ints cell.
+static size_t axis_bytes(const AxisTables& t)
 {
-    size_t nc = t.cell[0].size() + t.cell[1].size() + t.cell[2].size();
-    size_t nq = 0;
-    for (int k = 0; k < NQL; k++) nq += t.ql[k].size();
-    CHK(w.ax_cell.ensure(sizeof(int) * nc));
-    CHK(w.ax_zi.ensure(sizeof(double) * nc));
-    CHK(w.ax_ql.ensure(sizeof(QL) * nq));
-    if (w.ax_cell.arena) {
-        // a workspace that must not allocate: copy from the tables
-        // themselves, not through the (growable) pinned staging buffer
-        size_t oc = 0, oq = 0;
-        for (int k = 0; k < NQL; k++) {
-            d->ql[k] = w.ax_ql.as<QL>() + oq;
-            HIPCHK(hipMemcpyAsync((void*)d->ql[k], t.ql[k].data(), sizeof(QL) * t.ql[k].size(),
-                                  hipMemcpyHostToDevice, s));
-            oq += t.ql[k].size();
-        }
-        for (int a = 0; a < 3; a++) {
-            d->cell[a] = w.ax_cell.as<int>() + oc;
-            d->zi[a] = w.ax_zi.as<double>() + oc;
-            HIPCHK(hipMemcpyAsync((void*)d->cell[a], t.cell[a].data(), sizeof(int) * t.cell[a].size(),
-                                  hipMemcpyHostToDevice, s));
-            HIPCHK(hipMemcpyAsync((void*)d->zi[a], t.zi[a].data(), sizeof(double) * t.zi[a].size(),
-                                  hipMemcpyHostToDevice, s));
-            oc += t.cell[a].size();
-        }
-        return D2BI_OK;
+    size_t n = 0;
+    for (int k = 0; k < NQL; k++) n += sizeof(QL) * t.ql[k].size();
+    for (int a = 0; a < 3; a++) n += (sizeof(double) + sizeof(int)) * t.cell[a].size();
+    return (n + 15) & ~(size_t)15;
+}
+
+// Write the block into host memory h, and d's pointers for a block at dev.
+static void axis_pack(const AxisTables& t, char* h, const char* dev, AxisDev* d)
+{
+    size_t o = 0;
+    auto put = [&](const auto& v, auto* ptr) {
+        const size_t bytes = sizeof(v[0]) * v.size();
+        std::memcpy(h + o, v.data(), bytes);
+        *ptr = reinterpret_cast<std::remove_reference_t<decltype(*ptr)>>(dev + o);
+        o += bytes;
+    };
+    for (int a = 0; a < 3; a++) put(t.zi[a], &d->zi[a]);
+    for (int k = 0; k < NQL; k++) put(t.ql[k], &d->ql[k]);
+    for (int a = 0; a < 3; a++) put(t.cell[a], &d->cell[a]);
+}
+
+// Copy the axis tables into workspace w.  t must stay alive until the
+// stream has executed the copy.
+static int upload_axis(AxisTables& t, AxisDev* d, hipStream_t s, Workspace& w)
+{
+    const size_t bytes = axis_bytes(t);
+    CHK(w.ax_tab.ensure(bytes));
+    void* h;
+    if (w.ax_tab.arena) {
+        // a workspace that must not allocate: copy from pageable memory, not
+        // through the (growable) pinned staging buffer
+        t.packed.resize(bytes);
+        h = t.packed.data();
+    } else {
+        CHK(pinned(bytes, &h));
     }
-    size_t bytes = sizeof(int) * nc + sizeof(double) * nc + sizeof(QL) * nq;
-    void* hp;
-    CHK(pinned(bytes, &hp));
-    char* h = (char*)hp;
-    double* hz = (double*)h;
-    QL* hq = (QL*)(h + sizeof(double) * nc);
-    int* hc = (int*)(h + sizeof(double) * nc + sizeof(QL) * nq);
-    size_t oc = 0, oq = 0;
-    for (int k = 0; k < NQL; k++) {
-        std::memcpy(hq + oq, t.ql[k].data(), sizeof(QL) * t.ql[k].size());
-        d->ql[k] = w.ax_ql.as<QL>() + oq;
-        oq += t.ql[k].size();
+    axis_pack(t, (char*)h, w.ax_tab.as<char>(), d);
+    HIPCHK(hipMemcpyAsync(w.ax_tab.p, h, bytes, hipMemcpyHostToDevice, s));
+    if (!w.ax_tab.arena) {
+        // the pinned buffer is reused by later calls: they wait for this event
+        HIPCHK(hipEventRecord(g.ev[9], s));
+        g.pinned_busy = true;
     }
-    for (int a = 0; a < 3; a++) {
-        std::memcpy(hc + oc, t.cell[a].data(), sizeof(int) * t.cell[a].size());
-        std::memcpy(hz + oc, t.zi[a].data(), sizeof(double) * t.zi[a].size());
-        d->cell[a] = w.ax_cell.as<int>() + oc;
-        d->zi[a] = w.ax_zi.as<double>() + oc;
-        oc += t.cell[a].size();
-    }
-    HIPCHK(hipMemcpyAsync(w.ax_cell.p, hc, sizeof(int) * nc, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(w.ax_zi.p, hz, sizeof(double) * nc, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(w.ax_ql.p, hq, sizeof(QL) * nq, hipMemcpyHostToDevice, s));
-    // the pinned buffer is reused by later calls: they wait for this event
-    HIPCHK(hipEventRecord(g.ev[9], s));
-    g.pinned_busy = true;
     return D2BI_OK;
 }
 

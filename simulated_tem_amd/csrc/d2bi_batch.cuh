@@ -1,4 +1,5 @@
-// d2bi_batch.cuh -- batched conditions, executed as one captured HIP graph per batch.
+// d2bi_batch.cuh -- batched conditions on concurrent branches: launched as they
+// are the first time, captured into one HIP graph when the batch comes again.
 //
 // One part of the single translation unit d2bi_gpu.hip, which includes the
 // parts in order so that kernels and the device helpers they call compile
@@ -19,24 +20,25 @@ struct Cond {
     int nblk = 0, ncell = 0, variant = 0;
     bool dens = false;
     int64_t nr = 0, nbc = 0, nvox = 0, plane = 0;
-    int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axq = 0, o_img = 0;
+    int64_t o_mask = 0, o_blk = 0, o_scan = 0, o_img = 0;
+    size_t o_ax = 0;
     AxisDev ax;
 };
 
-// Conditions of a batch run on up to MAX_BRANCH concurrent branches of the
-// graph, each a chain of conditions on its own stream and workspace (branch 0
+// Conditions of a batch run on up to MAX_BRANCH concurrent branches, each a
+// chain of conditions on its own stream and workspace (branch 0
 // on the library's stream and workspace), so that small conditions fill the
 // GPU together.  A condition's arithmetic does not depend on its branch.
 static constexpr int MAX_BRANCH = 4;
 
 struct Batch {
-    Buf mask, blkcnt, blkoff, axc, axz, axq, img, guard, mpc;
+    Buf mask, blkcnt, blkoff, scan, ax, img, counters, tot;
     std::vector<unsigned char> key;
     uint64_t gen = 0;
-    hipGraphExec_t exec = nullptr;
-    std::vector<int64_t> nr;
+    std::vector<Cond> conds;                    // the planned conditions of key
+    hipGraphExec_t exec = nullptr;              // their graph, from the second call on
     int64_t total_plane = 0;
-    int nbr = 1;                                // branches of the captured graph
+    int nbr = 1;                                // branches the conditions run on
     int64_t branch_bytes = 0;                   // device bytes of one branch's workspace
     Workspace ws[MAX_BRANCH - 1];               // branches 1..MAX_BRANCH-1
     hipStream_t stream[MAX_BRANCH - 1] = {};
@@ -46,11 +48,12 @@ struct Batch {
         if (exec) (void)hipGraphExecDestroy(exec);
         exec = nullptr;
         key.clear();
+        conds.clear();
     }
     void release()
     {
         reset();
-        Buf* all[] = {&mask, &blkcnt, &blkoff, &axc, &axz, &axq, &img, &guard, &mpc};
+        Buf* all[] = {&mask, &blkcnt, &blkoff, &scan, &ax, &img, &counters, &tot};
         for (Buf* b : all) b->release();
         for (int k = 0; k < MAX_BRANCH - 1; k++) {
             ws[k].release_all();
@@ -84,8 +87,9 @@ static void key_append(std::vector<unsigned char>& k, const void* p, size_t n)
     k.insert(k.end(), c, c + n);
 }
 
-// counting pass of one condition: replica predicate and per-block offsets
-static int enqueue_count(const Cond& c, Batch& B, int* scan_tmp, hipStream_t s)
+// counting pass of one condition: replica predicate, per-block offsets, and
+// the number of points in the batch's totals
+static int enqueue_count(const Cond& c, int idx, Batch& B, hipStream_t s)
 {
     uint32_t* mask = B.mask.as<uint32_t>() + c.o_mask;
     int* cnt = B.blkcnt.as<int>() + c.o_blk;
@@ -95,22 +99,19 @@ static int enqueue_count(const Cond& c, Batch& B, int* scan_tmp, hipStream_t s)
     else
         zero_i32(s, cnt, c.nbc);
     HIPCHK(hipGetLastError());
-    return scan_exclusive_tmp(cnt, off, c.nbc, scan_tmp, s);
+    return scan_exclusive_tmp(cnt, off, c.nbc, B.scan.as<int>() + c.o_scan, s,
+                              ScanEnds{B.tot.as<int>() + idx, nullptr, nullptr, 0});
 }
 
 // the rest of one condition: bin, voxelise, integrate into its image slice,
 // on workspace w
 static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w, hipStream_t s)
 {
-    int* scan_tmp = w.scan_tmp.as<int>();
     const d2bi_plan* p = &c.plan;
-    int* mpc = B.mpc.as<int>() + idx;
-    unsigned long long* gc = B.guard.as<unsigned long long>() + idx;
-    unsigned long long* gp = w.guard_part.as<unsigned long long>();
-    zero_i32(s, w.cell_cnt.as<int>(), c.ncell + 1, mpc, 1, (int*)gc, 2, (int*)gp,
-             mode == D2BI_MODE_FAST ? 2 * GUARD_SLOTS * GUARD_STRIDE : 0);
+    Counters* ct = B.counters.as<Counters>() + idx;
+    zero_i32(s, w.cell_cnt.as<int>(), c.ncell + 1, (int*)ct, sizeof(Counters) / sizeof(int));
     CHK(launch_bin_points(c.d_x, c.BP, B.mask.as<uint32_t>() + c.o_mask, B.blkoff.as<int>() + c.o_blk, c.nblk, c.ncell,
-                          c.nr, scan_tmp, mpc, s, w));
+                          PointCount{B.tot.as<int>() + idx, c.nr}, w.scan_tmp.as<int>(), &ct->max_per_cell, s, w));
     VoxParams V;
     d2bi_record dummy;
     dummy.use_density = c.dens ? 1 : 0;
@@ -128,9 +129,8 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w
                                    2, false, s, [](int) {}));
     launch_tile<false>(F, variant, c.dens, w.cell_start.as<int>(), w.slot_frac.as<Frac3>(),
                        w.slot_p32.as<float4>(), w.slot_sn32.as<float>(), w.f32_field.as<float4>(), nullptr, nullptr,
-                       gp, s);
+                       ct->guard, s);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_sum_guard, dim3(1), dim3(256), 0, s, gp, GUARD_SLOTS, GUARD_STRIDE, gc);
     return launch_integrate_fast(p, c.dens, w.f32_field.p, d_img, s);
 }
 
@@ -144,14 +144,8 @@ struct BranchSizes {
 template <class F>
 static void branch_buffers(Workspace& w, const BranchSizes& z, F f)
 {
-    f(w.pt_cell, sizeof(int) * z.max_nr);
-    f(w.pt_slot, sizeof(int) * z.max_nr);
-    f(w.pt_j, sizeof(int) * z.max_nr);
-    f(w.cell_ids, sizeof(int) * z.max_nr);
-    f(w.slot_frac, sizeof(Frac3) * z.max_nr);
-    f(w.slot_p32, sizeof(float4) * z.max_nr);
-    if (z.mode == D2BI_MODE_FP64) f(w.slot_cs64, sizeof(double2) * z.max_nr);
-    else f(w.slot_sn32, sizeof(float) * z.max_nr);
+    point_buffers(w, z.mode == D2BI_MODE_FAST, false, false, false,
+                  [&](Buf& b, size_t bytes) { f(b, bytes * z.max_nr); });
     f(w.cell_cnt, sizeof(int) * z.max_cell);
     f(w.cell_start, sizeof(int) * z.max_cell);
     if (z.mode == D2BI_MODE_FP64) {
@@ -161,7 +155,6 @@ static void branch_buffers(Workspace& w, const BranchSizes& z, F f)
     } else {
         f(w.f32_field, sizeof(float4) * z.max_vox);
     }
-    f(w.guard_part, sizeof(unsigned long long) * GUARD_SLOTS * GUARD_STRIDE);
     f(w.scan_tmp, sizeof(int) * z.max_scan);
 }
 
@@ -182,12 +175,248 @@ static int64_t branch_bytes(const BranchSizes& z)
     return n;
 }
 
-// Batched conditions.  The first call with a given set of inputs plans every
-// condition, counts the points of each (one host synchronisation for the
-// sizes), sizes the workspace for the largest, and captures the whole batch
-// (counting, binning, voxelisation, integration of every condition) into one
-// HIP graph.  Later calls with the same inputs and an unchanged workspace
-// replay the graph: every replay recomputes everything from the atoms.
+// The batch of B.conds on nb branches, launched on the library's stream and
+// the branch streams (or captured from them): conditions to branches largest
+// first, each to the least loaded branch (a fixed rule: the same inputs give
+// the same assignment).  count: the counting passes too.
+static int enqueue_batch(Batch& B, int mode, int nb, bool count)
+{
+    const std::vector<Cond>& C = B.conds;
+    const int nRec = (int)C.size();
+    hipStream_t s = g.stream;
+    std::vector<int> order(nRec), branch(nRec, 0);
+    for (int i = 0; i < nRec; i++) order[i] = i;
+    auto work = [&](int i) { return (double)C[i].nvox * (1.0 + C[i].plan.nPrec / 8.0) + 8.0 * C[i].n; };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work(a) > work(b); });
+    std::vector<double> load(nb, 0.0);
+    for (int i : order) {
+        int k = 0;
+        for (int j = 1; j < nb; j++)
+            if (load[j] < load[k]) k = j;
+        branch[i] = k;
+        load[k] += work(i);
+    }
+    int rc = D2BI_OK;
+    auto bstream = [&](int k) { return k == 0 ? s : B.stream[k - 1]; };
+    if (nb > 1) {
+        if (hipEventRecord(B.fork, s) != hipSuccess) rc = seterr(D2BI_ERR_HIP, "batch fork failed");
+        for (int k = 1; k < nb && rc == D2BI_OK; k++)
+            if (hipStreamWaitEvent(bstream(k), B.fork, 0) != hipSuccess)
+                rc = seterr(D2BI_ERR_HIP, "batch fork failed");
+    }
+    for (int i = 0; i < nRec && rc == D2BI_OK; i++) {
+        if (count) rc = enqueue_count(C[i], i, B, bstream(branch[i]));
+        if (rc == D2BI_OK) rc = enqueue_rest(C[i], i, B, mode, B.branch_ws(branch[i]), bstream(branch[i]));
+    }
+    // join every branch back, also after an error, so that a capture can end
+    for (int k = 1; k < nb; k++)
+        if (hipEventRecord(B.join[k - 1], bstream(k)) != hipSuccess ||
+            hipStreamWaitEvent(s, B.join[k - 1], 0) != hipSuccess)
+            if (rc == D2BI_OK) rc = seterr(D2BI_ERR_HIP, "batch join failed");
+    return rc;
+}
+
+// Capture the batch (counting passes included) into B.exec.
+static int capture_batch(Batch& B, int mode)
+{
+    hipStream_t s = g.stream;
+    hipGraph_t graph;
+    g_capturing = true;
+    if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
+        g_capturing = false;
+        return seterr(D2BI_ERR_HIP, "graph capture failed to begin");
+    }
+    const int rc = enqueue_batch(B, mode, B.nbr, true);
+    hipError_t e = hipStreamEndCapture(s, &graph);
+    g_capturing = false;
+    if (rc != D2BI_OK) {
+        if (e == hipSuccess) (void)hipGraphDestroy(graph);
+        return rc;
+    }
+    if (e != hipSuccess) return seterr(D2BI_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
+    e = hipGraphInstantiate(&B.exec, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    if (e != hipSuccess) {
+        B.exec = nullptr;
+        return seterr(D2BI_ERR_HIP, "graph instantiation failed: %s", hipGetErrorString(e));
+    }
+    return D2BI_OK;
+}
+
+// Plan a batch's conditions, count their points (one host synchronisation for
+// the sizes), size the workspaces and image every condition, leaving the
+// images in B.img.  Launch choices not yet timed for a shape are timed here.
+static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms, int nRec, const double* precAngle,
+                     const int32_t* nPrec, int mode)
+{
+    hipStream_t s = g.stream;
+    std::vector<Cond>& C = B.conds;
+    C.assign(nRec, Cond());
+    int64_t o_mask = 0, o_blk = 0, o_scan = 0, o_img = 0;
+    size_t o_ax = 0;
+    int64_t max_scan = 1;
+    for (int i = 0; i < nRec; i++) {
+        Cond& c = C[i];
+        CHK(plan_image(&recs[i], atoms[i]->n, precAngle[i], nPrec[i], &c.plan));
+        CHK(axis_tables(&recs[i], &c.plan, &c.tab));
+        CHK(bin_params(&recs[i], &c.plan, &c.BP));
+        c.BP.fast = mode == D2BI_MODE_FAST ? 1 : 0;
+        c.d_x = atoms[i]->x;
+        c.n = atoms[i]->n;
+        c.BP.n = c.n;
+        c.nblk = bin_blocks(c.n);
+        c.nbc = (int64_t)c.BP.nuvw * c.nblk;
+        c.ncell = c.plan.Ex * c.plan.Ey * c.plan.Ez;
+        c.dens = recs[i].use_density != 0;
+        c.plane = (int64_t)c.plan.Mx * c.plan.My;
+        c.nvox = c.plane * c.plan.Mz;
+        c.o_mask = o_mask; o_mask += std::max<int64_t>(c.n, 1);
+        c.o_blk = o_blk; o_blk += c.nbc + 1;
+        c.o_scan = o_scan; o_scan += scan_tmp_ints(c.nbc);
+        c.o_ax = o_ax; o_ax += axis_bytes(c.tab);
+        c.o_img = o_img; o_img += c.plane;
+        max_scan = std::max(max_scan, scan_tmp_ints(c.ncell));
+    }
+    CHK(B.mask.ensure(sizeof(uint32_t) * o_mask));
+    CHK(B.blkcnt.ensure(sizeof(int) * o_blk));
+    CHK(B.blkoff.ensure(sizeof(int) * o_blk));
+    CHK(B.scan.ensure(sizeof(int) * o_scan));
+    CHK(B.ax.ensure(o_ax));
+    CHK(B.img.ensure(sizeof(double) * o_img));
+    CHK(B.counters.ensure(sizeof(Counters) * nRec));
+    CHK(B.tot.ensure(sizeof(int) * nRec));
+    B.total_plane = o_img;
+    // branch streams and the events that fork and join them (default priority)
+    int nbr = std::min(batch_branches(), nRec);
+    if (!B.fork) HIPCHK(hipEventCreateWithFlags(&B.fork, hipEventDisableTiming));
+    for (int k = 1; k < nbr; k++) {
+        if (!B.stream[k - 1]) HIPCHK(hipStreamCreateWithFlags(&B.stream[k - 1], hipStreamNonBlocking));
+        if (!B.join[k - 1]) HIPCHK(hipEventCreateWithFlags(&B.join[k - 1], hipEventDisableTiming));
+    }
+    // counting passes, dealt to the branch streams; the tables go up meanwhile
+    HIPCHK(hipEventRecord(B.fork, s));
+    for (int k = 1; k < nbr; k++) HIPCHK(hipStreamWaitEvent(B.stream[k - 1], B.fork, 0));
+    int rc = D2BI_OK;
+    for (int i = 0; i < nRec && rc == D2BI_OK; i++)
+        rc = enqueue_count(C[i], i, B, i % nbr == 0 ? s : B.stream[i % nbr - 1]);
+    for (int k = 1; k < nbr; k++) {
+        HIPCHK(hipEventRecord(B.join[k - 1], B.stream[k - 1]));
+        HIPCHK(hipStreamWaitEvent(s, B.join[k - 1], 0));
+    }
+    CHK(rc);
+    void* hp;
+    CHK(pinned(o_ax, &hp));
+    for (int i = 0; i < nRec; i++) axis_pack(C[i].tab, (char*)hp + C[i].o_ax, B.ax.as<char>() + C[i].o_ax, &C[i].ax);
+    HIPCHK(hipMemcpyAsync(B.ax.p, hp, o_ax, hipMemcpyHostToDevice, s));
+    void* hr;
+    CHK(pinned_result(sizeof(int) * nRec, &hr));
+    const int* tot = (const int*)hr;
+    HIPCHK(hipMemcpyAsync(hr, B.tot.p, sizeof(int) * nRec, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    int64_t max_nr = 1, max_cell = 1, max_vox = 1;
+    for (int i = 0; i < nRec; i++) {
+        if (tot[i] < 0) return seterr(D2BI_ERR_CAPACITY, "point count overflow");
+        C[i].nr = tot[i];
+        max_nr = std::max(max_nr, C[i].nr);
+        max_cell = std::max<int64_t>(max_cell, C[i].ncell + 1);
+        max_vox = std::max(max_vox, C[i].nvox);
+    }
+    const BranchSizes bz{mode, max_nr, max_cell, max_vox, max_scan};
+    // every branch gets a workspace sized for the largest condition; the
+    // branches beyond the first run only where what their workspaces
+    // would add (branch 0's growth included) fits in 85 % of the free
+    // device memory, so that a batch one workspace can hold does not
+    // fail for want of four
+    if (nbr > 1) {
+        size_t freeb = 0, totalb = 0;
+        const char* e = std::getenv("D2BI_BATCH_MEM");         // free bytes to assume (tests)
+        if (e && *e) freeb = (size_t)std::strtoull(e, nullptr, 10);
+        else if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) {
+            (void)hipGetLastError();
+            freeb = 0;
+        }
+        const double room = 0.85 * (double)freeb;
+        double used = branch_growth(B.branch_ws(0), bz);
+        int fit = 1;
+        for (int k = 1; k < nbr; k++) {
+            used += branch_growth(B.branch_ws(k), bz);
+            if (used > room) break;
+            fit = k + 1;
+        }
+        nbr = fit;
+    }
+    for (int k = 0; k < nbr; k++) {
+        int rc_ = D2BI_OK;
+        branch_buffers(B.branch_ws(k), bz, [&](Buf& b, size_t bytes) {
+            if (rc_ == D2BI_OK) rc_ = b.ensure(bytes);
+        });
+        CHK(rc_);
+    }
+    B.branch_bytes = branch_bytes(bz);
+    // FAST kernel variants (fixed, forced, or with D2BI_FAST_TUNE=1 tuned
+    // for unseen shapes), and the launch choices of shapes the tuner has not
+    // timed yet: one condition of each such shape, on its own, times them
+    for (int i = 0; i < nRec && mode == D2BI_MODE_FAST; i++) {
+        int v = known_variant(&C[i].plan, C[i].dens);
+        if (v < 0 || !condition_tuned(&C[i].plan, C[i].tab, C[i].dens, v)) {
+            d2bi_plan tmp;
+            CHK(image_condition(&recs[i], C[i].d_x, C[i].n, precAngle[i], nPrec[i], mode, nullptr, &tmp, g.ws));
+            v = known_variant(&C[i].plan, C[i].dens);
+            if (v < 0) v = 0;
+        }
+        C[i].variant = v;
+    }
+    // branch count: forced, cached, or tuned by timing a run on each count
+    // (images are the same on any count); the count that fits is kept unless
+    // another is 3 % faster
+    int chosen = nbr;
+    bool done = false;
+    HIPCHK(hipEventRecord(g.ev[0], s));
+    if (nbr > 1 && !std::getenv("D2BI_BATCH_BRANCHES") && tuning_on()) {
+        int64_t sum_vox = 0, max_vox_c = 0, sum_n = 0, sum_p = 0;
+        for (int i = 0; i < nRec; i++) {
+            sum_vox += C[i].nvox;
+            max_vox_c = std::max(max_vox_c, C[i].nvox);
+            sum_n += C[i].n;
+            sum_p += C[i].plan.nPrec;
+        }
+        const TuneKey bkey{TUNE_BRANCHES, nRec, mode, sum_vox, max_vox_c, sum_n, sum_p, nbr, 0};
+        const int c = tune_get(bkey);
+        if (c >= 1 && c <= nbr) {
+            chosen = c;
+        } else {
+            float tbest = 3.4e38f;
+            for (int q = 0; q < nbr; q++) {
+                const int nb = q == 0 ? nbr : q;            // the default first
+                int rq = D2BI_OK;
+                const float t = time_launch([&] { rq = enqueue_batch(B, mode, nb, false); }, s, 1);
+                CHK(rq);
+                if (q == 0) tbest = t >= 0.0f ? 0.97f * t : 3.4e38f;
+                else if (t >= 0.0f && t < tbest) {
+                    tbest = t;
+                    chosen = nb;
+                }
+            }
+            tune_put(bkey, chosen);
+            done = true;                                    // each run imaged every condition
+        }
+    }
+    if (!done) CHK(enqueue_batch(B, mode, chosen, false));
+    // workspaces of branches that are not used go back to the device
+    HIPCHK(hipStreamSynchronize(s));
+    for (int k = std::max(1, chosen); k < nbr; k++) B.branch_ws(k).release_all();
+    B.nbr = chosen;
+    return D2BI_OK;
+}
+
+// Batched conditions.  New inputs (records, atom uploads, precession) are
+// planned, counted and imaged with plain launches on the branches; when the
+// next call brings the same inputs and the workspaces are unchanged, the whole
+// batch (counting, binning, voxelisation, integration of every condition) is
+// captured into one HIP graph, which that call and later ones replay: every
+// replay recomputes everything from the atoms.  A batch that comes once, as
+// the frames of a series do, does not pay for a graph (capture and
+// instantiation took 0.6 ms of 2.4 for eight conditions of 1e4 to 4e5 atoms).
 // img_out: host memory, or device memory when dev_out.
 static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec, const double* precAngle,
                      const int32_t* nPrec, int mode, double* img_out, bool dev_out, d2bi_stats* st)
@@ -203,267 +432,46 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
     key_append(key, &nb, sizeof nb);
     for (int i = 0; i < nRec; i++) {
         key_append(key, &recs[i], sizeof(d2bi_record));
-        // the graph holds each set's point counts: key on the upload, not on
+        // the plan holds each set's point counts: key on the upload, not on
         // addresses that a later upload may reuse
         key_append(key, &atoms[i]->serial, sizeof(uint64_t));
         key_append(key, &atoms[i]->n, sizeof(int64_t));
         key_append(key, &precAngle[i], sizeof(double));
         key_append(key, &nPrec[i], sizeof(int32_t));
     }
-    const bool replay = B.exec && key == B.key && B.gen == g_alloc_gen;
-    if (!replay) {
+    if (B.conds.empty() || key != B.key || B.gen != g_alloc_gen) {
         B.reset();
-        std::vector<Cond> C(nRec);
-        int64_t o_mask = 0, o_blk = 0, o_ax = 0, o_axq = 0, o_img = 0;
-        int64_t max_scan = 1;
-        for (int i = 0; i < nRec; i++) {
-            Cond& c = C[i];
-            CHK(plan_image(&recs[i], atoms[i]->n, precAngle[i], nPrec[i], &c.plan));
-            CHK(axis_tables(&recs[i], &c.plan, &c.tab));
-            CHK(bin_params(&recs[i], &c.plan, &c.BP));
-            c.BP.fast = mode == D2BI_MODE_FAST ? 1 : 0;
-            c.d_x = atoms[i]->x;
-            c.n = atoms[i]->n;
-            c.BP.n = c.n;
-            c.nblk = bin_blocks(c.n);
-            c.nbc = (int64_t)c.BP.nuvw * c.nblk;
-            c.ncell = c.plan.Ex * c.plan.Ey * c.plan.Ez;
-            c.dens = recs[i].use_density != 0;
-            c.plane = (int64_t)c.plan.Mx * c.plan.My;
-            c.nvox = c.plane * c.plan.Mz;
-            c.o_mask = o_mask; o_mask += std::max<int64_t>(c.n, 1);
-            c.o_blk = o_blk; o_blk += c.nbc + 1;
-            c.o_ax = o_ax; o_ax += c.plan.Mx + c.plan.My + c.plan.Mz;
-            c.o_axq = o_axq; o_axq += 2 * (int64_t)c.plan.Mx + c.plan.My + 2 * (int64_t)c.plan.Mz;
-            c.o_img = o_img; o_img += c.plane;
-            max_scan = std::max(max_scan, std::max(scan_tmp_ints(c.nbc), scan_tmp_ints(c.ncell)));
+        const int rc = first_run(B, recs, atoms, nRec, precAngle, nPrec, mode);
+        if (rc != D2BI_OK) {
+            // nothing of the batch may run on: its inputs belong to the caller
+            (void)hipStreamSynchronize(s);
+            for (auto& bs : B.stream)
+                if (bs) (void)hipStreamSynchronize(bs);
+            B.reset();
+            return rc;
         }
-        CHK(B.mask.ensure(sizeof(uint32_t) * o_mask));
-        CHK(B.blkcnt.ensure(sizeof(int) * o_blk));
-        CHK(B.blkoff.ensure(sizeof(int) * o_blk));
-        CHK(B.axc.ensure(sizeof(int) * o_ax));
-        CHK(B.axz.ensure(sizeof(double) * o_ax));
-        CHK(B.axq.ensure(sizeof(QL) * o_axq));
-        CHK(B.img.ensure(sizeof(double) * o_img));
-        CHK(B.guard.ensure(sizeof(unsigned long long) * nRec));
-        CHK(B.mpc.ensure(sizeof(int) * nRec));
-        CHK(g.ws.scan_tmp.ensure(sizeof(int) * max_scan));       // the eager counting pass
-        // tables stay resident in the batch buffers
-        {
-            std::vector<int> hc(o_ax);
-            std::vector<double> hz(o_ax);
-            std::vector<QL> hq(o_axq);
-            for (int i = 0; i < nRec; i++) {
-                Cond& c = C[i];
-                int64_t oc = c.o_ax, oq = c.o_axq;
-                for (int k = 0; k < NQL; k++) {
-                    std::copy(c.tab.ql[k].begin(), c.tab.ql[k].end(), hq.begin() + oq);
-                    c.ax.ql[k] = B.axq.as<QL>() + oq;
-                    oq += (int64_t)c.tab.ql[k].size();
-                }
-                for (int a = 0; a < 3; a++) {
-                    std::copy(c.tab.cell[a].begin(), c.tab.cell[a].end(), hc.begin() + oc);
-                    std::copy(c.tab.zi[a].begin(), c.tab.zi[a].end(), hz.begin() + oc);
-                    c.ax.cell[a] = B.axc.as<int>() + oc;
-                    c.ax.zi[a] = B.axz.as<double>() + oc;
-                    oc += (int64_t)c.tab.cell[a].size();
-                }
-            }
-            HIPCHK(hipMemcpy(B.axc.p, hc.data(), sizeof(int) * o_ax, hipMemcpyHostToDevice));
-            HIPCHK(hipMemcpy(B.axz.p, hz.data(), sizeof(double) * o_ax, hipMemcpyHostToDevice));
-            HIPCHK(hipMemcpy(B.axq.p, hq.data(), sizeof(QL) * o_axq, hipMemcpyHostToDevice));
-        }
-        // counting pass: sizes of every condition
-        int* scan_tmp = g.ws.scan_tmp.as<int>();
-        for (int i = 0; i < nRec; i++) CHK(enqueue_count(C[i], B, scan_tmp, s));
-        std::vector<int> tot(nRec);
-        for (int i = 0; i < nRec; i++)
-            HIPCHK(hipMemcpyAsync(&tot[i], B.blkoff.as<int>() + C[i].o_blk + C[i].nbc, sizeof(int),
-                                  hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        int64_t max_nr = 1, max_cell = 1, max_vox = 1;
-        for (int i = 0; i < nRec; i++) {
-            if (tot[i] < 0) return seterr(D2BI_ERR_CAPACITY, "point count overflow");
-            C[i].nr = tot[i];
-            max_nr = std::max(max_nr, C[i].nr);
-            max_cell = std::max<int64_t>(max_cell, C[i].ncell + 1);
-            max_vox = std::max(max_vox, C[i].nvox);
-        }
-        int nbr = std::min(batch_branches(), nRec);
-        const BranchSizes bz{mode, max_nr, max_cell, max_vox, max_scan};
-        // every branch gets a workspace sized for the largest condition; the
-        // branches beyond the first run only where what their workspaces
-        // would add (branch 0's growth included) fits in 85 % of the free
-        // device memory, so that a batch one workspace can hold does not
-        // fail for want of four
-        if (nbr > 1) {
-            size_t freeb = 0, totalb = 0;
-            const char* e = std::getenv("D2BI_BATCH_MEM");         // free bytes to assume (tests)
-            if (e && *e) freeb = (size_t)std::strtoull(e, nullptr, 10);
-            else if (hipMemGetInfo(&freeb, &totalb) != hipSuccess) {
-                (void)hipGetLastError();
-                freeb = 0;
-            }
-            const double room = 0.85 * (double)freeb;
-            double used = branch_growth(B.branch_ws(0), bz);
-            int fit = 1;
-            for (int k = 1; k < nbr; k++) {
-                used += branch_growth(B.branch_ws(k), bz);
-                if (used > room) break;
-                fit = k + 1;
-            }
-            nbr = fit;
-        }
-        for (int k = 0; k < nbr; k++) {
-            int rc_ = D2BI_OK;
-            branch_buffers(B.branch_ws(k), bz, [&](Buf& b, size_t bytes) {
-                if (rc_ == D2BI_OK) rc_ = b.ensure(bytes);
-            });
-            CHK(rc_);
-        }
-        B.nbr = nbr;
-        B.branch_bytes = branch_bytes(bz);
-        // branch streams and the events that fork and join them in the graph
-        // (default priority)
-        if (!B.fork) HIPCHK(hipEventCreateWithFlags(&B.fork, hipEventDisableTiming));
-        for (int k = 1; k < nbr; k++) {
-            if (!B.stream[k - 1]) HIPCHK(hipStreamCreateWithFlags(&B.stream[k - 1], hipStreamNonBlocking));
-            if (!B.join[k - 1]) HIPCHK(hipEventCreateWithFlags(&B.join[k - 1], hipEventDisableTiming));
-        }
-        // FAST kernel variants (fixed, forced, or with D2BI_FAST_TUNE=1 tuned
-        // eagerly for unseen shapes, outside the graph), and the launch
-        // choices of shapes the tuner has not timed yet: one eager condition
-        // of each such shape times them (nothing is timed inside the graph)
-        for (int i = 0; i < nRec && mode == D2BI_MODE_FAST; i++) {
-            int v = known_variant(&C[i].plan, C[i].dens);
-            if (v < 0 || !condition_tuned(&C[i].plan, C[i].tab, C[i].dens, v)) {
-                d2bi_plan tmp;
-                CHK(image_condition(&recs[i], C[i].d_x, C[i].n, precAngle[i], nPrec[i], mode, nullptr, &tmp,
-                                    g.ws));
-                v = known_variant(&C[i].plan, C[i].dens);
-                if (v < 0) v = 0;
-            }
-            C[i].variant = v;
-        }
-        // capture the batch on nb branches: conditions to branches largest
-        // first, each to the least loaded branch (a fixed rule: the same
-        // inputs give the same graph); eager tuning may have grown workspace
-        // buffers, so this comes after it
-        auto capture = [&](int nb, hipGraphExec_t* exec) -> int {
-            std::vector<int> order(nRec), branch(nRec, 0);
-            for (int i = 0; i < nRec; i++) order[i] = i;
-            auto work = [&](int i) { return (double)C[i].nvox * (1.0 + C[i].plan.nPrec / 8.0) + 8.0 * C[i].n; };
-            std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return work(a) > work(b); });
-            std::vector<double> load(nb, 0.0);
-            for (int i : order) {
-                int k = 0;
-                for (int j = 1; j < nb; j++)
-                    if (load[j] < load[k]) k = j;
-                branch[i] = k;
-                load[k] += work(i);
-            }
-            hipGraph_t graph;
-            g_capturing = true;
-            if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-                g_capturing = false;
-                return seterr(D2BI_ERR_HIP, "graph capture failed to begin");
-            }
-            int rc = D2BI_OK;
-            auto bstream = [&](int k) { return k == 0 ? s : B.stream[k - 1]; };
-            if (nb > 1) {
-                if (hipEventRecord(B.fork, s) != hipSuccess) rc = seterr(D2BI_ERR_HIP, "graph fork failed");
-                for (int k = 1; k < nb && rc == D2BI_OK; k++)
-                    if (hipStreamWaitEvent(bstream(k), B.fork, 0) != hipSuccess)
-                        rc = seterr(D2BI_ERR_HIP, "graph fork failed");
-            }
-            for (int i = 0; i < nRec && rc == D2BI_OK; i++) {
-                Workspace& w = B.branch_ws(branch[i]);
-                rc = enqueue_count(C[i], B, w.scan_tmp.as<int>(), bstream(branch[i]));
-                if (rc == D2BI_OK) rc = enqueue_rest(C[i], i, B, mode, w, bstream(branch[i]));
-            }
-            for (int k = 1; k < nb; k++) {
-                // join every branch back, also after an error, so the capture can end
-                if (hipEventRecord(B.join[k - 1], bstream(k)) != hipSuccess ||
-                    hipStreamWaitEvent(s, B.join[k - 1], 0) != hipSuccess)
-                    if (rc == D2BI_OK) rc = seterr(D2BI_ERR_HIP, "graph join failed");
-            }
-            hipError_t e = hipStreamEndCapture(s, &graph);
-            g_capturing = false;
-            if (rc != D2BI_OK) {
-                if (e == hipSuccess) (void)hipGraphDestroy(graph);
-                return rc;
-            }
-            if (e != hipSuccess) return seterr(D2BI_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
-            e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(graph);
-            if (e != hipSuccess) {
-                *exec = nullptr;
-                return seterr(D2BI_ERR_HIP, "graph instantiation failed: %s", hipGetErrorString(e));
-            }
-            return D2BI_OK;
-        };
-        // branch count: forced, cached, or tuned by timing one run of each
-        // count's graph (images are the same on any count); the count that
-        // fits is kept unless another is 3 % faster
-        int chosen = nbr;
-        if (nbr > 1 && !std::getenv("D2BI_BATCH_BRANCHES") && tuning_on()) {
-            int64_t sum_vox = 0, max_vox_c = 0, sum_n = 0, sum_p = 0;
-            for (int i = 0; i < nRec; i++) {
-                sum_vox += C[i].nvox;
-                max_vox_c = std::max(max_vox_c, C[i].nvox);
-                sum_n += C[i].n;
-                sum_p += C[i].plan.nPrec;
-            }
-            const TuneKey bkey{TUNE_BRANCHES, nRec, mode, sum_vox, max_vox_c, sum_n, sum_p, nbr, 0};
-            const int c = tune_get(bkey);
-            if (c >= 1 && c <= nbr) {
-                chosen = c;
-            } else {
-                float tbest = 3.4e38f;
-                for (int q = 0; q < nbr; q++) {
-                    const int nb = q == 0 ? nbr : q;            // the default first
-                    hipGraphExec_t ex = nullptr;
-                    CHK(capture(nb, &ex));
-                    (void)hipGraphUpload(ex, s);
-                    const float t = time_launch([&] { (void)hipGraphLaunch(ex, s); }, s, 1);
-                    if (q == 0) tbest = t >= 0.0f ? 0.97f * t : 3.4e38f;
-                    if (t >= 0.0f && (q == 0 || t < tbest)) {
-                        if (q > 0) tbest = t;
-                        chosen = nb;
-                        if (B.exec) (void)hipGraphExecDestroy(B.exec);
-                        B.exec = ex;
-                    } else {
-                        (void)hipGraphExecDestroy(ex);
-                    }
-                }
-                tune_put(bkey, chosen);
-            }
-        }
-        if (!B.exec) CHK(capture(chosen, &B.exec));
-        // workspaces of branches the graph does not use go back to the device
-        for (int k = std::max(1, chosen); k < nbr; k++) B.branch_ws(k).release_all();
-        B.nbr = chosen;
         B.key = key;
         B.gen = g_alloc_gen;
-        B.nr.resize(nRec);
-        for (int i = 0; i < nRec; i++) B.nr[i] = C[i].nr;
-        B.total_plane = o_img;
+    } else {
+        if (!B.exec) CHK(capture_batch(B, mode));
+        HIPCHK(hipEventRecord(g.ev[0], s));
+        HIPCHK(hipGraphLaunch(B.exec, s));
     }
-    HIPCHK(hipEventRecord(g.ev[0], s));
-    HIPCHK(hipGraphLaunch(B.exec, s));
     HIPCHK(hipEventRecord(g.ev[1], s));
     HIPCHK(hipMemcpyAsync(img_out, B.img.p, sizeof(double) * B.total_plane,
                           dev_out ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
+    void* hr = nullptr;
+    if (st) {
+        CHK(pinned_result(sizeof(Counters) * nRec, &hr));
+        HIPCHK(hipMemcpyAsync(hr, B.counters.p, sizeof(Counters) * nRec, hipMemcpyDeviceToHost, s));
+    }
     HIPCHK(hipStreamSynchronize(s));
     if (st) {
-        std::vector<unsigned long long> gcv(nRec);
-        std::vector<int> mpc(nRec);
-        HIPCHK(hipMemcpy(gcv.data(), B.guard.p, sizeof(unsigned long long) * nRec, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(mpc.data(), B.mpc.p, sizeof(int) * nRec, hipMemcpyDeviceToHost));
+        const Counters* ct = (const Counters*)hr;
         for (int i = 0; i < nRec; i++) {
-            st->n_points += B.nr[i];
-            st->n_guard += (int64_t)gcv[i];
-            st->max_per_cell = std::max(st->max_per_cell, mpc[i]);
+            st->n_points += B.conds[i].nr;
+            st->n_guard += mode == D2BI_MODE_FAST ? ct[i].n_guard() : 0;
+            st->max_per_cell = std::max(st->max_per_cell, ct[i].max_per_cell);
         }
         float ms = 0.0f;
         (void)hipEventElapsedTime(&ms, g.ev[0], g.ev[1]);

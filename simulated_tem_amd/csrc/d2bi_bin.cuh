@@ -161,14 +161,15 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_classify(const double* __rest
 }
 
 // Pass 2: point number ii in (replica, atom) order, link cell, atom number and
-// a per-cell arrival slot from an atomic counter.
+// a per-cell arrival slot from an atomic counter.  Points past the cap of the
+// arrays are counted but not stored (their cells then come out empty).
 __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restrict__ x, BinParams P,
                                                            const uint32_t* __restrict__ mask,
                                                            const int* __restrict__ blk_off, int nblk,
                                                            int* __restrict__ pt_cell,
                                                            int* __restrict__ pt_slot,
                                                            int* __restrict__ pt_j,
-                                                           int* __restrict__ cell_cnt)
+                                                           int* __restrict__ cell_cnt, int64_t cap)
 {
     __shared__ int first[MAX_REPL];
     __shared__ int wcnt[BIN_BLOCK / 64][MAX_REPL];
@@ -204,8 +205,11 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
         const int cy = P.generic ? cell_of(fl[1], P.Ey) : (int)fl[1];
         const int cz = P.generic ? cell_of(fl[2], P.Ez) : (int)fl[2];
         const int cell = cx + P.Ex * (cy + P.Ey * cz);
-        pt_cell[ii] = cell;
-        pt_j[ii] = (int)j;
+        const bool held = (int64_t)(unsigned)ii < cap;
+        if (held) {
+            pt_cell[ii] = cell;
+            pt_j[ii] = (int)j;
+        }
         // arrival slot: lanes of this wave landing in one cell share
         // one atomic (the lowest such lane adds the group's size);
         // the grouping is ALU-only, so each lane waits for one atomic
@@ -222,31 +226,27 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
         int base = 0;
         if (lane == leader) base = atomicAdd(&cell_cnt[cell], (int)__popcll(grp));
         base = __shfl(base, leader, 64);
-        pt_slot[ii] = base + (int)__popcll(grp & lt);
+        if (held) pt_slot[ii] = base + (int)__popcll(grp & lt);
     }
 }
 
+// The number of points, which only the device knows when the passes after
+// the count are launched, and what the point arrays hold; a condition with
+// more points than that stores none and is binned again.
+struct PointCount {
+    const int* n;
+    int64_t cap;
+    // (a count that overflowed is negative)
+    __device__ int64_t stored() const { return (int64_t)(unsigned)*n > cap ? 0 : *n; }
+};
+
 // Pass 3: place each point at its cell's start + arrival slot.
-__global__ void k_bin_place(int64_t nr, const int* __restrict__ pt_cell, const int* __restrict__ pt_slot,
+__global__ void k_bin_place(PointCount N, const int* __restrict__ pt_cell, const int* __restrict__ pt_slot,
                             const int* __restrict__ cell_start, int* __restrict__ cell_ids)
 {
     int64_t ii = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (ii >= nr) return;
+    if (ii >= N.stored()) return;
     cell_ids[cell_start[pt_cell[ii]] + pt_slot[ii]] = (int)ii;
-}
-
-// Sum of the FAST guard counters into *out (one block).
-__global__ __launch_bounds__(256) void k_sum_guard(const unsigned long long* __restrict__ part, int n, int stride,
-                                                   unsigned long long* __restrict__ out)
-{
-    __shared__ unsigned long long ws[4];
-    unsigned long long v = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) v += part[(int64_t)i * stride];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) *out = (ws[0] + ws[1]) + (ws[2] + ws[3]);
 }
 
 // What pass 4 writes per slot (null: not wanted).
@@ -271,7 +271,7 @@ struct EmitOut {
 // (replica, atom) order; rep_first is padded to 32 entries with INT_MAX).
 // Bound: HBM and, in imaging, FP64 sincos with full argument reduction.
 template <bool FAST>
-__global__ __launch_bounds__(256) void k_bin_emit(int64_t nr, const int* __restrict__ cell_ids,
+__global__ __launch_bounds__(256) void k_bin_emit(PointCount N, const int* __restrict__ cell_ids,
                                                   const int* __restrict__ pt_cell, const int* __restrict__ pt_j,
                                                   const int* __restrict__ cell_start, const double* __restrict__ x,
                                                   BinParams P, const int* __restrict__ blk_off, int nblk, EmitOut O)
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(256) void k_bin_emit(int64_t nr, const int* __restr
         rep_first[threadIdx.x] = threadIdx.x < P.nuvw ? blk_off[(int64_t)threadIdx.x * nblk] : 0x7fffffff;
     __syncthreads();
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nr) return;
+    if (t >= N.stored()) return;
     const int ii = cell_ids[t];
     const int64_t j = pt_j[ii];
     const int c = pt_cell[ii];
@@ -358,26 +358,28 @@ __global__ __launch_bounds__(256) void k_app_phase(int64_t nr, const int2* __res
 }
 
 struct Binned {
-    int64_t nr = 0;
+    int64_t nr = -1;            // points; -1: not known on the host yet
+    int64_t cap = 0;            // what the point arrays hold
     int ncell = 0;
 };
 
-// Passes 2 to 4 on workspace w, once the points are counted: d_x, mask,
-// blk_off and nblk are the condition's atoms, replica predicates and
-// per-(replica, block) point offsets; w.cell_cnt is zero.  The largest cell
-// count goes to *mpc.
+// Passes 2 to 4 on workspace w, once the points are counted on the device (*N.n
+// of them): d_x, mask, blk_off and nblk are the condition's atoms, replica
+// predicates and per-(replica, block) point offsets; w.cell_cnt is zero.  The
+// largest cell count goes to *mpc.
 static int launch_bin_points(const double* d_x, const BinParams& P, const uint32_t* mask, const int* blk_off, int nblk,
-                             int ncell, int64_t nr, int* scan_tmp, int* mpc, hipStream_t s, Workspace& w)
+                             int ncell, PointCount N, int* scan_tmp, int* mpc, hipStream_t s, Workspace& w)
 {
-    if (P.n > 0 && nr > 0) {
+    if (P.n > 0 && N.cap > 0) {
         hipLaunchKernelGGL(k_bin_scatter, dim3(nblk), dim3(BIN_BLOCK), 0, s, d_x, P, mask, blk_off, nblk,
-                           w.pt_cell.as<int>(), w.pt_slot.as<int>(), w.pt_j.as<int>(), w.cell_cnt.as<int>());
+                           w.pt_cell.as<int>(), w.pt_slot.as<int>(), w.pt_j.as<int>(), w.cell_cnt.as<int>(), N.cap);
         HIPCHK(hipGetLastError());
     }
-    CHK(scan_exclusive_tmp(w.cell_cnt.as<int>(), w.cell_start.as<int>(), ncell, scan_tmp, s, mpc));
-    if (nr > 0) {
-        const dim3 grid((unsigned)((nr + 255) / 256));
-        hipLaunchKernelGGL(k_bin_place, grid, dim3(256), 0, s, nr, w.pt_cell.as<int>(), w.pt_slot.as<int>(),
+    CHK(scan_exclusive_tmp(w.cell_cnt.as<int>(), w.cell_start.as<int>(), ncell, scan_tmp, s,
+                           ScanEnds{nullptr, mpc, N.n, N.cap}));
+    if (P.n > 0 && N.cap > 0) {
+        const dim3 grid((unsigned)((N.cap + 255) / 256));
+        hipLaunchKernelGGL(k_bin_place, grid, dim3(256), 0, s, N, w.pt_cell.as<int>(), w.pt_slot.as<int>(),
                            w.cell_start.as<int>(), w.cell_ids.as<int>());
         EmitOut O{w.slot_p32.as<float4>(), w.slot_sn32.as<float>(), nullptr, w.slot_frac.as<Frac3>(),
                   P.keep_src ? w.slot_src.as<int2>() : nullptr, nullptr, nullptr};
@@ -391,7 +393,7 @@ static int launch_bin_points(const double* d_x, const BinParams& P, const uint32
             }
         }
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, nr, w.cell_ids.as<int>(), w.pt_cell.as<int>(),
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, N, w.cell_ids.as<int>(), w.pt_cell.as<int>(),
                                w.pt_j.as<int>(), w.cell_start.as<int>(), d_x, P, blk_off, nblk, O);
         };
         if (P.fast) go(k_bin_emit<true>);
@@ -401,9 +403,44 @@ static int launch_bin_points(const double* d_x, const BinParams& P, const uint32
     return D2BI_OK;
 }
 
+// The per-point and per-slot buffers of a condition and their bytes per point.
+template <class F>
+static void point_buffers(Workspace& w, bool fast, bool keep_ids, bool generic, bool keep_src, F f)
+{
+    f(w.pt_cell, sizeof(int));
+    f(w.pt_slot, sizeof(int));
+    f(w.pt_j, sizeof(int));
+    f(w.cell_ids, sizeof(int));
+    f(w.slot_p32, sizeof(float4));
+    f(w.slot_frac, sizeof(Frac3));
+    if (fast) f(w.slot_sn32, sizeof(float));
+    else if (!keep_ids) f(w.slot_cs64, sizeof(double2));
+    if (keep_ids) f(w.slot_id, sizeof(int));
+    if (keep_ids && !generic) f(w.pt_gdotr, sizeof(double));
+    if (keep_src) f(w.slot_src, sizeof(int2));
+}
+
+// Points a condition is expected to have, with a margin: its atoms' density
+// in the supercell times the link-cell box (at most all its replicas).
+static int64_t expected_points(const d2bi_record* r, const d2bi_plan* p, int64_t n)
+{
+    double A[9];
+    for (int j = 0; j < 3; j++)
+        for (int i = 0; i < 3; i++) A[3 * j + i] = r->super_a[3 * j + i] * r->super_n[j];
+    const double box = p->a_col[0] * p->Ex * (p->a_col[4] * p->Ey) * (p->a_col[8] * p->Ez), super = std::fabs(det3(A));
+    const double most = (double)r->nuvw * (double)n;
+    const double e = super > 0.0 ? 1.1 * (box / super) * (double)n + 4096.0 : most;
+    return (int64_t)std::min(std::min(e, most), 2147483647.0);
+}
+
 // Run binning for either a condition (generic = 0) or plain points, on
-// workspace w.
-static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, hipStream_t s, Workspace& w)
+// workspace w.  expect > 0: the point arrays are sized for that many points
+// (or what they hold) and nothing waits for the count, which stays in the
+// workspace's counters; the caller compares it with out->cap at its own end
+// and bins again with expect = 0 if they did not fit.  expect = 0: the host
+// waits for the count and sizes the arrays by it.
+static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, hipStream_t s, Workspace& w,
+                       int64_t expect = 0)
 {
     const int64_t ncell64 = (int64_t)P.Ex * P.Ey * P.Ez;
     if (ncell64 > (int64_t)INT32_MAX / 2) return seterr(D2BI_ERR_CAPACITY, "too many link cells");
@@ -411,40 +448,44 @@ static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, 
     const int nblk = bin_blocks(n);
     if (n > (int64_t)INT32_MAX) return seterr(D2BI_ERR_CAPACITY, "more than 2^31 - 1 atoms");
     P.n = n;
+    const int64_t nbc = (int64_t)P.nuvw * nblk;
     CHK(w.mask.ensure(sizeof(uint32_t) * std::max<int64_t>(n, 1)));
-    CHK(w.blk_cnt.ensure(sizeof(int) * ((int64_t)P.nuvw * nblk + 1)));
-    CHK(w.blk_off.ensure(sizeof(int) * ((int64_t)P.nuvw * nblk + 1)));
+    CHK(w.blk_cnt.ensure(sizeof(int) * (nbc + 1)));
+    CHK(w.blk_off.ensure(sizeof(int) * (nbc + 1)));
     CHK(w.cell_cnt.ensure(sizeof(int) * (ncell + 1)));
     CHK(w.cell_start.ensure(sizeof(int) * (ncell + 1)));
-    CHK(w.counters.ensure(64));
-    const int64_t nbc = (int64_t)P.nuvw * nblk;
-    zero_i32(s, w.cell_cnt.as<int>(), ncell + 1, w.counters.as<int>(), 16, w.blk_cnt.as<int>(), n > 0 ? 0 : nbc);
+    CHK(w.counters.ensure(sizeof(Counters)));
+    CHK(w.scan_tmp.ensure(sizeof(int) * std::max(scan_tmp_ints(nbc), scan_tmp_ints(ncell))));
+    Counters* ct = w.counters.as<Counters>();
+    zero_i32(s, w.cell_cnt.as<int>(), ncell + 1, (int*)ct, sizeof(Counters) / sizeof(int), w.blk_cnt.as<int>(),
+             n > 0 ? 0 : nbc);
     if (n > 0)
         hipLaunchKernelGGL(k_bin_classify, dim3(nblk), dim3(BIN_BLOCK), 0, s, d_x, P, w.mask.as<uint32_t>(),
                            w.blk_cnt.as<int>(), nblk);
     HIPCHK(hipGetLastError());
-    CHK(scan_exclusive(w.blk_cnt.as<int>(), w.blk_off.as<int>(), nbc, s, w));
-    int nr_host = 0;
-    HIPCHK(hipMemcpyAsync(&nr_host, w.blk_off.as<int>() + nbc, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    if (nr_host < 0) return seterr(D2BI_ERR_CAPACITY, "point count overflow");
-    const int64_t nr = nr_host;
-    const int64_t nrc = std::max<int64_t>(nr, 1);
-    CHK(w.pt_cell.ensure(sizeof(int) * nrc));
-    CHK(w.pt_slot.ensure(sizeof(int) * nrc));
-    CHK(w.pt_j.ensure(sizeof(int) * nrc));
-    CHK(w.cell_ids.ensure(sizeof(int) * nrc));
-    CHK(w.slot_p32.ensure(sizeof(float4) * nrc));
-    CHK(w.slot_frac.ensure(sizeof(Frac3) * nrc));
-    if (P.fast) CHK(w.slot_sn32.ensure(sizeof(float) * nrc));
-    else if (!P.keep_ids) CHK(w.slot_cs64.ensure(sizeof(double2) * nrc));
-    if (P.keep_ids) CHK(w.slot_id.ensure(sizeof(int) * nrc));
-    if (P.keep_ids && !P.generic) CHK(w.pt_gdotr.ensure(sizeof(double) * nrc));
-    if (P.keep_src) CHK(w.slot_src.ensure(sizeof(int2) * nrc));
-    CHK(w.scan_tmp.ensure(sizeof(int) * scan_tmp_ints(ncell)));
-    CHK(launch_bin_points(d_x, P, w.mask.as<uint32_t>(), w.blk_off.as<int>(), nblk, ncell, nr, w.scan_tmp.as<int>(),
-                          w.counters.as<int>(), s, w));
-    out->nr = nr;
+    CHK(scan_exclusive_tmp(w.blk_cnt.as<int>(), w.blk_off.as<int>(), nbc, w.scan_tmp.as<int>(), s,
+                           ScanEnds{&ct->n_points, nullptr, nullptr, 0}));
+    int64_t cap = expect;
+    if (expect <= 0) {
+        int nr_host = 0;
+        HIPCHK(hipMemcpyAsync(&nr_host, &ct->n_points, sizeof(int), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        if (nr_host < 0) return seterr(D2BI_ERR_CAPACITY, "point count overflow");
+        out->nr = cap = nr_host;
+    }
+    int rc = D2BI_OK;
+    int64_t held = INT64_MAX;
+    point_buffers(w, P.fast, P.keep_ids, P.generic, P.keep_src, [&](Buf& b, size_t bytes) {
+        if (rc == D2BI_OK) rc = b.ensure(bytes * std::max<int64_t>(cap, 1));
+        held = std::min(held, (int64_t)(b.cap / bytes));
+    });
+    CHK(rc);
+    // (twice the estimate at most: the passes over the points launch a thread
+    // for each that may be stored)
+    if (expect > 0) cap = std::min(held, 2 * expect);
+    CHK(launch_bin_points(d_x, P, w.mask.as<uint32_t>(), w.blk_off.as<int>(), nblk, ncell, PointCount{&ct->n_points, cap},
+                          w.scan_tmp.as<int>(), &ct->max_per_cell, s, w));
+    out->cap = cap;
     out->ncell = ncell;
     return D2BI_OK;
 }

@@ -108,10 +108,8 @@ struct Workspace {
     Buf slot_src;                           // atom and replica of each slot (aperture sums)
     Buf app_cs;                 // per-slot phases of the aperture points of one shared pass
     Buf scan_tmp;
-    Buf guard_part;             // FAST guard re-test counters, one per 128-byte line
-    Buf counters;               // misc device counters (guard count, max per cell)
-    // voxel axis tables
-    Buf ax_cell, ax_zi, ax_ql;
+    Buf counters;               // device counters of a condition (struct Counters)
+    Buf ax_tab;                 // voxel axis tables
     // fields and image
     Buf f64_re, f64_im, f64_rho, f32_field;
     Buf cnt, r2m;
@@ -125,7 +123,7 @@ struct Workspace {
     {
         Buf* all[] = {&x, &mask, &blk_cnt, &blk_off, &pt_cell, &pt_slot, &pt_j, &pt_gdotr,
                       &cell_cnt, &cell_start, &cell_ids, &slot_id, &slot_frac, &slot_cs64,
-                      &slot_p32, &slot_sn32, &slot_src, &app_cs, &scan_tmp, &guard_part, &counters, &ax_cell, &ax_zi, &ax_ql, &f64_re,
+                      &slot_p32, &slot_sn32, &slot_src, &app_cs, &scan_tmp, &counters, &ax_tab, &f64_re,
                       &f64_im, &f64_rho, &f32_field, &cnt, &r2m, &img, &tune_img, &blur_in, &blur_tmp,
                       &blur_out, &blur_w, &blur_wy, &blur_k};
         for (Buf* b : all) f(*b);
@@ -157,6 +155,8 @@ struct State {
     hipStream_t stream = nullptr;
     hipEvent_t ev[10] = {};
     bool pinned_busy = false;       // ev[9] marks the last copy out of the pinned staging buffer
+    void* res = nullptr;            // pinned memory that results are copied into
+    size_t res_cap = 0;
     Workspace ws;
 };
 
@@ -187,6 +187,40 @@ static int pinned(size_t bytes, void** out)
     *out = g.ws.pinned;
     return D2BI_OK;
 }
+
+// Pinned memory for results on their way to the caller (a call that copies
+// into it waits for its stream before it returns).
+static int pinned_result(size_t bytes, void** out)
+{
+    if (bytes > g.res_cap) {
+        if (g.res) (void)hipHostFree(g.res);
+        g.res = nullptr;
+        g.res_cap = 0;
+        HIPCHK(hipHostMalloc(&g.res, bytes, hipHostMallocDefault));
+        g.res_cap = bytes;
+    }
+    *out = g.res;
+    return D2BI_OK;
+}
+
+// Counters of one condition, cleared before it is binned.  The FAST guard
+// re-tests are spread over GUARD_SLOTS lines (many waves adding into one
+// address serialise) and added up on the host.
+static constexpr int GUARD_SLOTS = 16;               // power of two ...
+static constexpr int GUARD_STRIDE = 8;               // ... 64 bytes apart
+
+struct Counters {
+    int max_per_cell;           // largest link-cell population
+    int n_points;               // points in the link cells
+    int pad[14];
+    unsigned long long guard[GUARD_SLOTS * GUARD_STRIDE];
+    int64_t n_guard() const
+    {
+        unsigned long long v = 0;
+        for (int i = 0; i < GUARD_SLOTS; i++) v += guard[i * GUARD_STRIDE];
+        return (int64_t)v;
+    }
+};
 
 // ------------------------------------------------------------------ device atoms
 
@@ -282,6 +316,17 @@ __device__ inline int block_max(int v, int* lds)
     return v;
 }
 
+// What a scan hands on besides the array: its total and largest value (null:
+// not wanted); and the scan of the cell counts of more points than the point
+// arrays hold is that of empty cells, so that nothing reads past them.
+struct ScanEnds {
+    int* total_out;
+    int* max_out;
+    const int* points;          // null, or the number of points ...
+    int64_t cap;                // ... and what the point arrays hold
+    __device__ bool over() const { return points && (int64_t)(unsigned)*points > cap; }
+};
+
 // Short arrays (a small condition's block counts or link cells) in one
 // workgroup and one launch: on an 80^3 condition the launch gaps of a
 // three-phase scan cost more than its work (3 x ~5 us against 5).
@@ -290,13 +335,14 @@ static constexpr int SCAN_ONE_ITEMS = 16;
 static constexpr int SCAN_ONE = SCAN_ONE_BLOCK * SCAN_ONE_ITEMS;
 
 __global__ __launch_bounds__(SCAN_ONE_BLOCK) void k_scan_one(const int* __restrict__ in, int n, int* __restrict__ out,
-                                                             int* __restrict__ max_out)
+                                                             ScanEnds E)
 {
     __shared__ int lds[SCAN_ONE_BLOCK / 64 + 1];
     const int per = (n + SCAN_ONE_BLOCK - 1) / SCAN_ONE_BLOCK, base = (int)threadIdx.x * per;
+    const int end = E.over() ? 0 : n;
     int v[SCAN_ONE_ITEMS], s = 0, m = 0;
 #pragma unroll
-    for (int i = 0; i < SCAN_ONE_ITEMS; i++) v[i] = i < per && base + i < n ? in[base + i] : 0;
+    for (int i = 0; i < SCAN_ONE_ITEMS; i++) v[i] = i < per && base + i < end ? in[base + i] : 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ONE_ITEMS; i++) {
         s += v[i];
@@ -309,10 +355,13 @@ __global__ __launch_bounds__(SCAN_ONE_BLOCK) void k_scan_one(const int* __restri
         if (i < per && base + i < n) out[base + i] = e;
         e += v[i];
     }
-    if (threadIdx.x == 0) out[n] = tot;
-    if (max_out) {
+    if (threadIdx.x == 0) {
+        out[n] = tot;
+        if (E.total_out) *E.total_out = tot;
+    }
+    if (E.max_out) {
         m = block_max(m, lds);
-        if (threadIdx.x == 0) *max_out = m;
+        if (threadIdx.x == 0) *E.max_out = m;
     }
 }
 
@@ -322,9 +371,11 @@ __global__ __launch_bounds__(SCAN_ONE_BLOCK) void k_scan_one(const int* __restri
 static constexpr int SCAN_SELF = 4096;
 
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(const int* __restrict__ in, int64_t n,
-                                                            int* __restrict__ sums, int* __restrict__ maxs)
+                                                            int* __restrict__ sums, int* __restrict__ maxs,
+                                                            ScanEnds E)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
+    if (E.over()) n = 0;
     int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     int s = 0, m = 0;
 #pragma unroll
@@ -360,9 +411,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_sums(int* __restrict__ sums
 __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const int* __restrict__ in, int64_t n,
                                                            const int* __restrict__ sums, int scanned,
                                                            const int* __restrict__ maxs, int* __restrict__ out,
-                                                           int* __restrict__ max_out)
+                                                           ScanEnds E)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
+    const bool over = E.over();
     int before = 0;
     if (scanned) {
         before = sums[blockIdx.x];
@@ -376,7 +428,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const int* __restrict
     int s = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++) {
-        v[i] = base + i < n ? in[base + i] : 0;
+        v[i] = base + i < n && !over ? in[base + i] : 0;
         s += v[i];
     }
     int tot;
@@ -386,12 +438,15 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const int* __restrict
         if (base + i < n) out[base + i] = e;
         e += v[i];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + tot;
-    if (max_out && blockIdx.x == 0) {
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        out[n] = before + tot;
+        if (E.total_out) *E.total_out = before + tot;
+    }
+    if (E.max_out && blockIdx.x == 0) {
         int m = 0;
         for (int b = threadIdx.x; b < (int)gridDim.x; b += SCAN_BLOCK) m = max(m, maxs[b]);
         m = block_max(m, lds);
-        if (threadIdx.x == 0) *max_out = m;
+        if (threadIdx.x == 0) *E.max_out = m;
     }
 }
 
@@ -400,29 +455,23 @@ static int64_t scan_tmp_ints(int64_t n)
     return 2 * std::max<int64_t>(1, (n + SCAN_TILE - 1) / SCAN_TILE);
 }
 
-// out[0..n-1] = exclusive scan of in, out[n] = total, *max_out (optional) the
-// largest value, 0 if n = 0.  tmp: scan_tmp_ints(n) ints of scratch (no
-// allocation here, so the call can be captured into a graph).
-static int scan_exclusive_tmp(const int* in, int* out, int64_t n, int* tmp, hipStream_t s, int* max_out = nullptr)
+// out[0..n-1] = exclusive scan of in, out[n] = total, and what E asks for.
+// tmp: scan_tmp_ints(n) ints of scratch (no allocation here, so the call can
+// be captured into a graph).
+static int scan_exclusive_tmp(const int* in, int* out, int64_t n, int* tmp, hipStream_t s, const ScanEnds& E)
 {
     if (n <= SCAN_ONE) {
-        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_BLOCK), 0, s, in, (int)n, out, max_out);
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_BLOCK), 0, s, in, (int)n, out, E);
     } else {
         const int64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
         int *sums = tmp, *maxs = tmp + nb;
-        hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, maxs);
+        hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums, maxs, E);
         if (nb > SCAN_SELF) hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, s, sums, nb);
         hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_BLOCK), 0, s, in, n, sums,
-                           nb > SCAN_SELF ? 1 : 0, maxs, out, max_out);
+                           nb > SCAN_SELF ? 1 : 0, maxs, out, E);
     }
     HIPCHK(hipGetLastError());
     return D2BI_OK;
-}
-
-static int scan_exclusive(const int* in, int* out, int64_t n, hipStream_t s, Workspace& w, int* max_out = nullptr)
-{
-    CHK(w.scan_tmp.ensure(sizeof(int) * scan_tmp_ints(n)));
-    return scan_exclusive_tmp(in, out, n, w.scan_tmp.as<int>(), s, max_out);
 }
 
 }  // namespace d2bi

@@ -95,6 +95,8 @@ int d2bi_gpu_init(int device)
     if (scratch_address(device) != D2BI_OK) (void)hipGetLastError();
     HIPCHK(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
     for (auto& e : g.ev) HIPCHK(hipEventCreate(&e));
+    void* res;
+    CHK(pinned_result(sizeof(Counters) + 64 * 1024 * sizeof(double), &res));
     g.device = device;
     g.init = true;
     return D2BI_OK;
@@ -107,6 +109,9 @@ int d2bi_gpu_finalize(void)
     (void)hipStreamSynchronize(g.stream);
     g_batch.release();
     g.ws.release_all();
+    if (g.res) (void)hipHostFree(g.res);
+    g.res = nullptr;
+    g.res_cap = 0;
     for (auto& e : g.ev) { (void)hipEventDestroy(e); e = nullptr; }
     (void)hipStreamDestroy(g.stream);
     g.stream = nullptr;
@@ -158,9 +163,7 @@ int d2bi_gpu_image_dev(const d2bi_record* rec, d2bi_atoms atoms, double precAngl
     if (!rec || !atoms || !img) return seterr(D2BI_ERR_ARG, "null argument");
     if (stats) std::memset(stats, 0, sizeof *stats);
     d2bi_plan plan;
-    CHK(image_condition(rec, atoms->x, atoms->n, precAngle, nPrec, mode, stats, &plan, g.ws));
-    HIPCHK(hipMemcpy(img, g.ws.img.p, sizeof(double) * plan.Mx * plan.My, hipMemcpyDeviceToHost));
-    return D2BI_OK;
+    return image_condition(rec, atoms->x, atoms->n, precAngle, nPrec, mode, stats, &plan, g.ws, nullptr, img);
 }
 
 int d2bi_gpu_image_dev_out(const d2bi_record* rec, d2bi_atoms atoms, double precAngle, int32_t nPrec,
@@ -177,9 +180,7 @@ int d2bi_gpu_image_dev_out(const d2bi_record* rec, d2bi_atoms atoms, double prec
         return seterr(D2BI_ERR_ARG, "d_img is not memory of device %d", g.device);
     if (stats) std::memset(stats, 0, sizeof *stats);
     d2bi_plan plan;
-    CHK(image_condition(rec, atoms->x, atoms->n, precAngle, nPrec, mode, stats, &plan, g.ws, d_img));
-    HIPCHK(hipStreamSynchronize(g.stream));
-    return D2BI_OK;
+    return image_condition(rec, atoms->x, atoms->n, precAngle, nPrec, mode, stats, &plan, g.ws, d_img);
 }
 
 int d2bi_gpu_image_noalloc(const d2bi_record* rec, d2bi_atoms atoms, double precAngle, int32_t nPrec,
@@ -250,9 +251,7 @@ int d2bi_gpu_image(const d2bi_record* rec, const double* x, int64_t ld, int64_t 
     double* d_x;
     CHK(upload_atoms_tmp(x, ld, nAtoms, &d_x));
     d2bi_plan plan;
-    CHK(image_condition(rec, d_x, nAtoms, precAngle, nPrec, mode, stats, &plan, g.ws));
-    HIPCHK(hipMemcpy(img, g.ws.img.p, sizeof(double) * plan.Mx * plan.My, hipMemcpyDeviceToHost));
-    return D2BI_OK;
+    return image_condition(rec, d_x, nAtoms, precAngle, nPrec, mode, stats, &plan, g.ws, nullptr, img);
 }
 
 int d2bi_gpu_image_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int32_t nRec, const double* precAngle,
@@ -312,7 +311,7 @@ int d2bi_gpu_field(const d2bi_record* rec, const double* x, int64_t ld, int64_t 
     // FAST without count and r2min runs the imaging kernel itself (the
     // variant imaging uses)
     const bool diag = mode == D2BI_MODE_FP64 || count || r2min;
-    CHK(run_voxel(rec, &plan, tab, ax, mode, diag, nullptr, s, g.ws));
+    CHK(run_voxel(rec, &plan, tab, ax, mode, diag, true, s, g.ws));
     HIPCHK(hipStreamSynchronize(s));
     const int64_t nvox = (int64_t)plan.Mx * plan.My * plan.Mz;
     Workspace& w = g.ws;

@@ -315,9 +315,10 @@ static TuneKey tile_order_key(const d2bi_plan* p, const AxisTables& tab, bool de
 }
 
 // Voxelise into the mode's field buffers of workspace w; optional count /
-// r2min outputs.
+// r2min outputs.  fresh: the workspace's guard counters are zero (they were
+// cleared for this condition's binning).
 static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables& tab, const AxisDev& ax,
-                     int mode, bool want_diag, int64_t* n_guard, hipStream_t s, Workspace& w, Timer* T = nullptr)
+                     int mode, bool want_diag, bool fresh, hipStream_t s, Workspace& w)
 {
     const int64_t nvox = (int64_t)p->Mx * p->My * p->Mz;
     VoxParams V;
@@ -334,24 +335,18 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
         CHK(w.f64_re.ensure(sizeof(double) * nvox));
         CHK(w.f64_im.ensure(sizeof(double) * nvox));
         CHK(w.f64_rho.ensure(sizeof(double) * nvox));
-        if (T) CHK(T->record(2));
-        CHK(launch_voxel_fp64(p, tab, V, 1, w, w.slot_cs64.as<double2>(), 0, 0, dcnt, (double*)dr2, s));
-        if (T) CHK(T->record(3));
-        return D2BI_OK;
+        return launch_voxel_fp64(p, tab, V, 1, w, w.slot_cs64.as<double2>(), 0, 0, dcnt, (double*)dr2, s);
     }
     CHK(w.f32_field.ensure(sizeof(float4) * nvox));
     FastParams F;
     CHK(fast_params(p, tab, V, &F, 4));
-    CHK(w.counters.ensure(64));
-    unsigned long long* gc = (unsigned long long*)(w.counters.as<char>() + 8);
-    const size_t gp_bytes = sizeof(unsigned long long) * GUARD_SLOTS * GUARD_STRIDE;
-    CHK(w.guard_part.ensure(gp_bytes));
-    unsigned long long* gp = w.guard_part.as<unsigned long long>();
+    unsigned long long* gp = w.counters.as<Counters>()->guard;
     const bool dens = r->use_density != 0;
     // launch parameters follow the variant's tile depth; order: the tiles'
     // order over the workgroups (0 per XCD, 1 linear)
     auto run_variant = [&](int v, int order = 2) -> int {
         FastParams Fv;
+        fresh = false;
         CHK(variant_params(p, tab, V, &v, &Fv));
         set_tile_order(&Fv, order);
         pick_tile(want_diag, dens, v, Fv.thin_z != 0, [&](auto kern) {
@@ -380,18 +375,10 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
         order = tune_choose(tile_order_key(p, tab, dens, variant), "D2BI_TILE_ORDER", TILE_ORDERS, 3, 2, true, s,
                             [&](int o) { (void)run_variant(variant, o); });
     }
-    zero_i32(s, (int*)gp, (int64_t)(gp_bytes / sizeof(int)));   // tuning launches counted too
-    if (T) CHK(T->record(2));
+    // tuning launches counted too
+    if (!fresh) zero_i32(s, (int*)gp, (int64_t)(sizeof(Counters::guard) / (sizeof(int))));
     CHK(run_variant(variant, order));
     HIPCHK(hipGetLastError());
-    if (T) CHK(T->record(3));
-    hipLaunchKernelGGL(k_sum_guard, dim3(1), dim3(256), 0, s, gp, GUARD_SLOTS, GUARD_STRIDE, gc);
-    if (n_guard) {
-        unsigned long long v = 0;
-        HIPCHK(hipMemcpyAsync(&v, gc, 8, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        *n_guard = (int64_t)v;
-    }
     return D2BI_OK;
 }
 
@@ -552,26 +539,24 @@ static int launch_integrate_fp64(const d2bi_plan* p, bool dens, double* d_img, h
 }
 
 // Integrate the field of workspace w into d_img (Mx*My doubles).
-static int run_integrate(const d2bi_plan* p, bool dens, int mode, hipStream_t s, Workspace& w, double* d_img,
-                         Timer* T = nullptr)
+static int run_integrate(const d2bi_plan* p, bool dens, int mode, hipStream_t s, Workspace& w, double* d_img)
 {
-    if (mode == D2BI_MODE_FP64) {
-        if (T) CHK(T->record(4));
-        CHK(launch_integrate_fp64(p, dens, d_img, s, w));
-        if (T) CHK(T->record(5));
-        return D2BI_OK;
-    }
-    if (T) CHK(T->record(4));
-    CHK(launch_integrate_fast(p, dens, w.f32_field.p, d_img, s, false, 0.0, &w));
-    if (T) CHK(T->record(5));
-    return D2BI_OK;
+    if (mode == D2BI_MODE_FP64) return launch_integrate_fp64(p, dens, d_img, s, w);
+    return launch_integrate_fast(p, dens, w.f32_field.p, d_img, s, false, 0.0, &w);
 }
 
 // Whole condition: bin -> voxelise -> integrate on workspace w, the image
 // written to d_img (device memory of Mx*My doubles) or, when d_img is null,
-// left in w.img.
+// left in w.img; copied to h_img when that is given.  The host waits once, at
+// the end: the point arrays are sized by an estimate, and a condition that
+// has more points is imaged again with the exact count (the wait for the
+// count between the counting and the scatter left the GPU idle for 45-50 us).
+// The exact count comes first where the arrays are carved from a fixed block,
+// where the launch tuner has yet to time this shape (it should time real
+// work), or where the estimate does not fit in device memory.
 static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, double precAngle, int nPrec,
-                           int mode, d2bi_stats* st, d2bi_plan* plan_out, Workspace& w, double* d_img = nullptr)
+                           int mode, d2bi_stats* st, d2bi_plan* plan_out, Workspace& w, double* d_img = nullptr,
+                           double* h_img = nullptr)
 {
     if (mode != D2BI_MODE_FP64 && mode != D2BI_MODE_FAST) return seterr(D2BI_ERR_ARG, "unknown mode %d", mode);
     d2bi_plan plan;
@@ -580,37 +565,69 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
     CHK(axis_tables(r, &plan, &tab));
     BinParams BP;
     CHK(bin_params(r, &plan, &BP));
+    const bool dens = r->use_density != 0;
     BP.fast = mode == D2BI_MODE_FAST ? 1 : 0;
+    const int64_t plane = (int64_t)plan.Mx * plan.My;
     if (!d_img) {
-        CHK(w.img.ensure(sizeof(double) * (int64_t)plan.Mx * plan.My));
+        CHK(w.img.ensure(sizeof(double) * plane));
         d_img = w.img.as<double>();
     }
     hipStream_t s = g.stream;
     Timer T{g.ev, s};
-    CHK(T.record(0));
-    AxisDev ax;
-    CHK(upload_axis(tab, &ax, s, w));
+    // results come back through pinned memory, small images too
+    const bool small = h_img && plane <= 64 * 1024;
+    Counters* ct;
+    void* hp;
+    if (w.counters.arena) {
+        CHK(pinned_result(sizeof(Counters), &hp));       // held from initialisation on
+    } else {
+        CHK(pinned_result(sizeof(Counters) + (small ? sizeof(double) * plane : 0), &hp));
+    }
+    ct = (Counters*)hp;
+    double* hi = (double*)((char*)hp + sizeof(Counters));
     Binned b;
-    CHK(run_binning(d_x, n, BP, &b, s, w));
-    CHK(T.record(1));
-    CHK(run_voxel(r, &plan, tab, ax, mode, false, nullptr, s, w, &T));
-    CHK(run_integrate(&plan, r->use_density != 0, mode, s, w, d_img, &T));
-    CHK(T.record(6));
-    // counters (largest cell count at 0, FAST guard re-tests at 8) come back
-    // with the final synchronisation
-    int64_t hc[2] = {0, 0};
-    if (st) HIPCHK(hipMemcpyAsync(hc, w.counters.p, 16, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    auto enqueue = [&](int64_t expect) -> int {
+        CHK(T.record(0));
+        AxisDev ax;
+        CHK(upload_axis(tab, &ax, s, w));
+        b = Binned();
+        CHK(run_binning(d_x, n, BP, &b, s, w, expect));
+        CHK(T.record(1));
+        CHK(run_voxel(r, &plan, tab, ax, mode, false, true, s, w));
+        CHK(T.record(2));
+        CHK(run_integrate(&plan, dens, mode, s, w, d_img));
+        CHK(T.record(3));
+        HIPCHK(hipMemcpyAsync(ct, w.counters.p, sizeof(Counters), hipMemcpyDeviceToHost, s));
+        if (small) HIPCHK(hipMemcpyAsync(hi, d_img, sizeof(double) * plane, hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        return D2BI_OK;
+    };
+    const int v = known_variant(&plan, dens);
+    bool exact = w.counters.arena || n == 0;
+    if (mode == D2BI_MODE_FAST && (v < 0 || !condition_tuned(&plan, tab, dens, v))) exact = true;
+    if (!exact) {
+        const int rc = enqueue(expected_points(r, &plan, n));
+        if (rc != D2BI_OK) {
+            // memory for the estimate, or a failure the exact pass reports again
+            (void)hipGetLastError();
+            HIPCHK(hipStreamSynchronize(s));
+            exact = true;
+        } else if (ct->n_points < 0 || ct->n_points > b.cap) {
+            exact = true;
+        }
+    }
+    if (exact) CHK(enqueue(0));
+    if (small) std::memcpy(h_img, hi, sizeof(double) * plane);
+    else if (h_img) HIPCHK(hipMemcpy(h_img, d_img, sizeof(double) * plane, hipMemcpyDeviceToHost));
     if (st) {
-        const int mpc = (int)(hc[0] & 0xffffffff);
-        st->n_points += b.nr;
-        st->n_guard += mode == D2BI_MODE_FAST ? hc[1] : 0;
-        st->max_per_cell = std::max(st->max_per_cell, mpc);
+        st->n_points += ct->n_points;
+        st->n_guard += mode == D2BI_MODE_FAST ? ct->n_guard() : 0;
+        st->max_per_cell = std::max(st->max_per_cell, ct->max_per_cell);
         st->n_cells = b.ncell;
         st->ms_bin += T.ms(0, 1);
-        st->ms_voxel += T.ms(2, 3);          // the voxel kernel alone
-        st->ms_integrate += T.ms(4, 5);      // the integration kernels alone
-        st->ms_total += T.ms(0, 6);
+        st->ms_voxel += T.ms(1, 2);
+        st->ms_integrate += T.ms(2, 3);
+        st->ms_total += T.ms(0, 3);
     }
     if (plan_out) *plan_out = plan;
     return D2BI_OK;
@@ -656,12 +673,8 @@ static int run_voxel_apps(const d2bi_record* r, const d2bi_plan* p, const AxisTa
     F.field_stride = nvox;
     const int fo = forced_int("D2BI_TILE_ORDER", 0, 2);
     set_tile_order(&F, fo >= 0 ? fo : 2);
-    CHK(w.counters.ensure(64));
-    unsigned long long* gc = (unsigned long long*)(w.counters.as<char>() + 8);
-    const size_t gp_bytes = sizeof(unsigned long long) * GUARD_SLOTS * GUARD_STRIDE;
-    CHK(w.guard_part.ensure(gp_bytes));
-    unsigned long long* gp = w.guard_part.as<unsigned long long>();
-    zero_i32(s, (int*)gp, (int64_t)(gp_bytes / sizeof(int)));
+    unsigned long long* gp = w.counters.as<Counters>()->guard;
+    zero_i32(s, (int*)gp, (int64_t)(sizeof(Counters::guard) / (sizeof(int))));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(8 * F.per_xcd), dim3(64), 0, s, F, w.cell_start.as<int>(),
                            w.slot_frac.as<Frac3>(), w.slot_p32.as<float4>(), w.slot_sn32.as<float>(),
@@ -684,7 +697,6 @@ static int run_voxel_apps(const d2bi_record* r, const d2bi_plan* p, const AxisTa
     if (dens) pick_row_c(std::true_type{});
     else pick_row_c(std::false_type{});
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_sum_guard, dim3(1), dim3(256), 0, s, gp, GUARD_SLOTS, GUARD_STRIDE, gc);
     return D2BI_OK;
 }
 
@@ -741,13 +753,15 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
         return D2BI_OK;
     };
     auto add_stats = [&](const Binned& b, int points) -> int {
-        int64_t hc[2] = {0, 0};
-        if (st) HIPCHK(hipMemcpyAsync(hc, w.counters.p, 16, hipMemcpyDeviceToHost, s));
+        void* hp;
+        CHK(pinned_result(sizeof(Counters), &hp));
+        const Counters* ct = (const Counters*)hp;
+        if (st) HIPCHK(hipMemcpyAsync(hp, w.counters.p, sizeof(Counters), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         if (st) {
             st->n_points += b.nr * points;
-            st->n_guard += f64 ? 0 : hc[1];
-            st->max_per_cell = std::max(st->max_per_cell, (int)(hc[0] & 0xffffffff));
+            st->n_guard += f64 ? 0 : ct->n_guard();
+            st->max_per_cell = std::max(st->max_per_cell, ct->max_per_cell);
             st->n_cells = b.ncell;
         }
         return D2BI_OK;
@@ -762,7 +776,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
             BP.fast = f64 ? 0 : 1;
             Binned b;
             CHK(run_binning(d_x, n, BP, &b, s, w));
-            CHK(run_voxel(r, &pk, tab, ax, mode, false, nullptr, s, w));
+            CHK(run_voxel(r, &pk, tab, ax, mode, false, true, s, w));
             CHK(integrate_point(app, 0, w.f32_field.p));
             CHK(add_stats(b, 1));
         }
@@ -810,7 +824,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
             }
             if (na == 1) {
                 const d2bi_plan pk = point_plan(app);
-                CHK(run_voxel(r, &pk, tab, ax, mode, false, nullptr, s, w));
+                CHK(run_voxel(r, &pk, tab, ax, mode, false, false, s, w));
                 CHK(integrate_point(app, 0, w.f32_field.p));
             } else {
                 CHK(run_voxel_apps(r, &plan, tab, ax, mode, na, variant, nr, s, w));

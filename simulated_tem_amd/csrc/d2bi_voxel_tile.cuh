@@ -11,8 +11,6 @@ namespace d2bi {
 // ------------------------------------------------------------------ (b) voxelise, FAST
 
 static constexpr int TILE_CAP = 160;                 // staged candidates per pass (lane per voxel)
-static constexpr int GUARD_SLOTS = 1024;             // guard counters (power of two) ...
-static constexpr int GUARD_STRIDE = 16;              // ... 16 x 8 B = 128 B apart
 static constexpr int TILE_MAXC = 128;                // cells in a tile's unwrapped range (<= 5^3)
 static constexpr int ROW_BLOCK = 32;                 // row kernel: steps per guard test and Kahan merge
 

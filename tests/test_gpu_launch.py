@@ -1,0 +1,64 @@
+"""Launch paths that do not wait for the host.
+
+A single condition's point arrays are sized by an estimate and the count is
+looked at when the image is done: a cluster that fills a small part of its
+supercell has many times the estimate, and its image must be that of the exact
+count.  A batch is launched as it is the first time and captured into a graph
+the second: every call gives the same images, and so do batches that take
+turns (each is new again after the other).
+"""
+import os
+
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from simulated_tem_amd import abi, imaging, synth
+
+pytestmark = pytest.mark.gpu
+
+NTH = min(16, os.cpu_count() or 1)
+
+
+def cluster():
+    """30,000 atoms in a 40 A cube amid a 240 A supercell, imaged over 24 A."""
+    cfg = synth.scaled("c0", cells=(7, 7, 7))
+    cfg.update(sg=[0.01], d=(24.0, 25.0, 23.0))
+    box = np.array([240.0, 240.0, 240.0])
+    x = 100.0 + 40.0 * np.random.default_rng(5).random((30000, 3))
+    x, conds = synth.conditions(cfg, x, box)
+    return x, conds[0][0]
+
+
+@pytest.mark.parametrize("mode,tol", [("fp64", 1e-10), ("fast", 1e-4)])
+def test_more_points_than_expected(mode, tol):
+    x, im = cluster()
+    oc = orc.Condition(im.rec, x, 0.005, 2)
+    ref = oc.image(nthreads=NTH)
+    st = abi.D2biStats()
+    first = im.computeD2BI_img(x, 0.005, 2, mode=mode, stats=st)
+    assert st.n_points == oc.n_points
+    for _ in range(2):
+        st = abi.D2biStats()
+        assert np.array_equal(im.computeD2BI_img(x, 0.005, 2, mode=mode, stats=st), first)
+        assert st.n_points == oc.n_points
+    assert np.max(np.abs(first - ref)) <= tol
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fast"])
+def test_batches_taking_turns(mode):
+    batches = []
+    for seed in (3, 4):
+        todo = []
+        for cells, density, points in (((9, 8, 10), False, 3), ((6, 7, 6), True, 1), ((8, 6, 7), False, 9)):
+            cfg = synth.scaled("c0", cells=cells)
+            cfg.update(seed=seed, density=density, sg=[0.01], n_prec=points)
+            x, box = synth.make_atoms(cfg)
+            x, conds = synth.conditions(cfg, x, box)
+            todo.append((conds[0][0], imaging.Atoms(x), 0.005, points))
+        batches.append(todo)
+    alone = [[im.computeD2BI_img(at, pa, n, mode=mode) for im, at, pa, n in b] for b in batches]
+    for turn in (0, 1, 0, 0, 0, 1, 1, 0):
+        out = imaging.computeD2BI_img_batch(batches[turn], mode=mode)
+        for got, want in zip(out, alone[turn]):
+            assert np.array_equal(got, want), turn
