@@ -17,7 +17,7 @@ namespace d2bi {
 //   cell = mod(floor(zi) + 16*Ex, Ex), zi = zi - cell
 // (neighbourList1b, Lib_LinkCell3D.f90:1549-1565).  The zero off-diagonal
 // terms of the reference's 3x3 products add +-0 and change no bit.
-static constexpr int TILE = 4;                       // FAST voxel tiles: 4 voxels along x and y (z: 4 or 8)
+static constexpr int TILE = 4;                       // FAST voxel tiles: 4 voxels along x (y and z: 4 or 8)
 
 // FP32 voxel position along one axis relative to the link cell of its
 // FAST tile's first voxel, and that cell offset
@@ -29,13 +29,13 @@ struct QL {
 // Voxel positions relative to the first link cell of their tile: table k
 // holds axis QL_AXIS[k] for tiles of QL_TILE[k] voxels along it.
 static constexpr int NQL = 5;
-static constexpr int QL_AXIS[NQL] = {0, 1, 2, 2, 0};
+static constexpr int QL_AXIS[NQL] = {0, 1, 2, 2, 1};
 static constexpr int QL_TILE[NQL] = {4, 4, 4, 8, 8};
 
 struct AxisTables {
     std::vector<int> cell[3];
     std::vector<double> zi[3];
-    std::vector<QL> ql[NQL];       // x, y, z for 4-voxel tiles; z, x for 8-voxel tiles
+    std::vector<QL> ql[NQL];       // x, y, z for 4-voxel tiles; z, y for 8-voxel tiles
     std::vector<char> packed;      // the tables as uploaded without pinned memory
 };
 

@@ -36,11 +36,10 @@ static void fill_vox_params(const d2bi_record* r, const d2bi_plan* p, const Axis
     V->ax = ax;
 }
 
-// Tile depth of a FAST kernel variant: 0 (a lane per voxel) and 1 (rows of
-// 4 x 4 x 4 tiles) use 4 voxels, 2 (rows of 4 x 4 x 8 tiles) 8.
-static int variant_tz(int variant) { return variant == 2 ? 8 : 4; }
-// Voxels along x of a variant's tiles: 8 for variant 3 (rows of 8 x 4 x 4 tiles).
-static int variant_tx(int variant) { return variant == 3 ? 8 : 4; }
+// Tile of a FAST kernel variant, 4 voxels along x: variants 0 (a lane per
+// voxel) and 1 (rows) use 4 x 4 x 4, 2 4 x 4 x 8 and 3 4 x 8 x 8.
+static int variant_tz(int variant) { return variant >= 2 ? 8 : 4; }
+static int variant_ty(int variant) { return variant == 3 ? 8 : 4; }
 
 // The order of the FAST voxel kernel's tiles over its workgroups and the
 // grid it needs (8 per_xcd workgroups): orders 0 and 1 launch one workgroup
@@ -57,13 +56,13 @@ static void set_tile_order(FastParams* F, int order)
     }
 }
 
-// Link cells in the largest unwrapped cell range of a tx x 4 x tz tile.
-static int tile_cells(const d2bi_plan* p, const AxisTables& tab, int tz, int tx = TILE)
+// Link cells in the largest unwrapped cell range of a 4 x ty x tz tile.
+static int tile_cells(const d2bi_plan* p, const AxisTables& tab, int tz, int ty = TILE)
 {
     int worst = 1;
     for (int a = 0; a < 3; a++) {
         const int M = a == 0 ? p->Mx : a == 1 ? p->My : p->Mz;
-        const int ts = a == 2 ? tz : a == 0 ? tx : TILE;
+        const int ts = a == 2 ? tz : a == 1 ? ty : TILE;
         int mx = 0;
         for (int t0 = 0; t0 < M; t0 += ts)
             mx = std::max(mx, tab.cell[a][std::min(M, t0 + ts) - 1] - tab.cell[a][t0] + 3);
@@ -72,15 +71,15 @@ static int tile_cells(const d2bi_plan* p, const AxisTables& tab, int tz, int tx 
     return worst;
 }
 
-// Launch parameters of the FAST voxel kernel for a plan, tiles of tx x 4 x tz.
+// Launch parameters of the FAST voxel kernel for a plan, tiles of 4 x ty x tz.
 static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParams& V, FastParams* Fo, int tz,
-                       int tx = TILE)
+                       int ty = TILE)
 {
     FastParams& F = *Fo;
     F.v = V;
     F.tz = tz;
-    F.ntx = (p->Mx + tx - 1) / tx;
-    F.nty = (p->My + TILE - 1) / TILE;
+    F.ntx = (p->Mx + TILE - 1) / TILE;
+    F.nty = (p->My + ty - 1) / ty;
     F.ntz = (p->Mz + tz - 1) / tz;
     F.ntiles = F.ntx * F.nty * F.ntz;
     set_tile_order(&F, 2);
@@ -106,7 +105,7 @@ static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParam
                       p->a_col[4], rc);
     F.thin_z = p->a_col[8] < thin ? 1 : 0;
     // the unwrapped cell range of a tile must fit the per-tile cell table
-    const int worst = tile_cells(p, tab, tz, tx);
+    const int worst = tile_cells(p, tab, tz, ty);
     if (worst > TILE_MAXC) return seterr(D2BI_ERR_CAPACITY, "voxel tile spans %d link cells (max %d)", worst, TILE_MAXC);
     return D2BI_OK;
 }
@@ -180,13 +179,11 @@ static int launch_voxel_fp64(const d2bi_plan* p, const AxisTables& tab, const Vo
     return D2BI_OK;
 }
 
-// Launch parameters of a variant.  A 4 x 4 x 8 tile that spans more link
-// cells than the per-tile table holds falls back to the 4 x 4 x 4 row kernel
-// (*variant becomes 1), and so does an 8 x 4 x 4 tile (variant 3) that
-// spans too many.
+// A variant whose tiles span more link cells than the per-tile table holds
+// gives way to the next smaller tile (3 to 2, 2 to 1).
 static int effective_variant(const d2bi_plan* p, const AxisTables& tab, int variant)
 {
-    if (variant == 3 && tile_cells(p, tab, 4, 8) > TILE_MAXC) variant = 1;
+    if (variant == 3 && tile_cells(p, tab, 8, 8) > TILE_MAXC) variant = 2;
     if (variant == 2 && tile_cells(p, tab, 8) > TILE_MAXC) variant = 1;
     return variant;
 }
@@ -195,16 +192,16 @@ static int variant_params(const d2bi_plan* p, const AxisTables& tab, const VoxPa
                           FastParams* F)
 {
     *variant = effective_variant(p, tab, *variant);
-    return fast_params(p, tab, V, F, variant_tz(*variant), variant_tx(*variant));
+    return fast_params(p, tab, V, F, variant_tz(*variant), variant_ty(*variant));
 }
 
 // Kernel instance for (diagnostics, density, variant); link cells thinner
 // than 3 sigma along z take a row kernel (variant 1, 2 or 3) with the
 // z-offset test.
 template <bool DENS, int ROW, class Go>
-static void pick_row(int tz, int tx, Go go)
+static void pick_row(int tz, int ty, Go go)
 {
-    if (tx == 8) go(k_voxel_tile<DENS, false, ROW, 4, 8>);
+    if (ty == 8) go(k_voxel_tile<DENS, false, ROW, 8, 8>);
     else if (tz == 8) go(k_voxel_tile<DENS, false, ROW, 8>);
     else go(k_voxel_tile<DENS, false, ROW, 4>);
 }
@@ -213,16 +210,16 @@ template <class Go>
 static void pick_tile(bool diag, bool dens, int variant, bool thin_z, Go go)
 {
     if (diag) { go(k_voxel_tile<true, true, 0, 4>); return; }
-    const int tz = variant_tz(variant), tx = variant_tx(variant);
+    const int tz = variant_tz(variant), ty = variant_ty(variant);
     if (!thin_z && variant == 0) {
         if (dens) go(k_voxel_tile<true, false, 0, 4>);
         else go(k_voxel_tile<false, false, 0, 4>);
     } else if (thin_z) {
-        if (dens) pick_row<true, 2>(tz, tx, go);
-        else pick_row<false, 2>(tz, tx, go);
+        if (dens) pick_row<true, 2>(tz, ty, go);
+        else pick_row<false, 2>(tz, ty, go);
     } else {
-        if (dens) pick_row<true, 1>(tz, tx, go);
-        else pick_row<false, 1>(tz, tx, go);
+        if (dens) pick_row<true, 1>(tz, ty, go);
+        else pick_row<false, 1>(tz, ty, go);
     }
 }
 
@@ -237,16 +234,36 @@ static void launch_tile(const FastParams& F, int variant, bool dens, const int* 
     });
 }
 
-// Choice of the FAST voxel kernel variant (0: a lane per voxel, 1: a lane
-// per row of four voxels and quarter of the candidates of a 4 x 4 x 4 tile,
-// 2: a lane per row and half of the candidates of a 4 x 4 x 8 tile).  The
-// variants sum the same atoms in different orders, so their fields agree to
-// FP32 rounding, not bit for bit; the choice is therefore fixed, variant 2
-// (the fastest on every measured workload; variant_params falls back to 1 for
-// a tile whose cell range does not fit), so that a condition images the same
-// in every process.  D2BI_FAST_VARIANT=0|1|2 forces a variant;
-// D2BI_FAST_TUNE=1 instead times all three on the first condition of each
-// voxel-grid shape and keeps the fastest (results then depend on the timing).
+// Choice of the FAST voxel kernel variant (0: a lane per voxel; rows of four
+// voxels: 1: a lane per row and quarter of the candidates of a 4 x 4 x 4 tile,
+// 2: per row and half of the candidates of a 4 x 4 x 8 tile, 3: per row of a
+// 4 x 8 x 8 tile).  The variants sum the same atoms in different orders, so
+// their fields agree to FP32 rounding, not bit for bit; the choice is
+// therefore fixed by the grid's size, so that a condition images the same in
+// every process (variant_params falls back to a smaller tile where a cell
+// range does not fit).  A larger tile stages fewer candidates per voxel, but
+// needs enough tiles to fill the chip: 16 waves of variant 3 fit a CU, 20 of
+// 1 and 2, and below a few rounds of 4096 the waves' own latency counts.
+// Measured (voxel kernel, us, variants 1/2/3 at four voxels per lattice
+// parameter; tiles of variant 3): 14^3 cells 16/20/28 (686), 20^3 25/25/31
+// (2000), 28^3 48/44/47 (5488), 36^3 82/69/70 (11664), 40^3 109/89/88 (16000),
+// 50^3 204/163/153 (31250), 150 x 150 x 100 3463/2528/2292 (562500).
+// D2BI_FAST_VARIANT=0|1|2|3 forces a variant; D2BI_FAST_TUNE=1 instead times
+// all on the first condition of each voxel-grid shape and keeps the fastest
+// (results then depend on the timing).
+static int default_variant(const d2bi_plan* p, int most = 3)
+{
+    const int64_t t2 = (int64_t)((p->Mx + 3) / 4) * ((p->My + 3) / 4) * ((p->Mz + 7) / 8);
+    const int64_t t3 = (int64_t)((p->Mx + 3) / 4) * ((p->My + 7) / 8) * ((p->Mz + 7) / 8);
+    return std::min(most, t3 >= 16000 ? 3 : t2 >= 5000 ? 2 : 1);
+}
+
+// The aperture sum's variant, the same for a shared pass and for a pass per
+// point: tiles of 4 x 8 x 8 with four points' sums leave room for two or
+// three waves per SIMD and are no faster (60 x 60 x 40 cells, eight points,
+// whole call: 1377 us, variant 2 1338, variant 1 1537).
+static constexpr int APERTURE_VARIANT = 2;
+
 static std::map<std::array<int, 7>, int> g_variant_cache;
 
 static bool tune_variants()
@@ -267,20 +284,20 @@ static int known_variant(const d2bi_plan* p, bool dens)
 {
     const int f = forced_variant();
     if (f >= 0) return f;
-    if (!tune_variants()) return 2;
+    if (!tune_variants()) return default_variant(p);
     const std::array<int, 7> key{p->Mx, p->My, p->Mz, p->Ex, p->Ey, p->Ez, dens ? 1 : 0};
     auto it = g_variant_cache.find(key);
     return it == g_variant_cache.end() ? -1 : it->second;
 }
 
 template <class TimeFn>
-static int fast_variant(const d2bi_plan* p, bool dens, bool diag, bool thin_z, TimeFn time_variant)
+static int fast_variant(const d2bi_plan* p, bool dens, bool diag, bool thin_z, int most, TimeFn time_variant)
 {
     auto& cache = g_variant_cache;
     const int f = forced_variant();
     if (f >= 0) return f;
     if (diag) return 0;
-    if (!tune_variants()) return 2;
+    if (!tune_variants()) return default_variant(p, most);
     const std::array<int, 7> key{p->Mx, p->My, p->Mz, p->Ex, p->Ey, p->Ez, dens ? 1 : 0};
     auto it = cache.find(key);
     if (it != cache.end()) return it->second;
@@ -316,9 +333,10 @@ static TuneKey tile_order_key(const d2bi_plan* p, const AxisTables& tab, bool de
 
 // Voxelise into the mode's field buffers of workspace w; optional count /
 // r2min outputs.  fresh: the workspace's guard counters are zero (they were
-// cleared for this condition's binning).
+// cleared for this condition's binning).  most: the largest variant the
+// default choice may take.
 static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables& tab, const AxisDev& ax,
-                     int mode, bool want_diag, bool fresh, hipStream_t s, Workspace& w)
+                     int mode, bool want_diag, bool fresh, hipStream_t s, Workspace& w, int most = 3)
 {
     const int64_t nvox = (int64_t)p->Mx * p->My * p->Mz;
     VoxParams V;
@@ -356,9 +374,9 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
         });
         return D2BI_OK;
     };
-    const int variant = fast_variant(p, dens, want_diag, F.thin_z != 0, [&](int v) -> float {
+    const int variant = fast_variant(p, dens, want_diag, F.thin_z != 0, most, [&](int v) -> float {
         // a variant whose tiles span too many link cells is not timed
-        if (tile_cells(p, tab, variant_tz(v), variant_tx(v)) > TILE_MAXC) return 3.4e38f;
+        if (tile_cells(p, tab, variant_tz(v), variant_ty(v)) > TILE_MAXC) return 3.4e38f;
         HIPCHK(hipEventRecord(g.ev[7], s));
         CHK(run_variant(v));
         HIPCHK(hipEventRecord(g.ev[8], s));
@@ -767,6 +785,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
         return D2BI_OK;
     };
 
+    const int most = nApp > 1 ? APERTURE_VARIANT : 3;      // a single point is the plain image
     if (!aperture_shared()) {
         // every point binned and voxelised on its own
         for (int app = 0; app < nApp; app++) {
@@ -776,7 +795,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
             BP.fast = f64 ? 0 : 1;
             Binned b;
             CHK(run_binning(d_x, n, BP, &b, s, w));
-            CHK(run_voxel(r, &pk, tab, ax, mode, false, true, s, w));
+            CHK(run_voxel(r, &pk, tab, ax, mode, false, true, s, w, most));
             CHK(integrate_point(app, 0, w.f32_field.p));
             CHK(add_stats(b, 1));
         }
@@ -791,9 +810,9 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
         CHK(run_binning(d_x, n, BP, &b, s, w));
         const int64_t nr = b.nr;
         // shared passes of four or two points: FP64, or the FAST row kernels
-        // of rows of four voxels (the default variant 2, or a forced 1 or 2)
+        // of rows (variants 1 and 2; a forced 0 or 3 walks once per point)
         int variant = forced_variant();
-        if (variant < 0) variant = 2;
+        if (variant < 0) variant = default_variant(&plan, most);
         variant = effective_variant(&plan, tab, variant);
         const int na_max = (f64 || variant == 1 || variant == 2) ? 4 : 1;
         if (na_max > 1) CHK(w.app_cs.ensure((f64 ? sizeof(double2) : sizeof(float2)) * std::max<int64_t>(nr, 1) * na_max));
@@ -824,7 +843,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
             }
             if (na == 1) {
                 const d2bi_plan pk = point_plan(app);
-                CHK(run_voxel(r, &pk, tab, ax, mode, false, false, s, w));
+                CHK(run_voxel(r, &pk, tab, ax, mode, false, false, s, w, most));
                 CHK(integrate_point(app, 0, w.f32_field.p));
             } else {
                 CHK(run_voxel_apps(r, &plan, tab, ax, mode, na, variant, nr, s, w));

@@ -10,9 +10,9 @@ namespace d2bi {
 
 // ------------------------------------------------------------------ (b) voxelise, FAST
 
-static constexpr int TILE_CAP = 160;                 // staged candidates per pass (lane per voxel)
 static constexpr int TILE_MAXC = 128;                // cells in a tile's unwrapped range (<= 5^3)
 static constexpr int ROW_BLOCK = 32;                 // row kernel: steps per guard test and Kahan merge
+static constexpr int TILE_WIN = 1024;                // candidates whose cell starts are flagged at once
 
 struct FastParams {
     VoxParams v;
@@ -26,7 +26,7 @@ struct FastParams {
     float inv_k2;               // 1 / k2
     float cellf[3];             // link-cell sides in FP32
     int thin_z;                 // link cells thinner than 3 sigma along z
-    int tz;                     // tile depth in voxels (4, or 8 for the 4 x 4 x 8 row kernel)
+    int tz;                     // tile depth in voxels
     int order;                  // tiles over workgroups: 0 contiguous ranges per XCD, 1 linear, 2 rows dealt to XCDs
     // aperture points sharing one pass (kernels with NA > 1): point a's
     // (cos, sin) of g.r at app_cs[a app_stride + slot], its field at
@@ -35,22 +35,35 @@ struct FastParams {
     int64_t app_stride, field_stride;
 };
 
-// One wave per voxel tile: 4x4x4 voxels, or 4x4x8 for the row kernel with
-// TZ = 8 (x, y, z; x fastest).  The tile's candidates are the points of
+// One wave per voxel tile: 4x4x4 voxels, 4x4x8 or 4x8x8 for the row kernel
+// (x, y, z; x fastest).  The tile's candidates are the points of
 // every link cell in the unwrapped range [cell(first voxel)-1,
 // cell(last voxel)+1] on each axis; an unwrapped cell u stands for cell
 // mod(u, E) displaced by u - mod(u, E) cells, which is exactly the periodic
 // image neighbourList1b sees through its mod() (Lib_LinkCell3D.f90:1567-1575).
 // Cells, then points, farther than 3 sigma from the tile's voxel box are
-// dropped; the rest are compacted into LDS (ballot + popcount) and every
-// voxel of the tile tests them all.
+// dropped; the rest are compacted into LDS (ballot + popcount).
+//
+// What bounds it: FP32 vector instructions, not memory or LDS (counters on
+// 800 x 800 x 400 voxels: the vector units issue all the time).  The tile
+// lists about 400 points, keeps about 127 of them, and a voxel has 28 members,
+// so the kernel is arranged to spend few instructions on a listed point, few
+// on a kept one, and to leave out most of the pairs beyond 3 sigma:
+//   - a listed point is only moved to the tile frame, culled and compacted
+//     (the Gaussian factors were once evaluated here, for a quarter of the
+//     lanes); the records are made for 64 kept candidates at a time;
+//   - the rows of voxels form groups (2 along y by TZ / 2 along z), each with
+//     its own list of the candidates within 3 sigma of its box: 59 instead of
+//     127 of a 4 x 8 x 8 tile, 59 instead of 95 of a 4 x 4 x 8;
+//   - the larger tile stages fewer points per voxel.
+// 800 x 800 x 400 voxels, ms (before all three, 4 x 4 x 8 tiles: 5.5): 5.0,
+// 4.65, 4.2; 2020 vector instructions per 128 voxels became 1300.
 //
 // Staging.  The kept non-empty cells are listed once per tile with their
 // origin in the tile frame and the offset from candidate index to point
 // slot.  Candidates are then taken 64 at a time; the cell of candidate t is
-// the number of kept cells starting at or before t, less one, found from a
-// 64-bit mask of the cells starting inside the round (a flag per lane, a
-// ballot and a popcount).
+// the number of kept cells, after the first, that start at or before t: a
+// 64-bit mask of starts, from flags set for TILE_WIN candidates at a time.
 //
 // Arithmetic.  Positions are taken relative to the tile centre c (FP32,
 // rounded once from FP64 values).  For a candidate p and voxel q the Gaussian
@@ -67,21 +80,21 @@ struct FastParams {
 // ROW = false: lane = voxel; S = sum w (cos, sin) is accumulated in blocks of
 // 32 candidates whose sums are merged with Kahan compensation.
 //
-// ROW = true: the wave is the tile's voxel rows along x (one per (y, z): 16
-// for TZ = 4, 32 for TZ = 8) times NQ candidate parts (4 or 2); lane (row, s)
-// walks candidates s, s+NQ, s+2NQ, ... for the TX voxels of its row (TX = 4,
-// or 8 for 8 x 4 x 4 tiles).  The Gaussian factorises along x:
+// ROW = true: the wave is the tile's voxel rows along x (one per (y, z): 16,
+// 32 or 64) times NQ candidate parts (4, 2 or 1); lane (row, s)
+// walks entries s, s+NQ, s+2NQ, ... of its group's list for the four voxels of
+// its row.  The Gaussian factorises along x:
 //     2^(e_i - e_rc) = X_i * 2^t,   X_i = 2^(k2 ((p_x - q_x,i)^2 + p_y^2 + p_z^2)),
 //     t = -2 k2 (p_y q_y + p_z q_z) + k2 (q_y^2 + q_z^2) - e_rc   (e_rc = k2 (3 sigma)^2),
-// and the TX x positions q_x,i are the tile's, common to every row, so
-// X_0..X_TX-1 (which carry the candidate's own y-z term) are evaluated once
+// and the four x positions q_x,i are the tile's, common to every row, so
+// X_0..X_3 (which carry the candidate's own y-z term) are evaluated once
 // per candidate when it is staged and a lane spends two FMAs and one
-// v_exp_f32 per candidate on TX voxels.  Membership e_i >= e_rc
+// v_exp_f32 per candidate on four voxels.  Membership e_i >= e_rc
 // is u_i = X_i 2^t - 1 >= 0; a block in which some |u_i| lies within the
 // guard band is walked again and the pairs of the band are re-tested in FP64,
 // correcting the sums where the FP64 test disagrees.  The parts' sums are
 // added in a fixed order through LDS at the end, after which lane (row, s)
-// holds voxels s NV .. s NV + NV - 1 of its row (NV = TX / NQ).
+// holds voxels s NV .. s NV + NV - 1 of its row (NV = 4 / NQ).
 //
 // Thin cells.  Link cells are at least 3 sigma wide along x and y (Ex <=
 // Dx/deltaM + 2 with deltaM >= 3 sigma / min(a_x, a_y)), so along those axes
@@ -94,7 +107,7 @@ struct FastParams {
 // cell of the row's along z gets weight 0 for the row.  The diagnostic kernel
 // tests the z offset of every pair when F.thin_z is set.
 //
-// Aperture points (NA = 2 or 4, row kernels with rows of four voxels): the NA
+// Aperture points (NA = 2 or 4, row kernels of 4 x 4 x TZ tiles): the NA
 // points of a condition's aperture sum share its binned points, weights and
 // membership and differ only in g.r (Lib_DynamicalTwoBeamImaging.f90:
 // 1905-1922 sums them in one neighbour loop).  Each staged candidate carries
@@ -102,7 +115,7 @@ struct FastParams {
 // guard correction is applied to each.  Point a's sums take the same terms in
 // the same order as an NA = 1 pass with that point's phases, so its field is
 // that pass's to the bit.
-template <bool DENSITY, bool DIAG, int ROW, int TZ, int TX = 4, int NA = 1>
+template <bool DENSITY, bool DIAG, int ROW, int TZ, int TY = 4, int NA = 1>
 __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __restrict__ cell_start,
                                                    const Frac3* __restrict__ slot_frac,
                                                    const float4* __restrict__ p32,
@@ -113,14 +126,20 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                                                    unsigned long long* __restrict__ guard_count)
 {
     static_assert(!(DIAG && ROW), "the diagnostic kernel tests every pair itself");
-    static_assert(TZ == 4 || (ROW && TZ == 8), "tiles of 4 x 4 x 4, or 4 x 4 x 8 for the row kernel");
-    static_assert(TX == 4 || (ROW && TX == 8 && TZ == 4), "rows of 8 voxels: 8 x 4 x 4 tiles of the row kernel");
-    static_assert(NA == 1 || ((NA == 2 || NA == 4) && ROW && TX == 4), "aperture points: 2 or 4, row kernels of 4");
-    // ROW: candidate parts per row (4 for 16 rows, 2 for 32 rows), voxels a
-    // lane finishes (4 / NQ)
-    constexpr int NQ = ROW ? (TZ == 8 ? 2 : 4) : 1;
+    static_assert(TZ == 4 || (ROW && TZ == 8), "tiles of 4 x 4 x 4, or deeper ones of the row kernel");
+    static_assert(TY == 4 || (ROW && TY == 8 && TZ == 8), "tiles of 4 x 8 x 8: a lane per row");
+    static_assert(NA == 1 || ((NA == 2 || NA == 4) && ROW && TY == 4), "aperture points: 2 or 4, tiles 4 voxels wide");
+    constexpr int TX = 4;
+    // ROW: candidate parts per row, voxels a lane finishes
+    constexpr int NQ = ROW ? 256 / (TY * TZ * TX) : 1;
     constexpr int NV = ROW ? TX / NQ : 1;
-    constexpr int XR = TX / 4;                          // float4 records of a candidate's X factors
+    // ROW: groups of rows, 2 along y and TZ / 2 along z, with a list each
+    constexpr int GLANES = NQ * TZ, GROWS = TZ;
+    constexpr int NG = ROW ? 64 / GLANES : 1;
+    constexpr int GY = TY / 2;
+    // candidates staged at once: one pass for most tiles at four voxels per
+    // lattice parameter (about 95 candidates, 127 for 4 x 8 x 8)
+    constexpr int CAP = TY == 8 ? 144 : 112;
     // XCD-aware order: consecutive workgroups go round-robin to the 8 XCDs;
     // order 0 gives each XCD a contiguous range of tiles so neighbouring
     // tiles, which read the same link cells, share one L2 (the ranges are
@@ -140,28 +159,31 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
     const VoxParams& P = F.v;
     const int tx = L % F.ntx, ty = (L / F.ntx) % F.nty, tz = L / (F.ntx * F.nty);
     const int lane = threadIdx.x;
-    const int x0 = tx * TX, y0 = ty * TILE, z0 = tz * TZ;
-    const int x1 = min(P.Mx, x0 + TX) - 1, y1 = min(P.My, y0 + TILE) - 1, z1 = min(P.Mz, z0 + TZ) - 1;
+    const int x0 = tx * TX, y0 = ty * TY, z0 = tz * TZ;
+    const int x1 = min(P.Mx, x0 + TX) - 1, y1 = min(P.My, y0 + TY) - 1, z1 = min(P.Mz, z0 + TZ) - 1;
     // the lane's row of voxels along x (y fastest) and, lane per voxel, its x
     const int rrow = ROW ? lane / NQ : (lane >> 2);
-    const int ix = x0 + (lane & 3), iy = y0 + (rrow & 3), iz = z0 + (rrow >> 2);
+    const int grp = lane / GLANES, rg = rrow & (GROWS - 1);    // ROW: the lane's group and its row there
+    const int ix = x0 + (lane & 3);
+    const int iy = y0 + (ROW ? 2 * (grp % GY) + (rg & 1) : rrow & 3);
+    const int iz = z0 + (ROW ? (TZ / 2) * (grp / GY) + (rg >> 1) : rrow >> 2);
     const bool row_act = iy <= y1 && iz <= z1;
     const bool act = ix <= x1 && row_act;
     const int jx = min(ix, x1), jy = min(iy, y1), jz = min(iz, z1);
     const QL* const qlz_tab = TZ == 8 ? P.ax.ql[3] : P.ax.ql[2];   // z relative to the tile's first cell
-    const QL* const qlx_tab = TX == 8 ? P.ax.ql[4] : P.ax.ql[0];   // x relative to the tile's first cell
+    const QL* const qly_tab = TY == 8 ? P.ax.ql[4] : P.ax.ql[1];   // y relative to the tile's first cell
 
     // origin cell of the tile; the voxel's FP32 position relative to it and
     // its cell offset (host tables)
     const int c0x = P.ax.cell[0][x0], c0y = P.ax.cell[1][y0], c0z = P.ax.cell[2][z0];
-    const QL qlx = qlx_tab[jx], qly = P.ax.ql[1][jy], qlz = qlz_tab[jz];
+    const QL qlx = P.ax.ql[0][jx], qly = qly_tab[jy], qlz = qlz_tab[jz];
     const int lcx = qlx.lc, lcy = qly.lc, lcz = qlz.lc;
     const float qx = qlx.q, qy = qly.q, qz = qlz.q;
     // the tile's voxel box: positions do not decrease with the voxel index
     // (link cells are monotonic along each axis), so its corners are the
     // first and last voxels
-    const QL ex0 = qlx_tab[x0], ex1 = qlx_tab[x1];
-    const QL ey0 = P.ax.ql[1][y0], ey1 = P.ax.ql[1][y1];
+    const QL ex0 = P.ax.ql[0][x0], ex1 = P.ax.ql[0][x1];
+    const QL ey0 = qly_tab[y0], ey1 = qly_tab[y1];
     const QL ez0 = qlz_tab[z0], ez1 = qlz_tab[z1];
     const float bx0 = ex0.q, bx1 = ex1.q, by0 = ey0.q, by1 = ey1.q, bz0 = ez0.q, bz1 = ez1.q;
     // tile-centred frame
@@ -170,11 +192,6 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
     const float qcx = qx - ccx, qcy = qy - ccy, qcz = qz - ccz;
     const float k2 = F.k2;
     const float kq2 = k2 * fmaf(qcx, qcx, fmaf(qcy, qcy, qcz * qcz));
-    // ROW: the tile's four x positions (clamped at the grid's edge), the
-    // lane's candidate part and the y-z part of its exponent
-    float qxt[TX];
-#pragma unroll
-    for (int i = 0; i < TX; i++) qxt[i] = qlx_tab[min(x0 + i, x1)].q - ccx;
     const int squart = lane & (NQ - 1);
     const float kyz = fmaf(k2, fmaf(qcy, qcy, qcz * qcz), -F.e_rc);
 
@@ -183,29 +200,47 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
     const int ncx = ex1.lc + 3, ncy = ey1.lc + 3, ncz = ez1.lc + 3;
     const int ncell = ncx * ncy * ncz;                 // <= TILE_MAXC (checked on the host)
 
-    // staged candidates: ROW = false, (-2 k2 p, k2 |p|^2) tile-centred, then
-    // (cos, sin) of g.r, slot, cell offsets; ROW = true, (X_0..X_3), then
-    // (-2 k2 p_y, -2 k2 p_z, sin, cos), then (sin, slot, cell offsets, 0),
-    // NA > 1 then (cos, sin) of the aperture points two to a record, and four
-    // zero records after the last candidate of a pass
+    // records of the staged candidates, part c of candidate j at
+    // sM[c (CAP + 1) + j]: ROW = false, (-2 k2 p, k2 |p|^2) tile-centred,
+    // then (cos, sin) of g.r; ROW = true, (X_0..X_3), then (-2 k2 p_y,
+    // -2 k2 p_z, sin, cos), NA > 1 then (cos, sin) of the aperture points two
+    // to a part.  Until its record is made part 0 holds a candidate's position
+    // in the tile frame and its cosine.  ROW = true: candidate CAP is the
+    // zero record that fills the groups' lists.
     constexpr int NPH = NA > 1 ? NA / 2 : 0;
-    constexpr int REC = ROW ? XR + 2 + NPH : 2;
-    // ROW: 96 staged candidates per pass keep the wave's LDS at 7.6 KB, so
-    // its 88 VGPRs, not LDS, bound occupancy (20 waves per CU; 128 allowed 17
-    // and ran 15 % slower on c1)
-    constexpr int CAP = ROW ? 96 : TILE_CAP;
-    constexpr int NREC = ROW ? CAP + 4 : CAP;
+    constexpr int REC = ROW ? 2 + NPH : 2;
+    constexpr int RST = CAP + 1;
+    __shared__ float4 sM[RST * REC];
     __shared__ float4 crec[TILE_MAXC];         // kept cells: origin in the tile frame, slot - index
-    __shared__ int cupk[TILE_MAXC];            // kept cells: dx | dy << 8 | dz << 16
-    __shared__ int sflag[64];                  // cells starting at a lane's candidate this round
-    __shared__ float4 sA[REC * NREC];
-    int* const cstart = reinterpret_cast<int*>(sA);    // kept cells' first candidate (before staging)
-    static_assert(sizeof(int) * TILE_MAXC <= sizeof(float4) * REC * NREC, "cstart overlay");
-    static_assert(!ROW || 3 * 64 * TX * sizeof(float) <= sizeof(float4) * REC * NREC, "row sums overlay");
+    __shared__ unsigned short cupk[TILE_MAXC]; // kept cells: dx | dy << 4 | dz << 8 (each below 16)
+    __shared__ unsigned sflag[TILE_WIN / 32];  // bit s - 1 of the window: a cell starts at candidate s
+    __shared__ int sslot[CAP];            // staged candidates' slots ...
+    __shared__ unsigned char scell[CAP + 1];     // ... and kept cells
+    __shared__ __align__(16) unsigned short slist[ROW ? NG * CAP : 8];   // groups' candidates: 16 j
+    int* const cstart = reinterpret_cast<int*>(sM);
+    // ROW: the tile's x positions and the boxes of its GY parts along y and two
+    // along z (centre and half-width of each), tile-centred; clamped at the
+    // grid's edge.  Kept in LDS: as registers, live over the whole tile, they
+    // cost a wave per SIMD.
+    __shared__ __align__(16) float sbox[ROW ? TX + 2 * GY + 4 : 4];
+    if (ROW && lane < TX) sbox[lane] = P.ax.ql[0][min(x0 + lane, x1)].q - ccx;
+    if (ROW && lane < GY + 2) {
+        const bool z = lane >= GY;
+        const int v0 = z ? z0 + TZ / 2 * (lane - GY) : y0 + 2 * lane, v1 = z ? v0 + TZ / 2 - 1 : v0 + 1;
+        const float lo = z ? qlz_tab[min(v0, z1)].q : qly_tab[min(v0, y1)].q;
+        const float hi = z ? qlz_tab[min(v1, z1)].q : qly_tab[min(v1, y1)].q;
+        const float c = 0.5f * (lo + hi);
+        sbox[TX + 2 * lane] = c - (z ? ccz : ccy);
+        sbox[TX + 2 * lane + 1] = hi - c;
+    }
+    static_assert(TILE_MAXC / (3 * 3) < 16, "cell offsets in four bits");
+    static_assert(sizeof(int) * TILE_MAXC <= sizeof(sM), "cstart overlay");
+    static_assert(NQ == 1 || 3 * 64 * TX * sizeof(float) <= sizeof(sM), "row sums overlay");
+    static_assert(16 * CAP < 65536 && CAP % 8 == 0, "list entries, 16-byte stores");
 
-    // set bits of a wave mask below this lane (v_mbcnt)
-    auto below = [](unsigned long long m) -> int {
-        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    // base plus the set bits of a wave mask below this lane (v_mbcnt)
+    auto below = [](unsigned long long m, int base) -> int {
+        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)base));
     };
 
     // kept cells: in range of the tile box and not empty, in cell order
@@ -238,17 +273,17 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                     const int rc = rx + P.Ex * (ry + P.Ey * rz);
                     b = cell_start[rc];
                     cnt = cell_start[rc + 1] - b;
-                    upk = dx | (dy << 8) | (dz << 16);
+                    upk = dx | (dy << 4) | (dz << 8);
                 }
             }
             const int incl = wave_incl_scan(cnt);
             const unsigned long long m = __ballot(cnt > 0);
             if (cnt > 0) {
-                const int k = K + below(m);
+                const int k = below(m, K);
                 const int st = T + incl - cnt;
                 cstart[k] = st;
                 crec[k] = make_float4(lx, ly, lz, __int_as_float(b - st));
-                cupk[k] = upk;
+                cupk[k] = (unsigned short)upk;
             }
             K += (int)__popcll(m);
             T += __shfl(incl, 63, 64);
@@ -263,10 +298,10 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
     __syncthreads();
 
     // exact FP64 test of neighbourList1b (Lib_LinkCell3D.f90:1565-1596) for
-    // a staged candidate (packed unwrapped cell offsets u, point slot) and
-    // the voxel of x index vx (cell offset lx) in the lane's row
-    auto exact_at = [&](int lx, int vx, int u, int slot) -> bool {
-        const int kx = (u & 255) - 1 - lx, ky = ((u >> 8) & 255) - 1 - lcy, kz = (u >> 16) - 1 - lcz;
+    // staged candidate j and the voxel of x index vx (cell offset lx) in the lane's row
+    auto exact_at = [&](int lx, int vx, int j) -> bool {
+        const int slot = sslot[j], u = cupk[scell[j]];
+        const int kx = (u & 15) - 1 - lx, ky = ((u >> 4) & 15) - 1 - lcy, kz = (u >> 8) - 1 - lcz;
         if (kx < -1 || kx > 1 || ky < -1 || ky > 1 || kz < -1 || kz > 1) return false;
         const Frac3 f = slot_frac[slot];                              // FP64 offset in cell
         const double zix = P.ax.zi[0][vx], ziy = P.ax.zi[1][jy], ziz = P.ax.zi[2][jz];
@@ -299,77 +334,108 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
 
     int t_next = 0, kbase = 0;
     while (t_next < T) {
-        // stage: compact candidates within 3 sigma of the tile box
+        // compact the candidates within 3 sigma of the tile box
         int n = 0;
-        while (t_next < T && n <= CAP - 64) {
-            // cell of candidate t_next + lane
-            sflag[lane] = 0;
-            __syncthreads();
-            if (s_lo >= t_next && s_lo < t_next + 64) sflag[s_lo - t_next] = 1;
-            if (s_hi >= t_next && s_hi < t_next + 64) sflag[s_hi - t_next] = 1;
-            __syncthreads();
-            const unsigned long long sm = __ballot(sflag[lane] != 0);
-            const int k = kbase + below(sm) + ((sm >> lane) & 1ull ? 1 : 0) - 1;
-            kbase += (int)__popcll(sm);
-            const int t = t_next + lane;
-            bool keep = false;
-            float4 r0, r1, r2, r0b, rph[NPH > 0 ? NPH : 1];
-            if (t < T) {
-                const float4 cr = crec[k];
-                const int slot = t + __float_as_int(cr.w);
-                const float4 pc = p32[slot];
-                const float px = pc.x + cr.x, py = pc.y + cr.y, pz = pc.z + cr.z;
-                const float ex = fmaxf(0.0f, fabsf(px) - hx);
-                const float ey = fmaxf(0.0f, fabsf(py) - hy);
-                const float ez = fmaxf(0.0f, fabsf(pz) - hz);
-                keep = fmaf(ex, ex, fmaf(ey, ey, ez * ez)) <= F.rc_cull2;
-                if (keep) {
-                    const float m2k = -2.0f * k2;
-                    if (ROW) {
-                        float xv[TX];
-                        const float kyzp = k2 * fmaf(py, py, pz * pz);
-#pragma unroll
-                        for (int i = 0; i < TX; i++) {
-                            const float d = px - qxt[i];
-                            xv[i] = __builtin_amdgcn_exp2f(fmaf(k2, d * d, kyzp));
-                        }
-                        r0 = make_float4(xv[0], xv[1], xv[2], xv[3]);
-                        if (TX == 8) r0b = make_float4(xv[4 % TX], xv[5 % TX], xv[6 % TX], xv[7 % TX]);
-                        r1 = make_float4(m2k * py, m2k * pz, NA == 1 ? sn32[slot] : 0.0f, pc.w);
-                        r2 = make_float4(NA == 1 ? sn32[slot] : 0.0f, __int_as_float(slot),
-                                         __int_as_float(cupk[k]), 0.0f);
-#pragma unroll
-                        for (int h = 0; h < NPH; h++) {
-                            const float2 c0 = F.app_cs[(2 * h) * F.app_stride + slot];
-                            const float2 c1 = F.app_cs[(2 * h + 1) * F.app_stride + slot];
-                            rph[h] = make_float4(c0.x, c0.y, c1.x, c1.y);
-                        }
-                    } else {
-                        r0 = make_float4(m2k * px, m2k * py, m2k * pz, k2 * fmaf(px, px, fmaf(py, py, pz * pz)));
-                        r1 = make_float4(pc.w, sn32[slot], __int_as_float(slot), __int_as_float(cupk[k]));
-                    }
-                }
+        while (t_next < T) {
+            if ((t_next & (TILE_WIN - 1)) == 0) {
+                __syncthreads();
+                if (lane < TILE_WIN / 32) sflag[lane] = 0;
+                __syncthreads();
+                const int a = s_lo - 1 - t_next, b = s_hi - 1 - t_next;
+                if ((unsigned)a < (unsigned)TILE_WIN) atomicOr(&sflag[a >> 5], 1u << (a & 31));
+                if ((unsigned)b < (unsigned)TILE_WIN) atomicOr(&sflag[b >> 5], 1u << (b & 31));
+                __syncthreads();
             }
+            // cell of candidate t: the starts after the first at or before t
+            const int wd = (t_next & (TILE_WIN - 1)) >> 5;
+            const unsigned mlo = __builtin_amdgcn_readfirstlane(sflag[wd]);
+            const unsigned mhi = __builtin_amdgcn_readfirstlane(sflag[wd + 1]);
+            const int k = below((unsigned long long)mhi << 32 | mlo, kbase);
+            const int t = min(t_next + lane, T - 1);
+            const float4 cr = crec[k];
+            const int slot = t + __float_as_int(cr.w);
+            float4 pc = p32[slot];
+            pc.x += cr.x; pc.y += cr.y; pc.z += cr.z;
+            const float ex = fmaxf(0.0f, fabsf(pc.x) - hx);
+            const float ey = fmaxf(0.0f, fabsf(pc.y) - hy);
+            const float ez = fmaxf(0.0f, fabsf(pc.z) - hz);
+            const bool keep = fmaf(ex, ex, fmaf(ey, ey, ez * ez)) <= F.rc_cull2 && t_next + lane < T;
             const unsigned long long m = __ballot(keep);
+            const int nk = (int)__popcll(m);
+            if (n + nk > CAP) break;                  // these 64 open the next pass
             if (keep) {
-                const int p = n + below(m);
-                sA[REC * p] = r0;
-                if (ROW && TX == 8) sA[REC * p + 1] = r0b;
-                sA[REC * p + (ROW ? XR : 1)] = r1;
-                if (ROW) sA[REC * p + XR + 1] = r2;
-#pragma unroll
-                for (int h = 0; h < NPH; h++) sA[REC * p + XR + 2 + h] = rph[h];
+                const int p = below(m, n);
+                sM[p] = pc;
+                sslot[p] = slot;
+                scell[p] = (unsigned char)k;
             }
-            n += (int)__popcll(m);
+            n += nk;
+            kbase += __popc(mlo) + __popc(mhi);
             t_next += 64;
         }
-        n = __builtin_amdgcn_readfirstlane(n);
-        if (ROW && lane < 4) {
-            // zero records after the last candidate: X = 0, never a member
-            // and never in the guard band (u = -1)
-            const float4 z4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        __syncthreads();
+        // records, one candidate per lane, and the groups' lists of the
+        // candidates within 3 sigma of their voxels, filled up with the zero
+        // record (X = 0: never a member and never in the guard band, u = -1)
+        int gn[NG] = {0};
+        if (ROW) {
+            const unsigned z2 = 16u * CAP * 0x10001u;
+            for (int k = lane; k < NG * CAP / 8; k += 64) reinterpret_cast<uint4*>(slist)[k] = make_uint4(z2, z2, z2, z2);
+            if (lane < REC) sM[lane * RST + CAP] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (ROW == 2 && lane == 0) scell[CAP] = 0;
+            __syncthreads();
+        }
+        for (int jb = 0; jb < n; jb += 64) {
+            const bool live = jb + lane < n;
+            const int j = live ? jb + lane : n - 1;
+            const float4 pc = sM[j];
+            const int slot = sslot[j];
+            const float m2k = -2.0f * k2;
+            const float sn = NA == 1 ? sn32[slot] : 0.0f;
+            if (ROW) {
+                float ey2[GY], ez2[2];
+                const float ex = fmaxf(0.0f, fabsf(pc.x) - hx), ex2 = live ? ex * ex : 3.4028234663852886e38f;
 #pragma unroll
-            for (int k = 0; k < REC; k++) sA[REC * (n + lane) + k] = z4;
+                for (int h = 0; h < GY; h++) {
+                    const float ey = fmaxf(0.0f, fabsf(pc.y - sbox[TX + 2 * h]) - sbox[TX + 2 * h + 1]);
+                    ey2[h] = fmaf(ey, ey, ex2);
+                }
+#pragma unroll
+                for (int h = GY; h < GY + 2; h++) {
+                    const float ez = fmaxf(0.0f, fabsf(pc.z - sbox[TX + 2 * h]) - sbox[TX + 2 * h + 1]);
+                    ez2[h - GY] = ez * ez;
+                }
+#pragma unroll
+                for (int g = 0; g < NG; g++) {
+                    const bool in = ey2[g % GY] + ez2[g / GY] <= F.rc_cull2;
+                    const unsigned long long m = __ballot(in);
+                    if (in) slist[g * CAP + below(m, gn[g])] = (unsigned short)(16 * j);
+                    gn[g] += (int)__popcll(m);
+                }
+            }
+            if (live) {
+                if (ROW) {
+                    const float kyzp = k2 * fmaf(pc.y, pc.y, pc.z * pc.z);
+                    float xv[TX];
+#pragma unroll
+                    for (int i = 0; i < TX; i++) {
+                        const float d = pc.x - sbox[i];
+                        xv[i] = __builtin_amdgcn_exp2f(fmaf(k2, d * d, kyzp));
+                    }
+                    sM[j] = make_float4(xv[0], xv[1], xv[2], xv[3]);
+                    sM[RST + j] = make_float4(m2k * pc.y, m2k * pc.z, sn, pc.w);
+#pragma unroll
+                    for (int h = 0; h < NPH; h++) {
+                        const float2 c0 = F.app_cs[(2 * h) * F.app_stride + slot];
+                        const float2 c1 = F.app_cs[(2 * h + 1) * F.app_stride + slot];
+                        sM[(2 + h) * RST + j] = make_float4(c0.x, c0.y, c1.x, c1.y);
+                    }
+                } else {
+                    sM[j] = make_float4(m2k * pc.x, m2k * pc.y, m2k * pc.z,
+                                        k2 * fmaf(pc.x, pc.x, fmaf(pc.y, pc.y, pc.z * pc.z)));
+                    sM[RST + j] = make_float4(pc.w, sn, 0.0f, 0.0f);
+                }
+            }
         }
         __syncthreads();
         if (DIAG) {
@@ -379,15 +445,15 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                 const int je = min(jb + 16, n);
                 float pr = 0.0f, pi = 0.0f;
                 for (int j = jb; j < je; j++) {
-                    const float4 A = sA[REC * j];
-                    const float4 C = sA[REC * j + 1];
+                    const float4 A = sM[j];
+                    const float4 C = sM[RST + j];
                     const float e = fmaf(A.x, qcx, fmaf(A.y, qcy, fmaf(A.z, qcz, A.w + kq2)));
                     bool in = act && e >= F.e_rc;
                     if (act && fabsf(e - F.e_rc) <= F.e_band) {
                         nguard++;
-                        in = exact_at(lcx, jx, __float_as_int(C.w), __float_as_int(C.z));
+                        in = exact_at(lcx, jx, j);
                     }
-                    if (F.thin_z) in = in && (unsigned)((__float_as_int(C.w) >> 16) - lcz) <= 2u;
+                    if (F.thin_z) in = in && (unsigned)((cupk[scell[j]] >> 8) - lcz) <= 2u;
                     const float w = in ? __builtin_amdgcn_exp2f(e) : 0.0f;
                     pr = fmaf(w, C.x, pr);
                     pi = fmaf(w, C.y, pi);
@@ -409,8 +475,8 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                 float pr = 0.0f, pi = 0.0f, dmin = 3.4028234663852886e38f;
 #pragma unroll 4
                 for (int j = jb; j < je; j++) {
-                    const float4 A = sA[REC * j];
-                    const float4 C = sA[REC * j + 1];
+                    const float4 A = sM[j];
+                    const float4 C = sM[RST + j];
                     const float t = fmaf(A.x, qcx, fmaf(A.y, qcy, fmaf(A.z, qcz, A.w + kq2r)));
                     const float w = t >= 0.0f ? __builtin_amdgcn_exp2f(t) : 0.0f;
                     pr = fmaf(w, C.x, pr);
@@ -421,13 +487,13 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                 if (__ballot(dmin <= F.e_band)) {
                     pr = 0.0f; pi = 0.0f;
                     for (int j = jb; j < je; j++) {
-                        const float4 A = sA[REC * j];
-                        const float4 C = sA[REC * j + 1];
+                        const float4 A = sM[j];
+                        const float4 C = sM[RST + j];
                         const float t = fmaf(A.x, qcx, fmaf(A.y, qcy, fmaf(A.z, qcz, A.w + kq2r)));
                         bool in = t >= 0.0f;
                         if (fabsf(t) <= F.e_band) {
                             nguard++;
-                            in = exact_at(lcx, jx, __float_as_int(C.w), __float_as_int(C.z));
+                            in = exact_at(lcx, jx, j);
                         }
                         const float w = in ? __builtin_amdgcn_exp2f(t) : 0.0f;
                         pr = fmaf(w, C.x, pr);
@@ -448,30 +514,35 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
             // sums with Kahan compensation, and so are the re-walk's
             // corrections (the block sums are not live across the re-walk,
             // which sets the register peak).
-            const int nst = (n + NQ - 1) / NQ;
-            auto step = [](float u) { return __builtin_amdgcn_fmed3f(u * 1099511627776.0f, 0.0f, 1.0f); };
-            // the X factors of staged candidate j
-            auto load_x = [&](int j, float* xv) {
+            int gmax = gn[0];
 #pragma unroll
-                for (int c = 0; c < XR; c++) {
-                    const float4 X = sA[REC * j + c];
-                    xv[4 * c] = X.x; xv[4 * c + 1] = X.y; xv[4 * c + 2] = X.z; xv[4 * c + 3] = X.w;
-                }
+            for (int g = 1; g < NG; g++) gmax = max(gmax, gn[g]);
+            const int nst = (gmax + NQ - 1) / NQ;
+            const unsigned short* const list = slist + grp * CAP + squart;
+            auto step = [](float u) { return __builtin_amdgcn_fmed3f(u * 1099511627776.0f, 0.0f, 1.0f); };
+            // part c of the candidate with list entry e
+            auto part = [&](int e, int c) -> float4 {
+                return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(sM) + e + 16 * RST * c);
             };
-            // the (cos, sin) pairs of staged candidate j (B = its record XR,
-            // sn its sine when NA = 1)
-            auto load_ph = [&](int j, const float4& B, float sn, float* pc, float* ps) {
+            auto load_x = [&](int e, float* xv) {
+                const float4 X = part(e, 0);
+                xv[0] = X.x; xv[1] = X.y; xv[2] = X.z; xv[3] = X.w;
+            };
+            // its (cos, sin) pairs (B = its part 1)
+            auto load_ph = [&](int e, const float4& B, float* pc, float* ps) {
                 if (NA == 1) {
                     pc[0] = B.w;
-                    ps[0] = sn;
+                    ps[0] = B.z;
                 } else {
 #pragma unroll
                     for (int h = 0; h < NPH; h++) {
-                        const float4 Ph = sA[REC * j + XR + 2 + h];
+                        const float4 Ph = part(e, 2 + h);
                         pc[2 * h] = Ph.x; ps[2 * h] = Ph.y; pc[2 * h + 1] = Ph.z; ps[2 * h + 1] = Ph.w;
                     }
                 }
             };
+            // z offset of its cell
+            auto zoff = [&](int e) -> int { return cupk[scell[e >> 4]] >> 8; };
             for (int kb = 0; kb < nst; kb += ROW_BLOCK) {
                 const int ke = min(kb + ROW_BLOCK, nst);
                 float dmin = 3.4028234663852886e38f;
@@ -482,18 +553,16 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                     for (int a = 0; a < NA; a++) { bre[a][i] = 0.0f; bim[a][i] = 0.0f; }
 #pragma unroll 2
                 for (int kk = kb; kk < ke; kk++) {
-                    const int j = NQ * kk + squart;
+                    const int e = list[NQ * kk];
                     float xv[TX];
-                    load_x(j, xv);
-                    const float4 B = sA[REC * j + XR];
+                    load_x(e, xv);
+                    const float4 B = part(e, 1);
                     float E = __builtin_amdgcn_exp2f(fmaf(B.x, qcy, fmaf(B.y, qcz, kyz)));
-                    const float sn = B.z;
                     if (ROW == 2) {
-                        const float4 C = sA[REC * j + XR + 1];
-                        E = (unsigned)((__float_as_int(C.z) >> 16) - lcz) <= 2u ? E : 0.0f;
+                        E = (unsigned)(zoff(e) - lcz) <= 2u ? E : 0.0f;
                     }
                     float pc[NA], ps[NA];
-                    load_ph(j, B, sn, pc, ps);
+                    load_ph(e, B, pc, ps);
 #pragma unroll
                     for (int i = 0; i < TX; i++) {
                         const float u = fmaf(xv[i], E, -1.0f);
@@ -517,13 +586,12 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                     }
                 if (__ballot(dmin <= F.e_band)) {
                     for (int kk = kb; kk < ke; kk++) {
-                        const int j = NQ * kk + squart;
+                        const int e = list[NQ * kk];
                         float xv[TX];
-                        load_x(j, xv);
-                        const float4 B = sA[REC * j + XR];
-                        const float4 C = sA[REC * j + XR + 1];
+                        load_x(e, xv);
+                        const float4 B = part(e, 1);
                         float E = __builtin_amdgcn_exp2f(fmaf(B.x, qcy, fmaf(B.y, qcz, kyz)));
-                        if (ROW == 2) E = (unsigned)((__float_as_int(C.z) >> 16) - lcz) <= 2u ? E : 0.0f;
+                        if (ROW == 2) E = (unsigned)(zoff(e) - lcz) <= 2u ? E : 0.0f;
 #pragma unroll
                         for (int i = 0; i < TX; i++) {
                             const float u = fmaf(xv[i], E, -1.0f);
@@ -531,13 +599,12 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                                 const int vx = min(x0 + i, x1);
                                 // one re-test per aperture point it settles
                                 if (row_act && x0 + i <= x1) nguard += NA;
-                                const bool in = exact_at(qlx_tab[vx].lc, vx, __float_as_int(C.z),
-                                                         __float_as_int(C.y));
+                                const bool in = exact_at(P.ax.ql[0][vx].lc, vx, e >> 4);
                                 // replace the pass's s (u + 1) by the exact test's weight
                                 const float s = step(u);
                                 const float d = (in ? u + 1.0f : 0.0f) - fmaf(s, u, s);
                                 float pc[NA], ps[NA];
-                                load_ph(j, B, C.x, pc, ps);
+                                load_ph(e, B, pc, ps);
 #pragma unroll
                                 for (int a = 0; a < NA; a++) {
                                     kahan_add(rre[a][i], kre[a][i], d * pc[a]);
@@ -555,9 +622,9 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
     // the lane's voxels: ROW, voxels s NV .. s NV + NV - 1 of its row, from
     // the parts' sums added in part order through LDS; otherwise its own
     float vre[NA][NV], vim[NA][NV], vem[NV];
-    if (ROW) {
-        float2* red = reinterpret_cast<float2*>(sA);                  // [64 lanes][TX voxels]
-        float* redm = reinterpret_cast<float*>(sA) + 2 * 64 * TX;     // [64 lanes][TX voxels]
+    if (ROW && NQ > 1) {
+        float2* red = reinterpret_cast<float2*>(sM);                  // [64 lanes][TX voxels]
+        float* redm = reinterpret_cast<float*>(sM) + 2 * 64 * TX;     // [64 lanes][TX voxels]
         const int rb = lane & ~(NQ - 1);
 #pragma unroll
         for (int ap = 0; ap < NA; ap++) {
@@ -585,6 +652,16 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                 if (ap == 0)
                     vem[t] = (DENSITY && um > -1.0f) ? __builtin_amdgcn_logf(um + 1.0f) : -3.4028234663852886e38f;
             }
+        }
+    } else if (ROW) {
+#pragma unroll
+        for (int t = 0; t < NV; t++) {
+#pragma unroll
+            for (int ap = 0; ap < NA; ap++) {
+                vre[ap][t] = rre[ap][t];
+                vim[ap][t] = rim[ap][t];
+            }
+            vem[t] = (DENSITY && umax[t] > -1.0f) ? __builtin_amdgcn_logf(umax[t] + 1.0f) : -3.4028234663852886e38f;
         }
     } else {
         vre[0][0] = sre;
