@@ -11,11 +11,17 @@ namespace d2bi {
 
 // ------------------------------------------------------------------ (c) integrate
 
+// Points of one FAST integration launch, over all its fields, and the slots of
+// their deviations (a wave of NP points may read NP - 1 past its field's last).
+static constexpr int INT_POINTS = 32, INT_SLOTS = INT_POINTS + 31;
+
 struct FastIntParams {
-    int Mx, My, Mz, np;         // np: precession points in this pass
+    int Mx, My, Mz, np;         // np: precession points per field
+    int nsplit, split;          // waves per column, of them per field
     float b0, bg, dz;
-    float aa[32];               // 2 pi s_g per precession point
-    float al[32];               // 2 dz aa (k_integrate_poly)
+    int64_t stride;             // records from one field to the next
+    float aa[INT_SLOTS];        // 2 pi s_g per field and precession point
+    float al[INT_SLOTS];        // 2 dz aa (the shared step matrix)
 };
 
 __device__ __forceinline__ float fm(float a, float b, float c) { return fmaf(a, b, c); }
@@ -35,11 +41,15 @@ struct FastColumn {
     {
         const int64_t o = col + plane * (k == nz ? 0 : k);
         typedef float v2 __attribute__((ext_vector_type(2)));
-        typedef float v4 __attribute__((ext_vector_type(4)));
         if (DENS) {
-            const v4* f = static_cast<const v4*>(field) + o;
-            const v4 v = NT ? __builtin_nontemporal_load(f) : *f;
-            return make_float4(v.x, v.y, v.z, v.w);
+            // three words of the record: the fourth's register, free for other
+            // use at once, would make that use wait for the load in flight (8
+            // points: 73 us with three words, 85 with four)
+            const float* f = static_cast<const float*>(field) + 4 * o;
+            if (NT)
+                return make_float4(__builtin_nontemporal_load(f), __builtin_nontemporal_load(f + 1),
+                                   __builtin_nontemporal_load(f + 2), 0.0f);
+            return make_float4(f[0], f[1], f[2], 0.0f);
         }
         const v2* f = static_cast<const v2*>(field) + o;
         const v2 v = NT ? __builtin_nontemporal_load(f) : *f;
@@ -155,28 +165,6 @@ __device__ __forceinline__ double intensity_sum(int np, const T* p0r, const T* p
     return acc;
 }
 
-template <int NP>
-__device__ __forceinline__ void store_mean(int np, const float* p0r, const float* p0i, const float* pgr,
-                                           const float* pgi, double* __restrict__ img, int64_t col, int accumulate,
-                                           double inv_total)
-{
-    const double acc = intensity_sum<NP>(np, p0r, p0i, pgr, pgi) * inv_total;
-    img[col] = accumulate ? img[col] + acc : acc;
-}
-
-template <int NP, bool DENS>
-__global__ __launch_bounds__(256) void k_integrate_fast(FastIntParams P, const void* __restrict__ field,
-                                                        double* __restrict__ img, int accumulate,
-                                                        double inv_total)
-{
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t plane = (int64_t)P.Mx * P.My;
-    if (col >= plane) return;
-    float p0r[NP], p0i[NP], pgr[NP], pgi[NP];
-    march_stage<NP>(FastColumn<DENS, true>{field, col, plane, P.Mz, P.b0, P.bg}, P.Mz, P.dz, P.aa, p0r, p0i, pgr, pgi);
-    store_mean<NP>(P.np, p0r, p0i, pgr, pgi, img, col, accumulate, inv_total);
-}
-
 // Many precession points.  The system is phi' = i H(a) phi with
 // H(a) = [[c0, cg], [conj(cg), c0 + a]] (the derivative above), so one RK4
 // double step is phi <- M phi with
@@ -190,7 +178,7 @@ __global__ __launch_bounds__(256) void k_integrate_fast(FastIntParams P, const v
 // They are formed once per double step and shared: a precession point then
 // costs a Horner evaluation at its alpha and one matrix-vector product
 // (~40 FMAs) instead of four derivative evaluations and the stage updates
-// (~80).  Results differ from k_integrate_fast by rounding only.
+// (~80).  Results differ from the stage-by-stage march by rounding only.
 template <class T>
 struct cplx {
     T r, i;
@@ -362,17 +350,53 @@ __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al
     }
 }
 
-template <int NP, bool DENS>
-__global__ __launch_bounds__(256) void k_integrate_poly(FastIntParams P, const void* __restrict__ field,
-                                                        double* __restrict__ img, int accumulate,
-                                                        double inv_total)
+// Largest workgroup of an instance: what its registers leave room for.
+constexpr int int_threads(int np) { return np <= 2 ? 1024 : np <= 4 ? 512 : 256; }
+
+// FAST integration: one lane per pixel column and NP precession points, marched
+// stage by stage or (POLY) through the shared step matrix.  A column's points,
+// and those of several fields (the aperture points of one voxel pass), are
+// split over P.nsplit waves of its workgroup, P.split per field; the waves'
+// sums are scaled and added to the image in order.  One wave of the split
+// gives the bits of a launch of its own that adds to the image.
+//
+// Bound: one point, HBM; more, the FP32 vector units, and how evenly the waves
+// fill them: a wave alone on its SIMD issues an operation every 4.5 cycles,
+// several together one every 2.6, and 400 x 400 columns are 2500 waves for
+// 1024 SIMDs.  Splitting a column's points over waves evens the load, and
+// gives small images parallelism.
+template <int NP, bool DENS, bool POLY, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? int_threads(NP) : 256) void k_integrate_fast(FastIntParams P,
+                                                                                const void* __restrict__ field,
+                                                                                double* __restrict__ img,
+                                                                                int accumulate, double inv_total)
 {
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t plane = (int64_t)P.Mx * P.My;
-    if (col >= plane) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int ns = SPLIT ? P.nsplit : 1, cg = SPLIT ? wave / ns : wave, sp = SPLIT ? wave - cg * ns : 0;
+    const int ncg = (int)(blockDim.x >> 6) / ns;
+    const int64_t col = ((int64_t)blockIdx.x * ncg + cg) * 64 + lane;
+    const bool live = col < plane;
+    if (!SPLIT && !live) return;
+    const int fld = SPLIT ? sp / P.split : 0, p0 = SPLIT ? (sp - fld * P.split) * NP : 0, at = fld * P.np + p0;
+    const FastColumn<DENS, !SPLIT && !POLY> s{field, (live ? col : plane - 1) + fld * P.stride, plane, P.Mz, P.b0, P.bg};
     float p0r[NP], p0i[NP], pgr[NP], pgi[NP];
-    march_poly<NP>(FastColumn<DENS, false>{field, col, plane, P.Mz, P.b0, P.bg}, P.Mz, P.dz, P.al, p0r, p0i, pgr, pgi);
-    store_mean<NP>(P.np, p0r, p0i, pgr, pgi, img, col, accumulate, inv_total);
+    if constexpr (POLY) march_poly<NP>(s, P.Mz, P.dz, P.al + at, p0r, p0i, pgr, pgi);
+    else march_stage<NP>(s, P.Mz, P.dz, P.aa + at, p0r, p0i, pgr, pgi);
+    double acc = intensity_sum<NP>(min(NP, P.np - p0), p0r, p0i, pgr, pgi) * inv_total;
+    if constexpr (SPLIT) {
+        __shared__ double part[int_threads(NP)];
+        part[threadIdx.x] = acc;
+        __syncthreads();
+        if (sp > 0 || !live) return;
+        for (int k = 0; k < ns; k++) {
+            const double v = part[threadIdx.x + 64 * k];
+            acc = k > 0 ? acc + v : accumulate ? img[col] + v : v;
+        }
+        img[col] = acc;
+    } else {
+        img[col] = accumulate ? img[col] + acc : acc;
+    }
 }
 
 // ------------------------------------------------------------------ (c) integrate, FP64

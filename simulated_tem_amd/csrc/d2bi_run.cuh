@@ -400,20 +400,19 @@ static int run_voxel(const d2bi_record* r, const d2bi_plan* p, const AxisTables&
     return D2BI_OK;
 }
 
-// FAST integration of 8 or more precession points per pass through the
-// shared step matrix (k_integrate_poly); D2BI_FAST_INTEGRATOR=stage keeps the
-// stage-by-stage march for every pass.
+// FAST integration of 8 or more precession points per launch through the
+// shared step matrix, also where a column's points are split over waves that
+// fewer would march faster stage by stage (its images are nearer the FP64
+// ones: relative rms 4.3e-7 against 5.3e-7, 180^3 voxels, 8 points);
+// D2BI_FAST_INTEGRATOR=stage marches every point stage by stage.
 static bool fast_integrator_poly()
 {
     const char* e = std::getenv("D2BI_FAST_INTEGRATOR");
     return !(e && std::strcmp(e, "stage") == 0);
 }
 
-// Points of the next FAST integration pass when `left` remain.
-static int pass_points(int left)
-{
-    return left >= 32 ? 32 : left >= 16 ? 16 : left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
-}
+// Points of the next FAST integration launch when `left` remain.
+static int pass_points(int left) { return std::min(left, INT_POINTS); }
 
 // Tuner key of the FAST integrators' workgroup size for a pass of np points.
 static TuneKey int_block_key(const d2bi_plan* p, int np, bool dens)
@@ -436,57 +435,122 @@ static bool condition_tuned(const d2bi_plan* p, const AxisTables& tab, bool dens
     return true;
 }
 
-// One pass of the FAST integrators over NP points, workgroups of `block`
-// threads (a lane per pixel column; any block size gives the same image).
-template <int NP>
-static void launch_int_fast(const FastIntParams& P, bool dens, const void* field, double* img, int acc,
-                            double inv, int block, hipStream_t s)
+// How a FAST integration of np points over `plane` columns is split: points
+// per wave, waves per column, column groups per workgroup.
+struct IntSplit {
+    int n, ns, cg;
+};
+
+// The cheapest split by a model of k_integrate_fast: vector operations per
+// wave and double step (85 per point stage by stage, 40 per point after 230
+// through the step matrix, 60 for the density) times the cycles one takes on
+// the fullest SIMD (4.8 for a wave alone, 3.1 per wave together), workgroups
+// dealt to 256 CUs and a workgroup's waves to their four SIMDs; `waves` is
+// what an instance's registers let a SIMD hold.  More waves per column have to
+// win 7 %.  Measured, us by points per wave: 400 x 400 columns of 120 samples,
+// 5 points 1/2/4: 107/106/126, 32 points 8/16/32: 377/321/370; 80 x 80 of 80,
+// 5 points 1/2/4: 17/21/31; 800 x 800 of 120, 5 points 1/4/5: 353/447/285, 32
+// points 8/16/32: 1471/1215/1128; 236 x 268, 8 points of 4 per wave, 65 with
+// workgroups of two column groups, 95 of one.  Powers of two in passes, one
+// wave per column, took 110, 380, 40, 338, 1185 and 70.
+static IntSplit int_split(int64_t plane, int np, bool dens)
 {
-    const int64_t plane = (int64_t)P.Mx * P.My;
-    const dim3 grid((unsigned)((plane + block - 1) / block)), thr(block);
-    // from 8 points on, the shared step matrix costs less than it saves
-    if constexpr (NP >= 8) {
-        if (fast_integrator_poly()) {
-            if (dens) hipLaunchKernelGGL((k_integrate_poly<NP, true>), grid, thr, 0, s, P, field, img, acc, inv);
-            else hipLaunchKernelGGL((k_integrate_poly<NP, false>), grid, thr, 0, s, P, field, img, acc, inv);
-            return;
+    struct Inst {
+        int n, waves;
+    };
+    static const Inst stage[] = {{7, 7}, {6, 8}, {5, 8}, {4, 5}, {3, 6}, {2, 7}, {1, 7}};
+    static const Inst matrix[] = {{32, 2}, {16, 3}, {8, 4}, {4, 5}, {2, 5}};
+    const bool poly = np >= 8 && fast_integrator_poly();
+    const int64_t groups = (plane + 63) / 64;
+    IntSplit best{0, 1, 4};
+    double cost = 1.0e300;
+    for (int i = 0; i < (poly ? 5 : 7); i++) {
+        const int n = poly ? matrix[i].n : stage[i].n, waves = poly ? matrix[i].waves : stage[i].waves;
+        const int ns = (np + n - 1) / n, most = int_threads(n) / 64 / ns;
+        const double ops = (poly ? 230 + 40 * n : 15 + 85 * n) + (dens ? 60 : 0);
+        for (int cg = ns > 1 ? 1 : 4; cg <= (ns > 1 ? most : 4); cg++) {
+            const int64_t load = ((groups + cg - 1) / cg + 255) / 256 * ((ns * cg + 3) / 4);
+            auto cyc = [](int w) { return w > 0 ? std::max(4.8, 3.1 * w) : 0.0; };
+            const double c = ops * ((double)(load / waves) * cyc(waves) + cyc((int)(load % waves)));
+            if (c < (ns > best.ns ? 0.93 : 1.0) * cost) {
+                cost = c;
+                best = IntSplit{n, ns, cg};
+            }
         }
     }
-    if (dens) hipLaunchKernelGGL((k_integrate_fast<NP, true>), grid, thr, 0, s, P, field, img, acc, inv);
-    else hipLaunchKernelGGL((k_integrate_fast<NP, false>), grid, thr, 0, s, P, field, img, acc, inv);
+    return best;
 }
 
-static void launch_int_pass(int np, const FastIntParams& P, bool dens, const void* f, double* img, int acc,
-                            double inv, int block, hipStream_t s)
+// Whether one launch integrates nf fields of np points each: their
+// deviations fit its parameters and a column's waves one workgroup.
+static bool fields_fit(int64_t plane, int np, int nf, bool dens)
 {
-    switch (np) {
-        case 32: launch_int_fast<32>(P, dens, f, img, acc, inv, block, s); break;
-        case 16: launch_int_fast<16>(P, dens, f, img, acc, inv, block, s); break;
-        case 8: launch_int_fast<8>(P, dens, f, img, acc, inv, block, s); break;
-        case 4: launch_int_fast<4>(P, dens, f, img, acc, inv, block, s); break;
-        case 2: launch_int_fast<2>(P, dens, f, img, acc, inv, block, s); break;
-        default: launch_int_fast<1>(P, dens, f, img, acc, inv, block, s); break;
+    const IntSplit sp = int_split(plane, np, dens);
+    return nf * np <= INT_POINTS && 64 * nf * sp.ns <= int_threads(sp.n);
+}
+
+// One FAST integration launch, workgroups of about `block` threads (any size
+// gives the same image).
+static void launch_int_pass(FastIntParams P, int nf, bool dens, const void* f, double* img, int acc, double inv,
+                            int block, hipStream_t s)
+{
+    const int64_t plane = (int64_t)P.Mx * P.My;
+    const bool poly = P.np >= 8 && fast_integrator_poly();
+    const IntSplit sp = int_split(plane, P.np, dens);
+    P.split = sp.ns;
+    P.nsplit = nf * sp.ns;
+    // `block` sizes the workgroups of unsplit columns
+    const int cg = P.nsplit == 1 ? std::max(1, block / 64) : std::max(1, sp.cg / nf);
+    const dim3 grid((unsigned)((plane + 64 * cg - 1) / (64 * cg))), thr(64 * cg * P.nsplit);
+    auto go = [&](auto np_c, auto poly_c) {
+        constexpr int N = decltype(np_c)::value;
+        constexpr bool M = decltype(poly_c)::value;
+        auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, thr, 0, s, P, f, img, acc, inv); };
+        if (P.nsplit > 1 && dens) run(k_integrate_fast<N, true, M, true>);
+        else if (P.nsplit > 1) run(k_integrate_fast<N, false, M, true>);
+        else if (dens) run(k_integrate_fast<N, true, M, false>);
+        else run(k_integrate_fast<N, false, M, false>);
+    };
+    const std::true_type t{};
+    const std::false_type f_{};
+    switch (poly ? -sp.n : sp.n) {
+        case 1: go(std::integral_constant<int, 1>{}, f_); break;
+        case 2: go(std::integral_constant<int, 2>{}, f_); break;
+        case 3: go(std::integral_constant<int, 3>{}, f_); break;
+        case 4: go(std::integral_constant<int, 4>{}, f_); break;
+        case 5: go(std::integral_constant<int, 5>{}, f_); break;
+        case 6: go(std::integral_constant<int, 6>{}, f_); break;
+        case 7: go(std::integral_constant<int, 7>{}, f_); break;
+        case -2: go(std::integral_constant<int, 2>{}, t); break;
+        case -4: go(std::integral_constant<int, 4>{}, t); break;
+        case -8: go(std::integral_constant<int, 8>{}, t); break;
+        case -16: go(std::integral_constant<int, 16>{}, t); break;
+        default: go(std::integral_constant<int, 32>{}, t); break;
     }
 }
 
-// FAST integration of all precession points, in passes of up to 32.
+// FAST integration of all precession points, INT_POINTS a launch.
 // dens: the field holds float4 {x, rho} (density field on), else float2 x.
 // acc_in: add to d_img from the first pass on; inv: weight of one
 // integration (0: 1/nPrec).  tune_ws: a workspace whose tune_img buffer may
 // grow, for timing the workgroup sizes of a pass that adds to d_img (null:
-// such a pass is not timed).
+// such a pass is not timed).  nf > 1: fields at a stride of `stride` records
+// with nPrec deviations each in aa (fields_fit), one launch for all.
 static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, double* d_img, hipStream_t s,
-                                 bool acc_in = false, double inv = 0.0, Workspace* tune_ws = nullptr)
+                                 bool acc_in = false, double inv = 0.0, Workspace* tune_ws = nullptr, int nf = 1,
+                                 int64_t stride = 0, const double* aa = nullptr)
 {
+    if (!aa) aa = p->aa;
     if (inv == 0.0) inv = 1.0 / p->nPrec;
     for (int p0 = 0, first = acc_in ? 0 : 1; p0 < p->nPrec; first = 0) {
         const int np = pass_points(p->nPrec - p0);
         FastIntParams P;
         P.Mx = p->Mx; P.My = p->My; P.Mz = p->Mz; P.np = np;
         P.b0 = (float)p->b0; P.bg = (float)p->bg; P.dz = (float)p->dz;
-        for (int i = 0; i < 32; i++) {
-            P.aa[i] = i < np ? (float)p->aa[p0 + i] : 0.0f;
-            P.al[i] = i < np ? (float)(2.0 * p->dz * p->aa[p0 + i]) : 0.0f;
+        P.stride = stride;
+        for (int i = 0; i < INT_SLOTS; i++) {
+            P.aa[i] = i < nf * np ? (float)aa[p0 + i] : 0.0f;
+            P.al[i] = i < nf * np ? (float)(2.0 * p->dz * aa[p0 + i]) : 0.0f;
         }
         // workgroup size: timed on a launch that writes (not adds to) an
         // image, the output itself for the first pass, else a tuning buffer
@@ -498,9 +562,9 @@ static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, d
         }
         static const int cand[3] = {64, 128, 256};
         const int block = tune_choose(key, "D2BI_INT_BLOCK", cand, 3, 256, timg != nullptr, s, [&](int b) {
-            launch_int_pass(np, P, dens, f, timg, 0, inv, b, s);
+            launch_int_pass(P, nf, dens, f, timg, 0, inv, b, s);
         });
-        launch_int_pass(np, P, dens, f, d_img, !first, inv, block, s);
+        launch_int_pass(P, nf, dens, f, d_img, !first, inv, block, s);
         HIPCHK(hipGetLastError());
         p0 += np;
     }
@@ -848,8 +912,16 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
             } else {
                 CHK(run_voxel_apps(r, &plan, tab, ax, mode, na, variant, nr, s, w));
                 const size_t rec = dens ? sizeof(float4) : sizeof(float2);
-                for (int a = 0; a < na; a++)
-                    CHK(integrate_point(app + a, nvox * a, w.f32_field.as<char>() + rec * nvox * a));
+                if (!f64 && fields_fit(plane, nPrec, na, dens)) {
+                    std::vector<double> da((size_t)na * nPrec);
+                    for (int a = 0; a < na; a++)
+                        for (int q = 0; q < nPrec; q++) da[(size_t)nPrec * a + q] = aa[app + a + (size_t)nApp * q];
+                    CHK(launch_integrate_fast(&plan, dens, w.f32_field.p, d_img, s, app > 0, 1.0 / total, nullptr, na,
+                                              nvox, da.data()));
+                } else {
+                    for (int a = 0; a < na; a++)
+                        CHK(integrate_point(app + a, nvox * a, w.f32_field.as<char>() + rec * nvox * a));
+                }
             }
             CHK(add_stats(b, na));
             app += na;

@@ -35,3 +35,22 @@ def test_precession_points(mode, density, slices):
         e = float(np.max(np.abs(im.computeD2BI_img(x, 0.005, n, mode=mode) - ref)))
         print("[precession] %s n=%d max|dI| %.2e" % (mode, n, e), flush=True)
         assert e <= TOL[mode], n
+
+
+@pytest.mark.parametrize("columns", [(403, 397), (810, 790)])
+@pytest.mark.parametrize("density", [False, True])
+def test_fast_points_per_wave(columns, density):
+    """Large images march more points per wave, a small one splits a column's
+    points over waves; 160,000 and 640,000 columns take the instances the small
+    images above don't (several points per wave, the shared step matrix alone
+    and split).  Against the FP64 image, which is held to the oracle above."""
+    cfg = synth.scaled("c0", cells=(102, 100, 3))
+    cfg.update(density=density, sg=[0.01], d=(columns[0] * 3.1652 / 4, columns[1] * 3.1652 / 4, 13 * 3.1652 / 4))
+    x, box = synth.make_atoms(cfg)
+    x, conds = synth.conditions(cfg, x, box)
+    im = conds[0][0]
+    for n in (1, 2, 3, 4, 5, 6, 7, 8, 13, 16, 24, 32, 40):
+        ref = im.computeD2BI_img(x, 0.005, n, mode="fp64")
+        e = float(np.max(np.abs(im.computeD2BI_img(x, 0.005, n, mode="fast") - ref)))
+        print("[per wave] %s n=%d max|dI| %.2e of %.2e" % (columns, n, e, ref.max()), flush=True)
+        assert e <= TOL["fast"] * min(1.0, 10 * ref.max()), n
