@@ -132,7 +132,7 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
     double* __restrict__ out_im, int64_t out_stride, double* __restrict__ out_rho, int* __restrict__ out_cnt,
     double* __restrict__ out_r2m)
 {
-    constexpr int NW = F64R_NW, NT = 64 * NW, NS = REG / TILE;
+    constexpr int NW = F64R_NW, NS = REG / TILE;
     typedef F64Record<NA> Rec;
     __shared__ RegionStage<NW> S;
     // the link cells are done with once a pass is staged, the records after it
@@ -166,44 +166,48 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
             cnt[z][i] = 0;
         }
 
-    // records of a chunk: four threads per candidate, three for the axes, each
-    // also with a share of the phases.  A thread's inputs are loaded before
-    // the previous chunk's pairs.
-    constexpr int NI = (4 * F64R_REC + NT - 1) / NT, NC = NA > 2 ? NA / 2 : 1;
-    double in_f[NI], in_c[NI][NC];
+    // records of a chunk, a candidate per lane: three waves an axis each, the
+    // fourth the phases.  The parts go round the waves from chunk to chunk and
+    // region to region, so that no SIMD has the phases' share every time.  A
+    // lane's inputs are loaded before the previous chunk's pairs.
+    static_assert(NW == 4 && F64R_REC == 64, "a wave per part, a lane per candidate");
+    double in[2 * NA];
+    int turn = region;
     auto load = [&](int c0, int nc) {
+        const int part = (wave + turn + 1) & 3;
+        if (lane >= nc) return;
+        const int slot = __float_as_int(S.pos[c0 + lane].w);
+        if (part < 3) {
+            in[0] = reinterpret_cast<const double*>(frac + slot)[part];
+        } else {
 #pragma unroll
-        for (int j = 0; j < NI; j++) {
-            const int t = threadIdx.x + j * NT, role = t & 3;
-            if (t >= 4 * nc) continue;
-            const int slot = __float_as_int(S.pos[c0 + (t >> 2)].w);
-            in_f[j] = reinterpret_cast<const double*>(frac + slot)[min(role, 2)];
-#pragma unroll
-            for (int q = 0; q < NC; q++) {
-                const int e = (role * NC + q) & (2 * NA - 1);
-                in_c[j][q] = reinterpret_cast<const double*>(cs64 + (e >> 1) * cs_stride + slot)[e & 1];
+            for (int a = 0; a < NA; a++) {
+                const double2 c = cs64[a * cs_stride + slot];
+                in[2 * a] = c.x;
+                in[2 * a + 1] = c.y;
             }
         }
     };
     auto record = [&](int c0, int nc) {
+        turn++;
+        const int ax = (wave + turn) & 3;
+        Rec& q = U.rec[lane];
+        if (lane >= nc) {
+        } else if (ax == 3) {
 #pragma unroll
-        for (int j = 0; j < NI; j++) {
-            const int t = threadIdx.x + j * NT, i = t >> 2, role = t & 3;
-            if (t >= 4 * nc) continue;
-            const int ax = role;
-            if (ax == 3) continue;
-            Rec& q = U.rec[i];
-            const int u = ((S.upk[c0 + i] >> (8 * ax)) & 255) - 1;
+            for (int a = 0; a < NA; a++) q.cs[a] = make_double2(in[2 * a], in[2 * a + 1]);
+        } else {
+            const int u = ((S.upk[c0 + lane] >> (8 * ax)) & 255) - 1;
             const double side = ax == 0 ? P.a[0] : ax == 1 ? P.a[1] : P.a[2];
             const double h = ax == 0 ? R.h[0] : ax == 1 ? R.h[1] : R.h[2];
-            const double d0 = side * (in_f[j] + (u - S.zi[ax][0]));
+            const double d0 = side * (in[0] + (u - S.zi[ax][0]));
             const double ratio = exp((2.0 * d0) * (h * P.i2s2));
             double w = exp(-(d0 * d0) * P.i2s2);
             if (ax == 2) q.ratio = ratio;
 #pragma unroll
             for (int v = 0; v < REG; v++) {
                 const int k = u - S.lc[ax][v];
-                const double d = side * (in_f[j] + (k - S.zi[ax][v]));
+                const double d = side * (in[0] + (k - S.zi[ax][v]));
                 const double d2 = (unsigned)(k + 1) <= 2u ? d * d : HUGE_VAL;
                 if (ax == 2) {
                     q.z[v] = d2;
@@ -214,24 +218,13 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
                 w = w * ratio;
             }
         }
-        // phases
-#pragma unroll
-        for (int j = 0; j < NI; j++) {
-            const int t = threadIdx.x + j * NT;
-            if (t >= 4 * nc) continue;
-#pragma unroll
-            for (int q = 0; q < NC; q++) {
-                const int e = ((t & 3) * NC + q) & (2 * NA - 1);
-                reinterpret_cast<double*>(U.rec[t >> 2].cs)[e] = in_c[j][q];
-            }
-        }
         // the padding record: no voxel is in range of it
-        Rec& q = U.rec[F64R_REC];
+        Rec& e = U.rec[F64R_REC];
         if (threadIdx.x < REG) {
-            q.x[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
-            q.y[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
+            e.x[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
+            e.y[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
         } else if (threadIdx.x < sizeof(Rec) / 8 - 3 * REG) {
-            reinterpret_cast<double*>(&q)[threadIdx.x + 3 * REG] = 0.0;      // past x and y
+            reinterpret_cast<double*>(&e)[threadIdx.x + 3 * REG] = 0.0;      // past x and y
         }
     };
 
@@ -279,7 +272,9 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
                             sre[z][a][v] = fma(w, cs[a].x, sre[z][a][v]);
                             sim[z][a][v] = fma(w, cs[a].y, sim[z][a][v]);
                         }
-                        if (MIN) dmin[z][v] = fmin(dmin[z][v], dd);
+                        // fmin() would first quiet its operands, one more
+                        // operation per pair
+                        if (MIN) asm("v_min_f64 %0, %0, %1" : "+v"(dmin[z][v]) : "v"(dd));
                         if (DIAG) cnt[z][v] += in ? 1 : 0;
                         p = p * ratio;
                     }
@@ -302,7 +297,8 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
         for (int a = 0; a < NA; a++) {
             const double re = drop(part_sum(sre[z][a][0], sre[z][a][1], sre[z][a][2], sre[z][a][3])) * scale;
             const double im = drop(part_sum(sim[z][a][0], sim[z][a][1], sim[z][a][2], sim[z][a][3])) * scale;
-            double ww = hypot(re, im);
+            // (|S| counts from 1e-16 on, so its square is in range)
+            double ww = sqrt(fma(re, re, im * im));
             ww = 1 / (1.0e-16 > ww ? 1.0e-16 : ww);
             if (out) {
                 out_re[a * out_stride + o] = re * ww;
