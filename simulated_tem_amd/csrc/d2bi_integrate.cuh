@@ -402,10 +402,11 @@ __global__ __launch_bounds__(SPLIT ? int_threads(NP) : 256) void k_integrate_fas
 // ------------------------------------------------------------------ (c) integrate, FP64
 
 struct IntParams {
-    int Mx, My, Mz, np;         // np: precession points in this pass
+    int Mx, My, Mz, np;         // np: precession points in this launch
+    int nsplit;                 // waves per column
     double b0, bg, dz;
-    double aa[16];              // 2 pi s_g per precession point
-    double al[16];              // 2 dz aa
+    double aa[INT_SLOTS];       // 2 pi s_g per precession point
+    double al[INT_SLOTS];       // 2 dz aa
     int accumulate;             // add the column's sum to img
     double div;                 // and divide by it (0: not yet)
 };
@@ -438,29 +439,47 @@ struct Fp64Column {
     }
 };
 
+// Largest workgroup of an instance: what its registers leave room for.
+constexpr int int_threads64(int np) { return np <= 3 ? 1024 : np <= 8 ? 512 : 256; }
+
 // dynamicalTwoBeamIntegrationColumn_phaserho (Lib_DynamicalTwoBeamImaging.f90:
 // 2316-2480) and the precession average (:1897-1900, 1951): one lane per pixel
-// column, NP points per read of the column, stage by stage or, from six points
-// on, through the shared step matrix (40 FMAs per point instead of 80 after
-// ~230 to form the matrix: 5 points as 4 + 1 passes take 0.30 ms at 400 x 360
-// columns of 200 samples, 6 through the matrix 0.31); renormalised once at the
+// column and NP points, stage by stage or, from six points on, through the
+// shared step matrix (40 FMAs per point instead of 80 after ~230 to form the
+// matrix: 5 points as 4 + 1 passes take 0.30 ms at 400 x 360 columns of 200
+// samples, 6 through the matrix 0.31); a column's points split over P.nsplit
+// waves as k_integrate_fast's are; renormalised once at the
 // end, as the FAST march is.  Bound: FP64 VALU from two points on, HBM below
 // (1 point 0.079 ms, 5.8 TB/s).  A march per point with the reference's
 // divisions and a square root per step took 0.26 ms for 1 point, 2.00 for 8
 // and 8.7 for 32; this takes 0.079, 0.35 and 1.21.
-template <int NP, bool DENS>
-__global__ __launch_bounds__(256) void k_integrate_fp64(IntParams P, const double* __restrict__ fre,
-                                                        const double* __restrict__ fim,
-                                                        const double* __restrict__ frho, double* __restrict__ img)
+template <int NP, bool DENS, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? int_threads64(NP) : 256) void k_integrate_fp64(IntParams P,
+                                                                                  const double* __restrict__ fre,
+                                                                                  const double* __restrict__ fim,
+                                                                                  const double* __restrict__ frho,
+                                                                                  double* __restrict__ img)
 {
-    const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t plane = (int64_t)P.Mx * P.My;
-    if (col >= plane) return;
-    const Fp64Column<DENS> s{fre, fim, frho, col, plane, P.Mz, P.b0, P.bg};
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int ns = SPLIT ? P.nsplit : 1, cg = SPLIT ? wave / ns : wave, sp = SPLIT ? wave - cg * ns : 0;
+    const int ncg = (int)(blockDim.x >> 6) / ns;
+    const int64_t col = ((int64_t)blockIdx.x * ncg + cg) * 64 + lane;
+    const bool live = col < plane;
+    if (!SPLIT && !live) return;
+    const Fp64Column<DENS> s{fre, fim, frho, live ? col : plane - 1, plane, P.Mz, P.b0, P.bg};
+    const int p0 = sp * NP;
     double p0r[NP], p0i[NP], pgr[NP], pgi[NP];
-    if constexpr (NP >= 6) march_poly<NP>(s, P.Mz, P.dz, P.al, p0r, p0i, pgr, pgi);
-    else march_stage<NP>(s, P.Mz, P.dz, P.aa, p0r, p0i, pgr, pgi);
-    double acc = intensity_sum<NP>(P.np, p0r, p0i, pgr, pgi);
+    if constexpr (NP >= 6) march_poly<NP>(s, P.Mz, P.dz, P.al + p0, p0r, p0i, pgr, pgi);
+    else march_stage<NP>(s, P.Mz, P.dz, P.aa + p0, p0r, p0i, pgr, pgi);
+    double acc = intensity_sum<NP>(min(NP, P.np - p0), p0r, p0i, pgr, pgi);
+    if constexpr (SPLIT) {
+        __shared__ double part[int_threads64(NP)];
+        part[threadIdx.x] = acc;
+        __syncthreads();
+        if (sp > 0 || !live) return;
+        for (int k = 1; k < ns; k++) acc += part[threadIdx.x + 64 * k];
+    }
     if (P.accumulate) acc = img[col] + acc;
     img[col] = P.div != 0.0 ? acc / P.div : acc;
 }

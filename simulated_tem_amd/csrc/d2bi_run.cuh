@@ -453,32 +453,57 @@ struct IntSplit {
 // points 8/16/32: 1471/1215/1128; 236 x 268, 8 points of 4 per wave, 65 with
 // workgroups of two column groups, 95 of one.  Powers of two in passes, one
 // wave per column, took 110, 380, 40, 338, 1185 and 70.
-static IntSplit int_split(int64_t plane, int np, bool dens)
+struct IntInst {
+    int n, waves, most;         // points per wave, waves a SIMD holds, waves per workgroup
+    double ops;                 // vector operations per double step
+};
+
+// together: cycles per operation and wave where a SIMD holds several; gain:
+// what more waves per column have to come down to
+template <size_t N>
+static IntSplit cheapest_split(const IntInst (&inst)[N], int64_t plane, int np, double together, double gain)
 {
-    struct Inst {
-        int n, waves;
-    };
-    static const Inst stage[] = {{7, 7}, {6, 8}, {5, 8}, {4, 5}, {3, 6}, {2, 7}, {1, 7}};
-    static const Inst matrix[] = {{32, 2}, {16, 3}, {8, 4}, {4, 5}, {2, 5}};
-    const bool poly = np >= 8 && fast_integrator_poly();
     const int64_t groups = (plane + 63) / 64;
     IntSplit best{0, 1, 4};
     double cost = 1.0e300;
-    for (int i = 0; i < (poly ? 5 : 7); i++) {
-        const int n = poly ? matrix[i].n : stage[i].n, waves = poly ? matrix[i].waves : stage[i].waves;
-        const int ns = (np + n - 1) / n, most = int_threads(n) / 64 / ns;
-        const double ops = (poly ? 230 + 40 * n : 15 + 85 * n) + (dens ? 60 : 0);
-        for (int cg = ns > 1 ? 1 : 4; cg <= (ns > 1 ? most : 4); cg++) {
+    for (const IntInst& I : inst) {
+        const int ns = (np + I.n - 1) / I.n;
+        for (int cg = ns > 1 ? 1 : 4; cg <= (ns > 1 ? I.most / ns : 4); cg++) {
             const int64_t load = ((groups + cg - 1) / cg + 255) / 256 * ((ns * cg + 3) / 4);
-            auto cyc = [](int w) { return w > 0 ? std::max(4.8, 3.1 * w) : 0.0; };
-            const double c = ops * ((double)(load / waves) * cyc(waves) + cyc((int)(load % waves)));
-            if (c < (ns > best.ns ? 0.93 : 1.0) * cost) {
+            auto cyc = [&](int w) { return w > 0 ? std::max(4.8, together * w) : 0.0; };
+            const double c = I.ops * ((double)(load / I.waves) * cyc(I.waves) + cyc((int)(load % I.waves)));
+            if (c < (ns > best.ns ? gain : 1.0) * cost) {
                 cost = c;
-                best = IntSplit{n, ns, cg};
+                best = IntSplit{I.n, ns, cg};
             }
         }
     }
     return best;
+}
+
+static IntSplit int_split(int64_t plane, int np, bool dens)
+{
+    const double d = dens ? 60 : 0;
+    auto st = [&](int n, int waves) { return IntInst{n, waves, int_threads(n) / 64, 15 + 85.0 * n + d}; };
+    auto mx = [&](int n, int waves) { return IntInst{n, waves, int_threads(n) / 64, 230 + 40.0 * n + d}; };
+    const IntInst stage[] = {st(7, 7), st(6, 8), st(5, 8), st(4, 5), st(3, 6), st(2, 7), st(1, 7)};
+    const IntInst matrix[] = {mx(32, 2), mx(16, 3), mx(8, 4), mx(4, 5), mx(2, 5)};
+    if (np >= 8 && fast_integrator_poly()) return cheapest_split(matrix, plane, np, 3.1, 0.93);
+    return cheapest_split(stage, plane, np, 3.1, 0.93);
+}
+
+// The same for FP64, whose operations do not overlap (a SIMD's waves take 4.8
+// cycles each) and whose columns are 24 bytes a sample: splitting them has to
+// win 20 % (400 x 360 columns of 200 samples with density, 2 points: 135 us in
+// one wave, 196 in two).  136 x 136 of 136, one wave per column -> split: 2
+// points 32 -> 26, 4 51 -> 35, 8 81 -> 56; 400 x 360, 32 points 1213 -> 1050
+// (two launches before).
+static IntSplit int_split64(int64_t plane, int np)
+{
+    auto st = [&](int n, int waves) { return IntInst{n, waves, int_threads64(n) / 64, 15 + 80.0 * n}; };
+    auto mx = [&](int n, int waves) { return IntInst{n, waves, int_threads64(n) / 64, 230 + 40.0 * n}; };
+    const IntInst inst[] = {mx(16, 1), mx(12, 1), mx(8, 2), mx(6, 2), st(4, 3), st(3, 4), st(2, 4), st(1, 4)};
+    return cheapest_split(inst, plane, np, 4.8, 0.8);
 }
 
 // Whether one launch integrates nf fields of np points each: their
@@ -571,7 +596,7 @@ static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, d
     return D2BI_OK;
 }
 
-// FP64 integration of all precession points, in passes of up to 16.
+// FP64 integration of all precession points, INT_POINTS a launch.
 // accumulate: add each column's sum over precession points to d_img; otherwise
 // write sum / nPrec (div = 0) or sum / div.  The field is read from workspace
 // w, field_off voxels on.
@@ -579,32 +604,34 @@ static int launch_integrate_fp64(const d2bi_plan* p, bool dens, double* d_img, h
                                  int accumulate = 0, double div = 0.0, int64_t field_off = 0)
 {
     const int64_t plane = (int64_t)p->Mx * p->My;
-    // a lane per column: small workgroups spread a small image over the CUs
-    const int block = plane < 256 * 1024 ? 64 : 256;
     for (int p0 = 0; p0 < p->nPrec;) {
-        const int left = p->nPrec - p0;
-        const int inst = left <= 4 ? left : left <= 6 ? 6 : left <= 8 ? 8 : left <= 12 ? 12 : 16;
-        const int np = std::min(left, inst);
+        const int np = pass_points(p->nPrec - p0);
+        const IntSplit sp = int_split64(plane, np);
         IntParams P;
         P.Mx = p->Mx; P.My = p->My; P.Mz = p->Mz; P.np = np;
+        P.nsplit = sp.ns;
         P.b0 = p->b0; P.bg = p->bg; P.dz = p->dz;
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < INT_SLOTS; i++) {
             P.aa[i] = i < np ? p->aa[p0 + i] : 0.0;
             P.al[i] = 2.0 * p->dz * P.aa[i];
         }
         P.accumulate = accumulate || p0 > 0;
         P.div = accumulate || p0 + np < p->nPrec ? 0.0 : div == 0.0 ? (double)p->nPrec : div;
+        // unsplit: small workgroups spread a small image over the CUs
+        const int cg = sp.ns > 1 ? sp.cg : plane < 256 * 1024 ? 1 : 4;
         auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3((unsigned)((plane + block - 1) / block)), dim3(block), 0, s, P,
+            hipLaunchKernelGGL(kern, dim3((unsigned)((plane + 64 * cg - 1) / (64 * cg))), dim3(64 * cg * sp.ns), 0, s, P,
                                w.f64_re.as<double>() + field_off, w.f64_im.as<double>() + field_off,
                                w.f64_rho.as<double>(), d_img);
         };
         auto pick = [&](auto np_c) {
             constexpr int N = decltype(np_c)::value;
-            if (dens) go(k_integrate_fp64<N, true>);
-            else go(k_integrate_fp64<N, false>);
+            if (sp.ns > 1 && dens) go(k_integrate_fp64<N, true, true>);
+            else if (sp.ns > 1) go(k_integrate_fp64<N, false, true>);
+            else if (dens) go(k_integrate_fp64<N, true, false>);
+            else go(k_integrate_fp64<N, false, false>);
         };
-        switch (inst) {
+        switch (sp.n) {
             case 1: pick(std::integral_constant<int, 1>{}); break;
             case 2: pick(std::integral_constant<int, 2>{}); break;
             case 3: pick(std::integral_constant<int, 3>{}); break;
