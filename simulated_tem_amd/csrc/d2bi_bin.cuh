@@ -218,7 +218,7 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
         int leader = lane;
         while (rem) {
             const int l = __ffsll((long long)rem) - 1;
-            const int lc = __shfl(cell, l, 64);
+            const int lc = __builtin_amdgcn_readlane(cell, l);
             const unsigned long long gm = __ballot(cell == lc);
             if (cell == lc) { leader = l; grp = gm; }
             rem &= ~gm;
