@@ -545,14 +545,14 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
             auto zoff = [&](int e) -> int { return cupk[scell[e >> 4]] >> 8; };
             for (int kb = 0; kb < nst; kb += ROW_BLOCK) {
                 const int ke = min(kb + ROW_BLOCK, nst);
-                float dmin = 3.4028234663852886e38f;
+                // smallest |u| of the block's even and of its odd steps
+                float dmin[2] = {3.4028234663852886e38f, 3.4028234663852886e38f};
                 float bre[NA][TX], bim[NA][TX];
 #pragma unroll
                 for (int i = 0; i < TX; i++)
 #pragma unroll
                     for (int a = 0; a < NA; a++) { bre[a][i] = 0.0f; bim[a][i] = 0.0f; }
-#pragma unroll 2
-                for (int kk = kb; kk < ke; kk++) {
+                auto pairs = [&](int kk, float& near) {
                     const int e = list[NQ * kk];
                     float xv[TX];
                     load_x(e, xv);
@@ -573,10 +573,16 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                             bre[a][i] = fmaf(w, pc[a], bre[a][i]);
                             bim[a][i] = fmaf(w, ps[a], bim[a][i]);
                         }
-                        dmin = fminf(dmin, fabsf(u));
+                        near = fminf(near, fabsf(u));
                         if (DENSITY) umax[i] = fmaxf(umax[i], u);
                     }
+                };
+                int kk = kb;
+                for (; kk + 1 < ke; kk += 2) {
+                    pairs(kk, dmin[0]);
+                    pairs(kk + 1, dmin[1]);
                 }
+                if (kk < ke) pairs(kk, dmin[0]);
 #pragma unroll
                 for (int i = 0; i < TX; i++)
 #pragma unroll
@@ -584,8 +590,10 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                         kahan_add(rre[a][i], kre[a][i], bre[a][i]);
                         kahan_add(rim[a][i], kim[a][i], bim[a][i]);
                     }
-                if (__ballot(dmin <= F.e_band)) {
-                    for (int kk = kb; kk < ke; kk++) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    if (!__ballot(dmin[h] <= F.e_band)) continue;
+                    for (int kk = kb + h; kk < ke; kk += 2) {
                         const int e = list[NQ * kk];
                         float xv[TX];
                         load_x(e, xv);
