@@ -545,14 +545,15 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
             auto zoff = [&](int e) -> int { return cupk[scell[e >> 4]] >> 8; };
             for (int kb = 0; kb < nst; kb += ROW_BLOCK) {
                 const int ke = min(kb + ROW_BLOCK, nst);
-                // smallest |u| of the block's even and of its odd steps
-                float dmin[2] = {3.4028234663852886e38f, 3.4028234663852886e38f};
+                // smallest |u| of the block's even and odd steps, voxels 0-1 and 2-3
+                constexpr float far = 3.4028234663852886e38f;
+                float dmin[2][2] = {{far, far}, {far, far}};
                 float bre[NA][TX], bim[NA][TX];
 #pragma unroll
                 for (int i = 0; i < TX; i++)
 #pragma unroll
                     for (int a = 0; a < NA; a++) { bre[a][i] = 0.0f; bim[a][i] = 0.0f; }
-                auto pairs = [&](int kk, float& near) {
+                auto pairs = [&](int kk, float* near) {
                     const int e = list[NQ * kk];
                     float xv[TX];
                     load_x(e, xv);
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                             bre[a][i] = fmaf(w, pc[a], bre[a][i]);
                             bim[a][i] = fmaf(w, ps[a], bim[a][i]);
                         }
-                        near = fminf(near, fabsf(u));
+                        near[i >> 1] = fminf(near[i >> 1], fabsf(u));
                         if (DENSITY) umax[i] = fmaxf(umax[i], u);
                     }
                 };
@@ -591,8 +592,9 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                         kahan_add(rim[a][i], kim[a][i], bim[a][i]);
                     }
 #pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    if (!__ballot(dmin[h] <= F.e_band)) continue;
+                for (int hh = 0; hh < 4; hh++) {
+                    const int h = hh & 1, v0 = hh & 2;
+                    if (!__ballot(dmin[h][v0 >> 1] <= F.e_band)) continue;
                     for (int kk = kb + h; kk < ke; kk += 2) {
                         const int e = list[NQ * kk];
                         float xv[TX];
@@ -601,7 +603,7 @@ __global__ __launch_bounds__(64) void k_voxel_tile(FastParams F, const int* __re
                         float E = __builtin_amdgcn_exp2f(fmaf(B.x, qcy, fmaf(B.y, qcz, kyz)));
                         if (ROW == 2) E = (unsigned)(zoff(e) - lcz) <= 2u ? E : 0.0f;
 #pragma unroll
-                        for (int i = 0; i < TX; i++) {
+                        for (int i = v0; i < v0 + 2; i++) {
                             const float u = fmaf(xv[i], E, -1.0f);
                             if (fabsf(u) <= F.e_band) {
                                 const int vx = min(x0 + i, x1);
