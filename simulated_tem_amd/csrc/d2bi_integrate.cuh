@@ -197,12 +197,22 @@ __device__ __forceinline__ void static_for(F&& f)
     }
 }
 
+// Coefficients of one polynomial known to have no real (RE) or no imaginary
+// part (IM): bit k for alpha^k.  alpha multiplies the (2,2) element by i alone,
+// so the leading coefficients of the (2,2) entries are real or imaginary; an
+// operation with the zero part would still be made (0 x is not 0 for every x).
+template <unsigned RE, unsigned IM>
+struct NoPart {
+    static constexpr bool re(int k) { return (RE >> k) & 1u; }
+    static constexpr bool im(int k) { return (IM >> k) & 1u; }
+};
+
 // One column (P1, P2) of Q = s A_x P for a polynomial matrix P, with the
 // stage's scaled coefficients c = s c0, g = s cg and ax = s / (2 dz):
 //     Q1 = i (c P1 + g P2),   Q2 = i (conj(g) P1 + c P2 + ax alpha P2).
 // Terms are chained from the first present one, so structural zeros cost
-// nothing.
-template <int D1, int D2, class T, int E1 = (D1 > D2 ? D1 : D2), int E2 = (D1 > D2 + 1 ? D1 : D2 + 1)>
+// nothing; Z are the parts P2 lacks.
+template <class Z, int D1, int D2, class T, int E1 = (D1 > D2 ? D1 : D2), int E2 = (D1 > D2 + 1 ? D1 : D2 + 1)>
 __device__ __forceinline__ void rk_col(T c, T gr, T gi, T ax, const CPoly<D1, T>& P1, const CPoly<D2, T>& P2,
                                        CPoly<E1, T>& Q1, CPoly<E2, T>& Q2)
 {
@@ -210,8 +220,16 @@ __device__ __forceinline__ void rk_col(T c, T gr, T gi, T ax, const CPoly<D1, T>
         constexpr int k = decltype(kc)::value;
         T ur, ui;
         if constexpr (k <= D2) {
-            ur = fm(gr, P2.c[k].r, -gi * P2.c[k].i);
-            ui = fm(gr, P2.c[k].i, gi * P2.c[k].r);
+            if constexpr (Z::re(k)) {
+                ur = -gi * P2.c[k].i;
+                ui = gr * P2.c[k].i;
+            } else if constexpr (Z::im(k)) {
+                ur = gr * P2.c[k].r;
+                ui = gi * P2.c[k].r;
+            } else {
+                ur = fm(gr, P2.c[k].r, -gi * P2.c[k].i);
+                ui = fm(gr, P2.c[k].i, gi * P2.c[k].r);
+            }
             if constexpr (k <= D1) {
                 ur = fm(c, P1.c[k].r, ur);
                 ui = fm(c, P1.c[k].i, ui);
@@ -225,53 +243,42 @@ __device__ __forceinline__ void rk_col(T c, T gr, T gi, T ax, const CPoly<D1, T>
     static_for<0, E2>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
         constexpr bool ta = k <= D1, tb = k <= D2, tc = k >= 1 && k - 1 <= D2;
+        constexpr bool br = tb && !Z::re(k), bi = tb && !Z::im(k);
+        constexpr bool cr = tc && !Z::re(k - 1), ci = tc && !Z::im(k - 1);
         T ur = 0, ui = 0;
         if constexpr (ta) {
             ur = fm(gr, P1.c[k].r, gi * P1.c[k].i);
             ui = fm(gr, P1.c[k].i, -gi * P1.c[k].r);
         }
-        if constexpr (tb) {
-            if constexpr (ta) {
-                ur = fm(c, P2.c[k].r, ur);
-                ui = fm(c, P2.c[k].i, ui);
-            } else {
-                ur = c * P2.c[k].r;
-                ui = c * P2.c[k].i;
-            }
-        }
-        if constexpr (tc) {
-            if constexpr (ta || tb) {
-                ur = fm(ax, P2.c[k - 1].r, ur);
-                ui = fm(ax, P2.c[k - 1].i, ui);
-            } else {
-                ur = ax * P2.c[k - 1].r;
-                ui = ax * P2.c[k - 1].i;
-            }
-        }
+        if constexpr (br) ur = ta ? fm(c, P2.c[tb ? k : 0].r, ur) : c * P2.c[tb ? k : 0].r;
+        if constexpr (bi) ui = ta ? fm(c, P2.c[tb ? k : 0].i, ui) : c * P2.c[tb ? k : 0].i;
+        if constexpr (cr) ur = ta || br ? fm(ax, P2.c[tc ? k - 1 : 0].r, ur) : ax * P2.c[tc ? k - 1 : 0].r;
+        if constexpr (ci) ui = ta || bi ? fm(ax, P2.c[tc ? k - 1 : 0].i, ui) : ax * P2.c[tc ? k - 1 : 0].i;
         Q2.c[k] = cplx<T>{-ui, ur};
     });
 }
 
-// M += s P (degree of P <= degree of M)
-template <int DM, int DP, class T>
+// M += s P (degree of P <= degree of M; Z: the parts P lacks)
+template <class Z = NoPart<0, 0>, int DM, int DP, class T>
 __device__ __forceinline__ void poly_axpy(CPoly<DM, T>& M, T s, const CPoly<DP, T>& P)
 {
     static_assert(DP <= DM, "degree");
-#pragma unroll
-    for (int k = 0; k <= DP; k++) {
-        M.c[k].r = fm(s, P.c[k].r, M.c[k].r);
-        M.c[k].i = fm(s, P.c[k].i, M.c[k].i);
-    }
+    static_for<0, DP>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        if constexpr (!Z::re(k)) M.c[k].r = fm(s, P.c[k].r, M.c[k].r);
+        if constexpr (!Z::im(k)) M.c[k].i = fm(s, P.c[k].i, M.c[k].i);
+    });
 }
 
-template <int D, class T>
+// M at alpha (Z: parts its leading coefficient lacks)
+template <class Z = NoPart<0, 0>, int D, class T>
 __device__ __forceinline__ cplx<T> horner(const CPoly<D, T>& M, T al)
 {
     cplx<T> v = M.c[D];
 #pragma unroll
     for (int k = D - 1; k >= 0; k--) {
         v.r = fm(v.r, al, M.c[k].r);
-        v.i = fm(v.i, al, M.c[k].i);
+        v.i = Z::im(D) && k == D - 1 ? M.c[k].i : fm(v.i, al, M.c[k].i);
     }
     return v;
 }
@@ -285,6 +292,12 @@ __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al
     const T dz2 = 2 * dz, dz6 = dz / 3, third = T(1) / 3, two3 = T(2) / 3, sixth = T(1) / 6, half = T(0.5), one = T(1);
 #pragma unroll
     for (int p = 0; p < NP; p++) { p0r[p] = 1; p0i[p] = 0; pgr[p] = 0; pgi[p] = 0; }
+    // parts the leading coefficients of T22, K2_22, K3_22 and M22 lack
+    using Full = NoPart<0, 0>;
+    using Imag1 = NoPart<1u << 1, 0>;
+    using Real2 = NoPart<0, 1u << 2>;
+    using Imag3 = NoPart<1u << 3, 0>;
+    using Real4 = NoPart<0, 1u << 4>;
     T c0a = 0, cgra = 0, cgia = 0;
     typename S::Raw fb{}, fc{};
     if (nz >= 2) {
@@ -306,27 +319,27 @@ __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al
         CPoly<1, T> T22{{{one, ca}, {T(0), half}}};
         // K2 = dz A_b T1, T2 = I + K2
         CPoly<0, T> K2_11; CPoly<1, T> K2_21, K2_12; CPoly<2, T> K2_22;
-        rk_col(dz * c0b, dz * cgrb, dz * cgib, half, T11, T21, K2_11, K2_21);
-        rk_col(dz * c0b, dz * cgrb, dz * cgib, half, T12, T22, K2_12, K2_22);
+        rk_col<Full>(dz * c0b, dz * cgrb, dz * cgib, half, T11, T21, K2_11, K2_21);
+        rk_col<Imag1>(dz * c0b, dz * cgrb, dz * cgib, half, T12, T22, K2_12, K2_22);
         CPoly<0, T> U11 = K2_11; CPoly<1, T> U21 = K2_21, U12 = K2_12; CPoly<2, T> U22 = K2_22;
         U11.c[0].r += one;
         U22.c[0].r += one;
         // K3 = 2 dz A_b T2, T3 = I + K3
         CPoly<1, T> K3_11; CPoly<2, T> K3_21, K3_12; CPoly<3, T> K3_22;
-        rk_col(dz2 * c0b, dz2 * cgrb, dz2 * cgib, one, U11, U21, K3_11, K3_21);
-        rk_col(dz2 * c0b, dz2 * cgrb, dz2 * cgib, one, U12, U22, K3_12, K3_22);
+        rk_col<Full>(dz2 * c0b, dz2 * cgrb, dz2 * cgib, one, U11, U21, K3_11, K3_21);
+        rk_col<Real2>(dz2 * c0b, dz2 * cgrb, dz2 * cgib, one, U12, U22, K3_12, K3_22);
         CPoly<1, T> V11 = K3_11; CPoly<2, T> V21 = K3_21, V12 = K3_12; CPoly<3, T> V22 = K3_22;
         V11.c[0].r += one;
         V22.c[0].r += one;
         // K4/6 = (dz/3) A_c T3: the last term of M, which it starts
         CPoly<2, T> M11; CPoly<3, T> M21, M12; CPoly<4, T> M22;
-        rk_col(dz6 * c0c, dz6 * cgrc, dz6 * cgic, sixth, V11, V21, M11, M21);
-        rk_col(dz6 * c0c, dz6 * cgrc, dz6 * cgic, sixth, V12, V22, M12, M22);
+        rk_col<Full>(dz6 * c0c, dz6 * cgrc, dz6 * cgic, sixth, V11, V21, M11, M21);
+        rk_col<Imag3>(dz6 * c0c, dz6 * cgrc, dz6 * cgic, sixth, V12, V22, M12, M22);
         // + K3/3 + (2/3) K2 + Q1/3 + I
         poly_axpy(M11, third, K3_11); poly_axpy(M21, third, K3_21);
-        poly_axpy(M12, third, K3_12); poly_axpy(M22, third, K3_22);
+        poly_axpy(M12, third, K3_12); poly_axpy<Imag3>(M22, third, K3_22);
         poly_axpy(M11, two3, K2_11); poly_axpy(M21, two3, K2_21);
-        poly_axpy(M12, two3, K2_12); poly_axpy(M22, two3, K2_22);
+        poly_axpy(M12, two3, K2_12); poly_axpy<Real2>(M22, two3, K2_22);
         M11.c[0].r += one;
         M11.c[0].i = fm(ca, third, M11.c[0].i);
         M12.c[0].r = fm(-gai, third, M12.c[0].r);
@@ -339,7 +352,7 @@ __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al
 #pragma unroll
         for (int p = 0; p < NP; p++) {
             const T al = al_[p];
-            const cplx<T> m11 = horner(M11, al), m12 = horner(M12, al), m21 = horner(M21, al), m22 = horner(M22, al);
+            const cplx<T> m11 = horner(M11, al), m12 = horner(M12, al), m21 = horner(M21, al), m22 = horner<Real4>(M22, al);
             const T y0r = p0r[p], y0i = p0i[p], ygr = pgr[p], ygi = pgi[p];
             p0r[p] = fm(m11.r, y0r, fm(-m11.i, y0i, fm(m12.r, ygr, -m12.i * ygi)));
             p0i[p] = fm(m11.r, y0i, fm(m11.i, y0r, fm(m12.r, ygi, m12.i * ygr)));
