@@ -9,26 +9,27 @@ crystal (bcc, 200 x 200 x 100 cells, 8.0e6 atoms, Eshelby centres, voids,
 (110, 011) on a [001] zone = 42 conditions, each re-binned and re-voxelised
 (800 x 800 x 400 voxels) and integrated at 32 precession points (0.005 rad):
 1.344e3 integrations, 3.44e11 imaged voxels per batch.  A step is one whole
-batch through d2bi_gpu_image_batch_dev_out (one captured HIP graph; atoms
+batch through d2bi_gpu_image_batch_dev_out (plain launches on concurrent
+branches, from the second identical call on one captured HIP graph; atoms
 resident in HBM, the 42 images left in HBM), the window of the reference's
 T_D2BI timer (d2bi.f90:1392-1410) summed over the series.  The first call
-plans, counts and captures the graph; it is timed apart (first_call_s).
+plans, counts and tunes; it is timed apart (first_call_s).
 
 Beside the timed batch:
   fp64_value       the plain per-condition FP64 path (d2bi_gpu_image_dev_out,
                    FP64 mode, one condition per call) on conditions spread
                    over the series; fast_over_fp64 = value / fp64_value
   errors_vs_fp64   max and mean |I_FAST - I_FP64| per checked image
-  roofline         k_voxel_tile (the largest kernel of the batch), FP32 VALU:
+  roofline         k_voxel_tile, FP32 VALU:
                    algorithmic work 388 flop per voxel (28.27 in-sphere atoms
                    x 13 flop + 20) over its device time, measured with HIP
                    events around its launches on the library stream while
                    imaging conditions of the series one at a time (the same
                    kernels and launch shapes as in the graph)
   roofline_integrate
-                   k_integrate_poly<32> by its real operation count: per RK4
-                   double step and column, 399 flop to form the step matrix
-                   and 76 flop per precession point (Horner at the point's
+                   the FAST integrator by its operation count: per RK4
+                   double step and column, 374 flop to form the step matrix
+                   and 74 flop per precession point (Horner at the point's
                    alpha, one 2x2 complex product); the 78.5 flop per voxel
                    and condition of the stage-by-stage march would overstate
                    it
@@ -57,15 +58,15 @@ PEAK_FP32_TFLOPS = 157.3             # MI355X published FP32 vector/matrix peak
 PEAK_TRANS_PER_S = 157.3e12 / 16     # transcendentals at a quarter of the wave64 VALU rate
 FLOPS_PER_VOXEL = 388.0              # voxelisation, per voxel and field
 TRANS_PER_VOXEL = 30.0
-POLY_FORM_FLOPS = 399.0              # k_integrate_poly: step matrix, per double step and column
-POLY_POINT_FLOPS = 76.0              # k_integrate_poly: per precession point, double step and column
-STAGE_POINT_FLOPS = 140.0            # k_integrate_fast: per precession point, double step and column
+POLY_FORM_FLOPS = 374.0              # k_integrate_fast: step matrix, per double step and column
+POLY_POINT_FLOPS = 74.0              # ... and per precession point through it
+STAGE_POINT_FLOPS = 140.0            # ... per precession point stage by stage
 # HBM bytes per launch of k_voxel_tile from rocprofv3 FETCH_SIZE / WRITE_SIZE
 # passes, scaled by a 1 GiB copy's counts, with the library's default launch
 # choices (profiles/k_voxel_tile_c1_traffic.md, profiles/c3_batch_pmc.md); a
 # profiler cannot run inside the timed process, so the figure is recorded per
 # workload
-TRAFFIC_BYTES = {"c1": 4.557e9, "c3": 4.104e9}
+TRAFFIC_BYTES = {"c1": 3.590e9, "c3": 3.311e9}
 SINGLE = ("c0", "c1", "c2")
 
 
@@ -74,14 +75,14 @@ def log(*a):
 
 
 def integrate_flops(p, n_prec):
-    """Real flops of the FAST integration of one condition: passes of 32, 16
-    or 8 points through the shared step matrix, fewer stage by stage."""
+    """Flops of the FAST integration of one condition: launches of up to 32
+    points, from 8 on through the step matrix (formed once per column and
+    double step), fewer stage by stage."""
     cols = p.Mx * p.My
     ds = p.Mz // 2
     left, f = n_prec, 0.0
     while left > 0:
-        np_ = 32 if left >= 32 else 16 if left >= 16 else 8 if left >= 8 else 4 if left >= 4 else \
-            2 if left >= 2 else 1
+        np_ = min(left, 32)
         f += (POLY_FORM_FLOPS + POLY_POINT_FLOPS * np_) if np_ >= 8 else STAGE_POINT_FLOPS * np_
         left -= np_
     return cols * ds * f
@@ -236,7 +237,7 @@ def batch_main(args, imaging, synth, np):
     p0 = im0.plan(n0, pa0, npr0)
     vox0 = p0.Mx * p0.My * p0.Mz
     ach = vox0 * FLOPS_PER_VOXEL / (ms_vox * 1e-3) / 1e12
-    roof = {"bound": "valu", "pipe": "valu_fp32", "kernel": "k_voxel_tile<false,false,1,8,4,1>",
+    roof = {"bound": "valu", "pipe": "valu_fp32", "kernel": "k_voxel_tile<false,false,1,8,8,1>",
             "achieved": ach, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": ach / PEAK_FP32_TFLOPS,
             "traffic": TRAFFIC_BYTES.get(args.workload),
             "traffic_unit": "B per launch (rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, default launch choices)",
@@ -244,11 +245,11 @@ def batch_main(args, imaging, synth, np):
             "transcendental_frac": vox0 * TRANS_PER_VOXEL / (ms_vox * 1e-3) / PEAK_TRANS_PER_S}
     fi = integrate_flops(p0, npr0)
     ach_i = fi / (ms_int * 1e-3) / 1e12
-    roof_i = {"bound": "valu", "pipe": "valu_fp32", "kernel": "k_integrate_poly<%d,false>" % min(32, npr0),
+    roof_i = {"bound": "valu", "pipe": "valu_fp32", "kernel": "k_integrate_fast (%d points per launch)" % min(32, npr0),
               "achieved": ach_i, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": ach_i / PEAK_FP32_TFLOPS,
               "ms_per_launch": ms_int,
-              "work": "%d columns x %d double steps x (%g + %g x %d) flop" %
-                      (p0.Mx * p0.My, p0.Mz // 2, POLY_FORM_FLOPS, POLY_POINT_FLOPS, min(32, npr0))}
+              "work": "%d columns x %d double steps x %g flop" %
+                      (p0.Mx * p0.My, p0.Mz // 2, fi / (p0.Mx * p0.My) / (p0.Mz // 2))}
     log("[bench] per condition: voxel %.3f ms (%.3f of FP32 peak), integrate %.3f ms (%.3f), binning %.3f ms"
         % (ms_vox, roof["frac"], ms_int, roof_i["frac"], ms_bin))
     emax = max(e["max"] for e in errs)
@@ -316,7 +317,7 @@ def single_main(name, steps, warmup, imaging, synth, np, fp64_steps=3):
         log("[bench] %s fp64: %.3e imaged voxels/s, max err %.3e" % (name, out["fp64_value"], e.max()))
     t_vox = out["ms_voxel"] * 1e-3
     ach = vox * FLOPS_PER_VOXEL / t_vox / 1e12
-    out["roofline"] = {"bound": "valu", "pipe": "valu_fp32", "kernel": "k_voxel_tile<false,false,1,8,4,1>",
+    out["roofline"] = {"bound": "valu", "pipe": "valu_fp32", "kernel": "k_voxel_tile<false,false,1,8,8,1>",
                        "achieved": ach, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                        "frac": ach / PEAK_FP32_TFLOPS, "traffic": TRAFFIC_BYTES.get(name),
                        "ms_per_launch": out["ms_voxel"]}

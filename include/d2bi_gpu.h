@@ -250,9 +250,10 @@ int d2bi_gpu_image_noalloc(const d2bi_record* rec, d2bi_atoms atoms,
 /* Batched conditions: nRec records (tilts, g-vectors, s_g sweeps, ...)
  * over atom sets atoms[i] (entries may repeat), each integrated at nPrec[i]
  * precession points of angle precAngle[i].  img receives the images one
- * after another (sum of Mx*My over records).  The batch is executed as one
- * captured HIP graph per shape group; every record is re-voxelised, as the
- * reference re-voxelises each condition (d2bi.f90:1352-1394). */
+ * after another (sum of Mx*My over records).  The batch runs on
+ * concurrent branches, as plain launches the first time and as one captured
+ * HIP graph when the same batch comes again; every record is re-voxelised, as
+ * the reference re-voxelises each condition (d2bi.f90:1352-1394). */
 int d2bi_gpu_image_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int32_t nRec,
                          const double* precAngle, const int32_t* nPrec, int32_t mode,
                          double* img, d2bi_stats* stats);

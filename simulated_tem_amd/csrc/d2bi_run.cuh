@@ -77,7 +77,6 @@ static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParam
 {
     FastParams& F = *Fo;
     F.v = V;
-    F.tz = tz;
     F.ntx = (p->Mx + TILE - 1) / TILE;
     F.nty = (p->My + ty - 1) / ty;
     F.ntz = (p->Mz + tz - 1) / tz;

@@ -26,7 +26,6 @@ struct FastParams {
     float inv_k2;               // 1 / k2
     float cellf[3];             // link-cell sides in FP32
     int thin_z;                 // link cells thinner than 3 sigma along z
-    int tz;                     // tile depth in voxels
     int order;                  // tiles over workgroups: 0 contiguous ranges per XCD, 1 linear, 2 rows dealt to XCDs
     // aperture points sharing one pass (kernels with NA > 1): point a's
     // (cos, sin) of g.r at app_cs[a app_stride + slot], its field at
@@ -57,7 +56,8 @@ struct FastParams {
 //     127 of a 4 x 8 x 8 tile, 59 instead of 95 of a 4 x 4 x 8;
 //   - the larger tile stages fewer points per voxel.
 // 800 x 800 x 400 voxels, ms (before all three, 4 x 4 x 8 tiles: 5.5): 5.0,
-// 4.65, 4.2; 2020 vector instructions per 128 voxels became 1300.
+// 4.65, 4.2 (4.06 with the guard band watched by steps and voxels); 2020 vector
+// instructions per 128 voxels became 1280.
 //
 // Staging.  The kept non-empty cells are listed once per tile with their
 // origin in the tile frame and the offset from candidate index to point
@@ -90,9 +90,10 @@ struct FastParams {
 // X_0..X_3 (which carry the candidate's own y-z term) are evaluated once
 // per candidate when it is staged and a lane spends two FMAs and one
 // v_exp_f32 per candidate on four voxels.  Membership e_i >= e_rc
-// is u_i = X_i 2^t - 1 >= 0; a block in which some |u_i| lies within the
-// guard band is walked again and the pairs of the band are re-tested in FP64,
-// correcting the sums where the FP64 test disagrees.  The parts' sums are
+// is u_i = X_i 2^t - 1 >= 0; the steps and voxels of a block (even or
+// odd, 0-1 or 2-3) in which some |u_i| lies within the guard band are walked
+// again and the pairs of the band re-tested in FP64, correcting the sums where
+// the FP64 test disagrees.  The parts' sums are
 // added in a fixed order through LDS at the end, after which lane (row, s)
 // holds voxels s NV .. s NV + NV - 1 of its row (NV = 4 / NQ).
 //
