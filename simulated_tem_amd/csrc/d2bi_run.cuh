@@ -914,7 +914,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
                 std::memset(&G, 0, sizeof G);
                 for (int a = 0; a < na; a++)
                     for (int i = 0; i < 3; i++) G.g[a][i] = gshift[3 * (app + a) + i];
-                const dim3 grid((unsigned)((nr + 255) / 256));
+                const dim3 grid(xcd_grid(nr));
                 auto go = [&](auto kern) {
                     hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, nr, w.slot_src.as<int2>(), d_x, BP, G, nr,
                                        na > 1 ? w.app_cs.as<double2>() : w.slot_cs64.as<double2>(),
