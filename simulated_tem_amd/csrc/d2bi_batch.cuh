@@ -95,7 +95,8 @@ static int enqueue_count(const Cond& c, int idx, Batch& B, hipStream_t s)
     int* cnt = B.blkcnt.as<int>() + c.o_blk;
     int* off = B.blkoff.as<int>() + c.o_blk;
     if (c.n > 0)
-        hipLaunchKernelGGL(k_bin_classify, dim3(c.nblk), dim3(BIN_BLOCK), 0, s, c.d_x, c.BP, mask, cnt, c.nblk);
+        hipLaunchKernelGGL(k_bin_classify, dim3(c.nblk), dim3(BIN_BLOCK), 0, s, c.d_x, c.BP, mask, cnt, c.nblk,
+                           ZeroRanges{});
     else
         zero_i32(s, cnt, c.nbc);
     HIPCHK(hipGetLastError());

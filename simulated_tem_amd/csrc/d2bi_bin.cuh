@@ -102,12 +102,14 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t m)
     return __builtin_amdgcn_readfirstlane(m);
 }
 
-// Pass 1: replica predicate bits per atom and per-(replica, block) counts.
+// Pass 1: replica predicate bits per atom and per-(replica, block) counts.  It
+// also clears what the later passes count into (Z): a launch less.
 __global__ __launch_bounds__(BIN_BLOCK) void k_bin_classify(const double* __restrict__ x, BinParams P,
                                                             uint32_t* __restrict__ mask,
-                                                            int* __restrict__ blk_cnt, int nblk)
+                                                            int* __restrict__ blk_cnt, int nblk, ZeroRanges Z)
 {
     __shared__ int cnt[MAX_REPL];
+    zero_share(Z);
     if (threadIdx.x < MAX_REPL) cnt[threadIdx.x] = 0;
     __syncthreads();
     const int lane = threadIdx.x & 63;
@@ -472,11 +474,12 @@ static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, 
     CHK(w.counters.ensure(sizeof(Counters)));
     CHK(w.scan_tmp.ensure(sizeof(int) * std::max(scan_tmp_ints(nbc), scan_tmp_ints(ncell))));
     Counters* ct = w.counters.as<Counters>();
-    zero_i32(s, w.cell_cnt.as<int>(), ncell + 1, (int*)ct, sizeof(Counters) / sizeof(int), w.blk_cnt.as<int>(),
-             n > 0 ? 0 : nbc);
+    const ZeroRanges Z{{w.cell_cnt.as<int>(), (int*)ct}, {ncell + 1, sizeof(Counters) / sizeof(int)}};
     if (n > 0)
         hipLaunchKernelGGL(k_bin_classify, dim3(nblk), dim3(BIN_BLOCK), 0, s, d_x, P, w.mask.as<uint32_t>(),
-                           w.blk_cnt.as<int>(), nblk);
+                           w.blk_cnt.as<int>(), nblk, Z);
+    else
+        zero_i32(s, Z.p[0], Z.n[0], Z.p[1], Z.n[1], w.blk_cnt.as<int>(), nbc);
     HIPCHK(hipGetLastError());
     CHK(scan_exclusive_tmp(w.blk_cnt.as<int>(), w.blk_off.as<int>(), nbc, w.scan_tmp.as<int>(), s,
                            ScanEnds{&ct->n_points, nullptr, nullptr, 0}));

@@ -255,6 +255,15 @@ __global__ void k_zero(ZeroRanges Z)
     }
 }
 
+// The first two arrays, by a kernel that has other work too.
+__device__ __forceinline__ void zero_share(const ZeroRanges& Z)
+{
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+        for (int64_t i = first; i < Z.n[r]; i += step) Z.p[r][i] = 0;
+}
+
 static void zero_i32(hipStream_t s, int* p0, int64_t n0, int* p1 = nullptr, int64_t n1 = 0, int* p2 = nullptr,
                      int64_t n2 = 0, int* p3 = nullptr, int64_t n3 = 0)
 {
