@@ -655,7 +655,7 @@ static int run_integrate(const d2bi_plan* p, bool dens, int mode, hipStream_t s,
 
 // Whole condition: bin -> voxelise -> integrate on workspace w, the image
 // written to d_img (device memory of Mx*My doubles) or, when d_img is null,
-// left in w.img; copied to h_img when that is given.  The host waits once, at
+// left in w.img (copied to h_img when that is given).  The host waits once, at
 // the end: the point arrays are sized by an estimate, and a condition that
 // has more points is imaged again with the exact count (the wait for the
 // count between the counting and the scatter left the GPU idle for 45-50 us).
@@ -676,14 +676,18 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
     const bool dens = r->use_density != 0;
     BP.fast = mode == D2BI_MODE_FAST ? 1 : 0;
     const int64_t plane = (int64_t)plan.Mx * plan.My;
-    if (!d_img) {
+    // results come back through pinned memory, small images too: those are
+    // integrated right behind the counters, so that one copy brings both
+    const bool small = h_img && plane <= 64 * 1024, joint = small && !d_img && !w.counters.arena;
+    if (joint) {
+        CHK(w.counters.ensure(sizeof(Counters) + sizeof(double) * plane));
+        d_img = reinterpret_cast<double*>(w.counters.as<char>() + sizeof(Counters));
+    } else if (!d_img) {
         CHK(w.img.ensure(sizeof(double) * plane));
         d_img = w.img.as<double>();
     }
     hipStream_t s = g.stream;
     Timer T{g.ev, s};
-    // results come back through pinned memory, small images too
-    const bool small = h_img && plane <= 64 * 1024;
     Counters* ct;
     void* hp;
     if (w.counters.arena) {
@@ -705,8 +709,9 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
         CHK(T.record(2));
         CHK(run_integrate(&plan, dens, mode, s, w, d_img));
         CHK(T.record(3));
-        HIPCHK(hipMemcpyAsync(ct, w.counters.p, sizeof(Counters), hipMemcpyDeviceToHost, s));
-        if (small) HIPCHK(hipMemcpyAsync(hi, d_img, sizeof(double) * plane, hipMemcpyDeviceToHost, s));
+        HIPCHK(hipMemcpyAsync(ct, w.counters.p, sizeof(Counters) + (joint ? sizeof(double) * plane : 0),
+                              hipMemcpyDeviceToHost, s));
+        if (small && !joint) HIPCHK(hipMemcpyAsync(hi, d_img, sizeof(double) * plane, hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         return D2BI_OK;
     };
