@@ -62,3 +62,22 @@ def test_batches_taking_turns(mode):
         out = imaging.computeD2BI_img_batch(batches[turn], mode=mode)
         for got, want in zip(out, alone[turn]):
             assert np.array_equal(got, want), turn
+
+
+@pytest.mark.parametrize("mode", ["fp64", "fast"])
+def test_image_copies(mode):
+    """A small image comes back in one copy with the counters, from 65,536
+    pixels on in a copy of its own: both sides of that line, growing and
+    shrinking again, equal the image left in device memory to the bit."""
+    for voxels in ((256, 256), (256, 258), (40, 36), (256, 256), (300, 310), (40, 36)):
+        cfg = synth.scaled("c0", cells=(7, 7, 7))
+        cfg.update(sg=[0.01], d=(voxels[0] * 3.1652 / 4, voxels[1] * 3.1652 / 4, 21 * 3.1652 / 4))
+        x, box = synth.make_atoms(cfg)
+        x, conds = synth.conditions(cfg, x, box)
+        im = conds[0][0]
+        st = abi.D2biStats()
+        host = im.computeD2BI_img(x, 0.005, 40, mode=mode, stats=st)
+        assert host.shape == (voxels[1], voxels[0]) and st.n_points == orc.Condition(im.rec, x).n_points
+        d = imaging.DeviceBuffer(host.shape)
+        im.computeD2BI_img(imaging.Atoms(x), 0.005, 40, mode=mode, out=d)
+        assert np.array_equal(host, d.numpy())
