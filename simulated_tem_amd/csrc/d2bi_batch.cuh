@@ -288,7 +288,8 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
     CHK(B.tot.ensure(sizeof(int) * nRec));
     B.total_plane = o_img;
     // branch streams and the events that fork and join them (default priority)
-    int nbr = std::min(batch_branches(), nRec);
+    const int want = std::min(batch_branches(), nRec);
+    int nbr = want;
     if (!B.fork) HIPCHK(hipEventCreateWithFlags(&B.fork, hipEventDisableTiming));
     for (int k = 1; k < nbr; k++) {
         if (!B.stream[k - 1]) HIPCHK(hipStreamCreateWithFlags(&B.stream[k - 1], hipStreamNonBlocking));
@@ -346,7 +347,30 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
         }
         nbr = fit;
     }
-    for (int k = 0; k < nbr; k++) {
+    // branch count: forced, cached, or tuned below by timing a run on each
+    // count (images are the same on any count); the count that fits is kept
+    // unless another is 3 % faster.  A cached count sizes its own branches
+    // only: a workspace for the others, given back after the run, cost a
+    // batch of eight conditions of 1e4 to 4e5 atoms on three of four branches
+    // 1.89 ms a call against 1.37, in some processes 8.4
+    const bool pick = nbr > 1 && !std::getenv("D2BI_BATCH_BRANCHES") && tuning_on();
+    TuneKey bkey{};
+    int chosen = nbr;
+    bool tune = false;
+    if (pick) {
+        int64_t sum_vox = 0, max_vox_c = 0, sum_n = 0, sum_p = 0;
+        for (int i = 0; i < nRec; i++) {
+            sum_vox += C[i].nvox;
+            max_vox_c = std::max(max_vox_c, C[i].nvox);
+            sum_n += C[i].n;
+            sum_p += C[i].plan.nPrec;
+        }
+        bkey = TuneKey{TUNE_BRANCHES, nRec, mode, sum_vox, max_vox_c, sum_n, sum_p, nbr, 0};
+        const int c = tune_get(bkey);
+        tune = c < 1 || c > nbr;
+        if (!tune) chosen = c;
+    }
+    for (int k = 0; k < chosen; k++) {
         int rc_ = D2BI_OK;
         branch_buffers(B.branch_ws(k), bz, [&](Buf& b, size_t bytes) {
             if (rc_ == D2BI_OK) rc_ = b.ensure(bytes);
@@ -367,45 +391,29 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
         }
         C[i].variant = v;
     }
-    // branch count: forced, cached, or tuned by timing a run on each count
-    // (images are the same on any count); the count that fits is kept unless
-    // another is 3 % faster
-    int chosen = nbr;
-    bool done = false;
     HIPCHK(hipEventRecord(g.ev[0], s));
-    if (nbr > 1 && !std::getenv("D2BI_BATCH_BRANCHES") && tuning_on()) {
-        int64_t sum_vox = 0, max_vox_c = 0, sum_n = 0, sum_p = 0;
-        for (int i = 0; i < nRec; i++) {
-            sum_vox += C[i].nvox;
-            max_vox_c = std::max(max_vox_c, C[i].nvox);
-            sum_n += C[i].n;
-            sum_p += C[i].plan.nPrec;
-        }
-        const TuneKey bkey{TUNE_BRANCHES, nRec, mode, sum_vox, max_vox_c, sum_n, sum_p, nbr, 0};
-        const int c = tune_get(bkey);
-        if (c >= 1 && c <= nbr) {
-            chosen = c;
-        } else {
-            float tbest = 3.4e38f;
-            for (int q = 0; q < nbr; q++) {
-                const int nb = q == 0 ? nbr : q;            // the default first
-                int rq = D2BI_OK;
-                const float t = time_launch([&] { rq = enqueue_batch(B, mode, nb, false); }, s, 1);
-                CHK(rq);
-                if (q == 0) tbest = t >= 0.0f ? 0.97f * t : 3.4e38f;
-                else if (t >= 0.0f && t < tbest) {
-                    tbest = t;
-                    chosen = nb;
-                }
+    if (tune) {
+        float tbest = 3.4e38f;
+        for (int q = 0; q < nbr; q++) {
+            const int nb = q == 0 ? nbr : q;                // the default first
+            int rq = D2BI_OK;
+            const float t = time_launch([&] { rq = enqueue_batch(B, mode, nb, false); }, s, 1);
+            CHK(rq);
+            if (q == 0) tbest = t >= 0.0f ? 0.97f * t : 3.4e38f;
+            else if (t >= 0.0f && t < tbest) {
+                tbest = t;
+                chosen = nb;
             }
-            tune_put(bkey, chosen);
-            done = true;                                    // each run imaged every condition
         }
+        tune_put(bkey, chosen);
+    } else {                                                // (each timed run imaged every condition)
+        CHK(enqueue_batch(B, mode, chosen, false));
     }
-    if (!done) CHK(enqueue_batch(B, mode, chosen, false));
-    // workspaces of branches that are not used go back to the device
     HIPCHK(hipStreamSynchronize(s));
-    for (int k = std::max(1, chosen); k < nbr; k++) B.branch_ws(k).release_all();
+    // workspaces of branches that timing has just left unused, or that are
+    // unused where device memory is short, go back to the device
+    if (tune || nbr < want)
+        for (int k = std::max(1, chosen); k < nbr; k++) B.branch_ws(k).release_all();
     B.nbr = chosen;
     return D2BI_OK;
 }

@@ -149,3 +149,47 @@ def test_tuning_cache_file_and_fresh_processes(tmp_path):
         assert np.array_equal(a, c) and np.array_equal(b, c)
     for i in range(3):
         assert np.array_equal(tuned[i], tuned[3 + i])      # eager == batch
+
+
+_TURNS = r"""
+import sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+from simulated_tem_amd import imaging
+from tests.test_gpu_tune import _conds
+imaging.init(0)
+conds = _conds()
+ref = [im.computeD2BI_img(at, pa, npr, mode="fast") for (im, at, pa, npr) in conds]
+for turn in range(3):
+    for pick in ([0, 1, 2], [2, 1], [1, 0, 2], [1, 0, 2]):
+        st = imaging.D2biStats()
+        out = imaging.computeD2BI_img_batch([conds[i] for i in pick], mode="fast", stats=st)
+        for i, b in zip(pick, out):
+            assert np.array_equal(b, ref[i]), (turn, pick, i)
+        print(len(pick), st.n_branches, flush=True)
+"""
+
+
+@pytest.mark.parametrize("three,two", [(2, 1), (1, 2), (3, 1)])
+def test_batches_in_turn_on_cached_branch_counts(tmp_path, three, two):
+    """Batches on fewer branches than fit, as a cache file says (three
+    conditions on `three`, two on `two`), take turns in one process, the last
+    of them repeated as a graph: the counts are the cached ones and every image
+    is the condition's own, bit for bit."""
+    cache = tmp_path / "tune.txt"
+    env = {k: v for k, v in os.environ.items() if k not in TUNE_VARS}
+    env["D2BI_TUNE_CACHE"] = str(cache)
+
+    def turns():
+        r = subprocess.run([sys.executable, "-c", _TURNS, ROOT], env=env, cwd=ROOT, capture_output=True, text=True,
+                           timeout=100)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return [tuple(int(v) for v in ln.split()) for ln in r.stdout.splitlines()]
+
+    turns()
+    lines = [ln if ln[0] != 3 else ln[:9] + ((three if ln[1] == 3 else two),) for ln in _cache_lines(cache)]
+    cache.write_text("".join(" ".join(str(v) for v in ln) + "\n" for ln in lines))
+    print("\n[turns] three on %d, two on %d" % (three, two), flush=True)
+    got = turns()
+    assert len(got) == 12
+    assert all(nb == {3: three, 2: two}[n] for n, nb in got)
