@@ -94,12 +94,17 @@ __global__ __launch_bounds__(256) void k_voxel_fp64(VoxParams P, const int* __re
 // range is the reference's to the bit, and so are the members and the nearest
 // range.  A voxel whose cell is not next to the candidate's along an axis
 // gets an infinite square there (the 27-cell rule).  The weight factorises the
-// same way,
-//     exp(-(d0 - i h)^2 / 2s^2) = exp(-d0^2 / 2s^2) exp(d0 h / s^2)^i b_i,
-// two exponentials per candidate and axis; b_i = exp(-(i h)^2 / 2s^2) depends
-// on the voxel alone and multiplies its sums at the end.  Lane (xy, part) walks every fourth candidate of the subtile's list
-// for the four voxels along z at its x and y: an add, a compare, a select, a
-// multiply and two FMAs per pair, in FP64.
+// same way, into exp(-d^2 / 2s^2) of the three axes, each an exponential of its
+// own: of a member none is below exp(-4.5), whatever the voxels' sides, and the
+// product is nearer the exact weight than one exponential of the rounded range
+// (relative rms 1.8e-16 against 2.7e-16).  A recurrence along each axis,
+// exp(-d0^2 / 2s^2) exp(d0 h / s^2)^i from the region's first voxel, would take
+// two exponentials for eight, but carries exponents of the whole region: weights
+// off by up to 1e-14 at four voxels per lattice parameter, and under- and
+// overflow where voxels are taller than about 5 sigma.  Lane (xy, part) walks
+// every fourth candidate of the subtile's list for the four voxels along z at
+// its x and y: an add, a compare, a select, a multiply and two FMAs per pair, in
+// FP64.
 //
 // Bound: FP64 VALU issue (an add, multiply or compare ~4.7 cycles per wave,
 // measured) in the pair loop; the per-voxel 27-cell walk above evaluates 180
@@ -120,10 +125,7 @@ static constexpr int F64R_REC = 64;
 
 template <int NA>
 struct F64Record {
-    double2 x[REG], y[REG];                          // (square, weight) per voxel position
-    double z[REG];                                   // squares
-    double wz[REG / TILE];                           // weight of each subtile's first voxel
-    double ratio;                                    // weight ratio along z
+    double2 x[REG], y[REG], z[REG];                  // (square, weight) per voxel position
     double2 cs[NA];                                  // cos and sin of g.r
 };
 
@@ -201,33 +203,20 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
         } else {
             const int u = ((S.upk[c0 + lane] >> (8 * ax)) & 255) - 1;
             const double side = ax == 0 ? P.a[0] : ax == 1 ? P.a[1] : P.a[2];
-            const double h = ax == 0 ? R.h[0] : ax == 1 ? R.h[1] : R.h[2];
-            const double d0 = side * (in[0] + (u - S.zi[ax][0]));
-            const double ratio = exp((2.0 * d0) * (h * P.i2s2));
-            double w = exp(-(d0 * d0) * P.i2s2);
-            if (ax == 2) q.ratio = ratio;
+            double2* const out = ax == 0 ? q.x : ax == 1 ? q.y : q.z;
 #pragma unroll
             for (int v = 0; v < REG; v++) {
                 const int k = u - S.lc[ax][v];
                 const double d = side * (in[0] + (k - S.zi[ax][v]));
-                const double d2 = (unsigned)(k + 1) <= 2u ? d * d : HUGE_VAL;
-                if (ax == 2) {
-                    q.z[v] = d2;
-                    if (v % TILE == 0) q.wz[v / TILE] = w;
-                } else {
-                    (ax == 0 ? q.x : q.y)[v] = make_double2(d2, w);
-                }
-                w = w * ratio;
+                const double d2 = d * d;
+                out[v] = make_double2((unsigned)(k + 1) <= 2u ? d2 : HUGE_VAL, exp(-d2 * P.i2s2));
             }
         }
         // the padding record: no voxel is in range of it
-        Rec& e = U.rec[F64R_REC];
-        if (threadIdx.x < REG) {
-            e.x[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
-            e.y[threadIdx.x] = make_double2(HUGE_VAL, 0.0);
-        } else if (threadIdx.x < sizeof(Rec) / 8 - 3 * REG) {
-            reinterpret_cast<double*>(&e)[threadIdx.x + 3 * REG] = 0.0;      // past x and y
-        }
+        static_assert(sizeof(Rec) == sizeof(double2) * (3 * REG + NA), "x, y and z, then the phases");
+        if (threadIdx.x < 3 * REG + NA)
+            reinterpret_cast<double2*>(&U.rec[F64R_REC])[threadIdx.x] =
+                make_double2(threadIdx.x < 3 * REG ? HUGE_VAL : 0.0, 0.0);
     };
 
     for (int t_next = 0, T = 1; t_next < T;) {
@@ -257,14 +246,14 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
                 for (int k = 0; k < nl; k += 4) {
                     const Rec& q = *reinterpret_cast<const Rec*>(rec + lists[wave][k + part]);
                     const double2 qx = q.x[lx], qy = q.y[ly];
-                    const double s12 = qx.x + qy.x, ratio = q.ratio;
-                    double p = (qx.y * qy.y) * q.wz[z];
+                    const double s12 = qx.x + qy.x, wxy = qx.y * qy.y;
                     double2 cs[NA];
 #pragma unroll
                     for (int a = 0; a < NA; a++) cs[a] = q.cs[a];
 #pragma unroll
                     for (int v = 0; v < TILE; v++) {
-                        const double dd = s12 + q.z[z * TILE + v];
+                        const double2 qz = q.z[z * TILE + v];
+                        const double dd = s12 + qz.x, p = wxy * qz.y;
                         const bool in = dd <= P.rc2;
                         // a pair out of range keeps the low word of its
                         // weight: < 1e-313, dropped from the sums at the end
@@ -278,7 +267,6 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
                         // operation per pair
                         if (MIN) asm("v_min_f64 %0, %0, %1" : "+v"(dmin[z][v]) : "v"(dd));
                         if (DIAG) cnt[z][v] += in ? 1 : 0;
-                        p = p * ratio;
                     }
                 }
             }
@@ -292,13 +280,12 @@ __global__ __launch_bounds__(64 * F64R_NW, NA == 4 ? 2 : 4) void k_voxel_fp64_re
 #pragma unroll
     for (int z = 0; z < NS; z++) {
         const int vx = B.o[0] + lx, vy = B.o[1] + ly, vz = B.o[2] + z * TILE + part;
-        const double scale = (R.b[0][lx] * R.b[1][ly]) * R.b[2][z * TILE + part];
         const bool out = vx < P.Mx && vy < P.My && vz < P.Mz;
         const int64_t o = (int64_t)vx + (int64_t)P.Mx * (vy + (int64_t)P.My * vz);
 #pragma unroll
         for (int a = 0; a < NA; a++) {
-            const double re = drop(part_sum(sre[z][a][0], sre[z][a][1], sre[z][a][2], sre[z][a][3])) * scale;
-            const double im = drop(part_sum(sim[z][a][0], sim[z][a][1], sim[z][a][2], sim[z][a][3])) * scale;
+            const double re = drop(part_sum(sre[z][a][0], sre[z][a][1], sre[z][a][2], sre[z][a][3]));
+            const double im = drop(part_sum(sim[z][a][0], sim[z][a][1], sim[z][a][2], sim[z][a][3]));
             // (|S| counts from 1e-16 on, so its square is in range)
             double ww = sqrt(fma(re, re, im * im));
             ww = 1 / (1.0e-16 > ww ? 1.0e-16 : ww);

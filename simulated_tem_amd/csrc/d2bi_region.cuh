@@ -33,8 +33,6 @@ struct RegionParams {
     int nreg, per_xcd;          // regions; workgroups per XCD (the grid is 8 per_xcd)
     float rc_cull2;             // (3 sigma)^2 widened for the FP32 box culls
     float cellf[3];             // link-cell sides in FP32
-    double h[3];                // voxel sides
-    double b[3][REG];           // exp(-(i h)^2 / 2 sigma^2), i voxels from the region's first
 };
 
 // Region of a workgroup: rows of regions along x dealt to the XCDs in turn

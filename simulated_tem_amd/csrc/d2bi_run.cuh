@@ -115,7 +115,7 @@ static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParam
 static bool region_params(const d2bi_plan* p, const AxisTables& tab, const VoxParams& V, RegionParams* R)
 {
     R->v = V;
-    const int M[3] = {p->Mx, p->My, p->Mz}, E[3] = {p->Ex, p->Ey, p->Ez};
+    const int M[3] = {p->Mx, p->My, p->Mz};
     int n[3];
     int64_t worst = 1;
     for (int a = 0; a < 3; a++) {
@@ -125,10 +125,6 @@ static bool region_params(const d2bi_plan* p, const AxisTables& tab, const VoxPa
         worst *= mx;
         n[a] = (M[a] + REG - 1) / REG;
         R->cellf[a] = (float)p->a_col[4 * a];
-        // voxel sides: the link cells divide the voxel box, in x and y with a
-        // margin of deltaM voxels on both sides (plan_image)
-        R->h[a] = p->a_col[4 * a] * E[a] / (M[a] + (a < 2 ? 2 * p->deltaM : 0));
-        for (int i = 0; i < REG; i++) R->b[a][i] = std::exp(-((i * R->h[a]) * (i * R->h[a])) * p->i2s2);
     }
     if (worst > REG_MAXC) return false;
     R->nrx = n[0];
