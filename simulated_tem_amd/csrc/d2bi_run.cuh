@@ -111,7 +111,11 @@ static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParam
 
 // Launch parameters of the region kernels for a plan; false where they do not
 // apply: a region spanning more link cells than its table holds (voxels
-// coarser than about a third of the lattice parameter).
+// coarser than about a third of the lattice parameter), or so long that the
+// culls' FP32 positions might lose a member.  A position takes at most ten
+// roundings of 2^-24 of the range's length L, 1e-6 L over three axes, and the
+// culls allow half of 1e-4 of 3 sigma: 150 sigma, of which 100 are used (15 at
+// four voxels per lattice parameter, 28 at one).
 static bool region_params(const d2bi_plan* p, const AxisTables& tab, const VoxParams& V, RegionParams* R)
 {
     R->v = V;
@@ -123,6 +127,7 @@ static bool region_params(const d2bi_plan* p, const AxisTables& tab, const VoxPa
         for (int t0 = 0; t0 < M[a]; t0 += REG)
             mx = std::max(mx, tab.cell[a][std::min(M[a], t0 + REG) - 1] - tab.cell[a][t0] + 3);
         worst *= mx;
+        if (!(mx * p->a_col[4 * a] <= 100.0 * p->sigma)) return false;
         n[a] = (M[a] + REG - 1) / REG;
         R->cellf[a] = (float)p->a_col[4 * a];
     }

@@ -112,3 +112,29 @@ def test_weight_rounding(M):
         worst = max(worst, float(e / bound))
     print("[weights] M=%d members <= %d worst error / bound %.2f" % (M, cnt.max(), worst), flush=True)
     assert worst <= 1.0
+
+
+@pytest.mark.parametrize("height", [90.0, 1000.0, 1733.0, 3000.0])
+def test_members_at_the_rim(height):
+    """Points a hair inside 3 sigma above and below voxels many sigma tall: a
+    position is then larger than FP32 resolves the rim at, and every one of them
+    still counts."""
+    nz, hz = 16, height * SIGMA
+    d = np.array([8 * A0 / 4, 8 * A0 / 4, nz * hz])
+    cfg = synth.scaled("c0", cells=(7, 7, 7))
+    cfg.update(d=tuple(d), sg=[0.0])
+    _, conds = synth.conditions(cfg, np.zeros((1, 3)), np.array([40.0, 40.0, nz * hz]))
+    im = conds[0][0]
+    im.setSupercellTilt(np.eye(3), np.eye(3))
+    im.rec.gk_n[2] = nz
+    im.rec.gk_a[8] = d[2] / nz
+    side = np.array([im.rec.gk_a[0], im.rec.gk_a[4], im.rec.gk_a[8]])
+    rim = 3 * SIGMA * (1 - 1e-7)
+    v = np.array([(iz % 8, (3 * iz) % 8, iz) for iz in range(nz)])
+    up = np.array([0.0, 0.0, rim])
+    x = np.concatenate([v * side + up, v * side - up]) - np.array(im.rec.delta)
+    ph, _, cnt, r2m = im.field(x, "fp64")
+    oph, _, ocnt, or2m = orc.Condition(im.rec, x).field(nthreads=NTH)
+    print("[rim] %.0f sigma members %d of %d" % (height, cnt.sum(), ocnt.sum()), flush=True)
+    assert ocnt.sum() >= 2 * nz - 2
+    assert np.array_equal(cnt, ocnt) and np.array_equal(r2m, or2m)
