@@ -70,17 +70,38 @@ struct FastColumn {
     }
 };
 
+// Points scaled by a power of two each, so that their largest component lies
+// in [1/2, 1): no bit of what follows changes but the exponents.
+template <int NP>
+__device__ __forceinline__ void rescale(double* p0r, double* p0i, double* pgr, double* pgi)
+{
+#pragma unroll
+    for (int p = 0; p < NP; p++) {
+        const double m = fmax(fmax(fabs(p0r[p]), fabs(p0i[p])), fmax(fabs(pgr[p]), fabs(pgi[p])));
+        const int e = -__builtin_amdgcn_frexp_exp(m);
+        p0r[p] = __builtin_amdgcn_ldexp(p0r[p], e);
+        p0i[p] = __builtin_amdgcn_ldexp(p0i[p], e);
+        pgr[p] = __builtin_amdgcn_ldexp(pgr[p], e);
+        pgi[p] = __builtin_amdgcn_ldexp(pgi[p], e);
+    }
+}
+
 // One lane per pixel column, NP precession points marched together from
 // one read of the column (the field is shared by all precession points:
 // precession changes s_g only).  Classic RK4 with h = 2 dz; the per-step
 // renormalisation of the reference is a positive scalar on a linear map, so it
-// is applied once at the end: I = |phi_g|^2/|phi|^2.
+// is applied once at the end: I = |phi_g|^2/|phi|^2.  FP64 points are rescaled
+// every `every` double steps (RS), so that a column of any depth and deviation
+// stays in range; instances without are for those whose bound already does
+// (rescale_every), and take no branch and no register for it.
 // The mean-potential term c0 = b0 rho stays in, although in the exact ODE it
 // is a global phase: RK4's truncation error depends on the whole matrix, and
 // over 800 double steps leaving c0 out moves |phi_g|^2 by ~2e-4.
-template <int NP, class T, class S>
-__device__ __forceinline__ void march_stage(const S& s, int nz, T dz, const T* aa, T* p0r, T* p0i, T* pgr, T* pgi)
+template <int NP, bool RS = false, class T, class S>
+__device__ __forceinline__ void march_stage(const S& s, int nz, T dz, const T* aa, T* p0r, T* p0i, T* pgr, T* pgi,
+                                            int every = 0)
 {
+    [[maybe_unused]] int left = every;
     const T dz3 = dz / 3, dz23 = 2 * dz / 3, dz2 = 2 * dz;
 #pragma unroll
     for (int p = 0; p < NP; p++) { p0r[p] = 1; p0i[p] = 0; pgr[p] = 0; pgi[p] = 0; }
@@ -146,6 +167,12 @@ __device__ __forceinline__ void march_stage(const S& s, int nz, T dz, const T* a
             pgr[p] = fm(dgr, dz3, agr); pgi[p] = fm(dgi, dz3, agi);
         }
         c0a = c0c; cgra = cgrc; cgia = cgic;
+        if constexpr (RS) {
+            if (--left == 0) {
+                left = every;
+                rescale<NP>(p0r, p0i, pgr, pgi);
+            }
+        }
     }
     }
 }
@@ -286,9 +313,11 @@ __device__ __forceinline__ cplx<T> horner(const CPoly<D, T>& M, T al)
 // The column's march: NP points from (1, 0) through nz samples (sample nz is
 // sample 0); S gives a sample's coefficients (load(k) what is read, coef(raw)
 // c0 and cg).
-template <int NP, class T, class S>
-__device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al_, T* p0r, T* p0i, T* pgr, T* pgi)
+template <int NP, bool RS = false, class T, class S>
+__device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al_, T* p0r, T* p0i, T* pgr, T* pgi,
+                                           int every = 0)
 {
+    [[maybe_unused]] int left = every;
     const T dz2 = 2 * dz, dz6 = dz / 3, third = T(1) / 3, two3 = T(2) / 3, sixth = T(1) / 6, half = T(0.5), one = T(1);
 #pragma unroll
     for (int p = 0; p < NP; p++) { p0r[p] = 1; p0i[p] = 0; pgr[p] = 0; pgi[p] = 0; }
@@ -360,6 +389,12 @@ __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al
             pgi[p] = fm(m21.r, y0i, fm(m21.i, y0r, fm(m22.r, ygi, m22.i * ygr)));
         }
         c0a = c0c; cgra = cgrc; cgia = cgic;
+        if constexpr (RS) {
+            if (--left == 0) {
+                left = every;
+                rescale<NP>(p0r, p0i, pgr, pgi);
+            }
+        }
     }
 }
 
@@ -420,6 +455,7 @@ struct IntParams {
     double b0, bg, dz;
     double aa[INT_SLOTS];       // 2 pi s_g per precession point
     double al[INT_SLOTS];       // 2 dz aa
+    int every;                  // double steps between rescalings (0: none)
     int accumulate;             // add the column's sum to img
     double div;                 // and divide by it (0: not yet)
 };
@@ -466,7 +502,7 @@ constexpr int int_threads64(int np) { return np <= 3 ? 1024 : np <= 8 ? 512 : 25
 // (1 point 0.079 ms, 5.8 TB/s).  A march per point with the reference's
 // divisions and a square root per step took 0.26 ms for 1 point, 2.00 for 8
 // and 8.7 for 32; this takes 0.079, 0.35 and 1.21.
-template <int NP, bool DENS, bool SPLIT>
+template <int NP, bool DENS, bool SPLIT, bool RS>
 __global__ __launch_bounds__(SPLIT ? int_threads64(NP) : 256) void k_integrate_fp64(IntParams P,
                                                                                   const double* __restrict__ fre,
                                                                                   const double* __restrict__ fim,
@@ -483,8 +519,8 @@ __global__ __launch_bounds__(SPLIT ? int_threads64(NP) : 256) void k_integrate_f
     const Fp64Column<DENS> s{fre, fim, frho, live ? col : plane - 1, plane, P.Mz, P.b0, P.bg};
     const int p0 = sp * NP;
     double p0r[NP], p0i[NP], pgr[NP], pgi[NP];
-    if constexpr (NP >= 6) march_poly<NP>(s, P.Mz, P.dz, P.al + p0, p0r, p0i, pgr, pgi);
-    else march_stage<NP>(s, P.Mz, P.dz, P.aa + p0, p0r, p0i, pgr, pgi);
+    if constexpr (NP >= 6) march_poly<NP, RS>(s, P.Mz, P.dz, P.al + p0, p0r, p0i, pgr, pgi, P.every);
+    else march_stage<NP, RS>(s, P.Mz, P.dz, P.aa + p0, p0r, p0i, pgr, pgi, P.every);
     double acc = intensity_sum<NP>(min(NP, P.np - p0), p0r, p0i, pgr, pgi);
     if constexpr (SPLIT) {
         __shared__ double part[int_threads64(NP)];
