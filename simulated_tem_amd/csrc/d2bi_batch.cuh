@@ -17,7 +17,7 @@ struct Cond {
     BinParams BP;
     const double* d_x = nullptr;
     int64_t n = 0;
-    int nblk = 0, ncell = 0, variant = 0;
+    int nblk = 0, ncell = 0, variant = 0, mode = 0;
     bool dens = false;
     int64_t nr = 0, nbc = 0, nvox = 0, plane = 0;
     int64_t o_mask = 0, o_blk = 0, o_scan = 0, o_img = 0;
@@ -106,7 +106,7 @@ static int enqueue_count(const Cond& c, int idx, Batch& B, hipStream_t s)
 
 // the rest of one condition: bin, voxelise, integrate into its image slice,
 // on workspace w
-static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w, hipStream_t s)
+static int enqueue_rest(const Cond& c, int idx, Batch& B, Workspace& w, hipStream_t s)
 {
     const d2bi_plan* p = &c.plan;
     Counters* ct = B.counters.as<Counters>() + idx;
@@ -118,7 +118,7 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w
     dummy.use_density = c.dens ? 1 : 0;
     fill_vox_params(&dummy, p, c.ax, &V);
     double* d_img = B.img.as<double>() + c.o_img;
-    if (mode == D2BI_MODE_FP64) {
+    if (c.mode == D2BI_MODE_FP64) {
         CHK(launch_voxel_fp64(p, c.tab, V, 1, w, w.slot_cs64.as<double2>(), 0, 0, nullptr, nullptr, s));
         return launch_integrate_fp64(p, c.dens, d_img, s, w);
     }
@@ -137,7 +137,7 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, int mode, Workspace& w
 
 // Sizes of one branch's workspace: the largest condition of the batch.
 struct BranchSizes {
-    int mode;
+    bool fast, f64;             // what its conditions run in
     int64_t max_nr, max_cell, max_vox, max_scan;
 };
 
@@ -145,17 +145,19 @@ struct BranchSizes {
 template <class F>
 static void branch_buffers(Workspace& w, const BranchSizes& z, F f)
 {
-    point_buffers(w, z.mode == D2BI_MODE_FAST, false, false, false,
-                  [&](Buf& b, size_t bytes) { f(b, bytes * z.max_nr); });
+    for (int fast = 0; fast < 2; fast++)
+        if (fast ? z.fast : z.f64)
+            point_buffers(w, fast, false, false, false, [&](Buf& b, size_t bytes) {
+                if (!fast || !z.f64 || &b == &w.slot_sn32) f(b, bytes * z.max_nr);      // (each once)
+            });
     f(w.cell_cnt, sizeof(int) * z.max_cell);
     f(w.cell_start, sizeof(int) * z.max_cell);
-    if (z.mode == D2BI_MODE_FP64) {
+    if (z.f64) {
         f(w.f64_re, sizeof(double) * z.max_vox);
         f(w.f64_im, sizeof(double) * z.max_vox);
         f(w.f64_rho, sizeof(double) * z.max_vox);
-    } else {
-        f(w.f32_field, sizeof(float4) * z.max_vox);
     }
+    if (z.fast) f(w.f32_field, sizeof(float4) * z.max_vox);
     f(w.scan_tmp, sizeof(int) * z.max_scan);
 }
 
@@ -180,7 +182,7 @@ static int64_t branch_bytes(const BranchSizes& z)
 // the branch streams (or captured from them): conditions to branches largest
 // first, each to the least loaded branch (a fixed rule: the same inputs give
 // the same assignment).  count: the counting passes too.
-static int enqueue_batch(Batch& B, int mode, int nb, bool count)
+static int enqueue_batch(Batch& B, int nb, bool count)
 {
     const std::vector<Cond>& C = B.conds;
     const int nRec = (int)C.size();
@@ -207,7 +209,7 @@ static int enqueue_batch(Batch& B, int mode, int nb, bool count)
     }
     for (int i = 0; i < nRec && rc == D2BI_OK; i++) {
         if (count) rc = enqueue_count(C[i], i, B, bstream(branch[i]));
-        if (rc == D2BI_OK) rc = enqueue_rest(C[i], i, B, mode, B.branch_ws(branch[i]), bstream(branch[i]));
+        if (rc == D2BI_OK) rc = enqueue_rest(C[i], i, B, B.branch_ws(branch[i]), bstream(branch[i]));
     }
     // join every branch back, also after an error, so that a capture can end
     for (int k = 1; k < nb; k++)
@@ -218,7 +220,7 @@ static int enqueue_batch(Batch& B, int mode, int nb, bool count)
 }
 
 // Capture the batch (counting passes included) into B.exec.
-static int capture_batch(Batch& B, int mode)
+static int capture_batch(Batch& B)
 {
     hipStream_t s = g.stream;
     hipGraph_t graph;
@@ -227,7 +229,7 @@ static int capture_batch(Batch& B, int mode)
         g_capturing = false;
         return seterr(D2BI_ERR_HIP, "graph capture failed to begin");
     }
-    const int rc = enqueue_batch(B, mode, B.nbr, true);
+    const int rc = enqueue_batch(B, B.nbr, true);
     hipError_t e = hipStreamEndCapture(s, &graph);
     g_capturing = false;
     if (rc != D2BI_OK) {
@@ -261,7 +263,8 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
         CHK(plan_image(&recs[i], atoms[i]->n, precAngle[i], nPrec[i], &c.plan));
         CHK(axis_tables(&recs[i], &c.plan, &c.tab));
         CHK(bin_params(&recs[i], &c.plan, &c.BP));
-        c.BP.fast = mode == D2BI_MODE_FAST ? 1 : 0;
+        c.mode = condition_mode(&c.plan, mode);
+        c.BP.fast = c.mode == D2BI_MODE_FAST ? 1 : 0;
         c.d_x = atoms[i]->x;
         c.n = atoms[i]->n;
         c.BP.n = c.n;
@@ -316,14 +319,16 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
     HIPCHK(hipMemcpyAsync(hr, B.tot.p, sizeof(int) * nRec, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     int64_t max_nr = 1, max_cell = 1, max_vox = 1;
+    bool fast = false, f64 = false;
     for (int i = 0; i < nRec; i++) {
+        (C[i].mode == D2BI_MODE_FAST ? fast : f64) = true;
         if (tot[i] < 0) return seterr(D2BI_ERR_CAPACITY, "point count overflow");
         C[i].nr = tot[i];
         max_nr = std::max(max_nr, C[i].nr);
         max_cell = std::max<int64_t>(max_cell, C[i].ncell + 1);
         max_vox = std::max(max_vox, C[i].nvox);
     }
-    const BranchSizes bz{mode, max_nr, max_cell, max_vox, max_scan};
+    const BranchSizes bz{fast, f64, max_nr, max_cell, max_vox, max_scan};
     // every branch gets a workspace sized for the largest condition; the
     // branches beyond the first run only where what their workspaces
     // would add (branch 0's growth included) fits in 85 % of the free
@@ -381,7 +386,8 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
     // FAST kernel variants (fixed, forced, or with D2BI_FAST_TUNE=1 tuned
     // for unseen shapes), and the launch choices of shapes the tuner has not
     // timed yet: one condition of each such shape, on its own, times them
-    for (int i = 0; i < nRec && mode == D2BI_MODE_FAST; i++) {
+    for (int i = 0; i < nRec; i++) {
+        if (C[i].mode != D2BI_MODE_FAST) continue;
         int v = known_variant(&C[i].plan, C[i].dens);
         if (v < 0 || !condition_tuned(&C[i].plan, C[i].tab, C[i].dens, v)) {
             d2bi_plan tmp;
@@ -397,7 +403,7 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
         for (int q = 0; q < nbr; q++) {
             const int nb = q == 0 ? nbr : q;                // the default first
             int rq = D2BI_OK;
-            const float t = time_launch([&] { rq = enqueue_batch(B, mode, nb, false); }, s, 1);
+            const float t = time_launch([&] { rq = enqueue_batch(B, nb, false); }, s, 1);
             CHK(rq);
             if (q == 0) tbest = t >= 0.0f ? 0.97f * t : 3.4e38f;
             else if (t >= 0.0f && t < tbest) {
@@ -407,7 +413,7 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
         }
         tune_put(bkey, chosen);
     } else {                                                // (each timed run imaged every condition)
-        CHK(enqueue_batch(B, mode, chosen, false));
+        CHK(enqueue_batch(B, chosen, false));
     }
     HIPCHK(hipStreamSynchronize(s));
     // workspaces of branches that timing has just left unused, or that are
@@ -462,7 +468,7 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
         B.key = key;
         B.gen = g_alloc_gen;
     } else {
-        if (!B.exec) CHK(capture_batch(B, mode));
+        if (!B.exec) CHK(capture_batch(B));
         HIPCHK(hipEventRecord(g.ev[0], s));
         HIPCHK(hipGraphLaunch(B.exec, s));
     }
@@ -479,7 +485,7 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
         const Counters* ct = (const Counters*)hr;
         for (int i = 0; i < nRec; i++) {
             st->n_points += B.conds[i].nr;
-            st->n_guard += mode == D2BI_MODE_FAST ? ct[i].n_guard() : 0;
+            st->n_guard += B.conds[i].mode == D2BI_MODE_FAST ? ct[i].n_guard() : 0;
             st->max_per_cell = std::max(st->max_per_cell, ct[i].max_per_cell);
         }
         float ms = 0.0f;

@@ -71,6 +71,32 @@ static int tile_cells(const d2bi_plan* p, const AxisTables& tab, int tz, int ty 
     return worst;
 }
 
+// Binary exponents that the factors of a member's weight take in a tile of 4 x
+// ty x tz voxels: those of the range from the tile's centre (x: along x too;
+// the row kernels' factors take that from each voxel).
+static double tile_bits(const d2bi_plan* p, int tz, int ty, bool x)
+{
+    const double hx = x ? 0.5 * (std::min(TILE, p->Mx) - 1) * p->xmax[0] / p->Mx : 0.0;
+    const double hy = 0.5 * (std::min(ty, p->My) - 1) * p->xmax[1] / p->My;
+    const double hz = 0.5 * (std::min(tz, p->Mz) - 1) * p->xmax[2] / p->Mz;
+    const double q = std::sqrt(hx * hx + hy * hy + hz * hz) + 3.0 * p->sigma;
+    return q * q * p->i2s2 * 1.4426950408889634;
+}
+
+// What the FAST kernels allow them.  A member's X is at least 2^-bits and its
+// 2^t at most 2^(bits + 6.5), FP32's range ends at 2^-126, and eight roundings of
+// 85 leave u within half the guard band.  A 4 x 8 x 8 tile has 22 at four cubic
+// voxels per lattice parameter and 46 at two; 4 x 4 x 8 has 81 at one; voxels of
+// 1.4 x 1.4 x 2.7 sigma have 134 in a 4 x 8 x 8 tile (NaN) and 41 in 4 x 4 x 4.
+static constexpr double TILE_BITS = 85.0;
+
+// The arithmetic that images a condition in `mode`: FP64 where a voxel is so
+// tall (about 5 sigma) that even the smallest FAST tile has more.
+static int condition_mode(const d2bi_plan* p, int mode)
+{
+    return mode == D2BI_MODE_FAST && !(tile_bits(p, TILE, TILE, true) <= TILE_BITS) ? D2BI_MODE_FP64 : mode;
+}
+
 // Launch parameters of the FAST voxel kernel for a plan, tiles of 4 x ty x tz.
 static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParams& V, FastParams* Fo, int tz,
                        int ty = TILE)
@@ -179,12 +205,13 @@ static int launch_voxel_fp64(const d2bi_plan* p, const AxisTables& tab, const Vo
     return D2BI_OK;
 }
 
-// A variant whose tiles span more link cells than the per-tile table holds
-// gives way to the next smaller tile (3 to 2, 2 to 1).
+// A variant whose tiles span more link cells than the per-tile table holds, or
+// whose factors span more than TILE_BITS, gives way to the next smaller tile (3
+// to 2, 2 to 1).
 static int effective_variant(const d2bi_plan* p, const AxisTables& tab, int variant)
 {
-    if (variant == 3 && tile_cells(p, tab, 8, 8) > TILE_MAXC) variant = 2;
-    if (variant == 2 && tile_cells(p, tab, 8) > TILE_MAXC) variant = 1;
+    if (variant == 3 && (tile_cells(p, tab, 8, 8) > TILE_MAXC || tile_bits(p, 8, 8, false) > TILE_BITS)) variant = 2;
+    if (variant == 2 && (tile_cells(p, tab, 8) > TILE_MAXC || tile_bits(p, 8, 4, false) > TILE_BITS)) variant = 1;
     return variant;
 }
 
@@ -695,6 +722,7 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
     if (mode != D2BI_MODE_FP64 && mode != D2BI_MODE_FAST) return seterr(D2BI_ERR_ARG, "unknown mode %d", mode);
     d2bi_plan plan;
     CHK(plan_image(r, n, precAngle, nPrec, &plan));
+    mode = condition_mode(&plan, mode);
     AxisTables tab;
     CHK(axis_tables(r, &plan, &tab));
     BinParams BP;
@@ -857,6 +885,7 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
     if (mode != D2BI_MODE_FP64 && mode != D2BI_MODE_FAST) return seterr(D2BI_ERR_ARG, "unknown mode %d", mode);
     d2bi_plan plan;
     CHK(plan_image(r, n, precAngle, nPrec, &plan));
+    mode = condition_mode(&plan, mode);
     std::vector<double> gshift(3 * (size_t)nApp), aa((size_t)nApp * nPrec);
     CHK(aperture_setup(r, precAngle, nPrec, apAngle, nApp, gshift.data(), aa.data()));
     AxisTables tab;
