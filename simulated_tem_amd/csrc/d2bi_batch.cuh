@@ -442,9 +442,10 @@ static int run_batch(const d2bi_record* recs, const d2bi_atoms* atoms, int nRec,
     std::vector<unsigned char> key;
     key_append(key, &mode, sizeof mode);
     key_append(key, &nRec, sizeof nRec);
-    const int fv = forced_variant(), nb = batch_branches();
-    key_append(key, &fv, sizeof fv);
-    key_append(key, &nb, sizeof nb);
+    // settings that a graph holds as they were when it was captured
+    const int set[] = {forced_variant(), tune_variants() ? 1 : 0, batch_branches(), fast_integrator_poly() ? 1 : 0,
+                       tuning_on() ? 1 : 0, forced_int("D2BI_TILE_ORDER", 0, 2), forced_int("D2BI_INT_BLOCK", 64, 256)};
+    key_append(key, set, sizeof set);
     for (int i = 0; i < nRec; i++) {
         key_append(key, &recs[i], sizeof(d2bi_record));
         // the plan holds each set's point counts: key on the upload, not on

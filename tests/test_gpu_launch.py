@@ -81,3 +81,22 @@ def test_image_copies(mode):
         d = imaging.DeviceBuffer(host.shape)
         im.computeD2BI_img(imaging.Atoms(x), 0.005, 40, mode=mode, out=d)
         assert np.array_equal(host, d.numpy())
+
+
+def test_batch_follows_the_integrator_setting(monkeypatch):
+    """The integrator set when a batch is called is the one that images it, also
+    where a graph of the same batch was captured under the other."""
+    cfg = synth.scaled("c0", cells=(7, 6, 8))
+    cfg.update(sg=[0.01], n_prec=12)
+    x, box = synth.make_atoms(cfg)
+    x, conds = synth.conditions(cfg, x, box)
+    todo = [(conds[0][0], imaging.Atoms(x), 0.005, 12)] * 2
+    alone = {}
+    for how in ("stage", ""):
+        monkeypatch.setenv("D2BI_FAST_INTEGRATOR", how)
+        alone[how] = todo[0][0].computeD2BI_img(todo[0][1], 0.005, 12, mode="fast")
+    assert not np.array_equal(alone["stage"], alone[""])
+    for how in ("", "", "stage", "stage", "stage", "", "stage", "", ""):
+        monkeypatch.setenv("D2BI_FAST_INTEGRATOR", how)
+        for got in imaging.computeD2BI_img_batch(todo, mode="fast"):
+            assert np.array_equal(got, alone[how])
