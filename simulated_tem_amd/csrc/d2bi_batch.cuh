@@ -101,7 +101,7 @@ static int enqueue_count(const Cond& c, int idx, Batch& B, hipStream_t s)
         zero_i32(s, cnt, c.nbc);
     HIPCHK(hipGetLastError());
     return scan_exclusive_tmp(cnt, off, c.nbc, B.scan.as<int>() + c.o_scan, s,
-                              ScanEnds{B.tot.as<int>() + idx, nullptr, nullptr, 0});
+                              ScanEnds{B.tot.as<int>() + idx, nullptr, {}});
 }
 
 // the rest of one condition: bin, voxelise, integrate into its image slice,
@@ -112,7 +112,7 @@ static int enqueue_rest(const Cond& c, int idx, Batch& B, Workspace& w, hipStrea
     Counters* ct = B.counters.as<Counters>() + idx;
     zero_i32(s, w.cell_cnt.as<int>(), c.ncell + 1, (int*)ct, sizeof(Counters) / sizeof(int));
     CHK(launch_bin_points(c.d_x, c.BP, B.mask.as<uint32_t>() + c.o_mask, B.blkoff.as<int>() + c.o_blk, c.nblk, c.ncell,
-                          PointCount{B.tot.as<int>() + idx, c.nr}, w.scan_tmp.as<int>(), &ct->max_per_cell, s, w));
+                          PointCount{B.tot.as<int>() + idx, c.nr}, c.nr, w.scan_tmp.as<int>(), &ct->max_per_cell, s, w));
     VoxParams V;
     d2bi_record dummy;
     dummy.use_density = c.dens ? 1 : 0;

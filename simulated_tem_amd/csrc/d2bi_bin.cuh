@@ -163,15 +163,14 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_classify(const double* __rest
 }
 
 // Pass 2: point number ii in (replica, atom) order, link cell, atom number and
-// a per-cell arrival slot from an atomic counter.  Points past the cap of the
-// arrays are counted but not stored (their cells then come out empty).
+// a per-cell arrival slot from an atomic counter.
 __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restrict__ x, BinParams P,
                                                            const uint32_t* __restrict__ mask,
                                                            const int* __restrict__ blk_off, int nblk,
                                                            int* __restrict__ pt_cell,
                                                            int* __restrict__ pt_slot,
                                                            int* __restrict__ pt_j,
-                                                           int* __restrict__ cell_cnt, int64_t cap)
+                                                           int* __restrict__ cell_cnt, PointCount N)
 {
     __shared__ int first[MAX_REPL];
     __shared__ int wcnt[BIN_BLOCK / 64][MAX_REPL];
@@ -180,6 +179,7 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
     const unsigned long long lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const int64_t j = (int64_t)blockIdx.x * BIN_BLOCK + threadIdx.x;
     const uint32_t m = (j < P.n) ? mask[j] : 0u;
+    if (N.over()) return;
     // the wave's count per replica: zero, then the replicas some lane lies in
     const uint32_t wm0 = wave_or(m);
     if (lane < P.nuvw) wcnt[wave][lane] = 0;
@@ -207,11 +207,8 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
         const int cy = P.generic ? cell_of(fl[1], P.Ey) : (int)fl[1];
         const int cz = P.generic ? cell_of(fl[2], P.Ez) : (int)fl[2];
         const int cell = cx + P.Ex * (cy + P.Ey * cz);
-        const bool held = (int64_t)(unsigned)ii < cap;
-        if (held) {
-            pt_cell[ii] = cell;
-            pt_j[ii] = (int)j;
-        }
+        pt_cell[ii] = cell;
+        pt_j[ii] = (int)j;
         // arrival slot: lanes of this wave landing in one cell share
         // one atomic (the lowest such lane adds the group's size);
         // the grouping is ALU-only, so each lane waits for one atomic
@@ -228,42 +225,34 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
         int base = 0;
         if (lane == leader) base = atomicAdd(&cell_cnt[cell], (int)__popcll(grp));
         base = __shfl(base, leader, 64);
-        if (held) pt_slot[ii] = base + (int)__popcll(grp & lt);
+        pt_slot[ii] = base + (int)__popcll(grp & lt);
     }
 }
 
-// Item of a thread among n (-1: none), workgroups of 256: a contiguous range of
-// items per XCD (workgroups go round-robin to the eight), so that neighbours in
-// cell or atom order, which share lines of the arrays they gather from and
-// scatter into, share one L2.  Needs a grid of at least xcd_grid(n).  Against
+// f(t) for the items t of a thread among n, workgroups of 256 in a grid of
+// xcd_grid() (of n items or fewer; a thread goes on a grid's stride from its
+// first): a contiguous range of items per XCD (workgroups go round-robin to the
+// eight), so that neighbours in cell or atom order, which share lines of the
+// arrays they gather from and scatter into, share one L2.  Against
 // workgroups in order: k_bin_emit 39.5 -> 26.7 us and k_bin_place 9.6 -> 6.8 at
 // 1.2e6 atoms, 222 -> 211 and 54 -> 44 at 8e6 (k_bin_scatter, whose atomics
 // meet in memory either way, lost 7 % there and keeps its order).
-__device__ __forceinline__ int64_t xcd_item(int64_t n)
+template <class F>
+__device__ __forceinline__ void xcd_items(int64_t n, F f)
 {
-    const int64_t per = (n + 2047) / 2048, b = blockIdx.x >> 3;
-    const int64_t t = ((blockIdx.x & 7) * per + b) * 256 + threadIdx.x;
-    return b < per && t < n ? t : -1;
+    const int64_t per = (n + 2047) / 2048;
+    for (int64_t b = blockIdx.x >> 3; b < per; b += gridDim.x >> 3) {
+        const int64_t t = ((blockIdx.x & 7) * per + b) * 256 + threadIdx.x;
+        if (t < n) f(t);
+    }
 }
 static unsigned xcd_grid(int64_t n) { return (unsigned)(8 * ((n + 2047) / 2048)); }
-
-// The number of points, which only the device knows when the passes after
-// the count are launched, and what the point arrays hold; a condition with
-// more points than that stores none and is binned again.
-struct PointCount {
-    const int* n;
-    int64_t cap;
-    // (a count that overflowed is negative)
-    __device__ int64_t stored() const { return (int64_t)(unsigned)*n > cap ? 0 : *n; }
-};
 
 // Pass 3: place each point at its cell's start + arrival slot.
 __global__ void k_bin_place(PointCount N, const int* __restrict__ pt_cell, const int* __restrict__ pt_slot,
                             const int* __restrict__ cell_start, int* __restrict__ cell_ids)
 {
-    const int64_t ii = xcd_item(N.stored());
-    if (ii < 0) return;
-    cell_ids[cell_start[pt_cell[ii]] + pt_slot[ii]] = (int)ii;
+    xcd_items(N.stored(), [&](int64_t ii) { cell_ids[cell_start[pt_cell[ii]] + pt_slot[ii]] = (int)ii; });
 }
 
 // What pass 4 writes per slot (null: not wanted).
@@ -297,39 +286,39 @@ __global__ __launch_bounds__(256) void k_bin_emit(PointCount N, const int* __res
     if (threadIdx.x < MAX_REPL)
         rep_first[threadIdx.x] = threadIdx.x < P.nuvw ? blk_off[(int64_t)threadIdx.x * nblk] : 0x7fffffff;
     __syncthreads();
-    const int64_t t = xcd_item(N.stored());
-    if (t < 0) return;
-    const int ii = cell_ids[t];
-    const int64_t j = pt_j[ii];
-    const int c = pt_cell[ii];
-    const int s0 = cell_start[c], s1 = cell_start[c + 1];
-    int nn = 0;                                       // rep_first[0] = 0 <= ii
+    xcd_items(N.stored(), [&](int64_t t) {
+        const int ii = cell_ids[t];
+        const int64_t j = pt_j[ii];
+        const int c = pt_cell[ii];
+        const int s0 = cell_start[c], s1 = cell_start[c + 1];
+        int nn = 0;                                       // rep_first[0] = 0 <= ii
 #pragma unroll
-    for (int step = MAX_REPL / 2; step > 0; step >>= 1)
-        if (rep_first[nn + step] <= ii) nn += step;
-    const double x3[3] = {x[3 * j], x[3 * j + 1], x[3 * j + 2]};
-    int64_t s = s0;
-    for (int k = s0; k < s1; k++) s += cell_ids[k] < ii ? 1 : 0;
-    double yy[3], cyy[3];
-    bin_point(P, x3, nn, yy, cyy);
-    const Frac3 f{cyy[0] - floor(cyy[0]), cyy[1] - floor(cyy[1]), cyy[2] - floor(cyy[2])};
-    const double gd = (P.gg[0] * yy[0] + P.gg[1] * yy[1]) + P.gg[2] * yy[2];
-    O.frac[s] = f;
-    float4 p = make_float4((float)(P.cell_a[0] * f.x), (float)(P.cell_a[1] * f.y), (float)(P.cell_a[2] * f.z), 0.0f);
-    if (FAST) {
-        double sn, cs;
-        sincos(gd, &sn, &cs);
-        p.w = (float)cs;
-        O.sn32[s] = (float)sn;
-    } else if (O.cs64) {
-        double sn, cs;
-        sincos(gd, &sn, &cs);
-        O.cs64[s] = make_double2(cs, sn);
-    }
-    O.p32[s] = p;
-    if (O.src) O.src[s] = make_int2((int)j, nn);
-    if (O.id) O.id[s] = ii + 1;
-    if (O.gdotr) O.gdotr[ii] = gd;
+        for (int step = MAX_REPL / 2; step > 0; step >>= 1)
+            if (rep_first[nn + step] <= ii) nn += step;
+        const double x3[3] = {x[3 * j], x[3 * j + 1], x[3 * j + 2]};
+        int64_t s = s0;
+        for (int k = s0; k < s1; k++) s += cell_ids[k] < ii ? 1 : 0;
+        double yy[3], cyy[3];
+        bin_point(P, x3, nn, yy, cyy);
+        const Frac3 f{cyy[0] - floor(cyy[0]), cyy[1] - floor(cyy[1]), cyy[2] - floor(cyy[2])};
+        const double gd = (P.gg[0] * yy[0] + P.gg[1] * yy[1]) + P.gg[2] * yy[2];
+        O.frac[s] = f;
+        float4 p = make_float4((float)(P.cell_a[0] * f.x), (float)(P.cell_a[1] * f.y), (float)(P.cell_a[2] * f.z), 0.0f);
+        if (FAST) {
+            double sn, cs;
+            sincos(gd, &sn, &cs);
+            p.w = (float)cs;
+            O.sn32[s] = (float)sn;
+        } else if (O.cs64) {
+            double sn, cs;
+            sincos(gd, &sn, &cs);
+            O.cs64[s] = make_double2(cs, sn);
+        }
+        O.p32[s] = p;
+        if (O.src) O.src[s] = make_int2((int)j, nn);
+        if (O.id) O.id[s] = ii + 1;
+        if (O.gdotr) O.gdotr[ii] = gd;
+    });
 }
 
 // g-vectors of up to four aperture points (findGdotR_aperture,
@@ -351,51 +340,51 @@ __global__ __launch_bounds__(256) void k_app_phase(int64_t nr, const int2* __res
                                                    double2* __restrict__ out64, float2* __restrict__ out32,
                                                    float4* __restrict__ slot_p32, float* __restrict__ slot_sn32)
 {
-    const int64_t s = xcd_item(nr);
-    if (s < 0) return;
-    const int2 src = slot_src[s];
-    const int64_t j = src.x;
-    const double x3[3] = {x[3 * j], x[3 * j + 1], x[3 * j + 2]};
-    double yy[3], cyy[3];
-    bin_point(P, x3, src.y, yy, cyy);
+    xcd_items(nr, [&](int64_t s) {
+        const int2 src = slot_src[s];
+        const int64_t j = src.x;
+        const double x3[3] = {x[3 * j], x[3 * j + 1], x[3 * j + 2]};
+        double yy[3], cyy[3];
+        bin_point(P, x3, src.y, yy, cyy);
 #pragma unroll
-    for (int a = 0; a < NA; a++) {
-        const double gd = (G.g[a][0] * yy[0] + G.g[a][1] * yy[1]) + G.g[a][2] * yy[2];
-        double sn, cs;
-        sincos(gd, &sn, &cs);
-        if (F64) {
-            out64[a * stride + s] = make_double2(cs, sn);
-        } else if (NA == 1) {
-            reinterpret_cast<float*>(slot_p32 + s)[3] = (float)cs;
-            slot_sn32[s] = (float)sn;
-        } else {
-            out32[a * stride + s] = make_float2((float)cs, (float)sn);
+        for (int a = 0; a < NA; a++) {
+            const double gd = (G.g[a][0] * yy[0] + G.g[a][1] * yy[1]) + G.g[a][2] * yy[2];
+            double sn, cs;
+            sincos(gd, &sn, &cs);
+            if (F64) {
+                out64[a * stride + s] = make_double2(cs, sn);
+            } else if (NA == 1) {
+                reinterpret_cast<float*>(slot_p32 + s)[3] = (float)cs;
+                slot_sn32[s] = (float)sn;
+            } else {
+                out32[a * stride + s] = make_float2((float)cs, (float)sn);
+            }
         }
-    }
+    });
 }
 
 struct Binned {
     int64_t nr = -1;            // points; -1: not known on the host yet
-    int64_t cap = 0;            // what the point arrays hold
+    PointCount N{};             // on the device, and what the point arrays hold
     int ncell = 0;
 };
 
 // Passes 2 to 4 on workspace w, once the points are counted on the device (*N.n
-// of them): d_x, mask, blk_off and nblk are the condition's atoms, replica
-// predicates and per-(replica, block) point offsets; w.cell_cnt is zero.  The
-// largest cell count goes to *mpc.
+// of them, about `expect`): d_x, mask, blk_off and nblk are the condition's atoms,
+// replica predicates and per-(replica, block) point offsets; w.cell_cnt is zero.
+// The largest cell count goes to *mpc.
 static int launch_bin_points(const double* d_x, const BinParams& P, const uint32_t* mask, const int* blk_off, int nblk,
-                             int ncell, PointCount N, int* scan_tmp, int* mpc, hipStream_t s, Workspace& w)
+                             int ncell, PointCount N, int64_t expect, int* scan_tmp, int* mpc, hipStream_t s, Workspace& w)
 {
     if (P.n > 0 && N.cap > 0) {
         hipLaunchKernelGGL(k_bin_scatter, dim3(nblk), dim3(BIN_BLOCK), 0, s, d_x, P, mask, blk_off, nblk,
-                           w.pt_cell.as<int>(), w.pt_slot.as<int>(), w.pt_j.as<int>(), w.cell_cnt.as<int>(), N.cap);
+                           w.pt_cell.as<int>(), w.pt_slot.as<int>(), w.pt_j.as<int>(), w.cell_cnt.as<int>(), N);
         HIPCHK(hipGetLastError());
     }
     CHK(scan_exclusive_tmp(w.cell_cnt.as<int>(), w.cell_start.as<int>(), ncell, scan_tmp, s,
-                           ScanEnds{nullptr, mpc, N.n, N.cap}));
+                           ScanEnds{nullptr, mpc, N}));
     if (P.n > 0 && N.cap > 0) {
-        const dim3 grid(xcd_grid(N.cap));
+        const dim3 grid(xcd_grid(std::min(N.cap, expect)));
         hipLaunchKernelGGL(k_bin_place, grid, dim3(256), 0, s, N, w.pt_cell.as<int>(), w.pt_slot.as<int>(),
                            w.cell_start.as<int>(), w.cell_ids.as<int>());
         EmitOut O{w.slot_p32.as<float4>(), w.slot_sn32.as<float>(), nullptr, w.slot_frac.as<Frac3>(),
@@ -453,9 +442,10 @@ static int64_t expected_points(const d2bi_record* r, const d2bi_plan* p, int64_t
 // Run binning for either a condition (generic = 0) or plain points, on
 // workspace w.  expect > 0: the point arrays are sized for that many points
 // (or what they hold) and nothing waits for the count, which stays in the
-// workspace's counters; the caller compares it with out->cap at its own end
-// and bins again with expect = 0 if they did not fit.  expect = 0: the host
-// waits for the count and sizes the arrays by it.
+// workspace's counters; the caller compares it with out->N.cap at its own end
+// and bins again with expect = 0 if they did not fit (the kernels after the
+// count have then done nothing).  expect = 0: the host waits for the count and
+// sizes the arrays by it.
 static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, hipStream_t s, Workspace& w,
                        int64_t expect = 0)
 {
@@ -482,7 +472,7 @@ static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, 
         zero_i32(s, Z.p[0], Z.n[0], Z.p[1], Z.n[1], w.blk_cnt.as<int>(), nbc);
     HIPCHK(hipGetLastError());
     CHK(scan_exclusive_tmp(w.blk_cnt.as<int>(), w.blk_off.as<int>(), nbc, w.scan_tmp.as<int>(), s,
-                           ScanEnds{&ct->n_points, nullptr, nullptr, 0}));
+                           ScanEnds{&ct->n_points, nullptr, {}}));
     int64_t cap = expect;
     if (expect <= 0) {
         int nr_host = 0;
@@ -498,12 +488,9 @@ static int run_binning(const double* d_x, int64_t n, BinParams& P, Binned* out, 
         held = std::min(held, (int64_t)(b.cap / bytes));
     });
     CHK(rc);
-    // (twice the estimate at most: the passes over the points launch a thread
-    // for each that may be stored)
-    if (expect > 0) cap = std::min(held, 2 * expect);
-    CHK(launch_bin_points(d_x, P, w.mask.as<uint32_t>(), w.blk_off.as<int>(), nblk, ncell, PointCount{&ct->n_points, cap},
+    out->N = PointCount{&ct->n_points, expect > 0 ? held : cap};
+    CHK(launch_bin_points(d_x, P, w.mask.as<uint32_t>(), w.blk_off.as<int>(), nblk, ncell, out->N, cap,
                           w.scan_tmp.as<int>(), &ct->max_per_cell, s, w));
-    out->cap = cap;
     out->ncell = ncell;
     return D2BI_OK;
 }

@@ -325,15 +325,24 @@ __device__ inline int block_max(int v, int* lds)
     return v;
 }
 
+// The number of points, which only the device knows when the passes after the
+// count are launched, and what the point arrays hold.  A condition with more
+// points than that is imaged again: the kernels after the count return at once,
+// and the link cells come out empty, so that nothing reads past the arrays.
+struct PointCount {
+    const int* n = nullptr;     // null: no such limit
+    int64_t cap = 0;
+    // (a count that overflowed is negative)
+    __device__ bool over() const { return n && (int64_t)(unsigned)*n > cap; }
+    __device__ int64_t stored() const { return over() ? 0 : *n; }
+};
+
 // What a scan hands on besides the array: its total and largest value (null:
-// not wanted); and the scan of the cell counts of more points than the point
-// arrays hold is that of empty cells, so that nothing reads past them.
+// not wanted); N: the scan of the cell counts is that of empty cells if over.
 struct ScanEnds {
     int* total_out;
     int* max_out;
-    const int* points;          // null, or the number of points ...
-    int64_t cap;                // ... and what the point arrays hold
-    __device__ bool over() const { return points && (int64_t)(unsigned)*points > cap; }
+    PointCount N;
 };
 
 // Short arrays (a small condition's block counts or link cells) in one
@@ -348,7 +357,7 @@ __global__ __launch_bounds__(SCAN_ONE_BLOCK) void k_scan_one(const int* __restri
 {
     __shared__ int lds[SCAN_ONE_BLOCK / 64 + 1];
     const int per = (n + SCAN_ONE_BLOCK - 1) / SCAN_ONE_BLOCK, base = (int)threadIdx.x * per;
-    const int end = E.over() ? 0 : n;
+    const int end = E.N.over() ? 0 : n;
     int v[SCAN_ONE_ITEMS], s = 0, m = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ONE_ITEMS; i++) v[i] = i < per && base + i < end ? in[base + i] : 0;
@@ -384,7 +393,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_reduce(const int* __restric
                                                             ScanEnds E)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
-    if (E.over()) n = 0;
+    if (E.N.over()) n = 0;
     int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
     int s = 0, m = 0;
 #pragma unroll
@@ -423,7 +432,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_apply(const int* __restrict
                                                            ScanEnds E)
 {
     __shared__ int lds[SCAN_BLOCK / 64 + 1];
-    const bool over = E.over();
+    const bool over = E.N.over();
     int before = 0;
     if (scanned) {
         before = sums[blockIdx.x];

@@ -18,6 +18,7 @@ static constexpr int INT_POINTS = 32, INT_SLOTS = INT_POINTS + 31;
 struct FastIntParams {
     int Mx, My, Mz, np;         // np: precession points per field
     int nsplit, split;          // waves per column, of them per field
+    PointCount N;               // a field of no condition if over
     float b0, bg, dz;
     int64_t stride;             // records from one field to the next
     float aa[INT_SLOTS];        // 2 pi s_g per field and precession point
@@ -99,7 +100,7 @@ __device__ __forceinline__ void rescale(double* p0r, double* p0i, double* pgr, d
 // over 800 double steps leaving c0 out moves |phi_g|^2 by ~2e-4.
 template <int NP, bool RS = false, class T, class S>
 __device__ __forceinline__ void march_stage(const S& s, int nz, T dz, const T* aa, T* p0r, T* p0i, T* pgr, T* pgi,
-                                            int every = 0)
+                                            bool go, int every = 0)
 {
     [[maybe_unused]] int left = every;
     const T dz3 = dz / 3, dz23 = 2 * dz / 3, dz2 = 2 * dz;
@@ -121,7 +122,7 @@ __device__ __forceinline__ void march_stage(const S& s, int nz, T dz, const T* a
         for (int k = 0; k < 2 * PD; k++)
             if (k + 1 <= nz) ring[k] = s.load(k + 1);
     }
-    for (int i0 = 0; i0 <= nz - 2; i0 += 2 * PD) {
+    for (int i0 = 0; go && i0 <= nz - 2; i0 += 2 * PD) {
 #pragma unroll
     for (int u = 0; u < PD; u++) {
         const int ii = i0 + 2 * u;
@@ -311,11 +312,11 @@ __device__ __forceinline__ cplx<T> horner(const CPoly<D, T>& M, T al)
 }
 
 // The column's march: NP points from (1, 0) through nz samples (sample nz is
-// sample 0); S gives a sample's coefficients (load(k) what is read, coef(raw)
+// sample 0), or none if not go; S gives a sample's coefficients (load(k) what is read, coef(raw)
 // c0 and cg).
 template <int NP, bool RS = false, class T, class S>
 __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al_, T* p0r, T* p0i, T* pgr, T* pgi,
-                                           int every = 0)
+                                           bool go, int every = 0)
 {
     [[maybe_unused]] int left = every;
     const T dz2 = 2 * dz, dz6 = dz / 3, third = T(1) / 3, two3 = T(2) / 3, sixth = T(1) / 6, half = T(0.5), one = T(1);
@@ -334,7 +335,7 @@ __device__ __forceinline__ void march_poly(const S& s, int nz, T dz, const T* al
         fb = s.load(1);
         fc = s.load(2);
     }
-    for (int ii = 0; ii <= nz - 2; ii += 2) {
+    for (int ii = 0; go && ii <= nz - 2; ii += 2) {
         T c0b, cgrb, cgib, c0c, cgrc, cgic;
         s.coef(fb, c0b, cgrb, cgib);
         s.coef(fc, c0c, cgrc, cgic);
@@ -419,6 +420,7 @@ __global__ __launch_bounds__(SPLIT ? int_threads(NP) : 256) void k_integrate_fas
                                                                                 double* __restrict__ img,
                                                                                 int accumulate, double inv_total)
 {
+    const bool go = !P.N.over();                     // (looked at once the first samples are on their way)
     const int64_t plane = (int64_t)P.Mx * P.My;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int ns = SPLIT ? P.nsplit : 1, cg = SPLIT ? wave / ns : wave, sp = SPLIT ? wave - cg * ns : 0;
@@ -429,8 +431,8 @@ __global__ __launch_bounds__(SPLIT ? int_threads(NP) : 256) void k_integrate_fas
     const int fld = SPLIT ? sp / P.split : 0, p0 = SPLIT ? (sp - fld * P.split) * NP : 0, at = fld * P.np + p0;
     const FastColumn<DENS, !SPLIT && !POLY> s{field, (live ? col : plane - 1) + fld * P.stride, plane, P.Mz, P.b0, P.bg};
     float p0r[NP], p0i[NP], pgr[NP], pgi[NP];
-    if constexpr (POLY) march_poly<NP>(s, P.Mz, P.dz, P.al + at, p0r, p0i, pgr, pgi);
-    else march_stage<NP>(s, P.Mz, P.dz, P.aa + at, p0r, p0i, pgr, pgi);
+    if constexpr (POLY) march_poly<NP>(s, P.Mz, P.dz, P.al + at, p0r, p0i, pgr, pgi, go);
+    else march_stage<NP>(s, P.Mz, P.dz, P.aa + at, p0r, p0i, pgr, pgi, go);
     double acc = intensity_sum<NP>(min(NP, P.np - p0), p0r, p0i, pgr, pgi) * inv_total;
     if constexpr (SPLIT) {
         __shared__ double part[int_threads(NP)];
@@ -452,6 +454,7 @@ __global__ __launch_bounds__(SPLIT ? int_threads(NP) : 256) void k_integrate_fas
 struct IntParams {
     int Mx, My, Mz, np;         // np: precession points in this launch
     int nsplit;                 // waves per column
+    PointCount N;               // a field of no condition if over
     double b0, bg, dz;
     double aa[INT_SLOTS];       // 2 pi s_g per precession point
     double al[INT_SLOTS];       // 2 dz aa
@@ -509,6 +512,7 @@ __global__ __launch_bounds__(SPLIT ? int_threads64(NP) : 256) void k_integrate_f
                                                                                   const double* __restrict__ frho,
                                                                                   double* __restrict__ img)
 {
+    const bool go = !P.N.over();                     // (looked at once the first samples are on their way)
     const int64_t plane = (int64_t)P.Mx * P.My;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int ns = SPLIT ? P.nsplit : 1, cg = SPLIT ? wave / ns : wave, sp = SPLIT ? wave - cg * ns : 0;
@@ -519,8 +523,8 @@ __global__ __launch_bounds__(SPLIT ? int_threads64(NP) : 256) void k_integrate_f
     const Fp64Column<DENS> s{fre, fim, frho, live ? col : plane - 1, plane, P.Mz, P.b0, P.bg};
     const int p0 = sp * NP;
     double p0r[NP], p0i[NP], pgr[NP], pgi[NP];
-    if constexpr (NP >= 6) march_poly<NP, RS>(s, P.Mz, P.dz, P.al + p0, p0r, p0i, pgr, pgi, P.every);
-    else march_stage<NP, RS>(s, P.Mz, P.dz, P.aa + p0, p0r, p0i, pgr, pgi, P.every);
+    if constexpr (NP >= 6) march_poly<NP, RS>(s, P.Mz, P.dz, P.al + p0, p0r, p0i, pgr, pgi, go, P.every);
+    else march_stage<NP, RS>(s, P.Mz, P.dz, P.aa + p0, p0r, p0i, pgr, pgi, go, P.every);
     double acc = intensity_sum<NP>(min(NP, P.np - p0), p0r, p0i, pgr, pgi);
     if constexpr (SPLIT) {
         __shared__ double part[int_threads64(NP)];

@@ -590,7 +590,7 @@ static void launch_int_pass(FastIntParams P, int nf, bool dens, const void* f, d
 // with nPrec deviations each in aa (fields_fit), one launch for all.
 static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, double* d_img, hipStream_t s,
                                  bool acc_in = false, double inv = 0.0, Workspace* tune_ws = nullptr, int nf = 1,
-                                 int64_t stride = 0, const double* aa = nullptr)
+                                 int64_t stride = 0, const double* aa = nullptr, PointCount N = {})
 {
     if (!aa) aa = p->aa;
     if (inv == 0.0) inv = 1.0 / p->nPrec;
@@ -600,6 +600,7 @@ static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, d
         P.Mx = p->Mx; P.My = p->My; P.Mz = p->Mz; P.np = np;
         P.b0 = (float)p->b0; P.bg = (float)p->bg; P.dz = (float)p->dz;
         P.stride = stride;
+        P.N = N;
         for (int i = 0; i < INT_SLOTS; i++) {
             P.aa[i] = i < nf * np ? (float)aa[p0 + i] : 0.0f;
             P.al[i] = i < nf * np ? (float)(2.0 * p->dz * aa[p0 + i]) : 0.0f;
@@ -646,7 +647,7 @@ static int rescale_every(const d2bi_plan* p)
 // write sum / nPrec (div = 0) or sum / div.  The field is read from workspace
 // w, field_off voxels on.
 static int launch_integrate_fp64(const d2bi_plan* p, bool dens, double* d_img, hipStream_t s, Workspace& w,
-                                 int accumulate = 0, double div = 0.0, int64_t field_off = 0)
+                                 int accumulate = 0, double div = 0.0, int64_t field_off = 0, PointCount N = {})
 {
     const int64_t plane = (int64_t)p->Mx * p->My;
     const int every = rescale_every(p);
@@ -657,6 +658,7 @@ static int launch_integrate_fp64(const d2bi_plan* p, bool dens, double* d_img, h
         P.Mx = p->Mx; P.My = p->My; P.Mz = p->Mz; P.np = np;
         P.nsplit = sp.ns;
         P.every = every;
+        P.N = N;
         P.b0 = p->b0; P.bg = p->bg; P.dz = p->dz;
         for (int i = 0; i < INT_SLOTS; i++) {
             P.aa[i] = i < np ? p->aa[p0 + i] : 0.0;
@@ -700,10 +702,11 @@ static int launch_integrate_fp64(const d2bi_plan* p, bool dens, double* d_img, h
 }
 
 // Integrate the field of workspace w into d_img (Mx*My doubles).
-static int run_integrate(const d2bi_plan* p, bool dens, int mode, hipStream_t s, Workspace& w, double* d_img)
+static int run_integrate(const d2bi_plan* p, bool dens, int mode, PointCount N, hipStream_t s, Workspace& w,
+                         double* d_img)
 {
-    if (mode == D2BI_MODE_FP64) return launch_integrate_fp64(p, dens, d_img, s, w);
-    return launch_integrate_fast(p, dens, w.f32_field.p, d_img, s, false, 0.0, &w);
+    if (mode == D2BI_MODE_FP64) return launch_integrate_fp64(p, dens, d_img, s, w, 0, 0.0, 0, N);
+    return launch_integrate_fast(p, dens, w.f32_field.p, d_img, s, false, 0.0, &w, 1, 0, nullptr, N);
 }
 
 // Whole condition: bin -> voxelise -> integrate on workspace w, the image
@@ -761,7 +764,7 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
         CHK(T.record(1));
         CHK(run_voxel(r, &plan, tab, ax, mode, false, true, s, w));
         CHK(T.record(2));
-        CHK(run_integrate(&plan, dens, mode, s, w, d_img));
+        CHK(run_integrate(&plan, dens, mode, b.N, s, w, d_img));
         CHK(T.record(3));
         HIPCHK(hipMemcpyAsync(ct, w.counters.p, sizeof(Counters) + (joint ? sizeof(double) * plane : 0),
                               hipMemcpyDeviceToHost, s));
@@ -770,6 +773,7 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
         return D2BI_OK;
     };
     const int v = known_variant(&plan, dens);
+    double lost = 0.0;                                  // device time of a pass that did not fit
     bool exact = w.counters.arena || n == 0;
     if (mode == D2BI_MODE_FAST && (v < 0 || !condition_tuned(&plan, tab, dens, v))) exact = true;
     if (!exact) {
@@ -779,8 +783,9 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
             (void)hipGetLastError();
             HIPCHK(hipStreamSynchronize(s));
             exact = true;
-        } else if (ct->n_points < 0 || ct->n_points > b.cap) {
+        } else if (ct->n_points < 0 || ct->n_points > b.N.cap) {
             exact = true;
+            lost = T.ms(0, 3);
         }
     }
     if (exact) CHK(enqueue(0));
@@ -794,7 +799,7 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
         st->ms_bin += T.ms(0, 1);
         st->ms_voxel += T.ms(1, 2);
         st->ms_integrate += T.ms(2, 3);
-        st->ms_total += T.ms(0, 3);
+        st->ms_total += lost + T.ms(0, 3);
     }
     if (plan_out) *plan_out = plan;
     return D2BI_OK;
