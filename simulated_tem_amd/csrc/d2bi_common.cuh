@@ -38,6 +38,15 @@ int seterr(int code, const char* fmt, ...)
 // ------------------------------------------------------------------ device buffers
 
 static uint64_t g_alloc_gen = 0;         // bumped on every device reallocation
+static size_t g_alloc_bytes = 0;         // device bytes in buffers
+
+// hipMalloc of a buffer, within D2BI_MEM_LIMIT bytes for all of them (tests).
+static hipError_t alloc_device(void** p, size_t bytes)
+{
+    const char* e = std::getenv("D2BI_MEM_LIMIT");
+    if (e && *e && g_alloc_bytes + bytes > (size_t)std::strtoull(e, nullptr, 10)) return hipErrorOutOfMemory;
+    return hipMalloc(p, bytes);
+}
 
 // A fixed block of device memory handed out front to back (256-byte
 // aligned pieces); buffers bound to an arena never call the allocator.
@@ -66,19 +75,24 @@ struct Buf {
             return D2BI_OK;
         }
         g_alloc_gen++;
-        if (p) { (void)hipFree(p); p = nullptr; cap = 0; }
+        release();
         const size_t want = alloc_size(bytes);       // headroom for slightly larger conditions
-        hipError_t e = hipMalloc(&p, want);
+        hipError_t e = alloc_device(&p, want);
         if (e != hipSuccess) {
             p = nullptr;
-            return seterr(D2BI_ERR_HIP, "hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+            return seterr(D2BI_ERR_HIP, "hipMalloc(%zu) failed: %s (%zu bytes held)", want, hipGetErrorString(e),
+                          g_alloc_bytes);
         }
         cap = want;
+        g_alloc_bytes += cap;
         return D2BI_OK;
     }
     void release()
     {
-        if (p && !arena) (void)hipFree(p);
+        if (p && !arena) {
+            (void)hipFree(p);
+            g_alloc_bytes -= cap;
+        }
         p = nullptr;
         cap = 0;
     }

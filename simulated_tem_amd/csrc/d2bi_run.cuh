@@ -779,9 +779,14 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
     if (!exact) {
         const int rc = enqueue(expected_points(r, &plan, n));
         if (rc != D2BI_OK) {
-            // memory for the estimate, or a failure the exact pass reports again
+            // memory for the estimate, or a failure the exact pass reports again;
+            // arrays of the estimate would take the exact pass's room
             (void)hipGetLastError();
             HIPCHK(hipStreamSynchronize(s));
+            if (rc == D2BI_ERR_HIP) {
+                g_alloc_gen++;
+                point_buffers(w, BP.fast, false, false, false, [](Buf& q, size_t) { q.release(); });
+            }
             exact = true;
         } else if (ct->n_points < 0 || ct->n_points > b.N.cap) {
             exact = true;

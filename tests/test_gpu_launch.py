@@ -8,6 +8,8 @@ the second: every call gives the same images, and so do batches that take
 turns (each is new again after the other).
 """
 import os
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -19,6 +21,7 @@ from simulated_tem_amd import abi, imaging, synth
 pytestmark = pytest.mark.gpu
 
 NTH = min(16, os.cpu_count() or 1)
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def cluster():
@@ -133,3 +136,50 @@ def test_more_points_than_expected_once():
         assert st.ms_total <= 1.5 * stages
         took.append(wall / stages)
     assert min(took[1:]) <= 1.5
+
+
+_NO_ROOM = r"""
+import os, re, sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+from simulated_tem_amd import abi, imaging, synth
+cfg = synth.scaled("c0", cells=(20, 20, 20))
+cfg.update(sg=[0.01])
+x, box = synth.make_atoms(cfg)
+x, conds = synth.conditions(cfg, x, box)
+im, at = conds[0][0], imaging.Atoms(x)
+small = np.ones((300, 300))
+first = im.computeD2BI_img(at, 0.005, 1, mode="fast")       # not timed yet: sized by the exact count
+os.environ["D2BI_MEM_LIMIT"] = "1"
+try:
+    imaging.gaussianBlurImage(small, 2.0)
+    raise SystemExit("no failure")
+except abi.D2biError as e:
+    held = int(re.search(r"(\d+) bytes held", str(e)).group(1))
+print("[no room] %d bytes held" % held, flush=True)
+imaging.finalize()
+at = imaging.Atoms(x)
+os.environ["D2BI_MEM_LIMIT"] = str(held)
+for _ in range(2):
+    assert np.array_equal(im.computeD2BI_img(at, 0.005, 1, mode="fast"), first)
+os.environ["D2BI_MEM_LIMIT"] = str(held // 2)
+imaging.finalize()
+at = imaging.Atoms(x)
+try:
+    im.computeD2BI_img(at, 0.005, 1, mode="fast")
+    raise SystemExit("no failure")
+except abi.D2biError as e:
+    print("[no room] refused: %s" % e, flush=True)
+os.environ["D2BI_MEM_LIMIT"] = ""
+assert np.array_equal(im.computeD2BI_img(at, 0.005, 1, mode="fast"), first)
+"""
+
+
+def test_no_room_for_the_estimate():
+    """A condition that fits the device with arrays for its exact point count is
+    imaged there, also where those of the estimate do not leave room."""
+    env = {k: v for k, v in os.environ.items() if not k.startswith("D2BI_")}
+    r = subprocess.run([sys.executable, "-c", _NO_ROOM, ROOT], env=env, cwd=ROOT, capture_output=True, text=True,
+                       timeout=100)
+    print(r.stdout, flush=True)
+    assert r.returncode == 0, r.stdout + r.stderr
