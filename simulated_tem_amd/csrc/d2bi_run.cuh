@@ -543,12 +543,11 @@ static bool fields_fit(int64_t plane, int np, int nf, bool dens)
 
 // One FAST integration launch, workgroups of about `block` threads (any size
 // gives the same image).
-static void launch_int_pass(FastIntParams P, int nf, bool dens, const void* f, double* img, int acc, double inv,
-                            int block, hipStream_t s)
+static void launch_int_pass(FastIntParams P, const IntSplit& sp, int nf, bool dens, const void* f, double* img,
+                            int acc, double inv, int block, hipStream_t s)
 {
     const int64_t plane = (int64_t)P.Mx * P.My;
     const bool poly = P.np >= 8 && fast_integrator_poly();
-    const IntSplit sp = int_split(plane, P.np, dens);
     P.split = sp.ns;
     P.nsplit = nf * sp.ns;
     // `block` sizes the workgroups of unsplit columns
@@ -607,17 +606,23 @@ static int launch_integrate_fast(const d2bi_plan* p, bool dens, const void* f, d
         }
         // workgroup size: timed on a launch that writes (not adds to) an
         // image, the output itself for the first pass, else a tuning buffer
-        double* timg = first ? d_img : nullptr;
+        // (split columns size their own: nothing to time, and 256 stands for it
+        // in the key, which several fields share with one of their shape)
         const TuneKey key = int_block_key(p, np, dens);
-        if (!timg && tune_ws && !tune_ws->tune_img.arena && !g_capturing && tuning_on() && tune_get(key) < 0) {
+        const IntSplit sp = int_split((int64_t)P.Mx * P.My, np, dens);
+        const bool split = nf > 1 || sp.ns > 1;
+        if (split && nf == 1 && tuning_on() && forced_int("D2BI_INT_BLOCK", 64, 256) < 0 && tune_get(key) < 0)
+            tune_put(key, 256);
+        double* timg = first && !split ? d_img : nullptr;
+        if (!timg && !split && tune_ws && !tune_ws->tune_img.arena && !g_capturing && tuning_on() && tune_get(key) < 0) {
             CHK(tune_ws->tune_img.ensure(sizeof(double) * (int64_t)P.Mx * P.My));
             timg = tune_ws->tune_img.as<double>();
         }
         static const int cand[3] = {64, 128, 256};
-        const int block = tune_choose(key, "D2BI_INT_BLOCK", cand, 3, 256, timg != nullptr, s, [&](int b) {
-            launch_int_pass(P, nf, dens, f, timg, 0, inv, b, s);
+        const int block = split ? 256 : tune_choose(key, "D2BI_INT_BLOCK", cand, 3, 256, timg != nullptr, s, [&](int b) {
+            launch_int_pass(P, sp, nf, dens, f, timg, 0, inv, b, s);
         });
-        launch_int_pass(P, nf, dens, f, d_img, !first, inv, block, s);
+        launch_int_pass(P, sp, nf, dens, f, d_img, !first, inv, block, s);
         HIPCHK(hipGetLastError());
         p0 += np;
     }

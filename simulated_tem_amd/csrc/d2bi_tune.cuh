@@ -8,7 +8,9 @@
 // Tuned choices (each leaves every image bit-identical, because no thread's
 // arithmetic or summation order depends on it):
 //   TUNE_INT_BLOCK   threads per workgroup of the FAST integrators (64, 128
-//                    or 256): a lane integrates one pixel column on its own
+//                    or 256) where a lane integrates one pixel column on its
+//                    own; workgroups of columns split over waves have their
+//                    size from the split, and 256 is noted for them
 //   TUNE_TILE_ORDER  order of the FAST voxel kernel's tiles over the
 //                    workgroups (0: contiguous ranges per XCD, 1: linear, 2:
 //                    rows dealt to the XCDs in turn): a wave sums one tile on

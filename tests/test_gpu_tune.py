@@ -193,3 +193,34 @@ def test_batches_in_turn_on_cached_branch_counts(tmp_path, three, two):
     got = turns()
     assert len(got) == 12
     assert all(nb == {3: three, 2: two}[n] for n, nb in got)
+
+
+_APERTURE = r"""
+import sys
+sys.path.insert(0, sys.argv[1])
+from simulated_tem_amd import synth
+cfg = synth.scaled("c0", cells=(10, 10, 10))
+cfg.update(sg=[0.01])
+x, box = synth.make_atoms(cfg)
+x, conds = synth.conditions(cfg, x, box)
+im = conds[0][0]
+for n in (2, 5):        # four fields in a launch; a launch per field
+    im.computeD2BI_img(x, 0.005, n, apertureAngle=0.002, nAperturePoints=8)
+im.computeD2BI_img(x, 0.005, 7, mode="fast")
+"""
+
+
+def test_split_columns_are_not_timed(tmp_path):
+    """Workgroups of columns split over waves have one size: an aperture sum of
+    several fields per launch leaves no choice behind for a plain image of its
+    shape, and the plain image of split columns notes the default."""
+    cache = tmp_path / "tune.txt"
+    env = {k: v for k, v in os.environ.items() if k not in TUNE_VARS}
+    env["D2BI_TUNE_CACHE"] = str(cache)
+    r = subprocess.run([sys.executable, "-c", _APERTURE, ROOT], env=env, cwd=ROOT, capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    blocks = [ln for ln in _cache_lines(cache) if ln[0] == 1]
+    print("\n[split] %s" % blocks, flush=True)
+    assert [ln[4] for ln in blocks] == [5, 7]
+    assert all(ln[9] == 256 for ln in blocks)
