@@ -342,15 +342,25 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
             (void)hipGetLastError();
             freeb = 0;
         }
-        const double room = 0.85 * (double)freeb;
-        double used = branch_growth(B.branch_ws(0), bz);
-        int fit = 1;
-        for (int k = 1; k < nbr; k++) {
-            used += branch_growth(B.branch_ws(k), bz);
-            if (used > room) break;
-            fit = k + 1;
+        auto fitting = [&] {
+            double used = branch_growth(B.branch_ws(0), bz);
+            int fit = 1;
+            for (int k = 1; k < want; k++) {
+                used += branch_growth(B.branch_ws(k), bz);
+                if (used > 0.85 * (double)freeb) break;
+                fit = k + 1;
+            }
+            return fit;
+        };
+        nbr = fitting();
+        if (nbr < want) {
+            // what earlier batches left in the branches that do not fit
+            for (int k = nbr; k < MAX_BRANCH; k++) {
+                freeb += B.branch_ws(k).bytes();
+                B.branch_ws(k).release_all();
+            }
+            nbr = fitting();
         }
-        nbr = fit;
     }
     // branch count: forced, cached, or tuned below by timing a run on each
     // count (images are the same on any count); the count that fits is kept
@@ -417,7 +427,8 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
     }
     HIPCHK(hipStreamSynchronize(s));
     // workspaces of branches that timing has just left unused, or that are
-    // unused where device memory is short, go back to the device
+    // unused where device memory is short, go back to the device (the others
+    // already have)
     if (tune || nbr < want)
         for (int k = std::max(1, chosen); k < nbr; k++) B.branch_ws(k).release_all();
     B.nbr = chosen;

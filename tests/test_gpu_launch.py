@@ -7,6 +7,7 @@ count.  A batch is launched as it is the first time and captured into a graph
 the second: every call gives the same images, and so do batches that take
 turns (each is new again after the other).
 """
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -183,3 +184,47 @@ def test_no_room_for_the_estimate():
                        timeout=100)
     print(r.stdout, flush=True)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_short_memory_takes_back_idle_branches(monkeypatch):
+    """Where memory is too short for every branch, the workspaces that earlier
+    batches left in the others go back to the device, and their room counts."""
+    monkeypatch.setenv("D2BI_TUNE", "0")                # every branch that fits runs
+    hip = imaging._hip_runtime()
+
+    def batch(n, points, mem):
+        cfg = synth.scaled("c0", cells=(n, n, n))
+        cfg.update(sg=[0.01])
+        x, box = synth.make_atoms(cfg)
+        x, conds = synth.conditions(cfg, x, box)
+        monkeypatch.setenv("D2BI_BATCH_MEM", str(int(mem)))
+        at, st = imaging.Atoms(x), abi.D2biStats()
+        out = imaging.computeD2BI_img_batch([(conds[0][0], at, 0.005, points + i) for i in range(4)], stats=st)
+        del at
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        print("[branches] %d^3 cells, %.2e bytes free: %d branches of %.2e" % (n, mem, st.n_branches, st.branch_bytes), flush=True)
+        return out, st.n_branches, st.branch_bytes, free.value
+
+    try:
+        imaging.finalize()
+        large, nb, W2, _ = batch(38, 1, 1e15)
+        imaging.finalize()
+        _, nb, W, before = batch(30, 1, 1e15)
+        assert nb == 4 and 1.8 * W < W2 < 2.2 * W
+        # no room but that of three workspaces, which are given back: enough for
+        # branch 0 to grow and for one more of 1.2 W
+        small, nb, _, after = batch(30, 2, 0)
+        assert nb == 4                                  # nothing to add: the four are kept
+        got, nb, _, after = batch(32, 1, 0)
+        assert nb == 2 and after - before > 1.4 * W
+        # room for one larger workspace and the growth of another, and with
+        # what the others give back for a second
+        batch(30, 3, 1e15)
+        got, nb, _, _ = batch(38, 1, 1.5 * W / 0.85)
+        assert nb == 2
+        for a, b in zip(got, large):
+            assert np.array_equal(a, b)
+    finally:
+        monkeypatch.delenv("D2BI_BATCH_MEM", raising=False)
+        imaging.finalize()
