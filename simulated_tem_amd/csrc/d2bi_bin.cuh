@@ -230,29 +230,32 @@ __global__ __launch_bounds__(BIN_BLOCK) void k_bin_scatter(const double* __restr
 }
 
 // f(t) for the items t of a thread among n, workgroups of 256 in a grid of
-// xcd_grid() (of n items or fewer; a thread goes on a grid's stride from its
-// first): a contiguous range of items per XCD (workgroups go round-robin to the
+// xcd_grid(n) or more, or (LOOP) fewer, where a thread goes on at the grid's
+// stride: a contiguous range of items per XCD (workgroups go round-robin to the
 // eight), so that neighbours in cell or atom order, which share lines of the
 // arrays they gather from and scatter into, share one L2.  Against
 // workgroups in order: k_bin_emit 39.5 -> 26.7 us and k_bin_place 9.6 -> 6.8 at
-// 1.2e6 atoms, 222 -> 211 and 54 -> 44 at 8e6 (k_bin_scatter, whose atomics
+// 1.2e6 atoms, 222 -> 212 and 54 -> 46 at 8e6 (k_bin_scatter, whose atomics
 // meet in memory either way, lost 7 % there and keeps its order).
-template <class F>
+template <bool LOOP, class F>
 __device__ __forceinline__ void xcd_items(int64_t n, F f)
 {
     const int64_t per = (n + 2047) / 2048;
-    for (int64_t b = blockIdx.x >> 3; b < per; b += gridDim.x >> 3) {
+    int64_t b = blockIdx.x >> 3;
+    do {
         const int64_t t = ((blockIdx.x & 7) * per + b) * 256 + threadIdx.x;
-        if (t < n) f(t);
-    }
+        if (b < per && t < n) f(t);
+        b += gridDim.x >> 3;
+    } while (LOOP && b < per);
 }
 static unsigned xcd_grid(int64_t n) { return (unsigned)(8 * ((n + 2047) / 2048)); }
 
 // Pass 3: place each point at its cell's start + arrival slot.
+template <bool LOOP>
 __global__ void k_bin_place(PointCount N, const int* __restrict__ pt_cell, const int* __restrict__ pt_slot,
                             const int* __restrict__ cell_start, int* __restrict__ cell_ids)
 {
-    xcd_items(N.stored(), [&](int64_t ii) { cell_ids[cell_start[pt_cell[ii]] + pt_slot[ii]] = (int)ii; });
+    xcd_items<LOOP>(N.stored(), [&](int64_t ii) { cell_ids[cell_start[pt_cell[ii]] + pt_slot[ii]] = (int)ii; });
 }
 
 // What pass 4 writes per slot (null: not wanted).
@@ -276,7 +279,7 @@ struct EmitOut {
 // ii is the last one whose first point number is <= ii (numbers run in
 // (replica, atom) order; rep_first is padded to 32 entries with INT_MAX).
 // Bound: HBM and, in imaging, FP64 sincos with full argument reduction.
-template <bool FAST>
+template <bool FAST, bool LOOP>
 __global__ __launch_bounds__(256) void k_bin_emit(PointCount N, const int* __restrict__ cell_ids,
                                                   const int* __restrict__ pt_cell, const int* __restrict__ pt_j,
                                                   const int* __restrict__ cell_start, const double* __restrict__ x,
@@ -286,7 +289,7 @@ __global__ __launch_bounds__(256) void k_bin_emit(PointCount N, const int* __res
     if (threadIdx.x < MAX_REPL)
         rep_first[threadIdx.x] = threadIdx.x < P.nuvw ? blk_off[(int64_t)threadIdx.x * nblk] : 0x7fffffff;
     __syncthreads();
-    xcd_items(N.stored(), [&](int64_t t) {
+    xcd_items<LOOP>(N.stored(), [&](int64_t t) {
         const int ii = cell_ids[t];
         const int64_t j = pt_j[ii];
         const int c = pt_cell[ii];
@@ -340,7 +343,7 @@ __global__ __launch_bounds__(256) void k_app_phase(int64_t nr, const int2* __res
                                                    double2* __restrict__ out64, float2* __restrict__ out32,
                                                    float4* __restrict__ slot_p32, float* __restrict__ slot_sn32)
 {
-    xcd_items(nr, [&](int64_t s) {
+    xcd_items<false>(nr, [&](int64_t s) {
         const int2 src = slot_src[s];
         const int64_t j = src.x;
         const double x3[3] = {x[3 * j], x[3 * j + 1], x[3 * j + 2]};
@@ -384,9 +387,17 @@ static int launch_bin_points(const double* d_x, const BinParams& P, const uint32
     CHK(scan_exclusive_tmp(w.cell_cnt.as<int>(), w.cell_start.as<int>(), ncell, scan_tmp, s,
                            ScanEnds{nullptr, mpc, N}));
     if (P.n > 0 && N.cap > 0) {
-        const dim3 grid(xcd_grid(std::min(N.cap, expect)));
-        hipLaunchKernelGGL(k_bin_place, grid, dim3(256), 0, s, N, w.pt_cell.as<int>(), w.pt_slot.as<int>(),
-                           w.cell_start.as<int>(), w.cell_ids.as<int>());
+        // a thread per point that the arrays hold, or, where an earlier condition
+        // left them far larger, per point expected (k_bin_emit's loop costs it a
+        // wave per SIMD: 213 -> 220 us at 8e6 points)
+        const bool loop = N.cap > 2 * expect;
+        const dim3 grid(xcd_grid(loop ? expect : N.cap));
+        auto place = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, N, w.pt_cell.as<int>(), w.pt_slot.as<int>(),
+                               w.cell_start.as<int>(), w.cell_ids.as<int>());
+        };
+        if (loop) place(k_bin_place<true>);
+        else place(k_bin_place<false>);
         EmitOut O{w.slot_p32.as<float4>(), w.slot_sn32.as<float>(), nullptr, w.slot_frac.as<Frac3>(),
                   P.keep_src ? w.slot_src.as<int2>() : nullptr, nullptr, nullptr};
         if (!P.fast) {
@@ -402,8 +413,10 @@ static int launch_bin_points(const double* d_x, const BinParams& P, const uint32
             hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, N, w.cell_ids.as<int>(), w.pt_cell.as<int>(),
                                w.pt_j.as<int>(), w.cell_start.as<int>(), d_x, P, blk_off, nblk, O);
         };
-        if (P.fast) go(k_bin_emit<true>);
-        else go(k_bin_emit<false>);
+        if (loop && P.fast) go(k_bin_emit<true, true>);
+        else if (loop) go(k_bin_emit<false, true>);
+        else if (P.fast) go(k_bin_emit<true, false>);
+        else go(k_bin_emit<false, false>);
     }
     HIPCHK(hipGetLastError());
     return D2BI_OK;
