@@ -186,9 +186,9 @@ def batch_main(args, imaging, synth, np):
     dev = imaging.DeviceBuffer((imaging.batch_image_size(batch),))
     st = imaging.D2biStats()
     t0 = time.perf_counter()
-    imaging.computeD2BI_img_batch(batch, mode="fast", out=dev, stats=st)    # plans, counts, captures
+    imaging.computeD2BI_img_batch(batch, mode="fast", out=dev, stats=st)    # plans, counts, tunes
     first = time.perf_counter() - t0
-    log("[bench] first call (plan, count, capture, run) %.3f s, %d branches" % (first, st.n_branches))
+    log("[bench] first call (plan, count, tune, run) %.3f s, %d branches" % (first, st.n_branches))
     for _ in range(args.warmup):
         imaging.computeD2BI_img_batch(batch, mode="fast", out=dev)
     log("[bench] warmup done")

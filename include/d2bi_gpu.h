@@ -43,8 +43,9 @@ enum {
 };
 
 enum {
-    D2BI_MODE_FP64 = 0,         /* reference arithmetic in FP64: membership bit-exact, 1e-10 */
-    D2BI_MODE_FAST = 1          /* FP32 bulk, FP64 phase + FP64 guard-band membership        */
+    D2BI_MODE_FP64 = 0,         /* FP64: membership and ranges bit-exact, images to 1e-10    */
+    D2BI_MODE_FAST = 1          /* FP32 bulk, FP64 phase + FP64 guard-band membership; voxels
+                                   taller than about 5 sigma are imaged in FP64              */
 };
 
 /*

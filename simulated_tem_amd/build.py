@@ -5,8 +5,9 @@
 The library holds the HIP kernels, the C-ABI and the host setup code.
 Flags:
   --offload-arch=gfx950            MI355X only
-  -ffp-contract=off                FP64 kernels keep the reference's unfused
-                                   operation order; FAST kernels write fmaf
+  -ffp-contract=off                ranges and members keep the reference's
+                                   unfused operations; kernels that may fuse
+                                   write fmaf or fma
   -Xclang -target-feature -Xclang -packed-fp32-ops
                                    no packed FP32 (v_pk_*_f32) instructions
 """

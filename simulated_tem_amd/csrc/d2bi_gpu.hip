@@ -9,13 +9,15 @@
 //                    27 neighbour cells, rho from the nearest range
 //   (c) integrate    RK4 Howie-Whelan march down each pixel column
 //   (d) blur         separable Gaussian on the output image
-// FP64 mode reproduces the reference arithmetic (un-fused, same order).
-// FAST mode runs (b) and (c) in FP32 with FP64 phases and an FP64 re-test
+// FP64 mode evaluates positions, ranges, members and nearest ranges with the
+// reference's expressions (un-fused, same order, so to the bit); the weighted
+// sums and the march are FP64 in an order of their own, with fused
+// multiply-adds.  FAST mode runs (b) and (c) in FP32 with FP64 phases and an FP64 re-test
 // of every candidate whose FP32 range lies in a guard band around 3 sigma,
 // so voxel membership stays identical to FP64.
 //
 // The unit is compiled with -ffp-contract=off: every fused multiply-add in it
-// is written explicitly (fmaf) and only appears in FAST-mode FP32 code.
+// is written explicitly (fmaf, fma).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

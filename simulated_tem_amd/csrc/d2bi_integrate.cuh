@@ -501,7 +501,8 @@ constexpr int int_threads64(int np) { return np <= 3 ? 1024 : np <= 8 ? 512 : 25
 // matrix: 5 points as 4 + 1 passes take 0.30 ms at 400 x 360 columns of 200
 // samples, 6 through the matrix 0.31); a column's points split over P.nsplit
 // waves as k_integrate_fast's are; renormalised once at the
-// end, as the FAST march is.  Bound: FP64 VALU from two points on, HBM below
+// end, as the FAST march is, and (RS) rescaled by powers of two on the way where
+// the amplitudes might leave FP64's range.  Bound: FP64 VALU from two points on, HBM below
 // (1 point 0.079 ms, 5.8 TB/s).  A march per point with the reference's
 // divisions and a square root per step took 0.26 ms for 1 point, 2.00 for 8
 // and 8.7 for 32; this takes 0.079, 0.35 and 1.21.

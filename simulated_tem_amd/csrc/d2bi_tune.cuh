@@ -23,9 +23,9 @@
 // appended to that file and read back by later processes.  D2BI_TUNE=0 turns
 // tuning off (the defaults: 256 threads, rows dealt to the XCDs, four
 // branches where they fit); D2BI_INT_BLOCK, D2BI_TILE_ORDER and D2BI_BATCH_BRANCHES force a
-// choice.  Nothing is timed while a graph is being captured, or on a
-// workspace that must not allocate: those launches use cached or default
-// choices.
+// choice.  Nothing is timed while a graph is being captured: those launches
+// use cached or default choices.  Timing a pass that adds to an image takes a
+// buffer of its own, so a workspace that must not allocate does without.
 #pragma once
 
 namespace d2bi {
