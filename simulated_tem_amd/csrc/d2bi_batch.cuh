@@ -263,7 +263,8 @@ static int first_run(Batch& B, const d2bi_record* recs, const d2bi_atoms* atoms,
         CHK(plan_image(&recs[i], atoms[i]->n, precAngle[i], nPrec[i], &c.plan));
         CHK(axis_tables(&recs[i], &c.plan, &c.tab));
         CHK(bin_params(&recs[i], &c.plan, &c.BP));
-        c.mode = condition_mode(&c.plan, mode);
+        c.mode = mode;
+        CHK(condition_mode(&c.plan, c.tab, &c.mode));
         c.BP.fast = c.mode == D2BI_MODE_FAST ? 1 : 0;
         c.d_x = atoms[i]->x;
         c.n = atoms[i]->n;

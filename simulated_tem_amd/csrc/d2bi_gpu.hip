@@ -204,10 +204,9 @@ int d2bi_gpu_image_noalloc(const d2bi_record* rec, d2bi_atoms atoms, double prec
     // the rest (point arrays) when the point count is known
     d2bi_plan plan;
     CHK(plan_image(rec, atoms->n, precAngle, nPrec, &plan));
-    mode = condition_mode(&plan, mode);
     const double nvox = (double)plan.Mx * plan.My * plan.Mz;
     const double ncell = (double)plan.Ex * plan.Ey * plan.Ez;
-    const double need = nvox * (mode == D2BI_MODE_FP64 ? 24.0 : 16.0) + 8.0 * (ncell + 1) +
+    const double need = nvox * (mode == D2BI_MODE_FP64 || !fast_fits(&plan) ? 24.0 : 16.0) + 8.0 * (ncell + 1) +
                         4.0 * (double)atoms->n;
     if (need > (double)D2BI_SCRATCH_BYTES)
         return seterr(D2BI_ERR_CAPACITY,
@@ -301,9 +300,9 @@ int d2bi_gpu_field(const d2bi_record* rec, const double* x, int64_t ld, int64_t 
     CHK(upload_atoms_tmp(x, ld, nAtoms, &d_x));
     d2bi_plan plan;
     CHK(plan_image(rec, nAtoms, 0.0, 1, &plan));
-    mode = condition_mode(&plan, mode);
     AxisTables tab;
     CHK(axis_tables(rec, &plan, &tab));
+    CHK(condition_mode(&plan, tab, &mode));
     BinParams BP;
     CHK(bin_params(rec, &plan, &BP));
     BP.fast = mode == D2BI_MODE_FAST ? 1 : 0;

@@ -88,13 +88,14 @@ static double tile_bits(const d2bi_plan* p, int tz, int ty, bool x)
 // 85 leave u within half the guard band.  A 4 x 8 x 8 tile has 22 at four cubic
 // voxels per lattice parameter and 46 at two; 4 x 4 x 8 has 81 at one; voxels of
 // 1.4 x 1.4 x 2.7 sigma have 134 in a 4 x 8 x 8 tile (NaN) and 41 in 4 x 4 x 4.
-static constexpr double TILE_BITS = 85.0;
+// The kernel of a lane per voxel has no such factors, but its exponent is a
+// difference of the range from the tile's centre in x too: 130 keep its
+// roundings within the guard band.
+static constexpr double TILE_BITS = 85.0, VOXEL_BITS = 130.0;
 
-// The arithmetic that images a condition in `mode`: FP64 where a voxel is so
-// tall (about 5 sigma) that even the smallest FAST tile has more.
-static int condition_mode(const d2bi_plan* p, int mode)
+static bool fast_fits(const d2bi_plan* p)
 {
-    return mode == D2BI_MODE_FAST && !(tile_bits(p, TILE, TILE, true) <= TILE_BITS) ? D2BI_MODE_FP64 : mode;
+    return tile_bits(p, TILE, TILE, false) <= TILE_BITS && tile_bits(p, TILE, TILE, true) <= VOXEL_BITS;
 }
 
 // Launch parameters of the FAST voxel kernel for a plan, tiles of 4 x ty x tz.
@@ -132,6 +133,18 @@ static int fast_params(const d2bi_plan* p, const AxisTables& tab, const VoxParam
     // the unwrapped cell range of a tile must fit the per-tile cell table
     const int worst = tile_cells(p, tab, tz, ty);
     if (worst > TILE_MAXC) return seterr(D2BI_ERR_CAPACITY, "voxel tile spans %d link cells (max %d)", worst, TILE_MAXC);
+    return D2BI_OK;
+}
+
+// The arithmetic that images a condition in *mode: FP64 where a voxel is so
+// tall (about 5 sigma) that even the smallest FAST tile has too many bits.  What
+// the FAST kernels refuse is refused there too.
+static int condition_mode(const d2bi_plan* p, const AxisTables& tab, int* mode)
+{
+    if (*mode != D2BI_MODE_FAST || fast_fits(p)) return D2BI_OK;
+    FastParams F;
+    CHK(fast_params(p, tab, VoxParams{}, &F, TILE));
+    *mode = D2BI_MODE_FP64;
     return D2BI_OK;
 }
 
@@ -730,9 +743,9 @@ static int image_condition(const d2bi_record* r, const double* d_x, int64_t n, d
     if (mode != D2BI_MODE_FP64 && mode != D2BI_MODE_FAST) return seterr(D2BI_ERR_ARG, "unknown mode %d", mode);
     d2bi_plan plan;
     CHK(plan_image(r, n, precAngle, nPrec, &plan));
-    mode = condition_mode(&plan, mode);
     AxisTables tab;
     CHK(axis_tables(r, &plan, &tab));
+    CHK(condition_mode(&plan, tab, &mode));
     BinParams BP;
     CHK(bin_params(r, &plan, &BP));
     const bool dens = r->use_density != 0;
@@ -900,11 +913,11 @@ static int image_aperture(const d2bi_record* r, const double* d_x, int64_t n, do
     if (mode != D2BI_MODE_FP64 && mode != D2BI_MODE_FAST) return seterr(D2BI_ERR_ARG, "unknown mode %d", mode);
     d2bi_plan plan;
     CHK(plan_image(r, n, precAngle, nPrec, &plan));
-    mode = condition_mode(&plan, mode);
     std::vector<double> gshift(3 * (size_t)nApp), aa((size_t)nApp * nPrec);
     CHK(aperture_setup(r, precAngle, nPrec, apAngle, nApp, gshift.data(), aa.data()));
     AxisTables tab;
     CHK(axis_tables(r, &plan, &tab));
+    CHK(condition_mode(&plan, tab, &mode));
     hipStream_t s = g.stream;
     Workspace& w = g.ws;
     AxisDev ax;

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as orc
-from simulated_tem_amd import imaging, synth
+from simulated_tem_amd import abi, imaging, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -22,7 +22,7 @@ SIGMA = A0 / 2
 
 # voxel sides in sigma
 SIDES = [(0.5, 0.5, 2.87), (1.4, 1.4, 2.7), (1.0, 1.0, 2.8), (0.5, 0.5, 4.0), (0.5, 0.5, 8.0), (0.5, 0.5, 30.0),
-         (0.5, 2.9, 2.9), (0.5, 9.0, 0.5)]
+         (0.5, 2.9, 2.9), (0.5, 9.0, 0.5), (7.0, 1.0, 1.0), (9.0, 0.5, 0.5)]
 
 
 def boxes(sides, n=(18, 17, 19), density=False):
@@ -81,3 +81,18 @@ def test_voxel_sides_batch():
     for _ in range(3):
         for got, want in zip(imaging.computeD2BI_img_batch(todo, mode="fast"), alone):
             assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("side", [3.5, 5.0])
+def test_coarse_cubes_stay_refused(side):
+    """Cubes beyond 3 sigma have a link cell each, more to a tile than its table
+    holds: FAST says so, also where their weights would not fit its tiles; FP64
+    images them."""
+    x, im = boxes((side, side, side), n=(9, 9, 9))
+    at = imaging.Atoms(x)
+    for call in (lambda: im.computeD2BI_img(x, mode="fast"), lambda: im.field(x, "fast"),
+                 lambda: im.computeD2BI_img(x, 0.005, 2, apertureAngle=0.002, nAperturePoints=2),
+                 lambda: imaging.computeD2BI_img_batch([(im, at, 0.0, 1)] * 2, mode="fast")):
+        with pytest.raises(abi.D2biError, match="spans 2[0-9][0-9] link cells"):
+            call()
+    assert np.max(np.abs(im.computeD2BI_img(x, mode="fp64") - orc.compute_img(im.rec, x, nthreads=NTH))) <= 1e-10
